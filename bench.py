@@ -312,6 +312,14 @@ def run_encoder(args, name, hidden, heads, ffn, layers, dtype, seq_lens, max_pos
         bias = torch.zeros(ffn, dtype=dt, device="cuda")
         per["add_bias_act_kernel"] = time_kernel(lambda: pkg.capi.bias_gelu(inter, bias), 20, 3)
         gelu_note = "stand-alone launches on the step's [tokens, ffn] buffer (the steps fuse it into the GEMM)"
+    split_note = "launches inside the timed steps"
+    if "add_bias_and_transpose_kernel" not in per:
+        # the projection writes K and V^T itself: the stand-alone split kernel is timed on a projection output of this size
+        qkv, k, vt = new(3 * hidden), new(hidden), new(hidden)
+        qkv.normal_()
+        per["add_bias_and_transpose_kernel"] = time_kernel(
+            lambda: pkg.capi.qkv_bias_split(qkv, None, None, k, vt, spi_t, heads, pkg.capi.Q_SCALE), 20, 3)
+        split_note = "stand-alone launches on a projection output of the step's size (the steps fuse it into the projection)"
     pairs = block_pairs(spi, heads)
     att_us = per["attention"]
     att_flops = pairs * PAIR_FLOP
@@ -339,10 +347,10 @@ def run_encoder(args, name, hidden, heads, ffn, layers, dtype, seq_lens, max_pos
         "roofline_gelu": dict(hbm_roofline("bias_gelu_kernel", 2 * t * ffn * sz, per["add_bias_act_kernel"],
                                            traffic.get("bias_gelu_kernel")), measured=gelu_note),
         # K and V only (read + write) unless Q is materialised too
-        "roofline_qkv_split": hbm_roofline("qkv_bias_split_kernel", 2 * t * (3 if args.materialize_q else 2) * hidden * sz,
-                                           per["add_bias_and_transpose_kernel"],
-                                           traffic.get("qkv_bias_split_kernel_q" if args.materialize_q
-                                                       else "qkv_bias_split_kernel")),
+        "roofline_qkv_split": dict(hbm_roofline("qkv_bias_split_kernel", 2 * t * (3 if args.materialize_q else 2) * hidden * sz,
+                                                per["add_bias_and_transpose_kernel"],
+                                                traffic.get("qkv_bias_split_kernel_q" if args.materialize_q
+                                                            else "qkv_bias_split_kernel")), measured=split_note),
         "two_streams": two_streams,
         "kernel_us_per_launch": per,
         "kernel_us_per_step": {k: v[0] / args.steps for k, v in timing_all.items()},

@@ -155,6 +155,15 @@ int rt_qkv_bias_split(const void* qkv, const void* bias, void* q, void* k, void*
                       const int* seq_blocks_dev, int batch, int total_blocks, int heads,
                       float q_scale, int dtype, void* stream);
 
+/* The QKV projection and its head split as one kernel: x[T, k] . wt[3*H*64, k]^T + bias, the Q columns written to
+ * rows[T, 3*H*64] (its other columns are not touched), K and V straight to the packed tiles of rt_qkv_bias_split.
+ * The rows and tiles have the values of rt_gemm_bt (RT_EPILOGUE_BIAS) followed by rt_qkv_bias_split with
+ * q = NULL, bias = NULL; rows then goes to rt_bs_attention_fwd_qrows with a NULL bias.  fp16 / bf16, k a multiple
+ * of 64 and at least 128, 16-byte aligned pointers; RT_ENOSYS for what it does not take (use the pair then). */
+int rt_qkv_project(const void* x, const void* wt, const void* bias, void* rows, void* k_tiles, void* vt,
+                   const int* seq_blocks_dev, int batch, int total_blocks, int heads, int64_t k, int dtype,
+                   void* stream);
+
 /* Inverse of the packed layout: packed tiles -> dst[T, H*64] token-major; transposed = 0
  * for q / k, 1 for vt. */
 int rt_unpack_head_tiles(const void* packed, void* dst, const int* seq_blocks_dev, int batch,

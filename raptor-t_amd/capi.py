@@ -22,7 +22,7 @@ RT_GEMM_TUNE_ALL = -1
 EXPORTS = [
     "rt_last_error_string", "rt_abi_version", "rt_time_next_launch", "rt_meta_np_permutations", "rt_meta_seq_prefix_blocks",
     "rt_meta_rand_attn", "rt_meta_set_plan_cache", "rt_meta_to_index_size", "rt_meta_build_to_index", "rt_meta_block_costs",
-    "rt_meta_partition_lpt", "rt_meta_check_partition", "rt_meta_check_to_index", "rt_qkv_bias_split", "rt_unpack_head_tiles", "rt_bs_attention_fwd",
+    "rt_meta_partition_lpt", "rt_meta_check_partition", "rt_meta_check_to_index", "rt_qkv_bias_split", "rt_qkv_project", "rt_unpack_head_tiles", "rt_bs_attention_fwd",
     "rt_bs_attention_fwd_masked", "rt_bs_attention_fwd_qrows", "rt_bs_attention_fwd_no_alloc",
     "rt_bias_residual_layernorm", "rt_bias_gelu", "rt_embed_layernorm", "rt_gemm_create", "rt_gemm_destroy", "rt_gemm_set_tuning", "rt_gemm_set_retuning", "rt_gemm",
     "rt_gemm_bias_act", "rt_gemm_bt", "rt_sequence_pool", "rt_pooler_dense_tanh",
@@ -62,6 +62,7 @@ def lib():
         L.rt_meta_check_partition.argtypes = [i32p, i32p, I, I, I]
         L.rt_meta_check_to_index.argtypes = [i32p, i32p, L64, i32p, I, I]
         L.rt_qkv_bias_split.argtypes = [vp, vp, vp, vp, vp, vp, I, I, I, F, I, vp]
+        L.rt_qkv_project.argtypes = [vp, vp, vp, vp, vp, vp, vp, I, I, I, L64, I, vp]
         L.rt_unpack_head_tiles.argtypes = [vp, vp, vp, I, I, I, I, I, vp]
         L.rt_bs_attention_fwd.argtypes = [vp, vp, vp, vp, vp, I, I, I, vp, vp, I, vp, vp, I, I, vp]
         L.rt_bs_attention_fwd_masked.argtypes = [vp, vp, vp, vp, vp, vp, I, I, I, vp, vp, I, vp, vp, I, I, vp]
@@ -249,6 +250,18 @@ def qkv_bias_split(qkv, bias, q, k, vt, seq_blocks_dev, heads, q_scale):
     check(lib().rt_qkv_bias_split(_dp(qkv, name="qkv"), _dp(bias, dt, 3 * heads * 64, "bias"), _dp(q, dt, per, "q"),
                                   _dp(k, dt, per, "k"), _dp(vt, dt, per, "vt"), _ip(seq_blocks_dev, name="seq_blocks_dev"),
                                   batch, nb, heads, q_scale, _dtype_code(qkv), _stream()))
+
+
+def qkv_project(x, wt, bias, rows, k, vt, seq_blocks_dev, heads):
+    """x @ wt.T + bias with the head split: Q to rows[:, :heads * 64], K and V to the packed tiles."""
+    batch = seq_blocks_dev.numel() - 1
+    dt, width = x.dtype, 3 * heads * 64
+    if x.dim() != 2 or x.shape[0] % 64 or tuple(wt.shape) != (width, x.shape[1]) or tuple(rows.shape) != (x.shape[0], width):
+        raise ValueError("x must be [tokens (a multiple of 64), k], wt [3 * heads * 64, k] and rows [tokens, 3 * heads * 64]")
+    nb, per = x.shape[0] // 64, x.shape[0] * heads * 64
+    check(lib().rt_qkv_project(_dp(x, name="x"), _dp(wt, dt, name="wt"), _dp(bias, dt, width, "bias"), _dp(rows, dt, name="rows"),
+                               _dp(k, dt, per, "k"), _dp(vt, dt, per, "vt"), _ip(seq_blocks_dev, name="seq_blocks_dev"),
+                               batch, nb, heads, x.shape[1], _dtype_code(x), _stream()))
 
 
 def unpack_head_tiles(packed, dst, seq_blocks_dev, heads, transposed):

@@ -1,5 +1,6 @@
-// Dense GEMM of the layer through hipBLASLt: row-major C[M,N] = A[M,K] . B[K,N], inputs and
-// output in fp16 / bf16 / fp32, accumulation in fp32.
+// Dense GEMM of the layer: row-major C[M,N] = A[M,K] . B[K,N], inputs and output in fp16 / bf16 / fp32, accumulation
+// in fp32.  B[N,K]^T in a 16-bit type, which is what the layers run, goes to the kernels of gemm_mfma.hip; the
+// rest (fp32, B[K,N], shapes those kernels do not take) to hipBLASLt.
 //
 // Replaces kernels::MatMul (layers/kernels/mat_mul.cpp:9-96), which calls cublasGemmEx
 // with the operands swapped to express a row-major product in a column-major library and
@@ -12,8 +13,9 @@
 // the output.
 //
 // rt_gemm_bt takes B as Bt[N,K] (each output column's K weights contiguous), the b_trans = true
-// case of kernels::MatMul: with both operands K-contiguous the library's kernels for these shapes
-// run 8-20 % faster than with B[K,N], so a layer that owns its weights keeps them this way.
+// case of kernels::MatMul: with both operands K-contiguous a row of either is a run of memory that goes
+// to LDS as it is (and the library's kernels are 8-20 % faster than with B[K,N]), so a layer that owns its
+// weights keeps them this way.
 #include <hip/hip_runtime.h>
 #include <hipblaslt/hipblaslt.h>
 #include <hipblaslt/hipblaslt-ext.hpp>
@@ -24,6 +26,7 @@
 #include <mutex>
 #include <tuple>
 
+#include "gemm_mfma.h"
 #include "rt_common.h"
 
 struct rt_gemm_ctx {
@@ -207,6 +210,20 @@ int make_plan(rt_gemm_ctx* ctx, int64_t m, int64_t n, int64_t k, int dtype, int 
   return RT_OK;
 }
 
+// The library's handle and workspace, made when the first product needs them: a process whose products all run on the
+// kernels of gemm_mfma.hip never loads the library's solutions.  Caller holds ctx->m.
+int ensure_library(rt_gemm_ctx* ctx) {
+  if (!ctx->lt) LT_TRY(hipblasLtCreate(&ctx->lt));
+  if (!ctx->workspace) {
+    ctx->workspace_bytes = size_t(64) << 20;
+    if (hipMalloc(&ctx->workspace, ctx->workspace_bytes) != hipSuccess) {
+      ctx->workspace = nullptr;
+      return rt::fail(RT_ENOMEM, "could not allocate the 64 MiB GEMM workspace");
+    }
+  }
+  return RT_OK;
+}
+
 void free_plan(rt_gemm_ctx::Plan& p) {
   if (p.la) hipblasLtMatrixLayoutDestroy(p.la);
   if (p.lb) hipblasLtMatrixLayoutDestroy(p.lb);
@@ -223,14 +240,6 @@ int rt_gemm_create(rt_gemm_ctx** out) {
   RT_REQUIRE(out, RT_EINVAL, "NULL output");
   rt_gemm_ctx* ctx = new rt_gemm_ctx();
   if (hipGetDevice(&ctx->device) != hipSuccess) { delete ctx; return rt::fail(RT_EIO, "hipGetDevice failed: no usable GPU"); }
-  hipblasStatus_t s = hipblasLtCreate(&ctx->lt);
-  if (s != HIPBLAS_STATUS_SUCCESS) { delete ctx; return rt::fail(RT_EIO, "hipblasLtCreate failed with status %d", int(s)); }
-  ctx->workspace_bytes = size_t(64) << 20;
-  if (hipMalloc(&ctx->workspace, ctx->workspace_bytes) != hipSuccess) {
-    hipblasLtDestroy(ctx->lt);
-    delete ctx;
-    return rt::fail(RT_ENOMEM, "could not allocate the 64 MiB GEMM workspace");
-  }
   *out = ctx;
   return RT_OK;
 }
@@ -274,12 +283,14 @@ int run_gemm(rt_gemm_ctx* ctx, const void* a, const void* b, const void* bias, v
   const float alpha = 1.0f, beta = 0.0f;
   // the plan's descriptor carries the bias pointer: set and used under the lock
   std::lock_guard<std::mutex> lk(ctx->m);
+  int rc = ensure_library(ctx);
+  if (rc) return rc;
   const int mode = epilogue | (b_trans ? MODE_B_TRANS : 0);
   auto key = std::make_tuple(m, n, k, dtype, mode);
   auto it = ctx->plans.find(key);
   if (it == ctx->plans.end()) {
     rt_gemm_ctx::Plan p;
-    int rc = make_plan(ctx, m, n, k, dtype, mode, bias, p, a, b, c, static_cast<hipStream_t>(stream));
+    rc = make_plan(ctx, m, n, k, dtype, mode, bias, p, a, b, c, static_cast<hipStream_t>(stream));
     if (rc) { free_plan(p); return rc; }
     it = ctx->plans.emplace(key, p).first;
   }
@@ -307,11 +318,26 @@ int rt_gemm_bias_act(rt_gemm_ctx* ctx, const void* a, const void* b, const void*
   return run_gemm(ctx, a, b, bias, c, m, n, k, epilogue, false, dtype, stream);
 }
 
+int rt_qkv_project(const void* x, const void* wt, const void* bias, void* rows, void* k_tiles, void* vt,
+                   const int* seq_blocks_dev, int batch, int total_blocks, int heads, int64_t k, int dtype, void* stream) {
+  RT_REQUIRE(x && wt && rows && k_tiles && vt && seq_blocks_dev, RT_EINVAL, "NULL pointer");       // bias may be NULL
+  RT_REQUIRE(batch >= 1 && total_blocks >= batch && heads >= 1 && k >= 1, RT_EINVAL,
+             "bad geometry: batch=%d total_blocks=%d heads=%d k=%lld", batch, total_blocks, heads, (long long)k);
+  const int64_t m = int64_t(total_blocks) * RT_BLOCK, n = int64_t(heads) * 3 * RT_HEAD_DIM;
+  if (!rt::gemm_mfma_takes(x, wt, bias, rows, m, n, k, dtype) || !rt::gemm_mfma_takes(x, wt, k_tiles, vt, m, n, k, dtype))
+    return rt::fail(RT_ENOSYS, "rt_qkv_project does not take this problem");
+  return rt::gemm_mfma_qkv(x, wt, bias, rows, k_tiles, vt, seq_blocks_dev, batch, m, heads, k, dtype, stream);
+}
+
 int rt_gemm_bt(rt_gemm_ctx* ctx, const void* a, const void* bt, const void* bias, void* c, int64_t m, int64_t n,
                int64_t k, int epilogue, int dtype, void* stream) {
   RT_REQUIRE(epilogue == RT_EPILOGUE_NONE || epilogue == RT_EPILOGUE_BIAS || epilogue == RT_EPILOGUE_BIAS_GELU, RT_EINVAL,
              "unknown epilogue %d", epilogue);
   RT_REQUIRE(epilogue == RT_EPILOGUE_NONE || bias, RT_EINVAL, "NULL bias");
+  if (ctx && a && bt && c && m > 0 && n > 0 && k > 0 &&
+      rt::gemm_mfma_takes(a, bt, epilogue == RT_EPILOGUE_NONE ? nullptr : bias, c, m, n, k, dtype))
+    return rt::gemm_mfma_bt(a, bt, epilogue == RT_EPILOGUE_NONE ? nullptr : bias, c, m, n, k,
+                            epilogue == RT_EPILOGUE_BIAS_GELU, dtype, stream);
   return run_gemm(ctx, a, bt, epilogue == RT_EPILOGUE_NONE ? nullptr : bias, c, m, n, k, epilogue, true, dtype, stream);
 }
 

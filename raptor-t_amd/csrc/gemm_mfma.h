@@ -1,0 +1,17 @@
+// The library's own dense products (gemm_mfma.hip), called by the entry points in gemm.cpp.
+#pragma once
+#include <cstdint>
+
+namespace rt {
+
+// Whether gemm_mfma_bt computes this product: 64 tiles of output at least, 16-bit types, K a multiple of 64, N a multiple of 8, 16-byte aligned
+// operands whose byte offsets fit 31 bits.
+bool gemm_mfma_takes(const void* a, const void* bt, const void* bias, const void* c, int64_t m, int64_t n, int64_t k, int dtype);
+// C[M,N] = A[M,K] . Bt[N,K]^T (+ bias, + tanh GELU)
+int gemm_mfma_bt(const void* a, const void* bt, const void* bias, void* c, int64_t m, int64_t n, int64_t k, bool gelu, int dtype,
+                 void* stream);
+// QKV projection with the head split: the Q columns go to rows[M, 3 * heads * 64], K and V to the packed tiles.
+int gemm_mfma_qkv(const void* a, const void* bt, const void* bias, void* rows, void* kt, void* vt, const int* seq_blocks_dev,
+                  int batch, int64_t m, int heads, int64_t k, int dtype, void* stream);
+
+}  // namespace rt

@@ -243,6 +243,32 @@ void MatMulBias(const torch::Tensor& A, const torch::Tensor& B, bool b_trans, co
                            RT_EPILOGUE_BIAS, dtype_code(A), current_stream()), name.c_str());
 }
 
+bool ProjectQkv(const torch::Tensor& A, const torch::Tensor& B, const torch::Tensor& bias, torch::Tensor& qkv_rows,
+                torch::Tensor& k, torch::Tensor& v, const torch::Tensor& seq_len_info_tensor, int batch_size, int head_num,
+                int block_num) {
+  require_cuda_contiguous(A, "A");
+  const torch::ScalarType dt = A.scalar_type();
+  if (dt != torch::kHalf && dt != torch::kBFloat16) return false;
+  const int64_t width = int64_t(head_num) * 3 * RT_HEAD_DIM, tokens = int64_t(block_num) * RT_BLOCK;
+  if (batch_size < 1 || head_num < 1 || block_num < batch_size || A.dim() != 2 || B.dim() != 2 || A.size(0) != tokens ||
+      B.size(0) != width || B.size(1) != A.size(1))
+    throw std::invalid_argument("ProjectQkv: shape mismatch");
+  require_data(B, "qkv weight", dt, width * A.size(1));
+  require_data(bias, "qkv bias", dt, width);
+  require_data(qkv_rows, "qkv", dt, tokens * width);
+  require_data(k, "k", dt, tokens * head_num * RT_HEAD_DIM);
+  require_data(v, "v", dt, tokens * head_num * RT_HEAD_DIM);
+  require_index(seq_len_info_tensor, "seq_len_info_tensor", int64_t(batch_size) + 1);
+  static std::map<std::string, float> no_info;
+  ScopedGpuTimer timer(no_info, "MatMul");
+  const int rc = rt_qkv_project(A.data_ptr(), B.data_ptr(), bias.data_ptr(), qkv_rows.data_ptr(), k.data_ptr(), v.data_ptr(),
+                                seq_len_info_tensor.data_ptr<int>(), batch_size, block_num, head_num, A.size(1), dtype_code(A),
+                                current_stream());
+  if (rc == RT_ENOSYS) return false;
+  check(rc, "rt_qkv_project");
+  return true;
+}
+
 namespace {
 std::atomic<bool> g_epilogue_fusion{true};
 std::atomic<bool> g_q_from_rows{true};

@@ -71,6 +71,13 @@ void MatMul(const torch::Tensor& A, bool a_trans, const torch::Tensor& B, bool b
 void MatMulBias(const torch::Tensor& A, const torch::Tensor& B, bool b_trans, const torch::Tensor& bias, torch::Tensor& out,
                 rt_gemm_ctx* handle, const std::string& name);
 
+// The QKV projection and the head split in one kernel (rt_qkv_project): Q to qkv_rows' first columns, K and V to the
+// packed tiles.  False, with nothing launched, where the kernel does not take the problem (fp32, one head): then
+// MatMulBias + add_bias_and_transpose_kernel.  Times itself under "MatMul".
+bool ProjectQkv(const torch::Tensor& A, const torch::Tensor& B, const torch::Tensor& bias, torch::Tensor& qkv_rows,
+                torch::Tensor& k, torch::Tensor& v, const torch::Tensor& seq_len_info_tensor, int batch_size, int head_num,
+                int block_num);
+
 // MatMul followed by add_bias_act_kernel, as one GEMM with the bias add and the tanh GELU in
 // its epilogue (what BertIntermediate's pair of calls, layers/bert_intermediate.cpp:22-30,
 // computes).  Times itself under "MatMul_bias_gelu".

@@ -59,8 +59,13 @@ void MultiHeadedAttention::FuseGemm012AddBIasTranspose(const torch::Tensor& inpu
                                                        std::map<std::string, float>& info, bool kernel_fusion) const {
   torch::Tensor tmp_qkv_out1 = TensorSet::get_instance()->get_tensor("tmp_qkv_out1");
   // With both fusions on, the projection adds its bias in the GEMM's epilogue (one rounding of the fp32 sum, no
-  // extra pass) and the split kernel only changes the layout: the bias it is handed is undefined.
+  // extra pass).  Where the queries stay in its rows, it also writes K and V^T as the tiles the attention kernel reads;
+  // otherwise the split kernel changes the layout, and the bias it is handed is undefined.
   if (bias_in_projection(kernel_fusion)) {
+    if (kernels::attention_q_from_rows() &&
+        kernels::ProjectQkv(input_tensor, qkv_weight_, qkv_bias_, tmp_qkv_out1, k_out, v_out, seq_len_info_tensor, batch_size_,
+                            head_num_, block_num_))
+      return;
     kernels::MatMulBias(input_tensor, qkv_weight_, true, qkv_bias_, tmp_qkv_out1, kernels::shared_gemm_handle(),
                         "FuseGemm012AddBIasTranspose_MatMul");
     kernels::add_bias_and_transpose_kernel(torch::Tensor(), tmp_qkv_out1, q_out, k_out, v_out, seq_len_info_tensor,
