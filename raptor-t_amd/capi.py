@@ -25,7 +25,7 @@ EXPORTS = [
     "rt_meta_partition_lpt", "rt_meta_check_partition", "rt_meta_check_to_index", "rt_qkv_bias_split", "rt_qkv_project", "rt_unpack_head_tiles", "rt_bs_attention_fwd",
     "rt_bs_attention_fwd_masked", "rt_bs_attention_fwd_qrows", "rt_bs_attention_fwd_no_alloc",
     "rt_bias_residual_layernorm", "rt_bias_gelu", "rt_embed_layernorm", "rt_gemm_create", "rt_gemm_destroy", "rt_gemm_set_tuning", "rt_gemm_set_retuning", "rt_gemm",
-    "rt_gemm_bias_act", "rt_gemm_bt", "rt_sequence_pool", "rt_pooler_dense_tanh",
+    "rt_gemm_bias_act", "rt_gemm_bt", "rt_gemm_bt_slices", "rt_slices_residual_layernorm", "rt_sequence_pool", "rt_pooler_dense_tanh",
     "rt_pipeline_create", "rt_pipeline_publish", "rt_pipeline_acquire", "rt_pipeline_release",
     "rt_pipeline_destroy", "rt_pipeline_set_index_check",
 ]
@@ -78,6 +78,8 @@ def lib():
         L.rt_embed_layernorm.argtypes = [vp, vp, vp, vp, vp, vp, vp, vp, vp, L64, I, I, I, I, ctypes.c_float, I, I, vp]
         L.rt_gemm_bias_act.argtypes = [vp, vp, vp, vp, vp, L64, L64, L64, I, I, vp]
         L.rt_gemm_bt.argtypes = [vp, vp, vp, vp, vp, L64, L64, L64, I, I, vp]
+        L.rt_gemm_bt_slices.argtypes = [vp, vp, vp, L64, L64, L64, I, ctypes.POINTER(vp), i32p, vp]
+        L.rt_slices_residual_layernorm.argtypes = [vp, vp, I, vp, vp, vp, vp, L64, I, F, I, vp]
         L.rt_sequence_pool.argtypes = [vp, vp, vp, I, I, I, vp, I, vp]
         L.rt_pooler_dense_tanh.argtypes = [vp, vp, vp, vp, I, I, I, I, vp]
         L.rt_pipeline_create.argtypes = [ctypes.POINTER(vp), I, I, I, I, I, I, I]
@@ -427,6 +429,25 @@ class Gemm:
         check(lib().rt_gemm_bt(self._h, _dp(a), _dp(bt), None if bias is None else _dp(bias), _dp(c), m, n, k, epilogue,
                                _dtype_code(a), _stream()))
         return c
+
+    def bt_layernorm(self, a, bt, bias, residual, gamma, beta, out, eps):
+        """out = LN(a @ bt.T + bias + residual) * gamma + beta.  Returns the number of slices the product was cut into
+        (0: rt_gemm_bt and rt_bias_residual_layernorm)."""
+        m, k = a.shape
+        n = bt.shape[0]
+        self._operands(a, bt, out, m, n, k, bias)
+        for name, t, numel in (("residual", residual, m * n), ("gamma", gamma, n), ("beta", beta, n)):
+            _dp(t, a.dtype, numel, name)
+        parts, n_parts = ctypes.c_void_p(), ctypes.c_int()
+        check(lib().rt_gemm_bt_slices(self._h, _dp(a), _dp(bt), m, n, k, _dtype_code(a), ctypes.byref(parts),
+                                      ctypes.byref(n_parts), _stream()))
+        if n_parts.value == 0:
+            self.bt(a, bt, out)
+            bias_residual_layernorm(out, residual, bias, gamma, beta, eps)
+        else:
+            check(lib().rt_slices_residual_layernorm(_dp(out), parts, n_parts.value, _dp(residual), _dp(bias), _dp(gamma),
+                                                     _dp(beta), m, n, eps, _dtype_code(a), _stream()))
+        return n_parts.value
 
     def close(self):
         if self._h:

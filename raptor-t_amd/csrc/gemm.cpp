@@ -33,6 +33,7 @@ struct rt_gemm_ctx {
   hipblasLtHandle_t lt = nullptr;
   int tune_candidates = 64;         // heuristic results timed on a shape's first call (1 = take the first)
   void* workspace = nullptr;
+  float* slices = nullptr;          // rt_gemm_bt_slices
   size_t workspace_bytes = 0;
   int device = 0;
   std::mutex m;
@@ -248,6 +249,7 @@ int rt_gemm_destroy(rt_gemm_ctx* ctx) {
   if (!ctx) return RT_OK;
   for (auto& kv : ctx->plans) free_plan(kv.second);
   if (ctx->workspace) (void)hipFree(ctx->workspace);
+  if (ctx->slices) (void)hipFree(ctx->slices);
   if (ctx->lt) hipblasLtDestroy(ctx->lt);
   delete ctx;
   return RT_OK;
@@ -316,6 +318,28 @@ int rt_gemm_bias_act(rt_gemm_ctx* ctx, const void* a, const void* b, const void*
   RT_REQUIRE(epilogue == RT_EPILOGUE_BIAS || epilogue == RT_EPILOGUE_BIAS_GELU, RT_EINVAL, "unknown epilogue %d", epilogue);
   RT_REQUIRE(bias, RT_EINVAL, "NULL bias");
   return run_gemm(ctx, a, b, bias, c, m, n, k, epilogue, false, dtype, stream);
+}
+
+int rt_gemm_bt_slices(rt_gemm_ctx* ctx, const void* a, const void* bt, int64_t m, int64_t n, int64_t k, int dtype,
+                      const float** parts, int* n_parts, void* stream) {
+  constexpr int64_t SLICES_BYTES = int64_t(32) << 20;
+  RT_REQUIRE(ctx && a && bt && parts && n_parts, RT_EINVAL, "NULL argument");
+  RT_REQUIRE(m >= 0 && n > 0 && k > 0, RT_EINVAL, "bad shape M=%lld N=%lld K=%lld", (long long)m, (long long)n, (long long)k);
+  *parts = nullptr;
+  *n_parts = 0;
+  if (m == 0 || n % 256 != 0 || n > 1024 || !rt::gemm_mfma_takes(a, bt, nullptr, nullptr, m, n, k, dtype)) return RT_OK;
+  const int slices = rt::gemm_mfma_slices(m, n, k, SLICES_BYTES);
+  if (slices < 2) return RT_OK;
+  std::lock_guard<std::mutex> lk(ctx->m);
+  if (!ctx->slices && hipMalloc(reinterpret_cast<void**>(&ctx->slices), SLICES_BYTES) != hipSuccess) {
+    ctx->slices = nullptr;
+    return rt::fail(RT_ENOMEM, "could not allocate the 32 MiB workspace of product slices");
+  }
+  const int rc = rt::gemm_mfma_part(a, bt, ctx->slices, m, n, k, slices, dtype, stream);
+  if (rc) return rc;
+  *parts = ctx->slices;
+  *n_parts = slices;
+  return RT_OK;
 }
 
 int rt_qkv_project(const void* x, const void* wt, const void* bias, void* rows, void* k_tiles, void* vt,

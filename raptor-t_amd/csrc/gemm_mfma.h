@@ -4,7 +4,7 @@
 
 namespace rt {
 
-// Whether gemm_mfma_bt computes this product: 64 tiles of output at least, 16-bit types, K a multiple of 64, N a multiple of 8, 16-byte aligned
+// Whether gemm_mfma_bt computes this product: 16-bit types, K a multiple of 64, N a multiple of 8, 16-byte aligned
 // operands whose byte offsets fit 31 bits.
 bool gemm_mfma_takes(const void* a, const void* bt, const void* bias, const void* c, int64_t m, int64_t n, int64_t k, int dtype);
 // C[M,N] = A[M,K] . Bt[N,K]^T (+ bias, + tanh GELU)
@@ -13,5 +13,11 @@ int gemm_mfma_bt(const void* a, const void* bt, const void* bias, void* c, int64
 // QKV projection with the head split: the Q columns go to rows[M, 3 * heads * 64], K and V to the packed tiles.
 int gemm_mfma_qkv(const void* a, const void* bt, const void* bias, void* rows, void* kt, void* vt, const int* seq_blocks_dev,
                   int batch, int64_t m, int heads, int64_t k, int dtype, void* stream);
+
+// Into how many slices of the reduction this product should be cut if the caller can take fp32 slices [slices][M][N] of
+// up to max_bytes and add them up itself (1: not at all, use gemm_mfma_bt).
+int gemm_mfma_slices(int64_t m, int64_t n, int64_t k, int64_t max_bytes);
+// The slices; `slices` > 1 as gemm_mfma_slices gave it.
+int gemm_mfma_part(const void* a, const void* bt, float* parts, int64_t m, int64_t n, int64_t k, int slices, int dtype, void* stream);
 
 }  // namespace rt

@@ -36,7 +36,7 @@
 // against 340, 40768 x 4096 x 1024 274 against 282; the projection with the head split 141 against 114 + 38.
 #include <hip/hip_runtime.h>
 
-#include <mutex>
+#include <atomic>
 #include <type_traits>
 
 #include "gemm_mfma.h"
@@ -62,7 +62,8 @@ template <typename T> struct Mma;
 template <> struct Mma<_Float16> {
   typedef f16x8 v8;
   __device__ static void run(v8 a, v8 b, f32x4& c) { asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+v"(c) : "v"(a), "v"(b)); }
-  __device__ static void first(v8 a, v8 b, f32x4& d, f32x4 c) { asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %3" : "=v"(d) : "v"(a), "v"(b), "v"(c)); }
+  __device__ static void zero(v8 a, v8 b, f32x4& d) { asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, 0" : "=&v"(d) : "v"(a), "v"(b)); }
+  __device__ static void first(v8 a, v8 b, f32x4& d, f32x4 c) { asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %3" : "=&v"(d) : "v"(a), "v"(b), "v"(c)); }
   __device__ static uint32_t two(float a, float b) { return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{a, b}, f16x2)); }
   __device__ static float lo(uint32_t w) { return float(__builtin_bit_cast(f16x2, w).x); }
   __device__ static float hi(uint32_t w) { return float(__builtin_bit_cast(f16x2, w).y); }
@@ -70,7 +71,8 @@ template <> struct Mma<_Float16> {
 template <> struct Mma<__bf16> {
   typedef bf16x8 v8;
   __device__ static void run(v8 a, v8 b, f32x4& c) { asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(c) : "v"(a), "v"(b)); }
-  __device__ static void first(v8 a, v8 b, f32x4& d, f32x4 c) { asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %3" : "=v"(d) : "v"(a), "v"(b), "v"(c)); }
+  __device__ static void zero(v8 a, v8 b, f32x4& d) { asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, 0" : "=&v"(d) : "v"(a), "v"(b)); }
+  __device__ static void first(v8 a, v8 b, f32x4& d, f32x4 c) { asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %3" : "=&v"(d) : "v"(a), "v"(b), "v"(c)); }
   __device__ static uint32_t two(float a, float b) { return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{a, b}, bf16x2)); }
   __device__ static float lo(uint32_t w) { return __uint_as_float(w << 16); }
   __device__ static float hi(uint32_t w) { return __uint_as_float(w & 0xffff0000u); }
@@ -81,7 +83,7 @@ constexpr int BK = 64;                        // reduction steps of a stage
 constexpr int ROW = BK * 2;                   // bytes of an LDS row
 constexpr int EPI_BYTES = 32 * 64 * 2;        // a wave's room for turning a 32 x 64 block of outputs into whole rows
 constexpr int WAVES = 8;
-constexpr int NT = 2;                         // cache policy of the stores of C: non-temporal
+constexpr int NON_TEMPORAL = 2;               // cache policy of a store
 constexpr int B_STAGE = TN * ROW;
 
 // An A stage also has to hold the epilogue's blocks of all waves.
@@ -136,6 +138,7 @@ struct Params {
   void* c;                // [M, N]
   int m, n, k;
   int tiles_m, tiles_n;
+  int slices;             // parts the reduction is cut into (EPI_PART)
   // QKV split: N = 3 * heads * 64
   void* kt;
   void* vt;
@@ -197,7 +200,113 @@ template <int TM> struct Stages {
   __device__ __forceinline__ uint32_t next_b() const { return b == B0 ? B0 + B_STAGE : B0; }
 };
 
-enum { EPI_NONE = 0, EPI_GELU = 1, EPI_QKV = 2 };
+enum { EPI_NONE = 0, EPI_GELU = 1, EPI_QKV = 2, EPI_PART = 3 };
+
+// ---- epilogues of a wave's MT x 4 blocks of 16 x 16 outputs, rows from m0, columns from n0 --------------------------
+// Rows of C: 16 x 64 outputs at a time through the wave's LDS room (4 KB at `room`), stored as eight whole 128-byte rows
+// per instruction.  A block's rows are read back while the next one is written, and the stores pass no test:
+// offsets past the end of C are dropped by the range check.
+template <typename T, int MT, int EPI, int POLICY>
+__device__ __forceinline__ void store_rows(const f32x4 (&acc)[MT][4], __amdgpu_buffer_rsrc_t sc, int n, int m0, int n0, char* room) {
+  const int lane = again(threadIdx.x & 63), l16 = lane & 15, g4 = lane >> 4;
+  const bool col_ok = n0 + (lane & 7) * 8 < n;
+  uint32_t voff = col_ok ? (uint32_t(m0 + (lane >> 3)) * uint32_t(n) + uint32_t(n0 + (lane & 7) * 8)) * 2u : 0xfffffff0u;
+  const uint32_t ld8 = col_ok ? uint32_t(n) * 16u : 0u;         // eight rows
+  const int wr = l16 * 128 + 8 * (g4 & 1), wx = l16 >> 1, rr = (lane >> 3) * 128;
+#pragma unroll
+  for (int i = 0; i <= MT; ++i) {
+    u32x4 o[2];
+    if (i > 0) {
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+        o[j] = *reinterpret_cast<const u32x4*>(room + ((i - 1) & 1) * 2048 + j * 1024 + rr + (((lane & 7) ^ (((lane >> 4) + 4 * j) & 7)) << 4));
+    }
+    if (i < MT) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        f32x4 v = acc[i][j];
+        if (EPI == EPI_GELU) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[e] = gelu_tanh(v[e]);
+        }
+        *reinterpret_cast<u32x2*>(room + (i & 1) * 2048 + wr + (((2 * j + (g4 >> 1)) ^ wx) << 4)) =
+            u32x2{Mma<T>::two(v[0], v[1]), Mma<T>::two(v[2], v[3])};
+      }
+    }
+    if (i > 0) {
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        __builtin_amdgcn_raw_buffer_store_b128(o[j], sc, int(voff), 0, POLICY);
+        voff += ld8;
+      }
+    }
+    SB();
+  }
+}
+
+// K and V^T tiles: where the half tile of the 32 tokens from `row` on begins (lane's part), for head h.  seq_end: lane
+// l holds the end of sequence l (batches of up to 64 sequences).
+template <typename T> __device__ __forceinline__ T* half_tile(void* base, const Params& p, int seq_end, int row, int h) {
+  const int g = row >> 6, lane = again(threadIdx.x & 63);
+  int s, g0, end;                                          // the sequence block g belongs to
+  if (p.batch <= 64) {
+    s = __popcll(__ballot(lane < p.batch && seq_end <= g));
+    g0 = s == 0 ? 0 : __builtin_amdgcn_readlane(seq_end, s - 1);
+    end = __builtin_amdgcn_readlane(seq_end, s);
+  } else {
+    s = 0;
+    for (int b0 = 0; b0 < p.batch; b0 += 64)
+      s += __popcll(__ballot(b0 + lane < p.batch && p.seq_blocks[min(b0 + lane + 1, p.batch)] <= g));
+    g0 = p.seq_blocks[s];
+    end = p.seq_blocks[s + 1];
+  }
+  return static_cast<T*>(base) + (int64_t(g0) * p.heads + int64_t(h) * (end - g0) + (g - g0)) * 4096 + lane * 8;
+}
+
+// V^T tiles of head h (products taken with the tokens as rows): a lane's accumulators are 4 consecutive tokens of one
+// column; fragment 4 * (d >> 5) + (token >> 4) wants, in lane (d & 31) + 32 * x, the tokens 4 x .. + 4 and 8 + 4 x .. + 4
+// of its 16.
+template <typename T, int MT> __device__ __forceinline__ void store_v(const f32x4 (&acc)[MT][4], const Params& p, int seq_end, int m0, int h) {
+#pragma unroll
+  for (int i = 0; i < MT; i += 2) {
+    const int row = m0 + 16 * i;
+    if (row >= p.m) break;
+    T* const t = half_tile<T>(p.vt, p, seq_end, row, h) + ((row >> 5) & 1) * 1024;
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+#pragma unroll
+      for (int j = 0; j < 4; j += 2) {
+        const f32x4 &c = acc[i + q][j], &d = acc[i + q][j + 1];
+        uint32_t x0 = Mma<T>::two(c[0], c[1]), x1 = Mma<T>::two(c[2], c[3]);
+        uint32_t y0 = Mma<T>::two(d[0], d[1]), y1 = Mma<T>::two(d[2], d[3]);
+        permlane16_swap(x0, y0);
+        permlane16_swap(x1, y1);
+        permlane32_swap(x0, y0);
+        permlane32_swap(x1, y1);
+        *reinterpret_cast<u32x4*>(t + (2 * j + q) * 512) = u32x4{x0, x1, y0, y1};
+      }
+  }
+}
+
+// K tiles of head h (products taken with the columns as rows): a lane's accumulators are 4 consecutive columns of one
+// token; fragment 4 * (token >> 5) + (d >> 4) wants, in lane (token & 31) + 32 * x, the columns 8 x .. + 8 of its 16.
+template <typename T, int MT> __device__ __forceinline__ void store_k(const f32x4 (&acc)[MT][4], const Params& p, int seq_end, int m0, int h) {
+#pragma unroll
+  for (int i = 0; i < MT; i += 2) {
+    const int row = m0 + 16 * i;
+    if (row >= p.m) break;
+    T* const t = half_tile<T>(p.kt, p, seq_end, row, h) + ((row >> 5) & 1) * 2048;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const f32x4 &c = acc[i][j], &d = acc[i + 1][j];
+      uint32_t x0 = Mma<T>::two(c[0], c[1]), x1 = Mma<T>::two(c[2], c[3]);
+      uint32_t y0 = Mma<T>::two(d[0], d[1]), y1 = Mma<T>::two(d[2], d[3]);
+      permlane16_swap(x0, y0);
+      permlane16_swap(x1, y1);
+      *reinterpret_cast<u32x4*>(t + j * 512) = u32x4{x0, x1, y0, y1};
+    }
+  }
+}
 
 // What the epilogue needs from memory, requested a step ahead: the bias of a wave's columns (of column block j the 4
 // consecutive ones of a lane's accumulators, or (V) the one) for the tile after it, and where the batch's first 64
@@ -400,113 +509,23 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       const int following = tile + slots < last ? tile + slots : tile;
       auto next_bias = [&]() __attribute__((always_inline)) { load_bias(following); };
       f32x4 acc[MT][4];
-      // K and V^T tiles: where the half tile of the 32 tokens from `row` on begins (lane's part), for the wave's first head
-      auto half_tile = [&](void* base, int row, int h) __attribute__((always_inline)) {
-        const int g = row >> 6, lane = again(threadIdx.x & 63);
-        int s, g0, end;                                    // the sequence block g belongs to
-        if (p.batch <= 64) {
-          s = __popcll(__ballot(lane < p.batch && bias.seq_end <= g));
-          g0 = s == 0 ? 0 : __builtin_amdgcn_readlane(bias.seq_end, s - 1);
-          end = __builtin_amdgcn_readlane(bias.seq_end, s);
-        } else {
-          s = 0;
-          for (int b0 = 0; b0 < p.batch; b0 += 64)
-            s += __popcll(__ballot(b0 + lane < p.batch && p.seq_blocks[min(b0 + lane + 1, p.batch)] <= g));
-          g0 = p.seq_blocks[s];
-          end = p.seq_blocks[s + 1];
-        }
-        const int nb = end - g0;
-        return static_cast<T*>(base) + (int64_t(g0) * p.heads + int64_t(h) * nb + (g - g0)) * 4096 + lane * 8;
-      };
       // (The assembly comments keep the compiler from merging equal code of the branches, which costs it registers.)
       if (EPI == EPI_QKV && v_tile) {
         asm volatile("; V tile");
         main_loop<T, TM, MT, EPI, true>(acc, c0, bias, next_bias, lda, ldb, st, p, sa, sb, smem, lds0, w, lane, offa, offb);
-        if (n0 >= p.n) continue;
-        // A lane's accumulators are 4 consecutive tokens of one column; fragment 4 * (d >> 5) + (token >> 4) of the tile
-        // wants, in lane (d & 31) + 32 * x, the tokens 4 x .. + 4 and 8 + 4 x .. + 4 of its 16.
-#pragma unroll
-        for (int i = 0; i < MT; i += 2) {
-          const int row = m0 + 16 * i;
-          if (row >= p.m) break;
-          T* const t = half_tile(p.vt, row, (n0 - 2 * dm) >> 6) + ((row >> 5) & 1) * 1024;
-#pragma unroll
-          for (int q = 0; q < 2; ++q)
-#pragma unroll
-            for (int j = 0; j < 4; j += 2) {
-              const f32x4 &c = acc[i + q][j], &d = acc[i + q][j + 1];
-              uint32_t x0 = Mma<T>::two(c[0], c[1]), x1 = Mma<T>::two(c[2], c[3]);
-              uint32_t y0 = Mma<T>::two(d[0], d[1]), y1 = Mma<T>::two(d[2], d[3]);
-              permlane16_swap(x0, y0);
-              permlane16_swap(x1, y1);
-              permlane32_swap(x0, y0);
-              permlane32_swap(x1, y1);
-              *reinterpret_cast<u32x4*>(t + (2 * j + q) * 512) = u32x4{x0, x1, y0, y1};
-            }
-        }
+        if (n0 < p.n) store_v<T, MT>(acc, p, bias.seq_end, m0, (n0 - 2 * dm) >> 6);
         asm volatile("; V tile done");
         continue;
       }
       main_loop<T, TM, MT, EPI, false>(acc, c0, bias, next_bias, lda, ldb, st, p, sa, sb, smem, lds0, w, lane, offa, offb);
       if (EPI == EPI_QKV && n0 >= dm) {
-        // A lane's accumulators are 4 consecutive columns of one token; fragment 4 * (token >> 5) + (d >> 4) of the tile
-        // wants, in lane (token & 31) + 32 * x, the columns 8 x .. + 8 of its 16.
-#pragma unroll
-        for (int i = 0; i < MT; i += 2) {
-          const int row = m0 + 16 * i;
-          if (row >= p.m) break;
-          T* const t = half_tile(p.kt, row, (n0 - dm) >> 6) + ((row >> 5) & 1) * 2048;
-#pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            const f32x4 &c = acc[i][j], &d = acc[i + 1][j];
-            uint32_t x0 = Mma<T>::two(c[0], c[1]), x1 = Mma<T>::two(c[2], c[3]);
-            uint32_t y0 = Mma<T>::two(d[0], d[1]), y1 = Mma<T>::two(d[2], d[3]);
-            permlane16_swap(x0, y0);
-            permlane16_swap(x1, y1);
-            *reinterpret_cast<u32x4*>(t + j * 512) = u32x4{x0, x1, y0, y1};
-          }
-        }
+        store_k<T, MT>(acc, p, bias.seq_end, m0, (n0 - dm) >> 6);
         asm volatile("; K tile done");
         continue;
       }
-      // rows of C: 16 x 64 outputs at a time through the wave's LDS room (the A stage of the tile's last step; st has
-      // moved on by one), stored as eight whole 128-byte rows per instruction.  A block's rows are read back while the
-      // next one is written, and the stores pass no test: offsets past the end of C are dropped by the range check.
-      const int lane = again(threadIdx.x & 63), l16 = lane & 15, g4 = lane >> 4;
-      char* const epi = smem + (st.a == 0 ? 2u * a_stage<TM>() : st.a - a_stage<TM>()) + w * EPI_BYTES;
-      const bool col_ok = n0 + (lane & 7) * 8 < p.n;
-      uint32_t voff = col_ok ? (uint32_t(m0 + (lane >> 3)) * uint32_t(p.n) + uint32_t(n0 + (lane & 7) * 8)) * 2u : 0xfffffff0u;
-      const uint32_t ld8 = col_ok ? uint32_t(p.n) * 16u : 0u;       // eight rows
-      const int wr = l16 * 128 + 8 * (g4 & 1), wx = l16 >> 1, rr = (lane >> 3) * 128;
-#pragma unroll
-      for (int i = 0; i <= MT; ++i) {
-        u32x4 o[2];
-        if (i > 0) {
-#pragma unroll
-          for (int j = 0; j < 2; ++j)
-            o[j] = *reinterpret_cast<const u32x4*>(epi + ((i - 1) & 1) * 2048 + j * 1024 + rr + (((lane & 7) ^ (((lane >> 4) + 4 * j) & 7)) << 4));
-        }
-        if (i < MT) {
-#pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            f32x4 v = acc[i][j];
-            if (EPI == EPI_GELU) {
-#pragma unroll
-              for (int e = 0; e < 4; ++e) v[e] = gelu_tanh(v[e]);
-            }
-            *reinterpret_cast<u32x2*>(epi + (i & 1) * 2048 + wr + (((2 * j + (g4 >> 1)) ^ wx) << 4)) =
-                u32x2{Mma<T>::two(v[0], v[1]), Mma<T>::two(v[2], v[3])};
-          }
-        }
-        if (i > 0) {
-#pragma unroll
-          for (int j = 0; j < 2; ++j) {
-            __builtin_amdgcn_raw_buffer_store_b128(o[j], sc, int(voff), 0, NT);
-            voff += ld8;
-          }
-        }
-        SB();
-      }
+      // through the A stage of the tile's last step (st has moved on by one)
+      store_rows<T, MT, EPI, NON_TEMPORAL>(acc, sc, p.n, m0, n0,
+                                           smem + (st.a == 0 ? 2u * a_stage<TM>() : st.a - a_stage<TM>()) + w * EPI_BYTES);
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       // the trailing loads write LDS of this workgroup
   };
@@ -514,47 +533,288 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   else run(std::integral_constant<int, MT1>());
 }
 
-template <typename T, int TM, int MT0, int MT1, int EPI>
-int launch(const Params& base, hipStream_t st) {
-  Params p = base;
-  p.tiles_m = (p.m + TM - 1) / TM;
-  p.tiles_n = (p.n + TN - 1) / TN;
-  static std::once_flag once;
-  static hipError_t attr = hipSuccess;
-  std::call_once(once, [] {
-    attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_bt_kernel<T, TM, MT0, MT1, EPI>),
-                               hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes<TM>());
-  });
-  if (attr != hipSuccess) return rt::fail(RT_EIO, "gemm: %d bytes of LDS refused: %s", lds_bytes<TM>(), hipGetErrorString(attr));
-  const int total = p.tiles_m * p.tiles_n;
-  const int grid = total >= 256 ? 256 : (total + 7) / 8 * 8;
-  RT_LAUNCH((gemm_bt_kernel<T, TM, MT0, MT1, EPI>), dim3(grid), dim3(512), lds_bytes<TM>(), st, p);
+// ---- smaller products ------------------------------------------------------------------------------------------------
+// One workgroup of 4 waves per tile of TM x TC outputs and per slice of the reduction; a wave owns MT row blocks of 16
+// and 64 columns.  Where the kernel above would give too few CUs a tile each, what bounds a product is the latency of a
+// workgroup's chain of steps: STAGES of both operands are in flight, up to two workgroups share a CU, and a long
+// reduction is cut into slices (EPI_PART: the fp32 sums of slice s go to c[s][M][N] and the kernel that reads
+// them, the layer's LayerNorm, adds the slices).
+//   A step: fragments of half 1 requested, products of half 0; the own loads of the next step and the own reads of this
+//   one have arrived, barrier; fragments of the next step's half 0 and the loads of the step STAGES ahead requested,
+//   products of half 1.
+template <typename T, int TM, int TC, int NW, int STAGES, int EPI>
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) void gemm_bt_small_kernel(Params p) {
+  typedef typename Mma<T>::v8 v8;
+  extern __shared__ __align__(16) char smem[];
+  constexpr int WN = TC / 64, WM = NW / WN, MT = TM / 16 / WM;
+  constexpr int NA = TM / 8 / NW, NB = TC / 8 / NW, LOADS = NA + NB;      // load instructions of a wave and step
+  constexpr uint32_t STAGE = (TM + TC) * ROW;
+  static_assert(MT >= 1 && STAGES * STAGE >= NW * EPI_BYTES && NA >= 1 && NB >= 1, "tile");
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, l16 = lane & 15, g4 = lane >> 4;
+  // XCD x takes the x-th eighth of the list: slice, groups of 8 row panels, column, panel
+  const int tiles = p.tiles_m * p.tiles_n, total = tiles * p.slices, per = gridDim.x >> 3;
+  const int id = int(blockIdx.x & 7) * per + int(blockIdx.x >> 3);
+  if (id >= total) return;
+  const int slice = id / tiles, tile = id - slice * tiles;
+  constexpr int G = 8;
+  const int grp = tile / (G * p.tiles_n), in = tile - grp * G * p.tiles_n, h = min(G, p.tiles_m - grp * G);
+  const int tn = in / h, tm = grp * G + (in - tn * h);
+  const int all = p.k / BK, first = all * slice / p.slices, steps = all * (slice + 1) / p.slices - first;
+
+  const uint32_t lds0 = uint32_t(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) char*)smem));
+  const i32x4 sa = make_srd(p.a, uint32_t(p.m) * uint32_t(p.k) * 2u), sb = make_srd(p.bt, uint32_t(p.n) * uint32_t(p.k) * 2u);
+  int va[NA], vb[NB];
+  {
+    const int r = w * 8 + (lane >> 3), chunk = ((lane & 7) ^ ((r >> 1) & 7)) * 16;
+#pragma unroll
+    for (int j = 0; j < NA; ++j) va[j] = min(tm * TM + j * 8 * NW + r, p.m - 1) * p.k * 2 + chunk;
+#pragma unroll
+    for (int j = 0; j < NB; ++j) vb[j] = min(tn * TC + j * 8 * NW + r, p.n - 1) * p.k * 2 + chunk;
+  }
+  // loads [from, to) of a step: B's rows first
+  auto issue = [&](int s, uint32_t stage, int from, int to) __attribute__((always_inline)) {
+    const int soff = (first + s) * ROW;
+#pragma unroll
+    for (int j = 0; j < LOADS; ++j) {
+      if (j < from || j >= to) continue;
+      if (j < NB) load_to_lds(sb, vb[j % NB], soff, lds0 + stage + TM * ROW + (j * NW + w) * 1024);
+      else load_to_lds(sa, va[(j - NB) % NA], soff, lds0 + stage + ((j - NB) * NW + w) * 1024);
+    }
+  };
+#pragma unroll
+  for (int q = 0; q < STAGES; ++q)
+    if (q < steps) issue(q, q * STAGE, 0, LOADS);
+
+  const int m0 = tm * TM + (w / WN) * 16 * MT, n0 = tn * TC + (w % WN) * 64, dm = p.heads * 64;
+  const bool v_tile = EPI == EPI_QKV && n0 >= 2 * dm;
+  int offa[2], offb[2];
+#pragma unroll
+  for (int kk = 0; kk < 2; ++kk) {
+    const int c = ((4 * kk + g4) ^ (l16 >> 1)) << 4;
+    offa[kk] = ((w / WN) * 16 * MT + l16) * ROW + c;
+    offb[kk] = (TM + (w % WN) * 64 + l16) * ROW + c;
+  }
+  v8 a[2][MT], b[2][4];
+  f32x4 acc[MT][4];
+  auto read = [&](int kk, uint32_t stage) __attribute__((always_inline)) {
+    const char *la = smem + stage + offa[kk], *lb = smem + stage + offb[kk];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) b[kk][j] = *reinterpret_cast<const v8*>(lb + j * 16 * ROW);
+#pragma unroll
+    for (int i = 0; i < MT; ++i) a[kk][i] = *reinterpret_cast<const v8*>(la + i * 16 * ROW);
+  };
+  auto loop = [&](auto v_tag) __attribute__((always_inline)) {
+    constexpr bool V_TILE = decltype(v_tag)::value;
+    auto products = [&](int kk, int i, auto init) __attribute__((always_inline)) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int c = i & 1 ? 3 - j : j;
+        const v8 &x = V_TILE ? a[kk][i] : b[kk][c], &y = V_TILE ? b[kk][c] : a[kk][i];
+        if (decltype(init)::value) Mma<T>::zero(x, y, acc[i][c]);
+        else Mma<T>::run(x, y, acc[i][c]);
+      }
+      SB();
+    };
+    uint32_t cur = 0;
+    auto step = [&](int s, auto init) __attribute__((always_inline)) {
+      read(1, cur);
+      SB();
+      asm volatile("s_nop 1");
+#pragma unroll
+      for (int i = 0; i < MT; ++i) products(0, i, init);
+      if (s + STAGES <= steps) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" :: "n"((STAGES - 2) * LOADS) : "memory");
+      else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+      SB();
+      const uint32_t nxt = cur == (STAGES - 1) * STAGE ? 0u : cur + STAGE;
+      if (s + 1 < steps) read(0, nxt);
+      SB();
+      const bool more = s + STAGES < steps;
+      constexpr int PER_ROW = (LOADS + MT - 1) / MT;
+#pragma unroll
+      for (int i = 0; i < MT; ++i) {
+        products(1, i, std::false_type());
+        if (more) issue(s + STAGES, cur, i * PER_ROW, (i + 1) * PER_ROW);
+        SB();
+      }
+      cur = nxt;
+    };
+    if (STAGES <= steps) asm volatile("s_waitcnt vmcnt(%0)" :: "n"((STAGES - 1) * LOADS) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    SB();
+    read(0, 0);
+    step(0, std::true_type());
+#pragma clang loop unroll(disable)
+    for (int s = 1; s < steps; ++s) step(s, std::false_type());
+    asm volatile("s_nop 15\n\ts_nop 7");
+    SB();
+  };
+  if (v_tile) loop(std::true_type());
+  else loop(std::false_type());
+  if (n0 >= p.n) return;
+
+  if (EPI == EPI_PART) {
+    // whole 64-byte runs: 4 consecutive columns per lane
+    const __amdgpu_buffer_rsrc_t sc =
+        __builtin_amdgcn_make_buffer_rsrc(static_cast<float*>(p.c) + int64_t(slice) * p.m * p.n, 0, uint32_t(p.m) * uint32_t(p.n) * 4u, 0x00020000);
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int col = n0 + 16 * j + 4 * g4;
+        const uint32_t voff = col < p.n ? (uint32_t(m0 + 16 * i + l16) * uint32_t(p.n) + uint32_t(col)) * 4u : 0xfffffff0u;
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, acc[i][j]), sc, int(voff), 0, 0);
+      }
+    return;
+  }
+  if (p.bias) {
+    const T* bp = static_cast<const T*>(p.bias);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      f32x4 c;
+      if (v_tile) {
+        c = f32x4(Mma<T>::lo(reinterpret_cast<const uint16_t*>(bp)[min(n0 + 16 * j + l16, p.n - 1)]));
+      } else {
+        const u32x2 x = *reinterpret_cast<const u32x2*>(bp + min(n0 + 16 * j + 4 * g4, p.n - 4));
+        c = f32x4{Mma<T>::lo(x.x), Mma<T>::hi(x.x), Mma<T>::lo(x.y), Mma<T>::hi(x.y)};
+      }
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[i][j][e] += c[e];
+    }
+  }
+  if (EPI == EPI_QKV && n0 >= dm) {
+    const int seq_end = p.seq_blocks[min(lane + 1, p.batch)];
+    if constexpr (MT % 2 == 0) {
+      if (v_tile) store_v<T, MT>(acc, p, seq_end, m0, (n0 - 2 * dm) >> 6);
+      else store_k<T, MT>(acc, p, seq_end, m0, (n0 - dm) >> 6);
+    }
+    return;
+  }
+  const __amdgpu_buffer_rsrc_t sc = __builtin_amdgcn_make_buffer_rsrc(p.c, 0, uint32_t(p.m) * uint32_t(p.n) * 2u, 0x00020000);
+  store_rows<T, MT, EPI, 0>(acc, sc, p.n, m0, n0, smem + w * EPI_BYTES);
+}
+
+// More dynamic LDS than the default has to be asked for once per kernel and device.
+template <typename K> int allow_lds(K kernel, int bytes, std::atomic<uint64_t>& done) {
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return rt::fail(RT_EIO, "hipGetDevice failed: no usable GPU");
+  const uint64_t bit = uint64_t(1) << (dev & 63);
+  if (done.load(std::memory_order_relaxed) & bit) return RT_OK;
+  const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+  if (e != hipSuccess) return rt::fail(RT_EIO, "gemm: %d bytes of LDS refused: %s", bytes, hipGetErrorString(e));
+  done.fetch_or(bit, std::memory_order_relaxed);
+  return RT_OK;
+}
+
+int launched() {
   const hipError_t e = hipGetLastError();
   return e == hipSuccess ? RT_OK : rt::fail(RT_EIO, "gemm launch failed: %s", hipGetErrorString(e));
 }
 
-template <typename T, int EPI> int dispatch(const Params& p, hipStream_t st) {
-  // rounds of 256 workgroups x height of a tile: the shortest schedule
-  const int64_t tn = (p.n + TN - 1) / TN;
-  auto cost = [&](int tm) { return (((p.m + tm - 1) / tm) * tn + 255) / 256 * (tm + 24); };
-  const int heights[3] = {256, 224, 192};
-  int best = 0;
-  for (int i = 1; i < 3; ++i)
-    if (cost(heights[i]) < cost(heights[best])) best = i;
-  if (best == 0) return launch<T, 256, 8, 8, EPI>(p, st);
-  if (best == 1) return launch<T, 224, 8, 6, EPI>(p, st);
-  return launch<T, 192, 6, 6, EPI>(p, st);
+template <typename T, int TM, int MT0, int MT1, int EPI> int launch(const Params& base, hipStream_t st) {
+  Params p = base;
+  p.tiles_m = (p.m + TM - 1) / TM;
+  p.tiles_n = (p.n + TN - 1) / TN;
+  static std::atomic<uint64_t> done{0};
+  if (int rc = allow_lds(&gemm_bt_kernel<T, TM, MT0, MT1, EPI>, lds_bytes<TM>(), done)) return rc;
+  const int total = p.tiles_m * p.tiles_n;
+  const int grid = total >= 256 ? 256 : (total + 7) / 8 * 8;
+  RT_LAUNCH((gemm_bt_kernel<T, TM, MT0, MT1, EPI>), dim3(grid), dim3(512), lds_bytes<TM>(), st, p);
+  return launched();
+}
+
+template <typename T, int TM, int TC, int NW, int STAGES, int EPI> int launch_small(const Params& base, hipStream_t st) {
+  Params p = base;
+  p.tiles_m = (p.m + TM - 1) / TM;
+  p.tiles_n = (p.n + TC - 1) / TC;
+  constexpr int LDS = STAGES * (TM + TC) * ROW;
+  static std::atomic<uint64_t> done{0};
+  if (int rc = allow_lds(&gemm_bt_small_kernel<T, TM, TC, NW, STAGES, EPI>, LDS, done)) return rc;
+  const int total = p.tiles_m * p.tiles_n * p.slices;
+  RT_LAUNCH((gemm_bt_small_kernel<T, TM, TC, NW, STAGES, EPI>), dim3((total + 7) / 8 * 8), dim3(64 * NW), LDS, st, p);
+  return launched();
+}
+
+// ---- which kernel ----------------------------------------------------------------------------------------------------
+// A product's time is estimated for every kernel and number of slices from a model with three measured figures
+// each (microseconds, random fp16 operands): one step of a workgroup that has its CU to itself, how much longer it
+// takes when every CU has one, and a step of two workgroups that share a CU; plus the launch, its first loads and its
+// epilogue.  Where the lines fall, with both sides measured (us, before: hipBLASLt):
+//   512 x 2304 x 768    128 x 64: 7.0, 192 x 256: 13.7 (15.8)     4096 x 2304 x 768  192 x 256: 17.1, 128 x 64: 23 (21)
+//   512 x 768 x 3072    64 x 64 in 4 slices: 8.1, uncut 15.3 (16) 5568 x 768 x 3072  192 x 128: 33.6, 128 x 128: 41 (36)
+//   4096 x 768 x 3072   128 x 128: 27.4, 64 x 64: 34 (28.6)       8192 x 768 x 3072  256 x 128: 43, 192 x 256: 46 (41)
+struct Choice {
+  int tm, tc, waves, stages, slices;
+};
+struct Kernel {
+  Choice c;
+  float step, crowd, pair;      // pair 0: one workgroup per CU
+  float fixed;                  // per round
+  bool qkv;                     // has the head split (which needs 32 rows per wave)
+};
+const Kernel kKernels[] = {
+    {{256, 256, 8, 0, 1}, 1.05f, 0.20f, 0.f, 4.4f, true},
+    {{224, 256, 8, 0, 1}, 0.90f, 0.18f, 0.f, 4.2f, true},
+    {{192, 256, 8, 0, 1}, 0.78f, 0.16f, 0.f, 4.0f, true},
+    {{256, 128, 8, 3, 1}, 0.69f, 0.12f, 0.f, 3.4f, true},
+    {{192, 128, 8, 3, 1}, 0.58f, 0.11f, 0.f, 3.4f, false},
+    {{128, 128, 8, 4, 1}, 0.41f, 0.15f, 0.f, 3.4f, true},
+    {{128, 64, 4, 3, 1}, 0.35f, 0.02f, 0.54f, 3.4f, true},
+    {{64, 64, 4, 4, 1}, 0.27f, 0.02f, 0.37f, 3.4f, false},
+};
+
+// max_slices 1: the caller takes the product itself; more: fp32 slices will do, which the caller's next kernel reads.
+Choice choose(int64_t m, int64_t n, int64_t k, int epi, int max_slices) {
+  const int steps = int(k / BK);
+  Choice best = kKernels[0].c;
+  float best_us = 0.f;
+  for (const Kernel& kn : kKernels) {
+    if (epi == EPI_QKV && !kn.qkv) continue;
+    for (int s = 1; s <= (kn.c.stages == 0 ? 1 : max_slices); ++s) {
+      if (s > 1 && steps / s < 6) break;
+      const int64_t wgs = ((m + kn.c.tm - 1) / kn.c.tm) * ((n + kn.c.tc - 1) / kn.c.tc) * s;
+      const int64_t slots = kn.pair > 0.f ? 512 : 256, full = wgs / slots, rest = wgs % slots;
+      const float alone = kn.step + kn.crowd * float(rest < 256 ? rest : 256) / 256.f, both = kn.pair > 0.f ? kn.pair : kn.step + kn.crowd;
+      const float rounds = float(full) * both + (rest == 0 ? 0.f : rest <= 256 ? alone : both);
+      float us = rounds * float((steps + s - 1) / s) + kn.fixed * float(full + (rest ? 1 : 0));
+      if (s > 1) us += float(m) * float(n) * float(8 * s - 4) * 2e-7f;      // the slices' way to memory and back at 5 TB/s
+      if (best_us == 0.f || us < best_us) { best_us = us; best = kn.c; best.slices = s; }
+    }
+  }
+  return best;
+}
+
+template <typename T, int EPI> int dispatch(Params& p, const Choice& c, hipStream_t st) {
+  p.slices = c.slices;
+  if constexpr (EPI != EPI_PART) {
+    if (c.tc == TN) {
+      if (c.tm == 256) return launch<T, 256, 8, 8, EPI>(p, st);
+      if (c.tm == 224) return launch<T, 224, 8, 6, EPI>(p, st);
+      return launch<T, 192, 6, 6, EPI>(p, st);
+    }
+  }
+  if (c.tc == 128) {
+    if (c.tm == 256) return launch_small<T, 256, 128, 8, 3, EPI>(p, st);
+    if constexpr (EPI != EPI_QKV) {
+      if (c.tm == 192) return launch_small<T, 192, 128, 8, 3, EPI>(p, st);
+    }
+    return launch_small<T, 128, 128, 8, 4, EPI>(p, st);
+  }
+  if constexpr (EPI != EPI_QKV) {
+    if (c.tm == 64) return launch_small<T, 64, 64, 4, 4, EPI>(p, st);
+  }
+  return launch_small<T, 128, 64, 4, 3, EPI>(p, st);
 }
 
 }  // namespace
 
 namespace rt {
 
-// At least 64 tiles (a quarter of the CUs): with fewer, one CU's share of a long reduction is longer than what the
-// library's smaller tiles take (2816 x 768 x 3072, 45 tiles: 40 us against 22).
 bool gemm_mfma_takes(const void* a, const void* bt, const void* bias, const void* c, int64_t m, int64_t n, int64_t k, int dtype) {
   auto aligned = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; };
-  if ((m + 191) / 192 * ((n + TN - 1) / TN) < 64) return false;
   return (dtype == RT_F16 || dtype == RT_BF16) && k % BK == 0 && k >= 2 * BK && n % 8 == 0 && m * k < (int64_t(1) << 29) &&
          n * k < (int64_t(1) << 29) && (m + 256) * n < (int64_t(1) << 31) && aligned(a) && aligned(bt) && aligned(bias) && aligned(c);
 }
@@ -565,8 +825,9 @@ int gemm_mfma_bt(const void* a, const void* bt, const void* bias, void* c, int64
   p.a = a; p.bt = bt; p.bias = bias; p.c = c;
   p.m = int(m); p.n = int(n); p.k = int(k);
   hipStream_t st = static_cast<hipStream_t>(stream);
-  if (dtype == RT_F16) return gelu ? dispatch<_Float16, EPI_GELU>(p, st) : dispatch<_Float16, EPI_NONE>(p, st);
-  return gelu ? dispatch<__bf16, EPI_GELU>(p, st) : dispatch<__bf16, EPI_NONE>(p, st);
+  const Choice ch = choose(m, n, k, gelu ? EPI_GELU : EPI_NONE, 1);
+  if (dtype == RT_F16) return gelu ? dispatch<_Float16, EPI_GELU>(p, ch, st) : dispatch<_Float16, EPI_NONE>(p, ch, st);
+  return gelu ? dispatch<__bf16, EPI_GELU>(p, ch, st) : dispatch<__bf16, EPI_NONE>(p, ch, st);
 }
 
 int gemm_mfma_qkv(const void* a, const void* bt, const void* bias, void* rows, void* kt, void* vt, const int* seq_blocks_dev,
@@ -576,7 +837,24 @@ int gemm_mfma_qkv(const void* a, const void* bt, const void* bias, void* rows, v
   p.m = int(m); p.n = 3 * heads * 64; p.k = int(k);
   p.kt = kt; p.vt = vt; p.seq_blocks = seq_blocks_dev; p.batch = batch; p.heads = heads;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  return dtype == RT_F16 ? dispatch<_Float16, EPI_QKV>(p, st) : dispatch<__bf16, EPI_QKV>(p, st);
+  const Choice ch = choose(m, p.n, k, EPI_QKV, 1);
+  return dtype == RT_F16 ? dispatch<_Float16, EPI_QKV>(p, ch, st) : dispatch<__bf16, EPI_QKV>(p, ch, st);
+}
+
+int gemm_mfma_slices(int64_t m, int64_t n, int64_t k, int64_t max_bytes) {
+  if ((m + 256) * n * 4 >= (int64_t(1) << 32)) return 1;
+  const int64_t fit = max_bytes / (m * n * 4);
+  return choose(m, n, k, EPI_PART, int(fit < 1 ? 1 : fit > 8 ? 8 : fit)).slices;
+}
+
+int gemm_mfma_part(const void* a, const void* bt, float* parts, int64_t m, int64_t n, int64_t k, int slices, int dtype, void* stream) {
+  Params p{};
+  p.a = a; p.bt = bt; p.c = parts;
+  p.m = int(m); p.n = int(n); p.k = int(k);
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  const Choice ch = choose(m, n, k, EPI_PART, slices);
+  if (ch.slices != slices) return rt::fail(RT_EINVAL, "gemm: %d slices asked for, %d chosen", slices, ch.slices);
+  return dtype == RT_F16 ? dispatch<_Float16, EPI_PART>(p, ch, st) : dispatch<__bf16, EPI_PART>(p, ch, st);
 }
 
 }  // namespace rt

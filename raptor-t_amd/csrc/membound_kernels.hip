@@ -203,6 +203,115 @@ int ln_dispatch(void* out, const void* res, const void* bias, const void* gamma,
   return RT_OK;
 }
 
+// ---- the same, with the first operand as fp32 slices of a product -----------------------------------------------------
+// out = LN(sum of parts[s] + bias + residual): what a product cut along its reduction leaves (gemm_mfma.hip) is added
+// up where it is read anyway.  Such products have few rows (at most a few thousand), so a whole wave takes a row and
+// requests every slice of it before it waits; 4 consecutive columns per lane and trip, hidden = CH * 256.
+template <typename T> struct Quad;            // 4 elements of a 16-bit type
+template <> struct Quad<__half> {
+  __device__ static void load(const __half* p, float* f) {
+    const uint2 r = *reinterpret_cast<const uint2*>(p);
+    const __half2* h = reinterpret_cast<const __half2*>(&r);
+    const float2 a = __half22float2(h[0]), b = __half22float2(h[1]);
+    f[0] = a.x; f[1] = a.y; f[2] = b.x; f[3] = b.y;
+  }
+  __device__ static void store(__half* p, const float* f) {
+    uint2 r;
+    __half2* h = reinterpret_cast<__half2*>(&r);
+    h[0] = __floats2half2_rn(f[0], f[1]);
+    h[1] = __floats2half2_rn(f[2], f[3]);
+    *reinterpret_cast<uint2*>(p) = r;
+  }
+};
+template <> struct Quad<__hip_bfloat16> {
+  __device__ static void load(const __hip_bfloat16* p, float* f) {
+    const uint2 r = *reinterpret_cast<const uint2*>(p);
+    f[0] = __uint_as_float(r.x << 16); f[1] = __uint_as_float(r.x & 0xffff0000u);
+    f[2] = __uint_as_float(r.y << 16); f[3] = __uint_as_float(r.y & 0xffff0000u);
+  }
+  __device__ static void store(__hip_bfloat16* p, const float* f) {
+    *reinterpret_cast<uint2*>(p) = make_uint2(Vec<__hip_bfloat16>::pack2(f[0], f[1]), Vec<__hip_bfloat16>::pack2(f[2], f[3]));
+  }
+};
+
+template <typename T, int CH>
+__global__ __launch_bounds__(256) void slices_residual_layernorm_kernel(T* __restrict__ out, const float* __restrict__ parts,
+                                                                        int n_parts, const T* __restrict__ residual,
+                                                                        const T* __restrict__ bias, const T* __restrict__ gamma,
+                                                                        const T* __restrict__ beta, int64_t rows, float eps) {
+  constexpr int HIDDEN = CH * 256;
+  const int lane = threadIdx.x & 63;
+  const int64_t row = int64_t(blockIdx.x) * 4 + (threadIdx.x >> 6);
+  if (row >= rows) return;
+  const int64_t slice = rows * HIDDEN;
+  const float* src = parts + row * HIDDEN + lane * 4;
+  float x[CH][4];
+#pragma unroll
+  for (int c = 0; c < CH; ++c) {
+    float r[4], b[4];
+    Quad<T>::load(residual + row * HIDDEN + c * 256 + lane * 4, r);
+    Quad<T>::load(bias + c * 256 + lane * 4, b);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) x[c][i] = r[i] + b[i];
+  }
+  int s = 0;
+  for (; s + 4 <= n_parts; s += 4) {
+    float4 v[4][CH];
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int c = 0; c < CH; ++c) v[u][c] = *reinterpret_cast<const float4*>(src + (s + u) * slice + c * 256);
+#pragma unroll
+    for (int c = 0; c < CH; ++c) {
+      x[c][0] += (v[0][c].x + v[1][c].x) + (v[2][c].x + v[3][c].x);
+      x[c][1] += (v[0][c].y + v[1][c].y) + (v[2][c].y + v[3][c].y);
+      x[c][2] += (v[0][c].z + v[1][c].z) + (v[2][c].z + v[3][c].z);
+      x[c][3] += (v[0][c].w + v[1][c].w) + (v[2][c].w + v[3][c].w);
+    }
+  }
+#pragma unroll 3
+  for (; s < n_parts; ++s)
+#pragma unroll
+    for (int c = 0; c < CH; ++c) {
+      const float4 v = *reinterpret_cast<const float4*>(src + s * slice + c * 256);
+      x[c][0] += v.x; x[c][1] += v.y; x[c][2] += v.z; x[c][3] += v.w;
+    }
+  float sum = 0.f;
+#pragma unroll
+  for (int c = 0; c < CH; ++c) sum += (x[c][0] + x[c][1]) + (x[c][2] + x[c][3]);
+  const float mean = group_sum<64>(sum) * (1.0f / HIDDEN);
+  float sq = 0.f;
+#pragma unroll
+  for (int c = 0; c < CH; ++c)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) { const float t = x[c][i] - mean; sq += t * t; }
+  const float rstd = rsqrtf(group_sum<64>(sq) * (1.0f / HIDDEN) + eps);
+#pragma unroll
+  for (int c = 0; c < CH; ++c) {
+    float g[4], b[4], y[4];
+    Quad<T>::load(gamma + c * 256 + lane * 4, g);
+    Quad<T>::load(beta + c * 256 + lane * 4, b);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) y[i] = (x[c][i] - mean) * rstd * g[i] + b[i];
+    Quad<T>::store(out + row * HIDDEN + c * 256 + lane * 4, y);
+  }
+}
+
+template <typename T>
+bool slices_ln_dispatch(void* out, const float* parts, int n_parts, const void* res, const void* bias, const void* gamma,
+                        const void* beta, int64_t rows, int hidden, float eps, hipStream_t st) {
+  T* o = static_cast<T*>(out);
+  const T *r = static_cast<const T*>(res), *b = static_cast<const T*>(bias), *g = static_cast<const T*>(gamma),
+          *be = static_cast<const T*>(beta);
+  const dim3 grid(unsigned((rows + 3) / 4));
+#define RT_SLICES_LN(CH) case CH: RT_LAUNCH((slices_residual_layernorm_kernel<T, CH>), grid, dim3(256), 0, st, o, parts, n_parts, r, b, g, be, rows, eps); return true;
+  switch (hidden % 256 == 0 ? hidden / 256 : 0) {
+    RT_SLICES_LN(1) RT_SLICES_LN(2) RT_SLICES_LN(3) RT_SLICES_LN(4)
+    default: return false;
+  }
+#undef RT_SLICES_LN
+}
+
 // ---- embedding gather + LayerNorm ---------------------------------------------------------
 // out[t] = LN(word[ids[t]] + position[pos_ids[t]] + type[type_ids[t]]) * gamma + beta, written in
 // the encoder's dtype.  Tables, gamma and beta are of type TT (fp32 as the reference keeps them,
@@ -629,6 +738,21 @@ int rt_bias_residual_layernorm(void* out, const void* residual, const void* bias
   else if (dtype == RT_BF16) ln_dispatch<__hip_bfloat16>(out, residual, bias, gamma, beta, rows, hidden, eps, st);
   else ln_dispatch<float>(out, residual, bias, gamma, beta, rows, hidden, eps, st);
   return check_launch("bias_residual_layernorm");
+}
+
+int rt_slices_residual_layernorm(void* out, const float* parts, int n_parts, const void* residual, const void* bias,
+                                 const void* gamma, const void* beta, int64_t rows, int hidden, float eps, int dtype, void* stream) {
+  RT_REQUIRE(out && parts && residual && bias && gamma && beta, RT_EINVAL, "NULL pointer");
+  RT_REQUIRE(rows >= 0 && rows < (int64_t(1) << 31) && n_parts >= 1, RT_EINVAL, "rows=%lld or n_parts=%d out of range", (long long)rows, n_parts);
+  RT_REQUIRE(dtype == RT_F16 || dtype == RT_BF16, RT_EINVAL, "dtype %d is not a 16-bit type", dtype);
+  RT_REQUIRE(aligned16(out) && aligned16(parts) && aligned16(residual) && aligned16(bias) && aligned16(gamma) && aligned16(beta),
+             RT_EINVAL, "pointers must be 16-byte aligned");
+  RT_REQUIRE(hidden == 256 || hidden == 512 || hidden == 768 || hidden == 1024, RT_EINVAL, "hidden=%d must be 256, 512, 768 or 1024", hidden);
+  if (rows == 0) return RT_OK;
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  if (dtype == RT_F16) slices_ln_dispatch<__half>(out, parts, n_parts, residual, bias, gamma, beta, rows, hidden, eps, st);
+  else slices_ln_dispatch<__hip_bfloat16>(out, parts, n_parts, residual, bias, gamma, beta, rows, hidden, eps, st);
+  return check_launch("slices_residual_layernorm");
 }
 
 int rt_bias_gelu(void* out, const void* bias, int64_t rows, int width, int dtype, void* stream) {

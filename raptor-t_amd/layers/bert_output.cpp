@@ -19,11 +19,9 @@ BertOutput::BertOutput(torch::Tensor dense_weight, torch::Tensor dense_bias, tor
 std::map<std::string, float> BertOutput::operator()(const torch::Tensor& hidden_states, const torch::Tensor& input_tensor,
                                                     torch::Tensor& output_tensor, std::map<std::string, float>& info,
                                                     bool kernel_fusion) const {
-  kernels::MatMul(hidden_states, false, dense_weight_, true, 1.0, output_tensor, 0.0, kernels::shared_gemm_handle(),
-                  "BertOutput");
-  const int seq_len = int(input_tensor.size(0));
-  kernels::add_bias_and_layernorm_kernel(output_tensor, input_tensor, dense_bias_, seq_len, int(dense_weight_.size(0)),
-                                         eps_, layer_norm_weight_, layer_norm_bias_, info, kernel_fusion);
+  kernels::MatMulLayerNorm(hidden_states, dense_weight_, output_tensor, input_tensor, dense_bias_, int(input_tensor.size(0)),
+                           int(dense_weight_.size(0)), eps_, layer_norm_weight_, layer_norm_bias_,
+                           kernels::shared_gemm_handle(), info, kernel_fusion, "BertOutput");
   return info;
 }
 

@@ -393,25 +393,29 @@ void add_bias_and_transpose_kernel(const torch::Tensor& bias, torch::Tensor& inp
   }
 }
 
+static void check_layernorm_arguments(const torch::Tensor& out, const torch::Tensor& input_data, const torch::Tensor& bias,
+                                      int seq_len, int normalized_len, const torch::Tensor& layernorm_weight,
+                                      const torch::Tensor& layernorm_bias) {
+  if (seq_len < 0 || normalized_len < 1) throw std::invalid_argument("add_bias_and_layernorm_kernel: bad seq_len / width");
+  require_cuda_contiguous(out, "out");
+  const torch::ScalarType dt = out.scalar_type();
+  const int64_t n = int64_t(seq_len) * normalized_len;
+  if (out.numel() != n)
+    throw std::invalid_argument("add_bias_and_layernorm_kernel: out holds " + std::to_string(out.numel()) +
+                                " elements, seq_len x width is " + std::to_string(n));
+  require_data(input_data, "residual", dt, n);
+  if (input_data.numel() != n)
+    throw std::invalid_argument("add_bias_and_layernorm_kernel: the residual has other rows than out");
+  require_data(bias, "bias", dt, normalized_len);
+  require_data(layernorm_weight, "layernorm weight", dt, normalized_len);
+  require_data(layernorm_bias, "layernorm bias", dt, normalized_len);
+}
+
 void add_bias_and_layernorm_kernel(torch::Tensor& out, const torch::Tensor& input_data, const torch::Tensor& bias,
                                    int seq_len, int normalized_len, float eps, const torch::Tensor& layernorm_weight,
                                    const torch::Tensor& layernorm_bias, std::map<std::string, float>& info,
                                    bool kernel_fusion) {
-  if (seq_len < 0 || normalized_len < 1) throw std::invalid_argument("add_bias_and_layernorm_kernel: bad seq_len / width");
-  {
-    require_cuda_contiguous(out, "out");
-    const torch::ScalarType dt = out.scalar_type();
-    const int64_t n = int64_t(seq_len) * normalized_len;
-    if (out.numel() != n)
-      throw std::invalid_argument("add_bias_and_layernorm_kernel: out holds " + std::to_string(out.numel()) +
-                                  " elements, seq_len x width is " + std::to_string(n));
-    require_data(input_data, "residual", dt, n);
-    if (input_data.numel() != n)
-      throw std::invalid_argument("add_bias_and_layernorm_kernel: the residual has other rows than out");
-    require_data(bias, "bias", dt, normalized_len);
-    require_data(layernorm_weight, "layernorm weight", dt, normalized_len);
-    require_data(layernorm_bias, "layernorm bias", dt, normalized_len);
-  }
+  check_layernorm_arguments(out, input_data, bias, seq_len, normalized_len, layernorm_weight, layernorm_bias);
   ScopedGpuTimer timer(info, "add_bias_and_layernorm_kernel", kernel_fusion);
   if (kernel_fusion) {
     check(rt_bias_residual_layernorm(out.data_ptr(), input_data.data_ptr(), bias.data_ptr(),
@@ -422,6 +426,44 @@ void add_bias_and_layernorm_kernel(torch::Tensor& out, const torch::Tensor& inpu
   // Unfused: three library launches (add_bias_and_layernorm.cu:276-279)
   out.add_(input_data).add_(bias);
   out.copy_(torch::layer_norm(out, {normalized_len}, layernorm_weight, layernorm_bias, eps));
+}
+
+void MatMulLayerNorm(const torch::Tensor& A, const torch::Tensor& B, torch::Tensor& out, const torch::Tensor& input_data,
+                     const torch::Tensor& bias, int seq_len, int normalized_len, float eps, const torch::Tensor& layernorm_weight,
+                     const torch::Tensor& layernorm_bias, rt_gemm_ctx* handle, std::map<std::string, float>& info,
+                     bool kernel_fusion, const std::string& name) {
+  if (kernel_fusion && A.scalar_type() != torch::kFloat) {
+    check_layernorm_arguments(out, input_data, bias, seq_len, normalized_len, layernorm_weight, layernorm_bias);
+    const torch::ScalarType dt = out.scalar_type();
+    if (A.dim() != 2 || B.dim() != 2 || A.size(0) != seq_len || B.size(0) != normalized_len || B.size(1) != A.size(1))
+      throw std::invalid_argument(name + ": shape mismatch");
+    require_data(A, "A", dt, A.size(0) * A.size(1));
+    require_data(B, "B", dt, B.size(0) * B.size(1));
+    const float* parts = nullptr;
+    int n_parts = 0;
+    {
+      static std::map<std::string, float> no_info;
+      ScopedGpuTimer timer(no_info, "MatMul");
+      check(rt_gemm_bt_slices(handle, A.data_ptr(), B.data_ptr(), seq_len, normalized_len, A.size(1), dtype_code(A), &parts,
+                              &n_parts, current_stream()), name.c_str());
+      if (n_parts == 0)
+        check(rt_gemm_bt(handle, A.data_ptr(), B.data_ptr(), nullptr, out.data_ptr(), seq_len, normalized_len, A.size(1),
+                         RT_EPILOGUE_NONE, dtype_code(A), current_stream()), name.c_str());
+    }
+    ScopedGpuTimer timer(info, "add_bias_and_layernorm_kernel", true);
+    if (n_parts)
+      check(rt_slices_residual_layernorm(out.data_ptr(), parts, n_parts, input_data.data_ptr(), bias.data_ptr(),
+                                         layernorm_weight.data_ptr(), layernorm_bias.data_ptr(), seq_len, normalized_len, eps,
+                                         dtype_code(out), current_stream()), "rt_slices_residual_layernorm");
+    else
+      check(rt_bias_residual_layernorm(out.data_ptr(), input_data.data_ptr(), bias.data_ptr(), layernorm_weight.data_ptr(),
+                                       layernorm_bias.data_ptr(), seq_len, normalized_len, eps, dtype_code(out),
+                                       current_stream()), "rt_bias_residual_layernorm");
+    return;
+  }
+  MatMul(A, false, B, true, 1, out, 0, handle, name);
+  add_bias_and_layernorm_kernel(out, input_data, bias, seq_len, normalized_len, eps, layernorm_weight, layernorm_bias, info,
+                                kernel_fusion);
 }
 
 void add_bias_act_kernel(const torch::Tensor& bias, torch::Tensor& out, int total_seq_len, int dim_size,

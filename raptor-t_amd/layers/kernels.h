@@ -121,6 +121,14 @@ void add_bias_and_layernorm_kernel(torch::Tensor& out, const torch::Tensor& inpu
                                    const torch::Tensor& layernorm_bias, std::map<std::string, float>& info,
                                    bool kernel_fusion);
 
+// MatMul(A, B^T) into `out` followed by add_bias_and_layernorm_kernel: the pair that ends both halves of a layer.  With
+// kernel_fusion a product of few rows is cut into slices of its reduction, which the LayerNorm kernel adds up as it
+// reads them (rt_gemm_bt_slices); `out` is then written once.
+void MatMulLayerNorm(const torch::Tensor& A, const torch::Tensor& B, torch::Tensor& out, const torch::Tensor& input_data,
+                     const torch::Tensor& bias, int seq_len, int normalized_len, float eps, const torch::Tensor& layernorm_weight,
+                     const torch::Tensor& layernorm_bias, rt_gemm_ctx* handle, std::map<std::string, float>& info,
+                     bool kernel_fusion, const std::string& name);
+
 // layers/kernels/add_bias_act.cu:114-133
 void add_bias_act_kernel(const torch::Tensor& bias, torch::Tensor& out, int total_seq_len, int dim_size,
                          std::map<std::string, float>& info, bool kernel_fusion);

@@ -134,9 +134,8 @@ void MultiHeadedAttention::operator()(const torch::Tensor& input_tensor, const t
                             q_rows && !bias_in_projection(kernel_fusion) ? qkv_bias_ : torch::Tensor());
   semaphore->Release(layer_idx_, stream);
 
-  kernels::MatMul(attention_out, false, dense_weight_, true, 1, output, 0, handle_, "Attention Output");
-  kernels::add_bias_and_layernorm_kernel(output, input_tensor, dense_bias_, total_seq_len_, d_num_, eps_,
-                                         layernorm_gamma_, layernorm_beta_, info, kernel_fusion);
+  kernels::MatMulLayerNorm(attention_out, dense_weight_, output, input_tensor, dense_bias_, total_seq_len_, d_num_, eps_,
+                           layernorm_gamma_, layernorm_beta_, handle_, info, kernel_fusion, "Attention Output");
 }
 
 }  // namespace layers

@@ -46,6 +46,13 @@ def check(got, a, b, bias, gelu, dtype):
     (12295, 264, 192, torch.bfloat16),      # odd number of steps; 8 columns and 7 rows in tiles of their own
     (9409, 520, 768, torch.float16),        # tiles of 224 rows: one row in the last
     (16384 + 33, 1000, 256, torch.bfloat16),
+    (1, 8, 128, torch.float16),             # one row, one chunk of columns
+    (64, 768, 3072, torch.bfloat16),        # tiles of 64 x 64
+    (333, 776, 768, torch.float16),
+    (700, 2312, 192, torch.float16),        # tiles of 128 x 64
+    (1500, 2304, 768, torch.bfloat16),      # 128 x 128
+    (2049, 3080, 320, torch.float16),       # 256 x 128
+    (5600, 768, 1024, torch.bfloat16),      # 192 x 128
 ])
 @pytest.mark.parametrize("epilogue", [0, 1, 2])
 def test_gemm_bt_edges(capi, m, n, k, dtype, epilogue):
@@ -61,6 +68,10 @@ def test_gemm_bt_edges(capi, m, n, k, dtype, epilogue):
     (12, [832, 64, 3008, 1024], torch.float16),
     (5, [64] * 70 + [2048], torch.bfloat16),          # more sequences than one wave looks up at a time, K and V halves of a tile
     (16, [4096, 320], torch.float16),
+    (2, [64], torch.float16),                         # half a tile of 128 x 64
+    (12, [192, 320], torch.bfloat16),
+    (7, [960, 576], torch.float16),                   # 128 x 128
+    (12, [2048, 1088], torch.bfloat16),               # 256 x 128
 ])
 def test_qkv_project_equals_gemm_and_split(capi, heads, seq_lens, dtype):
     print("qkv_project", heads, len(seq_lens), dtype, flush=True)
@@ -75,3 +86,44 @@ def test_qkv_project_equals_gemm_and_split(capi, heads, seq_lens, dtype):
     capi.qkv_bias_split(rows2, None, None, k2, vt2, sb, heads, 1.0)
     assert torch.equal(rows[:, :d], rows2[:, :d]) and torch.equal(k, k2) and torch.equal(vt, vt2)
     assert bool((rows[:, d:] == 7.0).all())            # only the queries' columns are written
+
+
+@pytest.mark.parametrize("m,n,k,dtype", [
+    (1, 256, 768, torch.float16),
+    (64, 768, 3072, torch.bfloat16),                  # eight slices
+    (515, 768, 3072, torch.float16),
+    (1500, 1024, 4096, torch.bfloat16),
+    (2816, 768, 3072, torch.float16),
+    (1000, 512, 448, torch.float16),                  # seven steps
+    (64, 320, 1280, torch.float16),                   # a width the slices' LayerNorm does not have
+    (9000, 768, 768, torch.float16),                  # enough rows: not cut
+])
+def test_gemm_bt_layernorm(capi, m, n, k, dtype):
+    """rt_gemm_bt_slices + rt_slices_residual_layernorm against fp32.  The LayerNorm's input x is a sum of the product
+    (error of an fp32 sum as in check(); uncut, the product is also rounded to the stored type), bias and residual; an
+    error e of an element moves the output by at most e * gamma / std plus the shift of mean and variance by the row's
+    errors, less than as much again."""
+    print("gemm_bt_layernorm", m, n, k, dtype, flush=True)
+    a, b, bias = operands(m, n, k, dtype, seed=2)
+    g = torch.Generator(device="cuda").manual_seed(3)
+    res, gamma, beta = (torch.randn(*s, generator=g, device="cuda").to(dtype) for s in ((m, n), (n,), (n,)))
+    out = torch.full((m + 1, n), 7.0, dtype=dtype, device="cuda")
+    slices = capi.Gemm().bt_layernorm(a, b, bias, res, gamma, beta, out[:m], 1e-5)
+    print("  slices", slices, flush=True)
+    if n == 320 or m == 9000:
+        assert slices == 0
+    elif k >= 3072:
+        assert slices > 1
+    prod = a.float() @ b.float().t()
+    err = 2.0 ** -23 * k * (a.float().abs() @ b.float().abs().t())
+    if slices == 0:
+        err = err + 2.0 ** -(BITS[dtype] + 1) * prod.abs()
+    x = prod + bias.float() + res.float()
+    std = (x.var(dim=1, unbiased=False, keepdim=True) + 1e-5).sqrt()
+    want = (x - x.mean(dim=1, keepdim=True)) / std * gamma.float() + beta.float()
+    ulp = torch.exp2(torch.floor(torch.log2(want.abs().clamp_min(2.0 ** -14))) - BITS[dtype])
+    row = err.amax(dim=1, keepdim=True) / std
+    bound = 0.51 * ulp + row * (2 * gamma.float().abs() + (want - beta.float()).abs()) + 2.0 ** -18 * (want.abs() + 1)
+    over = ((out[:m].float() - want).abs() - bound).max().item()
+    assert over <= 0, over
+    assert bool((out[m] == 7.0).all())
