@@ -843,6 +843,37 @@ __device__ inline bool run_solo(const Args<T>& a, const Buffers<T>& b, const QSi
   return true;
 }
 
+// A wave's softmax state in LDS, and the merge of a parked state into the wave's own.
+constexpr int PARK_FLOATS = 68 * 64;
+__device__ inline void park_state(const State& st, float* slot, int lane) {
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int nt = 0; nt < 2; ++nt)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) slot[((t * 2 + nt) * 16 + e) * 64 + lane] = st.o[t][nt][e];
+#pragma unroll
+  for (int nt = 0; nt < 2; ++nt) {
+    slot[(64 + nt) * 64 + lane] = st.m[nt];
+    slot[(66 + nt) * 64 + lane] = st.l[nt];
+  }
+}
+__device__ inline void absorb_state(State& st, const float* slot, int lane) {
+#pragma unroll
+  for (int nt = 0; nt < 2; ++nt) {
+    const float m1 = slot[(64 + nt) * 64 + lane], l1 = slot[(66 + nt) * 64 + lane];
+    const float mt = fmaxf(fmaxf(st.m[nt], m1), -1e30f);        // finite even if both are empty
+    const float a0 = __builtin_amdgcn_exp2f(st.m[nt] - mt), a1 = __builtin_amdgcn_exp2f(m1 - mt);
+    st.m[nt] = mt;
+    st.l[nt] = st.l[nt] * a0 + l1 * a1;
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int e = 0; e < 16; ++e)
+        st.o[t][nt][e] = st.o[t][nt][e] * a0 + slot[((t * 2 + nt) * 16 + e) * 64 + lane] * a1;
+  }
+}
+
 // Four waves, one unit: wave w streams key blocks w, w+4, ...; tree merge through LDS.  FAST:
 // pipelined loop; false (the same in all four waves) = the unit has to be run again with FAST = false.
 template <typename T, bool MASKED, bool FAST>
@@ -861,42 +892,14 @@ __device__ inline bool run_split4(const Args<T>& a, const Buffers<T>& b, const Q
 #pragma unroll
   for (int nt = 0; nt < 2; ++nt) st.l[nt] = pair_sum(st.l[nt]);
 
-  auto dump = [&](float* slot) {
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-      for (int nt = 0; nt < 2; ++nt)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) slot[((t * 2 + nt) * 16 + e) * 64 + lane] = st.o[t][nt][e];
-#pragma unroll
-    for (int nt = 0; nt < 2; ++nt) {
-      slot[(64 + nt) * 64 + lane] = st.m[nt];
-      slot[(66 + nt) * 64 + lane] = st.l[nt];
-    }
-  };
-  auto absorb = [&](const float* slot) {
-#pragma unroll
-    for (int nt = 0; nt < 2; ++nt) {
-      const float m1 = slot[(64 + nt) * 64 + lane], l1 = slot[(66 + nt) * 64 + lane];
-      const float mt = fmaxf(fmaxf(st.m[nt], m1), -1e30f);        // finite even if both are empty
-      const float a0 = __builtin_amdgcn_exp2f(st.m[nt] - mt), a1 = __builtin_amdgcn_exp2f(m1 - mt);
-      st.m[nt] = mt;
-      st.l[nt] = st.l[nt] * a0 + l1 * a1;
-#pragma unroll
-      for (int t = 0; t < 2; ++t)
-#pragma unroll
-        for (int e = 0; e < 16; ++e)
-          st.o[t][nt][e] = st.o[t][nt][e] * a0 + slot[((t * 2 + nt) * 16 + e) * 64 + lane] * a1;
-    }
-  };
-  if (wave >= 2) dump(park + (wave - 2) * (68 * 64));
+  if (wave >= 2) park_state(st, park + (wave - 2) * PARK_FLOATS, lane);
   __syncthreads();
-  if (wave < 2) absorb(park + wave * (68 * 64));
+  if (wave < 2) absorb_state(st, park + wave * PARK_FLOATS, lane);
   __syncthreads();
-  if (wave == 1) dump(park);
+  if (wave == 1) park_state(st, park, lane);
   __syncthreads();
   if (wave == 0) {
-    absorb(park);
+    absorb_state(st, park, lane);
     float w[2];
 #pragma unroll
     for (int nt = 0; nt < 2; ++nt) w[nt] = __builtin_amdgcn_rcpf(fmaxf(st.l[nt], 1e-30f));
@@ -925,7 +928,7 @@ template <typename T, bool MASKED>
 __global__ __launch_bounds__(256, 2) void bs_attention_kernel(Args<T> a) {
   // 36864 bytes with two uses that never overlap in time: two parked wave states (2 x 17408 bytes) of the merge
   // that ends a row shared by the four waves, and each wave's room for a query tile in row order (finish_q)
-  static_assert(4 * Q_STAGE_BYTES >= 2 * 68 * 64 * int(sizeof(float)), "the park must hold two wave states");
+  static_assert(4 * Q_STAGE_BYTES >= 2 * PARK_FLOATS * int(sizeof(float)), "the park must hold two wave states");
   __shared__ __attribute__((aligned(16))) float park[4 * Q_STAGE_BYTES / 4];
   __shared__ Geometry geo;
   __shared__ __attribute__((aligned(16))) T qbias_lds[MAX_HEADS_QROWS * 64];
@@ -1286,6 +1289,128 @@ __global__ __launch_bounds__(256, 2) void bs_attention_kernel(Args<T> a) {
   }
 }
 
+// ---- batches with few units --------------------------------------------------------------------------------------------
+// Where the persistent kernel would leave most waves of the chip without a unit, its time is one unit's chain of tiles
+// (8 tiles, 13 us) or a global row's (a quarter of the sequence's blocks).  Here a unit's tiles are shared by several waves,
+// whose states merge through LDS: one workgroup of 8 waves (one per CU) takes one global row, or RPW other rows with
+// 8 / RPW waves each (rows_per_workgroup has the rule and the times of both kernels).  Nothing
+// persists and nothing is drawn: workgroup b looks its rows up from the batch's prefix, XCD x taking the x-th eighth of the
+// global rows and of the rest, both head-major, as the persistent kernel does.  With a caller's plan a workgroup takes one
+// unit of the list; the waves share it in the same way, so both give the same bits.  At most 64 sequences (a lane each).
+template <typename T, bool MASKED, int RPW>
+__global__ __launch_bounds__(512, 2) void bs_attention_few_kernel(Args<T> a, int n_wg) {
+  constexpr int WAVES_PER_ROW = 8 / RPW;
+  static_assert(8 * Q_STAGE_BYTES >= 4 * PARK_FLOATS * int(sizeof(float)), "the park must hold four wave states");
+  __shared__ __attribute__((aligned(16))) float park[8 * Q_STAGE_BYTES / 4];
+  __shared__ __attribute__((aligned(16))) T qbias_lds[MAX_HEADS_QROWS * 64];
+  __shared__ int failed[8];                            // per row: a wave's pipelined loop handed it back
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const QSide<T> qbias{qbias_lds, reinterpret_cast<char*>(park) + wave * Q_STAGE_BYTES};
+  // lane l: sequence l
+  const int sb0 = a.seq_blocks[min(lane, a.batch)], sb1 = a.seq_blocks[min(lane + 1, a.batch)];
+  if (a.q_rows)
+    for (int i = threadIdx.x; i < a.heads * 64; i += 512) qbias_lds[i] = a.q_bias ? a.q_bias[i] : static_cast<T>(0.f);
+  if (threadIdx.x < 8) failed[threadIdx.x] = 0;
+  const unsigned long long sparse = __ballot(lane < a.batch && sb1 - sb0 >= RT_MIN_SPARSE_BLOCKS);
+  const int n_sparse = __popcll(sparse), n_rows = a.nb_total - 2 * n_sparse;
+  const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
+
+  auto unit_at = [&](int s, int h, int i) {
+    Unit u;
+    u.g0 = __builtin_amdgcn_readlane(sb0, s);
+    u.n = __builtin_amdgcn_readlane(sb1, s) - u.g0;
+    u.h = h;
+    u.i = i;
+    u.tail = 64;
+    u.nbv = u.n;
+    if (MASKED) {
+      const int tokens = min(max(__builtin_amdgcn_readfirstlane(a.seq_tokens[s]), 1), 64 * u.n);
+      u.nbv = (tokens + 63) >> 6;
+      u.tail = tokens - 64 * (u.nbv - 1);
+    }
+    return u;
+  };
+  // sequence of a position in a per-lane ascending prefix (lane s: first position of sequence s)
+  auto seq_of = [&](int prefix, int x) { return __popcll(__ballot(lane < a.batch && prefix <= x)) - 1; };
+
+  Unit u;
+  bool valid = true, whole = false;                    // whole: all eight waves share one row
+  if (a.from_pos) {
+    const int n_units = a.nb_total * a.heads;
+    const int begin = min(max(a.from_pos[0], 0), n_units), end = min(max(a.from_pos[n_wg], begin), n_units);
+    if (begin + int(blockIdx.x) >= end) return;
+    const int id = __builtin_amdgcn_readfirstlane(a.from_idx[begin + int(blockIdx.x)]);
+    if (id < 0 || id >= n_units) return;
+    const int s = seq_of(sb0 * a.heads, id), g0 = __builtin_amdgcn_readlane(sb0, s), n = __builtin_amdgcn_readlane(sb1, s) - g0;
+    const int rem = id - g0 * a.heads, h = rem / n;
+    u = unit_at(s, h, rem - h * n);
+    whole = is_global_row(u);
+    valid = whole || wave < WAVES_PER_ROW;
+  } else {
+    const int n_pairs = n_sparse * a.heads;
+    const int p_lo = int(int64_t(n_pairs) * xcd / 8), p_hi = int(int64_t(n_pairs) * (xcd + 1) / 8), n_glob = 2 * (p_hi - p_lo);
+    whole = slot < n_glob;
+    if (whole) {
+      const int pair = p_lo + (slot >> 1), h = pair / n_sparse, k = pair - h * n_sparse;
+      // the k-th sparse sequence
+      const int s = __builtin_ctzll(__ballot((sparse >> lane & 1ull) && __popcll(sparse & ((1ull << lane) - 1ull)) == k));
+      u = unit_at(s, h, 0);
+      if (slot & 1) u.i = u.n - 1;
+    } else {
+      const int total = n_rows * a.heads;
+      const int lo = int(int64_t(total) * xcd / 8), hi = int(int64_t(total) * (xcd + 1) / 8);
+      const int first = lo + (slot - n_glob) * RPW;
+      if (first >= hi) return;
+      const int item = first + wave / WAVES_PER_ROW;
+      valid = item < hi;
+      const int it = valid ? item : first, h = it / n_rows, j = it - h * n_rows;
+      const int listed_before = sb0 - 2 * __popcll(sparse & ((1ull << lane) - 1ull));       // rows of earlier sequences
+      const int s = seq_of(listed_before, j);
+      u = unit_at(s, h, 0);
+      u.i = j - __builtin_amdgcn_readlane(listed_before, s) + ((sparse >> s & 1ull) ? 1 : 0);
+    }
+  }
+  __syncthreads();
+
+  Buffers<T> b;
+  {
+    const uint32_t kv_bytes = uint32_t(a.nb_total) * uint32_t(a.heads) * 8192u;
+    b.k = __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(a.k), 0, kv_bytes, 0x00020000);
+    b.v = __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(a.vt), 0, kv_bytes, 0x00020000);
+    b.q = a.q_rows ? __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(a.q_rows), 0, kv_bytes * 3u, 0x00020000)
+                   : __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(a.q), 0, kv_bytes, 0x00020000);
+  }
+  const int share = whole ? 8 : WAVES_PER_ROW, row = wave / share, part = wave - row * share;
+  const Row r = describe<T>(a, u);
+  State st;
+  state_init(st);
+  if (valid && !fast_row<T, MASKED>(a, b, qbias, r, part, share, lane, st) && lane == 0) failed[row] = 1;
+  __syncthreads();                                     // the query rooms are read
+  if (valid && failed[row]) {
+    typename Mma<T>::v8 qf[2][4];
+    slow_row<T, MASKED>(a, b, qbias, r, part, share, lane, false, qf, st);
+  }
+#pragma unroll
+  for (int nt = 0; nt < 2; ++nt) st.l[nt] = pair_sum(st.l[nt]);
+#pragma unroll
+  for (int half = 4; half >= 1; half >>= 1) {
+    if (2 * half > WAVES_PER_ROW && !whole) continue;
+    __syncthreads();                                   // the park is free
+    float* const place = park + (row * half + (part & (half - 1))) * PARK_FLOATS;
+    if (part >= half && part < 2 * half) park_state(st, place, lane);
+    __syncthreads();
+    if (part < half) absorb_state(st, place, lane);
+  }
+  __syncthreads();
+  if (valid && part == 0) {
+    float w[2];
+#pragma unroll
+    for (int nt = 0; nt < 2; ++nt) w[nt] = __builtin_amdgcn_rcpf(fmaxf(st.l[nt], 1e-30f));
+    const int64_t stride = int64_t(a.heads) * 64;
+    store_output<T>(a.out + int64_t(u.g0 + u.i) * 64 * stride + u.h * 64, stride, lane, st, w, qbias.stage);
+  }
+}
+
 // Two persistent workgroups per CU, a multiple of 8 so that every XCD gets the same number.
 unsigned plan_free_workgroups() {
   static unsigned cached = 0;
@@ -1325,6 +1450,49 @@ int* library_queues(int* err) {
 
 namespace {
 
+// Pairs of global rows the batch can have at most: the host knows the block count, not the sequences' lengths.
+int64_t most_pairs(int batch, int total_blocks, int heads) {
+  const int sparse = total_blocks / RT_MIN_SPARSE_BLOCKS;
+  return int64_t(sparse < batch ? sparse : batch) * heads;
+}
+
+// Rows that share a workgroup of bs_attention_few_kernel, as few as still give every workgroup a CU of its own and every
+// wave a tile (1 x 64 tokens: 6.7, 7.1, 5.7, 4.3 us with 1, 2, 4, 8; persistent kernel 13.2); 0: the persistent kernel.
+// Measured (us, 12 heads, persistent kernel / this one with 1, 2, 4, 8 rows to a workgroup): 1 x 512
+// tokens 18.2 / 8.1, 9.0, 10.5, 13.3; 1 x 2048 19.7 / 16.0, 12.3, 12.3, 14.0; 4 x 256-1024 22.5 / 23.1, 18.3, 13.1,
+// 16.7; 1 x 4096 25.6 / 29.5, 18.5, 17.7, 17.2; 8 x 150-1700 27.5 / 34.7, 26.8, 23.1, 16.8; 2 x 4096 35.4 / -, -, 25.9,
+// 22.7; 6 x 2048 42.0 / -, -, 40.9, 35.9.  From 3072 units on (16 heads, 6 x 2048: 50.9 / 51.5) a row is no longer the
+// shorter chain, and the persistent kernel's schedule is the better one.
+int rows_per_workgroup(int batch, int total_blocks, int heads) {
+  const int64_t units = int64_t(total_blocks) * heads;
+  if (batch > 64 || units > 2816) return 0;
+  const int64_t global = 2 * most_pairs(batch, total_blocks, heads);
+  const int longest = total_blocks - batch + 1;         // tiles that a row can have at most
+  for (int rows = 1; rows <= 4; rows *= 2)
+    if (8 / rows <= longest && global + (units - global + rows - 1) / rows <= 256) return rows;
+  return 8;
+}
+
+template <typename T> int launch_few(const Args<T>& a, int rpw, int n_wg, hipStream_t st) {
+  // every XCD's share of the global rows (two per head of each sequence that may have them) and of the others
+  const int64_t units = int64_t(a.nb_total) * a.heads, pairs = most_pairs(a.batch, a.nb_total, a.heads);
+  const int64_t per_xcd = 2 * ((pairs + 7) / 8) + ((units + 7) / 8 + rpw - 1) / rpw;
+  const dim3 grid(unsigned(a.from_pos ? units : 8 * per_xcd));
+  auto go = [&](auto masked, auto rows) {
+    RT_LAUNCH((bs_attention_few_kernel<T, decltype(masked)::value, decltype(rows)::value>), grid, dim3(512), 0, st, a, n_wg);
+  };
+  auto pick = [&](auto masked) {
+    if (rpw == 1) go(masked, std::integral_constant<int, 1>());
+    else if (rpw == 2) go(masked, std::integral_constant<int, 2>());
+    else if (rpw == 4) go(masked, std::integral_constant<int, 4>());
+    else go(masked, std::integral_constant<int, 8>());
+  };
+  if (a.seq_tokens) pick(std::true_type());
+  else pick(std::false_type());
+  const hipError_t e = hipGetLastError();
+  return e == hipSuccess ? RT_OK : rt::fail(RT_EIO, "bs_attention launch failed: %s", hipGetErrorString(e));
+}
+
 int launch_attention(const void* q, const void* q_rows, const void* q_bias, float q_scale, const void* k, const void* vt,
                      void* out, const int* seq_blocks_dev, const int* seq_tokens_dev, int batch, int total_blocks,
                      int heads, const int* to_idx, const int* to_pos, int plan_heads, const int* from_idx,
@@ -1350,10 +1518,21 @@ int launch_attention(const void* q, const void* q_rows, const void* q_bias, floa
     return rt::launch_attention_f32(q, q_rows, q_bias, q_scale, k, vt, out, seq_blocks_dev, seq_tokens_dev, batch,
                                     total_blocks, heads, to_idx, to_pos, plan_heads, from_idx, from_pos, n_wg, stream);
   }
+  RT_REQUIRE(!from_idx || n_wg >= 1, RT_EINVAL, "balanced launch needs n_wg >= 1, got %d", n_wg);
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  if (const int rpw = rows_per_workgroup(batch, total_blocks, heads)) {
+    auto few = [&](auto tag) {
+      typedef decltype(tag) T;
+      return launch_few(Args<T>{(const T*)q, (const T*)k, (const T*)vt, (T*)out, seq_blocks_dev, batch, heads, total_blocks, to_idx,
+                                to_pos, plan_heads, from_idx, from_pos, seq_tokens_dev, (const T*)q_rows, (const T*)q_bias,
+                                q_scale, nullptr},
+                        rpw, n_wg, st);
+    };
+    return dtype == RT_F16 ? few(_Float16()) : few(__bf16());
+  }
   unsigned grid;
   int* queues = nullptr;
   if (from_idx) {
-    RT_REQUIRE(n_wg >= 1, RT_EINVAL, "balanced launch needs n_wg >= 1, got %d", n_wg);
     grid = unsigned(n_wg);
   } else {
     grid = plan_free_workgroups();
@@ -1365,7 +1544,6 @@ int launch_attention(const void* q, const void* q_rows, const void* q_bias, floa
       if (!queues) return rt::fail(RT_ENOMEM, "no device memory for the work queues (step %d)", err);
     }
   }
-  hipStream_t st = static_cast<hipStream_t>(stream);
   if (dtype == RT_F16) {
     Args<_Float16> a{(const _Float16*)q, (const _Float16*)k, (const _Float16*)vt, (_Float16*)out, seq_blocks_dev, batch,
                      heads, total_blocks, to_idx, to_pos, plan_heads, from_idx, from_pos, seq_tokens_dev,
