@@ -308,8 +308,7 @@ int rt_gemm_bt(rt_gemm_ctx* ctx, const void* a, const void* bt, const void* bias
  * step is rt_slices_residual_layernorm: with few rows, cutting a long reduction is what gives every CU a share.
  * *n_parts = 0: the product is better not cut (or cannot be: hidden sizes other than 256 / 512 / 768 / 1024), nothing
  * was launched, use rt_gemm_bt + rt_bias_residual_layernorm.  Otherwise the slices parts[n_parts][m][n] are being
- * written on `stream`, in a workspace of the context (32 MiB, allocated the first time): they are valid until the next
- * call on the context. */
+ * written on `stream`, in a workspace of the context (32 MiB): they are valid until the next call on the context. */
 int rt_gemm_bt_slices(rt_gemm_ctx* ctx, const void* a, const void* bt, int64_t m, int64_t n, int64_t k, int dtype,
                       const float** parts, int* n_parts, void* stream);
 /* rt_bias_residual_layernorm with the sum of those slices in place of its input: out = LN(sum + bias + residual). */

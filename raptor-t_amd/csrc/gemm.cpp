@@ -33,7 +33,7 @@ struct rt_gemm_ctx {
   hipblasLtHandle_t lt = nullptr;
   int tune_candidates = 64;         // heuristic results timed on a shape's first call (1 = take the first)
   void* workspace = nullptr;
-  float* slices = nullptr;          // rt_gemm_bt_slices
+  float* slices = nullptr;          // rt_gemm_bt_slices, SLICES_BYTES
   size_t workspace_bytes = 0;
   int device = 0;
   std::mutex m;
@@ -55,6 +55,7 @@ struct rt_gemm_ctx {
 namespace {
 
 constexpr int MODE_B_TRANS = 16;   // B is handed over as Bt[N,K]
+constexpr int64_t SLICES_BYTES = int64_t(32) << 20;
 
 #define LT_TRY(expr)                                                                     \
   do {                                                                                   \
@@ -241,6 +242,11 @@ int rt_gemm_create(rt_gemm_ctx** out) {
   RT_REQUIRE(out, RT_EINVAL, "NULL output");
   rt_gemm_ctx* ctx = new rt_gemm_ctx();
   if (hipGetDevice(&ctx->device) != hipSuccess) { delete ctx; return rt::fail(RT_EIO, "hipGetDevice failed: no usable GPU"); }
+  // here and not at the first product that is cut: that one may be the first of its size inside a graph capture
+  if (hipMalloc(reinterpret_cast<void**>(&ctx->slices), SLICES_BYTES) != hipSuccess) {
+    delete ctx;
+    return rt::fail(RT_ENOMEM, "could not allocate the 32 MiB workspace of product slices");
+  }
   *out = ctx;
   return RT_OK;
 }
@@ -322,7 +328,6 @@ int rt_gemm_bias_act(rt_gemm_ctx* ctx, const void* a, const void* b, const void*
 
 int rt_gemm_bt_slices(rt_gemm_ctx* ctx, const void* a, const void* bt, int64_t m, int64_t n, int64_t k, int dtype,
                       const float** parts, int* n_parts, void* stream) {
-  constexpr int64_t SLICES_BYTES = int64_t(32) << 20;
   RT_REQUIRE(ctx && a && bt && parts && n_parts, RT_EINVAL, "NULL argument");
   RT_REQUIRE(m >= 0 && n > 0 && k > 0, RT_EINVAL, "bad shape M=%lld N=%lld K=%lld", (long long)m, (long long)n, (long long)k);
   *parts = nullptr;
@@ -331,10 +336,6 @@ int rt_gemm_bt_slices(rt_gemm_ctx* ctx, const void* a, const void* bt, int64_t m
   const int slices = rt::gemm_mfma_slices(m, n, k, SLICES_BYTES);
   if (slices < 2) return RT_OK;
   std::lock_guard<std::mutex> lk(ctx->m);
-  if (!ctx->slices && hipMalloc(reinterpret_cast<void**>(&ctx->slices), SLICES_BYTES) != hipSuccess) {
-    ctx->slices = nullptr;
-    return rt::fail(RT_ENOMEM, "could not allocate the 32 MiB workspace of product slices");
-  }
   const int rc = rt::gemm_mfma_part(a, bt, ctx->slices, m, n, k, slices, dtype, stream);
   if (rc) return rc;
   *parts = ctx->slices;

@@ -127,3 +127,21 @@ def test_gemm_bt_layernorm(capi, m, n, k, dtype):
     over = ((out[:m].float() - want).abs() - bound).max().item()
     assert over <= 0, over
     assert bool((out[m] == 7.0).all())
+
+
+def test_cut_product_as_first_call_in_a_capture(capi):
+    """A context's first product that is cut may be met inside a capture, which allows no allocation."""
+    m, n, k = 512, 768, 3072
+    a, b, bias = operands(m, n, k, torch.float16)
+    residual, out, want = (torch.randn(m, n, device="cuda").half() for _ in range(3))
+    args = (a, b, bias, residual, 1 + 0 * bias, 0 * bias)
+    assert capi.Gemm().bt_layernorm(*args, want, 1e-5) > 1
+    fresh, graph = capi.Gemm(), torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        fresh.bt_layernorm(*args, out, 1e-5)
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
