@@ -136,6 +136,11 @@ struct State {
   float m[2], l[2];      // per query tile: reference maximum (log2 units), partial row sum
 };
 
+// Reference of a query that has met keys, all of them with a score of minus infinity; -INFINITY: it has met none.  No
+// finite score lies below it, so it gives way to any, and a share of a row's tiles that holds nothing but such keys adds
+// nothing to the other shares.
+constexpr float LOWEST = -3.402823466e+38f;
+
 __device__ inline void state_init(State& st) {
 #pragma unroll
   for (int t = 0; t < 2; ++t)
@@ -245,7 +250,7 @@ __device__ inline void stream_tiles(const T* __restrict__ kbase, const T* __rest
 #pragma unroll
           for (int e = 0; e < 16; ++e) mx = fmaxf(mx, sc[t][e]);
         mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-        const float m_new = fresh ? mx : fmaxf(mx, st.m[nt]);
+        const float m_new = fmaxf(mx, fresh ? LOWEST : st.m[nt]);
 #pragma unroll
         for (int t = 0; t < 2; ++t)
 #pragma unroll
@@ -809,12 +814,21 @@ __device__ inline bool fast_row(const Args<T>& a, const Buffers<T>& b, const QSi
   return sums_finite(st);
 }
 
-// normalises the state and writes the unit's output tile
-template <typename T>
+// One over a row's whole sum.  A row that has met nothing but padding writes zeros; one whose keys all have a score
+// of minus infinity has no softmax (only the moving-maximum loop meets such rows).
+__device__ inline float row_weight(float l, float m) {
+  return l == 0.f && m == LOWEST ? __builtin_nanf("") : __builtin_amdgcn_rcpf(fmaxf(l, 1e-30f));
+}
+
+// normalises the state and writes the unit's output tile; FAST: the state comes from the pipelined loop
+template <typename T, bool FAST>
 __device__ inline void finish_unit(const Args<T>& a, const QSide<T>& qs, const Unit& u, int lane, State& st) {
   float w[2];
 #pragma unroll
-  for (int nt = 0; nt < 2; ++nt) w[nt] = __builtin_amdgcn_rcpf(fmaxf(pair_sum(st.l[nt]), 1e-30f));
+  for (int nt = 0; nt < 2; ++nt) {
+    const float l = pair_sum(st.l[nt]);
+    w[nt] = FAST ? __builtin_amdgcn_rcpf(fmaxf(l, 1e-30f)) : row_weight(l, st.m[nt]);
+  }
   const int64_t stride = int64_t(a.heads) * 64;
   store_output<T>(a.out + int64_t(u.g0 + u.i) * 64 * stride + u.h * 64, stride, lane, st, w, qs.stage);
 }
@@ -839,7 +853,7 @@ __device__ inline bool run_solo(const Args<T>& a, const Buffers<T>& b, const QSi
     typename Mma<T>::v8 qf[2][4];
     slow_row<T, MASKED>(a, b, qbias, r, 0, 1, lane, false, qf, st);
   }
-  finish_unit<T>(a, qbias, u, lane, st);
+  finish_unit<T, FAST>(a, qbias, u, lane, st);
   return true;
 }
 
@@ -862,9 +876,9 @@ __device__ inline void absorb_state(State& st, const float* slot, int lane) {
 #pragma unroll
   for (int nt = 0; nt < 2; ++nt) {
     const float m1 = slot[(64 + nt) * 64 + lane], l1 = slot[(66 + nt) * 64 + lane];
-    const float mt = fmaxf(fmaxf(st.m[nt], m1), -1e30f);        // finite even if both are empty
+    const float m = fmaxf(st.m[nt], m1), mt = fmaxf(m, LOWEST);        // mt: finite even if both are empty
     const float a0 = __builtin_amdgcn_exp2f(st.m[nt] - mt), a1 = __builtin_amdgcn_exp2f(m1 - mt);
-    st.m[nt] = mt;
+    st.m[nt] = m;
     st.l[nt] = st.l[nt] * a0 + l1 * a1;
 #pragma unroll
     for (int t = 0; t < 2; ++t)
@@ -902,7 +916,7 @@ __device__ inline bool run_split4(const Args<T>& a, const Buffers<T>& b, const Q
     absorb_state(st, park, lane);
     float w[2];
 #pragma unroll
-    for (int nt = 0; nt < 2; ++nt) w[nt] = __builtin_amdgcn_rcpf(fmaxf(st.l[nt], 1e-30f));
+    for (int nt = 0; nt < 2; ++nt) w[nt] = row_weight(st.l[nt], st.m[nt]);
     const int64_t stride = int64_t(a.heads) * 64;
     // wave 0's room is the start of the park, which it has just finished reading
     store_output<T>(a.out + int64_t(u.g0 + u.i) * 64 * stride + u.h * 64, stride, lane, st, w, qbias.stage);
@@ -1243,7 +1257,7 @@ __global__ __launch_bounds__(256, 2) void bs_attention_kernel(Args<T> a) {
             SB();
             primed = nx_short;
             if (sums_finite(st)) {
-              finish_unit<T>(a, qbias, cur.u, lane, st);
+              finish_unit<T, true>(a, qbias, cur.u, lane, st);
               SB();
             } else {
               if (lane == 0) redo[wave][n_redo] = item;
@@ -1405,7 +1419,7 @@ __global__ __launch_bounds__(512, 2) void bs_attention_few_kernel(Args<T> a, int
   if (valid && part == 0) {
     float w[2];
 #pragma unroll
-    for (int nt = 0; nt < 2; ++nt) w[nt] = __builtin_amdgcn_rcpf(fmaxf(st.l[nt], 1e-30f));
+    for (int nt = 0; nt < 2; ++nt) w[nt] = row_weight(st.l[nt], st.m[nt]);
     const int64_t stride = int64_t(a.heads) * 64;
     store_output<T>(a.out + int64_t(u.g0 + u.i) * 64 * stride + u.h * 64, stride, lane, st, w, qbias.stage);
   }

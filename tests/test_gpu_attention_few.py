@@ -48,3 +48,39 @@ def test_few_units(capi, heads, lens, scale, padded):
     assert (plan.float().cpu() - ref).abs().max().item() <= tol
     if len(lens) <= 64:
         assert torch.equal(plan, out)                 # the caller's plan changes the order, not a unit's arithmetic
+
+
+@pytest.mark.parametrize("heads,lens", [
+    (2, [512]),                                       # 8 waves to a row: every tile is the first of its wave
+    (12, [1024, 256]),                                # 4 waves to a row, global rows by 8
+    (12, [512, 1024, 1280]),                          # 2
+    (12, [2048, 3008, 384]),                          # 1
+    (16, [2048] * 6),                                 # the persistent kernel
+])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_infinite_and_very_low_scores(capi, heads, lens, dtype):
+    """Key blocks that a query scores with minus infinity throughout (first, in the middle, last in a wave's share),
+    queries with no other keys, infinite and undefined values and, where the type reaches so far, rows whose scores
+    all lie below -1e30: weights as a softmax over the whole row gives them."""
+    print("infinities", heads, lens, dtype, flush=True)
+    g = torch.Generator().manual_seed(1)
+    t = sum(lens)
+    q, k, v = (torch.randn(t, heads, 64, generator=g).to(dtype) for _ in range(3))
+    inf = float("inf")
+    for block in (0, 2, lens[0] // 64 - 1):
+        k[64 * block:64 * block + 64, 0, 3] = inf      # by the sign of a query's element: no weight, or no number
+    k[320, 1, 5] = inf
+    v[400, 1, 7] = inf
+    v[410, 1, 9] = float("nan")
+    if dtype == torch.bfloat16:
+        q[:64, 1] = q[:64, 1].abs()
+        k[:lens[0], 1] = -2e35 * k[:lens[0], 1].abs().clamp_min(.1)
+        k[lens[0]:, 0, 9] = inf                        # the later sequences' head 0: every key, zeros or NaN
+    out, ref = lh.run_attention(capi, q.cuda(), k.cuda(), v.cuda(), lens, heads, seed=3)
+    out = out.float().cpu()
+    assert torch.equal(out.isnan(), ref.isnan()) and torch.equal(out.isinf(), ref.isinf())
+    ok = out.isfinite()                                # of the two heads with infinite keys half the queries, about
+    assert int(out.isnan().sum()) > 0 and int(ok.sum()) > out.numel() // 4
+    # weights and output rounded to the type (half a unit in the last place of values up to max |v| each)
+    tol = 4 * (2.0 ** -11 if dtype == torch.float16 else 2.0 ** -8) * v[v.isfinite()].abs().max().item()
+    assert (out - ref)[ok].abs().max().item() <= tol
