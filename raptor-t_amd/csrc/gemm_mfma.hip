@@ -328,8 +328,10 @@ __device__ __forceinline__ void main_loop(f32x4 (&acc)[MT][4], const f32x4 (&c0)
   typedef typename Mma<T>::v8 v8;
   v8 a[MT], b[2][4];
   // What may still be on its way at a step's barrier: the loads of A(s+2), which every wave has issued behind those of
-  // s+1, or in a tile's first step the stores of the last tile's outputs, which are as young.
-  constexpr int LEFT = TM / 64, STORES = EPI == EPI_QKV ? LEFT : 2 * MT;
+  // s+1, or in a tile's first step, behind its loads of B(s+1), the stores of the last tile's outputs.  store_rows issues
+  // 2 * MT of them whatever it stores (past the ends of C the range check drops them); store_v and store_k issue none for
+  // rows and columns past the end, so behind them nothing may be left: B(s+1) could be what is.
+  constexpr int LEFT = TM / 64, STORES = EPI == EPI_QKV ? 0 : 2 * MT;
   enum { FIRST, INNER, LAST };
   // row i of a half: its four products, the columns in alternating direction (a row's last weights fragment is the
   // next row's first: fewer operand bits toggle)

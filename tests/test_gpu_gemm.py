@@ -72,6 +72,12 @@ def test_gemm_bt_edges(capi, m, n, k, dtype, epilogue):
     (12, [192, 320], torch.bfloat16),
     (7, [960, 576], torch.float16),                   # 128 x 128
     (12, [2048, 1088], torch.bfloat16),               # 256 x 128
+    # More tiles than workgroups, so that a tile is followed by another one, where some waves store nothing of it:
+    (6, [14464], torch.float16),                      # tiles of 192: columns past the end, and a last panel with its lower half past the end
+    (10, [4096, 4096, 4160], torch.bfloat16),         # 224: the same
+    (6, [22976], torch.bfloat16),                     # 256: columns past the end
+    (24, [3712], torch.float16),                      # 192: rows past the end only
+    (24, [4096, 2368], torch.bfloat16),               # 256: the same
 ])
 def test_qkv_project_equals_gemm_and_split(capi, heads, seq_lens, dtype):
     print("qkv_project", heads, len(seq_lens), dtype, flush=True)
