@@ -212,20 +212,6 @@ int make_plan(rt_gemm_ctx* ctx, int64_t m, int64_t n, int64_t k, int dtype, int 
   return RT_OK;
 }
 
-// The library's handle and workspace, made when the first product needs them: a process whose products all run on the
-// kernels of gemm_mfma.hip never loads the library's solutions.  Caller holds ctx->m.
-int ensure_library(rt_gemm_ctx* ctx) {
-  if (!ctx->lt) LT_TRY(hipblasLtCreate(&ctx->lt));
-  if (!ctx->workspace) {
-    ctx->workspace_bytes = size_t(64) << 20;
-    if (hipMalloc(&ctx->workspace, ctx->workspace_bytes) != hipSuccess) {
-      ctx->workspace = nullptr;
-      return rt::fail(RT_ENOMEM, "could not allocate the 64 MiB GEMM workspace");
-    }
-  }
-  return RT_OK;
-}
-
 void free_plan(rt_gemm_ctx::Plan& p) {
   if (p.la) hipblasLtMatrixLayoutDestroy(p.la);
   if (p.lb) hipblasLtMatrixLayoutDestroy(p.lb);
@@ -242,9 +228,19 @@ int rt_gemm_create(rt_gemm_ctx** out) {
   RT_REQUIRE(out, RT_EINVAL, "NULL output");
   rt_gemm_ctx* ctx = new rt_gemm_ctx();
   if (hipGetDevice(&ctx->device) != hipSuccess) { delete ctx; return rt::fail(RT_EIO, "hipGetDevice failed: no usable GPU"); }
-  // here and not at the first product that is cut: that one may be the first of its size inside a graph capture
+  // All of it here and not at the first product that needs it: that one may be inside a graph capture, which allows
+  // neither the allocations nor the library's start.
+  hipblasStatus_t s = hipblasLtCreate(&ctx->lt);
+  if (s != HIPBLAS_STATUS_SUCCESS) { delete ctx; return rt::fail(RT_EIO, "hipblasLtCreate failed with status %d", int(s)); }
+  ctx->workspace_bytes = size_t(64) << 20;
+  if (hipMalloc(&ctx->workspace, ctx->workspace_bytes) != hipSuccess) {
+    ctx->workspace = nullptr;
+    rt_gemm_destroy(ctx);
+    return rt::fail(RT_ENOMEM, "could not allocate the 64 MiB GEMM workspace");
+  }
   if (hipMalloc(reinterpret_cast<void**>(&ctx->slices), SLICES_BYTES) != hipSuccess) {
-    delete ctx;
+    ctx->slices = nullptr;
+    rt_gemm_destroy(ctx);
     return rt::fail(RT_ENOMEM, "could not allocate the 32 MiB workspace of product slices");
   }
   *out = ctx;
@@ -291,14 +287,12 @@ int run_gemm(rt_gemm_ctx* ctx, const void* a, const void* b, const void* bias, v
   const float alpha = 1.0f, beta = 0.0f;
   // the plan's descriptor carries the bias pointer: set and used under the lock
   std::lock_guard<std::mutex> lk(ctx->m);
-  int rc = ensure_library(ctx);
-  if (rc) return rc;
   const int mode = epilogue | (b_trans ? MODE_B_TRANS : 0);
   auto key = std::make_tuple(m, n, k, dtype, mode);
   auto it = ctx->plans.find(key);
   if (it == ctx->plans.end()) {
     rt_gemm_ctx::Plan p;
-    rc = make_plan(ctx, m, n, k, dtype, mode, bias, p, a, b, c, static_cast<hipStream_t>(stream));
+    int rc = make_plan(ctx, m, n, k, dtype, mode, bias, p, a, b, c, static_cast<hipStream_t>(stream));
     if (rc) { free_plan(p); return rc; }
     it = ctx->plans.emplace(key, p).first;
   }

@@ -151,3 +151,34 @@ def test_cut_product_as_first_call_in_a_capture(capi):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, want)
+
+
+@pytest.mark.parametrize("call,dtype", [("bt", torch.float32), ("plain", torch.float16), ("bias_gelu", torch.bfloat16)])
+def test_library_product_as_first_call_in_a_capture(capi, call, dtype):
+    """The same for the products left to the library: fp32, and B[K, N]."""
+    m, n, k = 128, 192, 256
+    a, bt, bias = operands(m, n, k, dtype, seed=4)
+    b, out, want = bt.t().contiguous(), *(torch.empty(m, n, dtype=dtype, device="cuda") for _ in range(2))
+
+    def run(gemm, c):
+        if call == "bt":
+            gemm.bt(a, bt, c)
+        elif call == "plain":
+            gemm(a, b, c)
+        else:
+            gemm.bias_act(a, b, bias, c)
+
+    eager = capi.Gemm()
+    eager.set_tuning(1)                                # as in a capture, where no candidate can be timed
+    run(eager, want)
+    fresh, graph = capi.Gemm(), torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        run(fresh, out)
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        run(eager, want)
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
