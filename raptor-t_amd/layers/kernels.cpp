@@ -316,17 +316,32 @@ double tune_layer_gemms(const std::vector<int64_t>& token_counts, int64_t hidden
   // random operands: an all-zero product draws less power and would be timed at other clocks
   torch::Tensor a = torch::randn({max_m, wide}, opt), out = torch::empty({max_m, wide}, opt);
   torch::Tensor w = torch::randn({wide, wide}, opt) * 0.05, bias = torch::zeros({wide}, opt);
+  torch::Tensor tiles = torch::empty({2, max_m, hidden}, opt), seq_blocks = torch::zeros({2}, opt.dtype(torch::kInt32));
   rt_gemm_ctx* handle = shared_gemm_handle();
   void* stream = current_stream();
   const int dt = dtype_code(a);
+  auto product = [&](int64_t m, int64_t n, int64_t k, int epilogue) {
+    check(rt_gemm_bt(handle, a.data_ptr(), w.data_ptr(), epilogue == RT_EPILOGUE_NONE ? nullptr : bias.data_ptr(),
+                     out.data_ptr(), m, n, k, epilogue, dt, stream), "tune_layer_gemms");
+  };
+  // the products the layers run with the present switches, through the calls they make for them
   for (int64_t m : token_counts) {
-    // the shapes and epilogues the layers run with the present switches
-    const int64_t qkv_epilogue = gemm_epilogue_fusion() ? RT_EPILOGUE_BIAS : RT_EPILOGUE_NONE;
-    const int64_t shapes[4][3] = {{3 * hidden, hidden, qkv_epilogue}, {hidden, hidden, RT_EPILOGUE_NONE},
-                                  {ffn, hidden, RT_EPILOGUE_BIAS_GELU}, {hidden, ffn, RT_EPILOGUE_NONE}};
-    for (const auto& sh : shapes)
-      check(rt_gemm_bt(handle, a.data_ptr(), w.data_ptr(), sh[2] == RT_EPILOGUE_NONE ? nullptr : bias.data_ptr(),
-                       out.data_ptr(), m, sh[0], sh[1], int(sh[2]), dt, stream), "tune_layer_gemms");
+    int rc = RT_ENOSYS;
+    if (gemm_epilogue_fusion() && attention_q_from_rows() && m % RT_BLOCK == 0 && hidden % RT_HEAD_DIM == 0) {
+      seq_blocks.select(0, 1).fill_(m / RT_BLOCK);             // the rows as one sequence
+      rc = rt_qkv_project(a.data_ptr(), w.data_ptr(), bias.data_ptr(), out.data_ptr(), tiles[0].data_ptr(), tiles[1].data_ptr(),
+                          seq_blocks.data_ptr<int>(), 1, int(m / RT_BLOCK), int(hidden / RT_HEAD_DIM), hidden, dt, stream);
+      if (rc != RT_ENOSYS) check(rc, "tune_layer_gemms");
+    }
+    if (rc == RT_ENOSYS) product(m, 3 * hidden, hidden, gemm_epilogue_fusion() ? RT_EPILOGUE_BIAS : RT_EPILOGUE_NONE);
+    product(m, ffn, hidden, RT_EPILOGUE_BIAS_GELU);
+    for (int64_t k : {hidden, ffn}) {                          // the two that end in a LayerNorm (MatMulLayerNorm)
+      const float* parts = nullptr;
+      int n_parts = 0;
+      if (dt != RT_F32)
+        check(rt_gemm_bt_slices(handle, a.data_ptr(), w.data_ptr(), m, hidden, k, dt, &parts, &n_parts, stream), "tune_layer_gemms");
+      if (n_parts == 0) product(m, hidden, k, RT_EPILOGUE_NONE);
+    }
   }
   check(hipStreamSynchronize(static_cast<hipStream_t>(stream)) == hipSuccess ? 0 : RT_EIO, "tune_layer_gemms");
   return std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();

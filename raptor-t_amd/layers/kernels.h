@@ -95,10 +95,11 @@ bool gemm_epilogue_fusion();
 void set_attention_q_from_rows(bool on);
 bool attention_q_from_rows();
 
-// Start-up tuning for a server: runs the four GEMMs of an encoder layer (hidden -> 3*hidden,
-// hidden -> hidden, hidden -> ffn with bias + GELU, ffn -> hidden; weights as [out, in]) once for every
-// token count in `token_counts` on the shared context, so that no later batch of one of these sizes
-// pays for the timing of candidates.  Uses scratch operands of its own; returns the seconds it took.
+// Start-up for a server: runs the four products of an encoder layer (hidden -> 3*hidden, hidden -> hidden,
+// hidden -> ffn with bias + GELU, ffn -> hidden; weights as [out, in]) once for every token count in
+// `token_counts` on the shared context, through the calls that the layers make for them, so that no later batch
+// of one of these sizes meets a kernel for the first time or, where the library computes it, pays for the timing
+// of candidates.  Uses scratch operands of its own; returns the seconds it took.
 double tune_layer_gemms(const std::vector<int64_t>& token_counts, int64_t hidden, int64_t ffn, torch::ScalarType dtype);
 
 // What `balanced = true` means for the attention launch.  The reference's balanced kernel walks the

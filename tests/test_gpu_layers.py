@@ -348,6 +348,24 @@ def test_startup_gemm_tuning_runs(mb):
         mb.cxx.tune_layer_gemms([0], 256, 512, torch.float16)
 
 
+@pytest.mark.parametrize("q_from_rows,fusion", [(True, True), (False, True), (True, False)])
+def test_startup_products_of_every_route(mb, q_from_rows, fusion):
+    """The layers' own calls (head split in the projection, cut products) and the ones they fall back to: rows or a
+    width that are no whole blocks, fp32, a width the slices' LayerNorm does not have."""
+    say("tune_layer_gemms routes", q_from_rows, fusion)
+    mb.cxx.set_attention_q_from_rows(q_from_rows)
+    mb.cxx.set_gemm_epilogue_fusion(fusion)
+    try:
+        for counts, hidden, ffn, dtype in (([64, 512, 4096], 768, 3072, torch.float16), ([100, 1], 768, 3072, torch.bfloat16),
+                                           ([128], 320, 640, torch.float16), ([64], 96, 200, torch.float16),
+                                           ([128, 33], 256, 512, torch.float32)):
+            assert mb.cxx.tune_layer_gemms(counts, hidden, ffn, dtype) > 0.0
+        torch.cuda.synchronize()
+    finally:
+        mb.cxx.set_attention_q_from_rows(True)
+        mb.cxx.set_gemm_epilogue_fusion(True)
+
+
 def test_api_rejects_mismatched_batch(mb, ut):
     hidden, heads, ffn, dtype = 768, 12, 3072, torch.float16
     g = torch.Generator().manual_seed(2)
