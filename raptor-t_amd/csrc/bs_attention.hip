@@ -790,10 +790,10 @@ __device__ inline void slow_row(const Args<T>& a, const Buffers<T>& b, const QSi
 // Entries first, first + step, ... of row r through the state with the pipelined loop, no hand-over
 // from or to another row.  False: the row has to be run with the moving-maximum loop instead (more
 // than 64 entries for this wave, or scores that outgrew the reference); the state is then undefined.
-template <typename T, bool MASKED>
-__device__ inline bool fast_row(const Args<T>& a, const Buffers<T>& b, const QSide<T>& qbias, const Row& r, int first, int step,
-                                int lane, State& st) {
-  Tiles<T> t;
+// HAVE_Q: the queries are in t.qf already; they are there afterwards too.
+template <typename T, bool MASKED, bool HAVE_Q>
+__device__ inline bool fast_share(const Args<T>& a, const Buffers<T>& b, const QSide<T>& qbias, const Row& r, int first, int step,
+                                  int lane, Tiles<T>& t, State& st) {
   state_init(st);
   first = __builtin_amdgcn_readfirstlane(first);
   int my = __builtin_amdgcn_readfirstlane((r.cnt - first + step - 1) / step);           // this wave's entries
@@ -805,13 +805,19 @@ __device__ inline bool fast_row(const Args<T>& a, const Buffers<T>& b, const QSi
     if (!pad_to_end(ids, my, lane, pd)) return false;
     if (my == 0) return true;                          // every tile of this wave's share is padding
   }
-  request_q<T>(a, b, r.u, lane, t.qf);
+  if (!HAVE_Q) request_q<T>(a, b, r.u, lane, t.qf);
   request_first<T>(b, __builtin_amdgcn_readlane(ids, 0), lane, t);
-  finish_q<T>(a, qbias, r.u, lane, t.qf);
+  if (!HAVE_Q) finish_q<T>(a, qbias, r.u, lane, t.qf);
   float mref;
   if (!fast_reference<T, MASKED>(t, mref, pd.last && my == 1, pd.tail, lane)) return false;
   fast_loop<T, MASKED>(b, ids, my, -1, lane, mref, t, st, NoNextQ{}, pd);
   return sums_finite(st);
+}
+template <typename T, bool MASKED>
+__device__ inline bool fast_row(const Args<T>& a, const Buffers<T>& b, const QSide<T>& qbias, const Row& r, int first, int step,
+                                int lane, State& st) {
+  Tiles<T> t;
+  return fast_share<T, MASKED, false>(a, b, qbias, r, first, step, lane, t, st);
 }
 
 // One over a row's whole sum.  A row that has met nothing but padding writes zeros; one whose keys all have a score
@@ -1307,29 +1313,27 @@ __global__ __launch_bounds__(256, 2) void bs_attention_kernel(Args<T> a) {
 // Where the persistent kernel would leave most waves of the chip without a unit, its time is one unit's chain of tiles
 // (8 tiles, 13 us) or a global row's (a quarter of the sequence's blocks).  Here a unit's tiles are shared by several waves,
 // whose states merge through LDS: one workgroup of 8 waves (one per CU) takes one global row, or RPW other rows with
-// 8 / RPW waves each (rows_per_workgroup has the rule and the times of both kernels).  Nothing
-// persists and nothing is drawn: workgroup b looks its rows up from the batch's prefix, XCD x taking the x-th eighth of the
-// global rows and of the rest, both head-major, as the persistent kernel does.  With a caller's plan a workgroup takes one
-// unit of the list; the waves share it in the same way, so both give the same bits.  At most 64 sequences (a lane each).
-template <typename T, bool MASKED, int RPW>
-__global__ __launch_bounds__(512, 2) void bs_attention_few_kernel(Args<T> a, int n_wg) {
-  constexpr int WAVES_PER_ROW = 8 / RPW;
-  static_assert(8 * Q_STAGE_BYTES >= 4 * PARK_FLOATS * int(sizeof(float)), "the park must hold four wave states");
-  __shared__ __attribute__((aligned(16))) float park[8 * Q_STAGE_BYTES / 4];
-  __shared__ __attribute__((aligned(16))) T qbias_lds[MAX_HEADS_QROWS * 64];
-  __shared__ int failed[8];                            // per row: a wave's pipelined loop handed it back
-  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const QSide<T> qbias{qbias_lds, reinterpret_cast<char*>(park) + wave * Q_STAGE_BYTES};
-  // lane l: sequence l
-  const int sb0 = a.seq_blocks[min(lane, a.batch)], sb1 = a.seq_blocks[min(lane + 1, a.batch)];
-  if (a.q_rows)
-    for (int i = threadIdx.x; i < a.heads * 64; i += 512) qbias_lds[i] = a.q_bias ? a.q_bias[i] : static_cast<T>(0.f);
-  if (threadIdx.x < 8) failed[threadIdx.x] = 0;
-  const unsigned long long sparse = __ballot(lane < a.batch && sb1 - sb0 >= RT_MIN_SPARSE_BLOCKS);
-  const int n_sparse = __popcll(sparse), n_rows = a.nb_total - 2 * n_sparse;
-  const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
+// 8 / RPW waves each (rows_per_workgroup has the rule and the times of both kernels).  At most 64 sequences (a lane each).
+template <typename T, int NW> struct FewRoom {
+  // four wave states in a merge; each wave's room for a query tile
+  static constexpr int PARK = 4 * PARK_FLOATS > NW * Q_STAGE_BYTES / 4 ? 4 * PARK_FLOATS : NW * Q_STAGE_BYTES / 4;
+  __attribute__((aligned(16))) float park[PARK];
+  __attribute__((aligned(16))) T qbias[MAX_HEADS_QROWS * 64];
+  int failed[8];                                       // per row: a wave's pipelined loop handed it back
+};
 
-  auto unit_at = [&](int s, int h, int i) {
+// Lane l: where sequence l begins and ends.  Also fills the bias copy; the caller's barrier follows.
+template <typename T> struct FewBatch {
+  int lane, sb0, sb1;
+  template <int NW> __device__ __forceinline__ FewBatch(const Args<T>& a, FewRoom<T, NW>& room) {
+    lane = threadIdx.x & 63;
+    sb0 = a.seq_blocks[min(lane, a.batch)];
+    sb1 = a.seq_blocks[min(lane + 1, a.batch)];
+    if (a.q_rows)
+      for (int i = threadIdx.x; i < a.heads * 64; i += 64 * NW) room.qbias[i] = a.q_bias ? a.q_bias[i] : static_cast<T>(0.f);
+    if (threadIdx.x < 8) room.failed[threadIdx.x] = 0;
+  }
+  template <bool MASKED> __device__ __forceinline__ Unit unit_at(const Args<T>& a, int s, int h, int i) const {
     Unit u;
     u.g0 = __builtin_amdgcn_readlane(sb0, s);
     u.n = __builtin_amdgcn_readlane(sb1, s) - u.g0;
@@ -1343,74 +1347,70 @@ __global__ __launch_bounds__(512, 2) void bs_attention_few_kernel(Args<T> a, int
       u.tail = tokens - 64 * (u.nbv - 1);
     }
     return u;
-  };
+  }
   // sequence of a position in a per-lane ascending prefix (lane s: first position of sequence s)
-  auto seq_of = [&](int prefix, int x) { return __popcll(__ballot(lane < a.batch && prefix <= x)) - 1; };
-
-  Unit u;
-  bool valid = true, whole = false;                    // whole: all eight waves share one row
-  if (a.from_pos) {
-    const int n_units = a.nb_total * a.heads;
-    const int begin = min(max(a.from_pos[0], 0), n_units), end = min(max(a.from_pos[n_wg], begin), n_units);
-    if (begin + int(blockIdx.x) >= end) return;
-    const int id = __builtin_amdgcn_readfirstlane(a.from_idx[begin + int(blockIdx.x)]);
-    if (id < 0 || id >= n_units) return;
-    const int s = seq_of(sb0 * a.heads, id), g0 = __builtin_amdgcn_readlane(sb0, s), n = __builtin_amdgcn_readlane(sb1, s) - g0;
-    const int rem = id - g0 * a.heads, h = rem / n;
-    u = unit_at(s, h, rem - h * n);
-    whole = is_global_row(u);
-    valid = whole || wave < WAVES_PER_ROW;
-  } else {
-    const int n_pairs = n_sparse * a.heads;
-    const int p_lo = int(int64_t(n_pairs) * xcd / 8), p_hi = int(int64_t(n_pairs) * (xcd + 1) / 8), n_glob = 2 * (p_hi - p_lo);
-    whole = slot < n_glob;
-    if (whole) {
-      const int pair = p_lo + (slot >> 1), h = pair / n_sparse, k = pair - h * n_sparse;
-      // the k-th sparse sequence
-      const int s = __builtin_ctzll(__ballot((sparse >> lane & 1ull) && __popcll(sparse & ((1ull << lane) - 1ull)) == k));
-      u = unit_at(s, h, 0);
-      if (slot & 1) u.i = u.n - 1;
-    } else {
-      const int total = n_rows * a.heads;
-      const int lo = int(int64_t(total) * xcd / 8), hi = int(int64_t(total) * (xcd + 1) / 8);
-      const int first = lo + (slot - n_glob) * RPW;
-      if (first >= hi) return;
-      const int item = first + wave / WAVES_PER_ROW;
-      valid = item < hi;
-      const int it = valid ? item : first, h = it / n_rows, j = it - h * n_rows;
-      const int listed_before = sb0 - 2 * __popcll(sparse & ((1ull << lane) - 1ull));       // rows of earlier sequences
-      const int s = seq_of(listed_before, j);
-      u = unit_at(s, h, 0);
-      u.i = j - __builtin_amdgcn_readlane(listed_before, s) + ((sparse >> s & 1ull) ? 1 : 0);
-    }
+  __device__ __forceinline__ int seq_of(const Args<T>& a, int prefix, int x) const {
+    return __popcll(__ballot(lane < a.batch && prefix <= x)) - 1;
   }
-  __syncthreads();
+};
 
+template <typename T> __device__ __forceinline__ Buffers<T> few_buffers(const Args<T>& a) {
   Buffers<T> b;
-  {
-    const uint32_t kv_bytes = uint32_t(a.nb_total) * uint32_t(a.heads) * 8192u;
-    b.k = __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(a.k), 0, kv_bytes, 0x00020000);
-    b.v = __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(a.vt), 0, kv_bytes, 0x00020000);
-    b.q = a.q_rows ? __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(a.q_rows), 0, kv_bytes * 3u, 0x00020000)
-                   : __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(a.q), 0, kv_bytes, 0x00020000);
-  }
-  const int share = whole ? 8 : WAVES_PER_ROW, row = wave / share, part = wave - row * share;
+  const uint32_t kv_bytes = uint32_t(a.nb_total) * uint32_t(a.heads) * 8192u;
+  b.k = __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(a.k), 0, kv_bytes, 0x00020000);
+  b.v = __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(a.vt), 0, kv_bytes, 0x00020000);
+  b.q = a.q_rows ? __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(a.q_rows), 0, kv_bytes * 3u, 0x00020000)
+                 : __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(a.q), 0, kv_bytes, 0x00020000);
+  return b;
+}
+
+// The workgroup's NW waves on their rows, from the first tile to the output.  `whole`: unit u is the same in all
+// waves, which take its eight shares; else 8 / RPW waves (but no more than there are) take the shares of one row and u is
+// theirs.  `valid`: the wave has a row.
+template <typename T, bool MASKED, int RPW, int NW>
+__device__ __forceinline__ void share_rows(const Args<T>& a, const Buffers<T>& b, FewRoom<T, NW>& room, const QSide<T>& qbias,
+                                           const Unit& u, bool valid, bool whole, int lane, int wave) {
+  const int share = whole ? 8 : 8 / RPW, waves = share < NW ? share : NW, row = wave / waves, part = wave - row * waves;
   const Row r = describe<T>(a, u);
   State st;
-  state_init(st);
-  if (valid && !fast_row<T, MASKED>(a, b, qbias, r, part, share, lane, st) && lane == 0) failed[row] = 1;
-  __syncthreads();                                     // the query rooms are read
-  if (valid && failed[row]) {
-    typename Mma<T>::v8 qf[2][4];
-    slow_row<T, MASKED>(a, b, qbias, r, part, share, lane, false, qf, st);
+  if (NW < 8 && share > NW) {
+    // two shares per wave: the later one first, whose state waits in the wave's own park place (u is valid in all waves)
+    static_assert(NW == 8 || NW == 4, "eight shares are one or two per wave");
+    Tiles<T> t;
+    request_q<T>(a, b, u, lane, t.qf);
+    finish_q<T>(a, qbias, u, lane, t.qf);
+    __syncthreads();                                   // the query rooms are read
+    float* const own = room.park + wave * PARK_FLOATS;
+    auto two_shares = [&](auto one) {
+      bool ok = one(wave + 4);
+#pragma unroll
+      for (int nt = 0; nt < 2; ++nt) st.l[nt] = pair_sum(st.l[nt]);
+      park_state(st, own, lane);
+      ok = one(wave) && ok;
+#pragma unroll
+      for (int nt = 0; nt < 2; ++nt) st.l[nt] = pair_sum(st.l[nt]);
+      return ok;
+    };
+    const bool ok = two_shares([&](int p) { return fast_share<T, MASKED, true>(a, b, qbias, r, p, 8, lane, t, st); });
+    if (__syncthreads_or(!ok))
+      two_shares([&](int p) { slow_row<T, MASKED>(a, b, qbias, r, p, 8, lane, true, t.qf, st); return true; });
+    absorb_state(st, own, lane);
+  } else {
+    state_init(st);
+    if (valid && !fast_row<T, MASKED>(a, b, qbias, r, part, share, lane, st) && lane == 0) room.failed[row] = 1;
+    __syncthreads();                                   // the query rooms are read
+    if (valid && room.failed[row]) {
+      typename Mma<T>::v8 qf[2][4];
+      slow_row<T, MASKED>(a, b, qbias, r, part, share, lane, false, qf, st);
+    }
+#pragma unroll
+    for (int nt = 0; nt < 2; ++nt) st.l[nt] = pair_sum(st.l[nt]);
   }
 #pragma unroll
-  for (int nt = 0; nt < 2; ++nt) st.l[nt] = pair_sum(st.l[nt]);
-#pragma unroll
-  for (int half = 4; half >= 1; half >>= 1) {
-    if (2 * half > WAVES_PER_ROW && !whole) continue;
+  for (int half = NW / 2; half >= 1; half >>= 1) {
+    if (2 * half > 8 / RPW && !whole) continue;
     __syncthreads();                                   // the park is free
-    float* const place = park + (row * half + (part & (half - 1))) * PARK_FLOATS;
+    float* const place = room.park + (row * half + (part & (half - 1))) * PARK_FLOATS;
     if (part >= half && part < 2 * half) park_state(st, place, lane);
     __syncthreads();
     if (part < half) absorb_state(st, place, lane);
@@ -1422,6 +1422,105 @@ __global__ __launch_bounds__(512, 2) void bs_attention_few_kernel(Args<T> a, int
     for (int nt = 0; nt < 2; ++nt) w[nt] = row_weight(st.l[nt], st.m[nt]);
     const int64_t stride = int64_t(a.heads) * 64;
     store_output<T>(a.out + int64_t(u.g0 + u.i) * 64 * stride + u.h * 64, stride, lane, st, w, qbias.stage);
+  }
+}
+
+// Without a plan nothing persists and nothing is drawn: workgroup b looks its rows up from the batch's prefix, XCD x
+// taking the x-th eighth of the global rows and of the rest, both head-major, as the persistent kernel does.
+template <typename T, bool MASKED, int RPW>
+__global__ __launch_bounds__(512, 2) void bs_attention_few_kernel(Args<T> a) {
+  constexpr int WAVES_PER_ROW = 8 / RPW;
+  __shared__ FewRoom<T, 8> room;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const FewBatch<T> batch(a, room);
+  const int lane = batch.lane, sb0 = batch.sb0, sb1 = batch.sb1;
+  const QSide<T> qbias{room.qbias, reinterpret_cast<char*>(room.park) + wave * Q_STAGE_BYTES};
+  const unsigned long long sparse = __ballot(lane < a.batch && sb1 - sb0 >= RT_MIN_SPARSE_BLOCKS);
+  const int n_sparse = __popcll(sparse), n_rows = a.nb_total - 2 * n_sparse;
+  const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
+
+  Unit u;
+  bool valid = true;
+  const int n_pairs = n_sparse * a.heads;
+  const int p_lo = int(int64_t(n_pairs) * xcd / 8), p_hi = int(int64_t(n_pairs) * (xcd + 1) / 8), n_glob = 2 * (p_hi - p_lo);
+  const bool whole = slot < n_glob;
+  if (whole) {
+    const int pair = p_lo + (slot >> 1), h = pair / n_sparse, k = pair - h * n_sparse;
+    // the k-th sparse sequence
+    const int s = __builtin_ctzll(__ballot((sparse >> lane & 1ull) && __popcll(sparse & ((1ull << lane) - 1ull)) == k));
+    u = batch.template unit_at<MASKED>(a, s, h, 0);
+    if (slot & 1) u.i = u.n - 1;
+  } else {
+    const int total = n_rows * a.heads;
+    const int lo = int(int64_t(total) * xcd / 8), hi = int(int64_t(total) * (xcd + 1) / 8);
+    const int first = lo + (slot - n_glob) * RPW;
+    if (first >= hi) return;
+    const int item = first + wave / WAVES_PER_ROW;
+    valid = item < hi;
+    const int it = valid ? item : first, h = it / n_rows, j = it - h * n_rows;
+    const int listed_before = sb0 - 2 * __popcll(sparse & ((1ull << lane) - 1ull));       // rows of earlier sequences
+    const int s = batch.seq_of(a, listed_before, j);
+    u = batch.template unit_at<MASKED>(a, s, h, 0);
+    u.i = j - __builtin_amdgcn_readlane(listed_before, s) + ((sparse >> s & 1ull) ? 1 : 0);
+  }
+  __syncthreads();
+  share_rows<T, MASKED, RPW, 8>(a, few_buffers(a), room, qbias, u, valid, whole, lane, wave);
+}
+
+// With a caller's plan workgroup c walks its slice, as in the persistent kernel: four waves, two workgroups per CU, a global
+// row by all of them, other entries side by side as far as there are waves for them.  A unit's tiles are cut into as many
+// shares as without a plan, so the bits are the same; a wave takes two of eight.  The slice is clamped to the list, ids
+// outside it are skipped.  Measured (us a call, 12 heads, rt_meta_partition_lpt into 512 and 256; persistent kernel / this one):
+// 1 x 4096 tokens 22.7, 21.1 / 23.7, 21.1; 8 x 150-1700 28.8, 35.6 / 28.7, 32.1; 2 x 4096 31.9, 34.7 / 32.7, 32.0;
+// 6 x 2048 44.5, 50.4 / 42.1, 41.9; 7 x 2048 50.7, 60.6 / 46.8, 52.1 (one workgroup of 8 waves per unit: 96).  Behind it: plans
+// of fewer workgroups than CUs for few units (1 x 2048 into 64: 21.7 / 41.8), whose rows are cut finer than they need.
+template <typename T, bool MASKED, int RPW>
+__global__ __launch_bounds__(256, 2) void bs_attention_few_plan_kernel(Args<T> a) {
+  constexpr int SIDE = RPW > 2 ? RPW / 2 : 1;          // rows side by side
+  __shared__ FewRoom<T, 4> room;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int n_units = a.nb_total * a.heads;
+  const int begin = min(max(a.from_pos[blockIdx.x], 0), n_units);
+  const int end = min(max(a.from_pos[blockIdx.x + 1], begin), n_units);
+  if (begin == end) return;
+  const FewBatch<T> batch(a, room);
+  const QSide<T> qbias{room.qbias, reinterpret_cast<char*>(room.park) + wave * Q_STAGE_BYTES};
+  const Buffers<T> b = few_buffers(a);
+  auto unit_of_flat = [&](int id) {
+    const int s = batch.seq_of(a, batch.sb0 * a.heads, id);
+    const int g0 = __builtin_amdgcn_readlane(batch.sb0, s), n = __builtin_amdgcn_readlane(batch.sb1, s) - g0;
+    const int rem = id - g0 * a.heads, h = rem / n;
+    return batch.template unit_at<MASKED>(a, s, h, rem - h * n);
+  };
+  for (int p = begin; p < end;) {
+    int ids[SIDE];                                     // the next entries in one round trip
+#pragma unroll
+    for (int w = 0; w < SIDE; ++w) {
+      ids[w] = __builtin_amdgcn_readfirstlane(p + w < end ? a.from_idx[p + w] : -1);
+      if (ids[w] >= n_units) ids[w] = -1;
+    }
+    if (ids[0] < 0) { ++p; continue; }
+    Unit u = unit_of_flat(ids[0]);
+    const bool whole = is_global_row(u);
+    int run = 1;
+    if (!whole) {
+      const int mine = SIDE * wave / 4;
+      bool more = true;
+#pragma unroll
+      for (int w = 1; w < SIDE; ++w) {
+        more = more && ids[w] >= 0;
+        if (more) {
+          const Unit v = unit_of_flat(ids[w]);
+          more = !is_global_row(v);
+          if (more) ++run;
+          if (more && w == mine) u = v;
+        }
+      }
+    }
+    if (threadIdx.x < 8) room.failed[threadIdx.x] = 0;           // (the last rows' flags were read several barriers ago)
+    __syncthreads();
+    share_rows<T, MASKED, RPW, 4>(a, b, room, qbias, u, whole || SIDE * wave / 4 < run, whole, batch.lane, wave);
+    p += run;
   }
 }
 
@@ -1488,12 +1587,17 @@ int rows_per_workgroup(int batch, int total_blocks, int heads) {
 }
 
 template <typename T> int launch_few(const Args<T>& a, int rpw, int n_wg, hipStream_t st) {
-  // every XCD's share of the global rows (two per head of each sequence that may have them) and of the others
-  const int64_t units = int64_t(a.nb_total) * a.heads, pairs = most_pairs(a.batch, a.nb_total, a.heads);
-  const int64_t per_xcd = 2 * ((pairs + 7) / 8) + ((units + 7) / 8 + rpw - 1) / rpw;
-  const dim3 grid(unsigned(a.from_pos ? units : 8 * per_xcd));
   auto go = [&](auto masked, auto rows) {
-    RT_LAUNCH((bs_attention_few_kernel<T, decltype(masked)::value, decltype(rows)::value>), grid, dim3(512), 0, st, a, n_wg);
+    constexpr bool MASKED = decltype(masked)::value;
+    constexpr int RPW = decltype(rows)::value;
+    if (a.from_pos) {
+      RT_LAUNCH((bs_attention_few_plan_kernel<T, MASKED, RPW>), dim3(unsigned(n_wg)), dim3(256), 0, st, a);
+      return;
+    }
+    // every XCD's share of the global rows (two per head of each sequence that may have them) and of the others
+    const int64_t units = int64_t(a.nb_total) * a.heads, pairs = most_pairs(a.batch, a.nb_total, a.heads);
+    const int64_t per_xcd = 2 * ((pairs + 7) / 8) + ((units + 7) / 8 + rpw - 1) / rpw;
+    RT_LAUNCH((bs_attention_few_kernel<T, MASKED, RPW>), dim3(unsigned(8 * per_xcd)), dim3(512), 0, st, a);
   };
   auto pick = [&](auto masked) {
     if (rpw == 1) go(masked, std::integral_constant<int, 1>());

@@ -50,6 +50,42 @@ def test_few_units(capi, heads, lens, scale, padded):
         assert torch.equal(plan, out)                 # the caller's plan changes the order, not a unit's arithmetic
 
 
+@pytest.mark.parametrize("heads,lens,scale", [
+    (2, [512], 1.0),                                  # a unit in 8 shares: two to each of the workgroup's four waves
+    (2, [512], 40.0),                                 # the same with scores beyond the pipelined loop's range
+    (12, [1024, 1088], 1.0),                          # 4
+    (12, [256, 1024, 640, 896], 1.0),                 # 2: two units side by side
+    (12, [2048, 3008, 384], 6.0),                     # 1: four
+])
+@pytest.mark.parametrize("padded", [False, True])
+def test_few_units_walk_the_plan(capi, heads, lens, scale, padded):
+    """Every workgroup walks the slice that the partition gives it, whatever its neighbours have: one slice with all units,
+    more slices than units, and slices whose ends do not meet (the first is empty, the second begins before its end)."""
+    print("plan walk", heads, lens, scale, padded, flush=True)
+    g = torch.Generator(device="cuda").manual_seed(3)
+    t = sum(lens)
+    sb, _, _, ph, sb_d, idx_d, pos_d = lh.device_plan(capi, lens, heads, 3)
+    q, k, v = (torch.randn(t, heads, 64, generator=g, device="cuda").half() for _ in range(3))
+    operands = lh.pack_heads(q * (scale * lh.LOG2E / 8), sb), lh.pack_heads(k, sb), lh.pack_heads(v, sb, transpose_v=True)
+    tokens = torch.tensor([max(1, n - 81 - 3 * i) for i, n in enumerate(lens)], dtype=torch.int32).cuda() if padded else None
+    units = t // 64 * heads
+
+    def run(*plan):
+        out = torch.full((t, heads * 64), float("nan"), dtype=torch.float16, device="cuda")
+        capi.bs_attention_fwd(*operands, out, sb_d, heads, idx_d, pos_d, ph, *plan, seq_tokens_dev=tokens)
+        torch.cuda.synchronize()
+        return out
+
+    want = run(None, None)
+    assert not bool(want.isnan().any())
+    for n_wg in (1, 5, units + 3):
+        fp, fi = capi.partition_lpt(sb, heads, n_wg)
+        assert torch.equal(run(torch.from_numpy(fi).cuda(), torch.from_numpy(fp).cuda()), want), n_wg
+    ids = torch.arange(units, dtype=torch.int32).cuda()
+    ends = torch.tensor([units // 2, 0, units], dtype=torch.int32).cuda()
+    assert torch.equal(run(ids, ends), want)
+
+
 @pytest.mark.parametrize("heads,lens", [
     (2, [512]),                                       # 8 waves to a row: every tile is the first of its wave
     (12, [1024, 256]),                                # 4 waves to a row, global rows by 8
