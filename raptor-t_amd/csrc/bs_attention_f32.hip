@@ -4,9 +4,11 @@
 // fp16 / bf16 kernel of bs_attention.hip, with every tensor in fp32.
 //
 // The products run on the bf16 matrix instructions without losing fp32's digits: an operand is cut, exactly, into
-// three bf16 parts of eight bits each (hi + mid + lo), and of the nine products of parts the six largest are added
-// up in fp32; what is left out is below 2^-22 of a product, 2^-25 on average, less than the roundings of
-// an fp32 sum.  Six products of 16x16x32 take 96 cycles of a SIMD's matrix pipe where v_mfma_f32_16x16x4_f32 takes 256.
+// three bf16 parts (hi + mid + lo), and of the nine products of parts the six largest are added up in fp32.  The parts are
+// rounded, not truncated, so what is left out (mid * lo twice, lo * lo) is at most 2^-24 of a product, of either sign: less
+// than the roundings of an fp32 sum.  (Truncated parts leave out up to 2^-21, always towards zero: operands whose low bits
+// are all ones were then twice as far from 64 bits as on the fp32 instruction, 8.8e-7 against 4.4e-7; now 2.2e-7.)  Six
+// products of 16x16x32 take 96 cycles of a SIMD's matrix pipe where v_mfma_f32_16x16x4_f32 takes 256.
 //
 // One workgroup of eight waves per unit (64 queries of one head against the unit's list of key blocks).  A key
 // block's K and V^T tiles are cut once for the whole workgroup, 8 + 8 numbers per thread, on their way into LDS, in
@@ -26,8 +28,9 @@
 //
 // Bound by the matrix pipe at 1 540 cycles per tile and SIMD (with the cutting, 700 vector cycles, beside it) and, with
 // few units, by the longest row on one CU.  Measured (us, before: one tile at a time on v_mfma_f32_16x16x4_f32, units in flat
-// order): 12 heads x 1024 tokens 82 -> 29, x 4 x 2048 493 -> 143, x 128 + 832 + 1984 178 -> 68; the error against 64 bits
-// 5.0e-7 -> 3.2e-7 of the result (the longer steps of the matrix instruction add up fewer partial sums).
+// order): 12 heads x 1024 tokens 82 -> 32, x 4 x 2048 493 -> 142, x 128 + 832 + 1984 178 -> 68 (with truncated parts 30, 135,
+// 64); the error against 64 bits 5.0e-7 -> 3.0e-7 of the result (the longer steps of the matrix instruction add up fewer
+// partial sums), 0.4 to 0.65 of the fp32 instruction's over scores of size 0.1 to 10 and the mantissas above.
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
@@ -36,9 +39,11 @@
 
 namespace {
 
+typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 constexpr int THREADS = 512;
@@ -218,19 +223,19 @@ __device__ void run_plain(const ArgsF32& a, const Unit& u, float (*ks)[PITCH], f
   for (int dt = 0; dt < 4; ++dt) *reinterpret_cast<f32x4*>(dst + 16 * dt + 4 * grp) = o[dt] * inv;
 }
 
-// Eight numbers as three bf16 parts; p[0] + p[1] + p[2] is the number.  Cutting, not rounding: no part can be
-// larger than the number.
+// Eight numbers as three bf16 parts; p[0] + p[1] + p[2] is the number.  Each part is what is left, rounded to nearest: the
+// second is at most 2^-8 of the number and the third 2^-17, with either sign, and the third is exact.
 __device__ __forceinline__ void cut8(const f32x4& x, const f32x4& y, u32x4 (&p)[3]) {
   float v[8] = {x[0], x[1], x[2], x[3], y[0], y[1], y[2], y[3]};
 #pragma unroll
   for (int part = 0; part < 3; ++part) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const uint32_t a = __float_as_uint(v[2 * i]), b = __float_as_uint(v[2 * i + 1]);
-      p[part][i] = __builtin_amdgcn_perm(b, a, 0x07060302u);
+      const uint32_t w = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{v[2 * i], v[2 * i + 1]}, bf16x2));
+      p[part][i] = w;
       if (part < 2) {
-        v[2 * i] -= __uint_as_float(a & 0xffff0000u);
-        v[2 * i + 1] -= __uint_as_float(b & 0xffff0000u);
+        v[2 * i] -= __uint_as_float(w << 16);
+        v[2 * i + 1] -= __uint_as_float(w & 0xffff0000u);
       }
     }
   }
@@ -260,6 +265,7 @@ __device__ void run_unit(const ArgsF32& a, int unit, char* smem) {
 
   // Q operand: step s, lane: Q[16 (wave & 3) + qcol][32 s + 8 grp .. + 8]
   u32x4 q[2][3];
+  bool bad = false;                                    // the unit has to be run again by the plain kernel
   {
     const int qrow = 16 * (wave & 3) + qcol;
 #pragma unroll
@@ -405,24 +411,25 @@ __device__ void run_unit(const ArgsF32& a, int unit, char* smem) {
     *reinterpret_cast<f32x4*>(room + 4096) = f32x4{m, l, 0.f, 0.f};
   }
   __syncthreads();
-  bool bad = false;
   if (!half) {
     const f32x4 ml = *reinterpret_cast<const f32x4*>(room + 4096);
     const float mm = fmaxf(m, ml[0]);
     const float c0 = m == -INFINITY ? 0.f : exp2f(m - mm), c1 = ml[0] == -INFINITY ? 0.f : exp2f(ml[0] - mm);
     l = l * c0 + ml[1] * c1;
-    bad = !(l < INFINITY);
+    bad = bad | !(l < INFINITY);
 #pragma unroll
     for (int dt = 0; dt < 4; ++dt) {
       o[dt] = o[dt] * c0 + *reinterpret_cast<const f32x4*>(room + dt * 1024) * c1;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) bad = bad || !(fabsf(o[dt][e]) < INFINITY);
+      for (int e = 0; e < 4; ++e) bad = bad | !(fabsf(o[dt][e]) < INFINITY);
     }
     // O^T accumulator dt: lane holds d = 16 dt + 4 grp + e for query qcol
     const float inv = 1.0f / fmaxf(l, 1e-30f);        // a row that lists nothing but padding writes zeros
     float* dst = a.out + (int64_t(u.block) * 64 + 16 * wave + qcol) * dm + u.h * 64;
 #pragma unroll
-    for (int dt = 0; dt < 4; ++dt) *reinterpret_cast<f32x4*>(dst + 16 * dt + 4 * grp) = o[dt] * inv;
+    for (int dt = 0; dt < 4; ++dt) {
+      *reinterpret_cast<f32x4*>(dst + 16 * dt + 4 * grp) = o[dt] * inv;
+    }
   }
   // (its barrier also lets the next unit have the LDS)
   if (__syncthreads_or(bad)) {
