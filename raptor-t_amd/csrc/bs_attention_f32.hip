@@ -23,8 +23,11 @@
 // 16 kt + 4 (lane >> 4) + i of query lane & 15: with a step's 32 keys taken in the order that makes these a lane's 8,
 // P never leaves its registers; V^T is laid out in LDS in the same order.
 //
-// The parts of an infinity are no numbers (inf - inf), so a unit whose result is not finite is run again by the
-// plain kernel below on v_mfma_f32_16x16x4_f32: rows that meet infinities give what fp32 arithmetic gives.
+// A unit is run again by the plain kernel below on v_mfma_f32_16x16x4_f32, which gives what fp32 arithmetic gives,
+//   if its result is not finite: the parts of an infinity are no numbers (inf - inf);
+//   if an output is below 2^-100 (values below 2^-109 lose digits: the bf16 instructions take a subnormal part for zero) or
+//   a query lies outside 2^-109 .. 2^80, where digits that it or a key loses could reach a score.
+// Values and weights below 2^-126 count as zero otherwise (exp2 is the hardware's instruction).
 //
 // Bound by the matrix pipe at 1 540 cycles per tile and SIMD (with the cutting, 700 vector cycles, beside it) and, with
 // few units, by the longest row on one CU.  Measured (us, before: one tile at a time on v_mfma_f32_16x16x4_f32, units in flat
@@ -284,6 +287,11 @@ __device__ void run_unit(const ArgsF32& a, int unit, char* smem) {
         x = *reinterpret_cast<const f32x4*>(src);
         y = *reinterpret_cast<const f32x4*>(src + 4);
       }
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float v = fabsf(e < 4 ? x[e & 3] : y[e & 3]);
+        bad = bad | ((v != 0.f) & !((v >= 0x1p-109f) & (v <= 0x1p80f)));
+      }
       cut8(x, y, q[s]);
     }
   }
@@ -428,7 +436,10 @@ __device__ void run_unit(const ArgsF32& a, int unit, char* smem) {
     float* dst = a.out + (int64_t(u.block) * 64 + 16 * wave + qcol) * dm + u.h * 64;
 #pragma unroll
     for (int dt = 0; dt < 4; ++dt) {
-      *reinterpret_cast<f32x4*>(dst + 16 * dt + 4 * grp) = o[dt] * inv;
+      const f32x4 r = o[dt] * inv;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) bad = bad | ((r[e] != 0.f) & (fabsf(r[e]) < 0x1p-100f));
+      *reinterpret_cast<f32x4*>(dst + 16 * dt + 4 * grp) = r;
     }
   }
   // (its barrier also lets the next unit have the LDS)

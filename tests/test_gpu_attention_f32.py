@@ -88,6 +88,9 @@ INPUTS = {
     "large mean": lambda r, sign, power: (r() + 4, r() + 4, r() + 4),
     "ones": lambda r, sign, power: (2 * sign() * ONES, sign() * ONES, sign() * ONES),
     "ones of many sizes": lambda r, sign, power: (sign() * power() * ONES, sign() * power() * ONES, sign() * power() * ONES),
+    "tiny values": lambda r, sign, power: (r(), r(), r() * 2.0 ** -118),
+    "tiny queries": lambda r, sign, power: (r() * 2.0 ** -120, r() * 2.0 ** 120, r()),
+    "huge queries": lambda r, sign, power: (r() * 2.0 ** 120, r() * 2.0 ** -120, r()),
 }
 
 
