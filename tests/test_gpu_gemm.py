@@ -42,10 +42,17 @@ def check(got, a, b, bias, gelu, dtype):
 
 
 @pytest.mark.parametrize("m,n,k,dtype", [
-    (12288, 256, 128, torch.float16),       # the shortest reduction: a tile's first step is followed by its last
-    (12295, 264, 192, torch.bfloat16),      # odd number of steps; 8 columns and 7 rows in tiles of their own
-    (9409, 520, 768, torch.float16),        # tiles of 224 rows: one row in the last
-    (16384 + 33, 1000, 256, torch.bfloat16),
+    (12288, 256, 128, torch.float16),       # 128 x 128, the shortest reduction
+    (12295, 264, 192, torch.bfloat16),      # 128 x 64, odd number of steps; 8 columns and 7 rows in tiles of their own
+    (9409, 520, 768, torch.float16),        # 192 x 128: one row in the last panel
+    (16384 + 33, 1000, 256, torch.bfloat16),        # 192 x 256
+    # More tiles than workgroups with the shortest reductions: a tile's first step is followed by its last (two steps, loads
+    # reach into the tile after the next) or by one more (three); one row, 8 columns in the last tiles
+    (8065, 2312, 128, torch.float16),       # 192 x 256
+    (16353, 2304, 128, torch.bfloat16),     # 224 x 256
+    (12289, 2312, 128, torch.float16),      # 256 x 256
+    (8065, 2312, 192, torch.bfloat16),
+    (12321, 3080, 192, torch.float16),
     (1, 8, 128, torch.float16),             # one row, one chunk of columns
     (64, 768, 3072, torch.bfloat16),        # tiles of 64 x 64
     (333, 776, 768, torch.float16),
@@ -70,7 +77,8 @@ def test_gemm_bt_edges(capi, m, n, k, dtype, epilogue):
     (16, [4096, 320], torch.float16),
     (2, [64], torch.float16),                         # half a tile of 128 x 64
     (12, [192, 320], torch.bfloat16),
-    (7, [960, 576], torch.float16),                   # 128 x 128
+    (7, [960, 576], torch.float16),                   # 128 x 64, 252 of 256 workgroups
+    (7, [960, 640], torch.float16),                   # 128 x 128
     (12, [2048, 1088], torch.bfloat16),               # 256 x 128
     # More tiles than workgroups, so that a tile is followed by another one, where some waves store nothing of it:
     (6, [14464], torch.float16),                      # tiles of 192: columns past the end, and a last panel with its lower half past the end
