@@ -354,7 +354,7 @@ def run_encoder(args, name, hidden, heads, ffn, layers, dtype, seq_lens, max_pos
         "two_streams": two_streams,
         "kernel_us_per_launch": per,
         "kernel_us_per_step": {k: v[0] / args.steps for k, v in timing_all.items()},
-        "kernel_timing": "HIP events holding each dispatch's own start and end (hipExtLaunchKernelGGL; the vendor GEMMs: "
+        "kernel_timing": "HIP events holding each dispatch's own start and end (hipExtLaunchKernelGGL; the products: "
                          "events recorded around the call).  attention: one launch in five inside the timed steps; "
                          "the others: a second pass over the same steps with every launcher timed",
     }

@@ -25,12 +25,17 @@
 //     and nobody reads step s any more
 //     half 1, rest   between its products the first fragment reads of step s+1 and the loads of B(s+2) and A(s+3) into
 //                    the stages just freed
-//   so the matrix pipe has work across the barrier, and the loads of the next tile's first steps are in flight
-//   while the epilogue of the present one runs.  A tile's last step leaves its A stage empty: the epilogue turns its
+//   so the matrix pipe has work across the barrier, and the loads of the next tile's first steps are requested before the
+//   epilogue of the present one.  A tile's last step leaves its A stage empty: the epilogue turns its
 //   outputs into whole rows there, and the load that belongs there follows in the next tile's first step.
+//   (The compiler waits for the bias, and so for every load and store before it, at the head of a tile: the first bias is
+//   requested outside the tile loop.  A tile therefore begins when the last one's outputs are stored.)
 //
-// Bound by the power the part may draw: with random operands it holds 1.7-1.85 GHz in these loops, at 2 600 cycles a
-// step where the matrix instructions alone take 2 240.  Measured against hipBLASLt's best of 64 suggestions for the
+// Bound by the boundaries of tiles and by power.  Within a tile a step takes 2 600 cycles where its matrix instructions
+// alone take 2 240, at 1.7-1.85 GHz with random operands; over a launch the matrix pipe is busy for 49 % (37184 x 2304 x 768
+// with the head split), 54 % (x 3072 x 768), 50 % (the same with GELU), 39 % (x 768 x 768) and 62 % (x 768 x 3072) of the
+// cycles at 1.9-2.3 GHz: the shorter the reduction, the more of it is first loads, epilogue and the last round.  Measured
+// against hipBLASLt's best of 64 suggestions for the
 // shape, in turn on one box (us): 37184 x 2304 x 768 113 against 127, 37184 x 3072 x 768 147 against 165 and with bias +
 // GELU 165 against 225, 37184 x 768 x 3072 130 against 132, 37184 x 768 x 768 41 against 44, 40768 x 1024 x 4096 268
 // against 340, 40768 x 4096 x 1024 274 against 282; the projection with the head split 141 against 114 + 38.
@@ -370,7 +375,9 @@ __device__ __forceinline__ void main_loop(f32x4 (&acc)[MT][4], const f32x4 (&c0)
     products(1, b[1], no);
     SB();
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" :: "n"(W == LAST ? 0 : W == FIRST ? STORES : LEFT) : "memory");
-    if (W == LAST) {                                 // the compiler's own wait for these comes here, where it costs nothing
+    // The compiler's own wait for these comes here, where everything has arrived already.  (With the head split it has
+    // waited before: load_bias' two ways to load share registers, so each load waits for the one before it.)
+    if (W == LAST) {
 #pragma unroll
       for (int j = 0; j < 4; ++j) asm volatile("" : "+v"(bias.w[j]));
       if (EPI == EPI_QKV) asm volatile("" : "+v"(bias.seq_end));
@@ -437,7 +444,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const uint32_t lds0 = uint32_t(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) char*)smem));
   const __amdgpu_buffer_rsrc_t sc = __builtin_amdgcn_make_buffer_rsrc(p.c, 0, uint32_t(p.m) * uint32_t(p.n) * 2u, 0x00020000);
   const i32x4 sa = make_srd(p.a, uint32_t(p.m) * uint32_t(p.k) * 2u), sb = make_srd(p.bt, uint32_t(p.n) * uint32_t(p.k) * 2u);
-  // Workgroups go to the 8 XCDs round-robin: XCD x takes the x-th eighth of the tiles (columns vary fastest), its
+  // Workgroups go to the 8 XCDs round-robin: XCD x takes the x-th eighth of the tiles (in tile_at's order), its
   // workgroups take neighbouring tiles, so the rows of A are fetched into one L2.
   const int total = p.tiles_m * p.tiles_n, xcd = blockIdx.x & 7, slot = blockIdx.x >> 3, slots = gridDim.x >> 3;
   int tile = int(int64_t(total) * xcd / 8) + slot;
@@ -536,7 +543,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 }
 
 // ---- smaller products ------------------------------------------------------------------------------------------------
-// One workgroup of 4 waves per tile of TM x TC outputs and per slice of the reduction; a wave owns MT row blocks of 16
+// One workgroup of NW (4 or 8) waves per tile of TM x TC outputs and per slice of the reduction; a wave owns MT row blocks of 16
 // and 64 columns.  Where the kernel above would give too few CUs a tile each, what bounds a product is the latency of a
 // workgroup's chain of steps: STAGES of both operands are in flight, up to two workgroups share a CU, and a long
 // reduction is cut into slices (EPI_PART: the fp32 sums of slice s go to c[s][M][N] and the kernel that reads
@@ -748,6 +755,9 @@ template <typename T, int TM, int TC, int NW, int STAGES, int EPI> int launch_sm
 //   512 x 2304 x 768    128 x 64: 7.0, 192 x 256: 13.7 (15.8)     4096 x 2304 x 768  192 x 256: 17.1, 128 x 64: 23 (21)
 //   512 x 768 x 3072    64 x 64 in 4 slices: 8.1, uncut 15.3 (16) 5568 x 768 x 3072  192 x 128: 33.6, 128 x 128: 41 (36)
 //   4096 x 768 x 3072   128 x 128: 27.4, 64 x 64: 34 (28.6)       8192 x 768 x 3072  256 x 128: 43, 192 x 256: 46 (41)
+// Both sides again for every kernel at 13 shapes (512-37184 rows, N 768-3072, K 768 and 3072) in fp16 and in bf16: bf16 is 0-6 %
+// faster throughout and the kernels stand in the same order, but for pairs within 3 %; what the rule picks is the
+// fastest or within 5 % of it in both types.
 struct Choice {
   int tm, tc, waves, stages, slices;
 };

@@ -43,7 +43,7 @@ std::map<std::string, std::pair<double, int64_t>> timing_collect();
 // RAII timer: accumulates into info[key] only when the key already exists (synchronous),
 // and feeds the deferred timing when it is active.  `own_dispatch`: the launcher starts exactly one kernel of
 // the library; its events then carry the dispatch's own start and end (rt_time_next_launch), the duration a
-// profiler reports.  Otherwise (vendor GEMMs) the events are recorded on the stream before and after the call
+// profiler reports.  Otherwise (products) the events are recorded on the stream before and after the call
 // and also count the gaps to the neighbouring kernels.
 class ScopedGpuTimer {
  public:
