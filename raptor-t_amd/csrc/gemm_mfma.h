@@ -7,6 +7,8 @@ namespace rt {
 // Whether gemm_mfma_bt computes this product: 16-bit types, K a multiple of 64, N a multiple of 8, 16-byte aligned
 // operands whose byte offsets fit 31 bits.
 bool gemm_mfma_takes(const void* a, const void* bt, const void* bias, const void* c, int64_t m, int64_t n, int64_t k, int dtype);
+// Whether it is also the faster way: not for a long reduction with few outputs, which hipBLASLt cuts.
+bool gemm_mfma_pays(int64_t m, int64_t n, int64_t k);
 // C[M,N] = A[M,K] . Bt[N,K]^T (+ bias, + tanh GELU)
 int gemm_mfma_bt(const void* a, const void* bt, const void* bias, void* c, int64_t m, int64_t n, int64_t k, bool gelu, int dtype,
                  void* stream);

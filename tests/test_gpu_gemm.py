@@ -54,8 +54,9 @@ def check(got, a, b, bias, gelu, dtype):
     (8065, 2312, 192, torch.bfloat16),
     (12321, 3080, 192, torch.float16),
     (1, 8, 128, torch.float16),             # one row, one chunk of columns
-    (64, 768, 3072, torch.bfloat16),        # tiles of 64 x 64
-    (333, 776, 768, torch.float16),
+    (64, 768, 3072, torch.bfloat16),        # a long reduction with few outputs: the library
+    (333, 776, 768, torch.float16),         # tiles of 64 x 64
+    (64, 5120, 1280, torch.bfloat16),
     (700, 2312, 192, torch.float16),        # tiles of 128 x 64
     (1500, 2304, 768, torch.bfloat16),      # 128 x 128
     (2049, 3080, 320, torch.float16),       # 256 x 128
@@ -69,6 +70,28 @@ def test_gemm_bt_edges(capi, m, n, k, dtype, epilogue):
     capi.Gemm().bt(a, b, c[:m], bias=bias if epilogue else None, epilogue=epilogue)
     check(c[:m], a, b, bias if epilogue else None, epilogue == 2, dtype)
     assert bool((c[m] == 7.0).all())                   # nothing past the last row
+
+
+@pytest.mark.parametrize("m,n,k,own", [
+    (64, 768, 1216, True), (64, 768, 1280, False), (1, 256, 16384, False), (1, 4096, 4096, False), (1, 4104, 4096, True),
+    (512, 512, 3072, False), (513, 512, 3072, True),
+])
+@pytest.mark.parametrize("epilogue", [0, 2])
+def test_long_reductions_with_few_outputs_go_to_the_library(capi, m, n, k, own, epilogue):
+    """They are slower as one chain of steps.  Which way a product went shows in the pair of events that the next launch
+    of the own kernels takes and a product of the library leaves waiting."""
+    print("gemm_bt route", m, n, k, epilogue, flush=True)
+    a, b, bias = operands(m, n, k, torch.float16)
+    c = torch.empty(m, n, dtype=torch.float16, device="cuda")
+    gemm = capi.Gemm()
+    gemm.set_tuning(1)
+    start, stop = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+    for e in (start, stop):
+        e.record()                                     # the handles exist from here on
+    assert capi.time_next_launch(start.cuda_event, stop.cuda_event) == 0
+    gemm.bt(a, b, c, bias=bias if epilogue else None, epilogue=epilogue)
+    assert capi.time_next_launch(None, None) == (0 if own else 1)
+    check(c, a, b, bias if epilogue else None, epilogue == 2, torch.float16)
 
 
 @pytest.mark.parametrize("heads,seq_lens,dtype", [
