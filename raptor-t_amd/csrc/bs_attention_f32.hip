@@ -31,8 +31,8 @@
 //
 // Bound by the matrix pipe at 1 540 cycles per tile and SIMD (with the cutting, 700 vector cycles, beside it) and, with
 // few units, by the longest row on one CU.  Measured (us, before: one tile at a time on v_mfma_f32_16x16x4_f32, units in flat
-// order): 12 heads x 1024 tokens 82 -> 32, x 4 x 2048 493 -> 142, x 128 + 832 + 1984 178 -> 68 (with truncated parts 30, 135,
-// 64); the error against 64 bits 5.0e-7 -> 3.0e-7 of the result (the longer steps of the matrix instruction add up fewer
+// order): 12 heads x 1024 tokens 82 -> 32, x 4 x 2048 493 -> 136, x 128 + 832 + 1984 178 -> 60 (the rounding of the parts
+// is 4 % of it); the error against 64 bits 5.0e-7 -> 3.0e-7 of the result (the longer steps of the matrix instruction add up fewer
 // partial sums), 0.4 to 0.65 of the fp32 instruction's over scores of size 0.1 to 10 and the mantissas above.
 #include <hip/hip_runtime.h>
 
@@ -105,33 +105,38 @@ __device__ __forceinline__ float group_sum(float v) {
 
 // Where a unit stands.
 struct Unit {
-  int g0, n, nbv, tail, block, h, p0, p1;        // its sequence's first block and blocks; see unit_at; its entries of the index
+  int g0, n, nbv, tail, block, h, p0, p1;        // its sequence's first block and blocks; see unit_of; its entries of the index
   int64_t head_base;                             // its head's tiles
 };
 
+// Row `i` of head h of sequence s, which has n blocks from g0 on.
+template <bool MASKED> __device__ __forceinline__ Unit unit_of(const ArgsF32& a, int s, int g0, int n, int h, int i) {
+  Unit u;
+  u.g0 = g0;
+  u.n = n;
+  u.h = h;
+  u.block = g0 + i;
+  // blocks that hold real tokens and the real tokens of the last of them; at least one (a tile with every key
+  // masked has no finite maximum); blocks from nbv on are padding as a whole and are left out
+  const int tokens = MASKED ? min(max(a.seq_tokens[s], 1), 64 * n) : 64 * n;
+  u.nbv = (tokens + 63) >> 6;
+  u.tail = tokens - 64 * (u.nbv - 1);
+  const int row = (a.plan_heads > 1 ? h : 0) * a.nb_total + u.block;
+  u.p0 = a.to_pos[row];
+  u.p1 = a.to_pos[row + 1];
+  u.head_base = (int64_t(g0) * a.heads + int64_t(h) * n) * 4096;
+  return u;
+}
+
+// flat unit id = block + head * n_s + first block of the sequence * heads
 template <bool MASKED> __device__ __forceinline__ Unit unit_at(const ArgsF32& a, int unit) {
-  // flat unit id = block + head * n_s + first block of the sequence * heads
   int lo = 0, hi = a.batch;
   while (hi - lo > 1) {
     const int mid = (lo + hi) >> 1;
     if (a.seq_blocks[mid] * a.heads <= unit) lo = mid; else hi = mid;
   }
-  Unit u;
-  u.g0 = a.seq_blocks[lo];
-  u.n = a.seq_blocks[lo + 1] - u.g0;
-  const int rem = unit - u.g0 * a.heads;
-  u.h = rem / u.n;
-  u.block = u.g0 + rem - u.h * u.n;
-  // blocks that hold real tokens and the real tokens of the last of them; at least one (a tile with every key
-  // masked has no finite maximum); blocks from nbv on are padding as a whole and are left out
-  const int tokens = MASKED ? min(max(a.seq_tokens[lo], 1), 64 * u.n) : 64 * u.n;
-  u.nbv = (tokens + 63) >> 6;
-  u.tail = tokens - 64 * (u.nbv - 1);
-  const int row = (a.plan_heads > 1 ? u.h : 0) * a.nb_total + u.block;
-  u.p0 = a.to_pos[row];
-  u.p1 = a.to_pos[row + 1];
-  u.head_base = (int64_t(u.g0) * a.heads + int64_t(u.h) * u.n) * 4096;
-  return u;
+  const int g0 = a.seq_blocks[lo], n = a.seq_blocks[lo + 1] - g0, rem = unit - g0 * a.heads, h = rem / n;
+  return unit_of<MASKED>(a, lo, g0, n, h, rem - h * n);
 }
 
 // The unit on fp32 matrix instructions, four waves, no overlap: the arithmetic of fp32 itself.
@@ -261,8 +266,7 @@ __device__ __forceinline__ f32x4 mma(const u32x4& a, const u32x4& b, const f32x4
 constexpr int PART_A[6] = {2, 1, 0, 1, 0, 0}, PART_B[6] = {0, 1, 2, 0, 1, 0};
 
 template <bool MASKED>
-__device__ void run_unit(const ArgsF32& a, int unit, char* smem) {
-  const Unit u = unit_at<MASKED>(a, unit);
+__device__ void run_unit(const ArgsF32& a, const Unit& u, char* smem) {
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int qcol = lane & 15, grp = lane >> 4, half = wave >> 2, dm = a.heads * 64;
 
@@ -460,30 +464,46 @@ __global__ __launch_bounds__(THREADS) void bs_attention_f32_kernel(ArgsF32 a) {
     const int end = min(max(a.from_pos[blockIdx.x + 1], begin), n_units);
     for (int p = begin; p < end; ++p) {
       const int unit = a.from_idx[p];
-      if (unit >= 0 && unit < n_units) run_unit<MASKED>(a, unit, smem);
+      if (unit >= 0 && unit < n_units) run_unit<MASKED>(a, unit_at<MASKED>(a, unit), smem);
     }
     return;
   }
   // Without a plan one unit per workgroup, the rows that list every block (the first and the last of a sequence) first:
-  // they take up to ten times as long as the others.  Slots: the two ends of every (sequence, head), then all units, of
-  // which the ends have been done.  Workgroups go to the XCDs round-robin: XCD x takes the x-th eighth of either list,
-  // so a head's tiles are read into one L2.  Measured at 12 heads x 4 x 2048: 346 us
-  // in flat order, 143 in this one.
-  const int ends = 2 * a.batch * a.heads, x = blockIdx.x & 7, slot = blockIdx.x >> 3, end_slots = (ends + 7) >> 3;
-  int unit;
-  if (slot < end_slots) {
-    const int e = x * end_slots + slot;
-    if (e >= ends) return;
-    const int seq = e / (2 * a.heads), h = (e >> 1) - seq * a.heads, g0 = a.seq_blocks[seq], n = a.seq_blocks[seq + 1] - g0;
-    if (n < 1 + (e & 1)) return;                       // a sequence of one row, or none
-    unit = g0 * a.heads + h * n + (e & 1 ? n - 1 : 0);
-  } else {
-    unit = x * ((n_units + 7) >> 3) + slot - end_slots;
-    if (slot - end_slots >= (n_units + 7) >> 3 || unit >= n_units) return;
-    const Unit u = unit_at<MASKED>(a, unit);
-    if (u.block == u.g0 || u.block == u.g0 + u.n - 1) return;
+  // they take up to ten times as long as the others.  Two lists, the two ends of every (sequence, head) and the rows
+  // between them.  Workgroups go to the XCDs round-robin: XCD x takes the x-th eighth of either list, so a head's tiles are
+  // read into one L2.  Measured at 12 heads x 4 x 2048: 346 us in flat order, 136 in this one.  Every workgroup has a unit: with
+  // a second list of all rows, whose ends returned at once, the workgroups at work came in a pattern that left a part
+  // of every XCD idle (12 heads x 60 x 256 tokens 188, 60 x 320 195, 60 x 64 37; now 133, 183, 20).
+  const int lane = threadIdx.x & 63, x = blockIdx.x & 7;
+  const unsigned long long upto = (2ull << lane) - 1ull;            // the lanes up to this one
+  int before = 0;                                                   // ends of earlier sequences
+  for (int s0 = 0; s0 < a.batch; s0 += 64) {
+    const int n = a.seq_blocks[min(s0 + lane + 1, a.batch)] - a.seq_blocks[min(s0 + lane, a.batch)];
+    before += __popcll(__ballot(n >= 1)) + __popcll(__ballot(n >= 2));
   }
-  run_unit<MASKED>(a, unit, smem);
+  const int64_t ends = int64_t(before) * a.heads, rows = n_units - ends;
+  const int end_lo = int(ends * x / 8), end_hi = int(ends * (x + 1) / 8), row_lo = int(rows * x / 8), row_hi = int(rows * (x + 1) / 8);
+  int j = int(blockIdx.x >> 3);
+  const bool is_end = j < end_hi - end_lo;
+  j = is_end ? j + end_lo : j - (end_hi - end_lo) + row_lo;
+  if (!is_end && j >= row_hi) return;
+  before = 0;
+  for (int s0 = 0; s0 < a.batch; s0 += 64) {
+    const int g0 = a.seq_blocks[min(s0 + lane, a.batch)], g1 = a.seq_blocks[min(s0 + lane + 1, a.batch)], n = g1 - g0;
+    const unsigned long long one = __ballot(n >= 1), two = __ballot(n >= 2);
+    const int ends_upto = before + __popcll(one & upto) + __popcll(two & upto);
+    const int count = is_end ? min(n, 2) : max(n - 2, 0), last = (is_end ? ends_upto : g1 - ends_upto) * a.heads;
+    const unsigned long long there = __ballot(last > j);
+    if (there) {
+      const int l = __builtin_ctzll(there), c = __builtin_amdgcn_readlane(count, l);
+      const int k = j - (__builtin_amdgcn_readlane(last, l) - c * a.heads), h = k / c, i = k - h * c;
+      const int first = __builtin_amdgcn_readlane(g0, l), blocks = __builtin_amdgcn_readlane(n, l);
+      if (first + blocks > a.nb_total) return;
+      run_unit<MASKED>(a, unit_of<MASKED>(a, s0 + l, first, blocks, h, !is_end ? i + 1 : i == 0 ? 0 : blocks - 1), smem);
+      return;
+    }
+    before += __popcll(one) + __popcll(two);
+  }
 }
 
 }  // namespace
@@ -497,8 +517,8 @@ int launch_attention_f32(const void* q, const void* q_rows, const void* q_bias, 
   const ArgsF32 a{(const float*)q, (const float*)k, (const float*)vt, (float*)out, seq_blocks_dev, batch, heads,
                   total_blocks, to_idx, to_pos, plan_heads, from_idx, from_pos, seq_tokens_dev,
                   (const float*)q_rows, (const float*)q_bias, q_scale};
-  const unsigned units = unsigned(total_blocks) * unsigned(heads), ends = 2u * unsigned(batch) * unsigned(heads);
-  const unsigned grid = from_idx ? unsigned(n_wg) : 8u * ((units + 7) / 8 + (ends + 7) / 8);
+  // an XCD's eighths of the two lists together: at most an eighth of the units and two more
+  const unsigned units = unsigned(total_blocks) * unsigned(heads), grid = from_idx ? unsigned(n_wg) : 8u * ((units + 14) / 8);
   hipStream_t st = static_cast<hipStream_t>(stream);
   if (seq_tokens_dev) RT_LAUNCH(bs_attention_f32_kernel<true>, dim3(grid), dim3(THREADS), 0, st, a);
   else RT_LAUNCH(bs_attention_f32_kernel<false>, dim3(grid), dim3(THREADS), 0, st, a);

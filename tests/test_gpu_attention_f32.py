@@ -26,6 +26,8 @@ def capi():
     (3, [64, 128, 192, 64], [1, 96, 161, 32], 1.0),             # no key, some and all keys in the upper half of the last tile
     (2, [768, 64 * 40], [768 - 31, 64 * 40 - 63], 3.0),         # sparse rows and global rows of 40 tiles
     (7, [832, 1088], [65, 1088], 1.0),                          # whole blocks of padding; unit counts no multiple of 8
+    (3, [64] * 70 + [192, 64, 448, 128], None, 1.0),            # more sequences than a wave looks up at a time, most of one row
+    (1, [256, 64] * 64 + [320], [256 - i for i in range(128)] + [300], 1.0),
 ])
 @pytest.mark.parametrize("n_wg", [0, 5])
 def test_fp32_attention(capi, heads, lens, tokens, scale, n_wg):
