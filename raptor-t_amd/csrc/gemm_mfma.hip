@@ -268,19 +268,20 @@ template <typename T> __device__ __forceinline__ T* half_tile(void* base, const 
   return static_cast<T*>(base) + (int64_t(g0) * p.heads + int64_t(h) * (end - g0) + (g - g0)) * 4096 + lane * 8;
 }
 
-// V^T tiles of head h (products taken with the tokens as rows): a lane's accumulators are 4 consecutive tokens of one
+// V^T tiles of head h from its column d0 (a multiple of 32) on (products taken with the tokens as rows): a lane's accumulators are 4 consecutive tokens of one
 // column; fragment 4 * (d >> 5) + (token >> 4) wants, in lane (d & 31) + 32 * x, the tokens 4 x .. + 4 and 8 + 4 x .. + 4
 // of its 16.
-template <typename T, int MT> __device__ __forceinline__ void store_v(const f32x4 (&acc)[MT][4], const Params& p, int seq_end, int m0, int h) {
+template <typename T, int MT, int NT>
+__device__ __forceinline__ void store_v(const f32x4 (&acc)[MT][NT], const Params& p, int seq_end, int m0, int h, int d0 = 0) {
 #pragma unroll
   for (int i = 0; i < MT; i += 2) {
     const int row = m0 + 16 * i;
     if (row >= p.m) break;
-    T* const t = half_tile<T>(p.vt, p, seq_end, row, h) + ((row >> 5) & 1) * 1024;
+    T* const t = half_tile<T>(p.vt, p, seq_end, row, h) + ((row >> 5) & 1) * 1024 + d0 * 64;
 #pragma unroll
     for (int q = 0; q < 2; ++q)
 #pragma unroll
-      for (int j = 0; j < 4; j += 2) {
+      for (int j = 0; j < NT; j += 2) {
         const f32x4 &c = acc[i + q][j], &d = acc[i + q][j + 1];
         uint32_t x0 = Mma<T>::two(c[0], c[1]), x1 = Mma<T>::two(c[2], c[3]);
         uint32_t y0 = Mma<T>::two(d[0], d[1]), y1 = Mma<T>::two(d[2], d[3]);
@@ -293,16 +294,17 @@ template <typename T, int MT> __device__ __forceinline__ void store_v(const f32x
   }
 }
 
-// K tiles of head h (products taken with the columns as rows): a lane's accumulators are 4 consecutive columns of one
+// K tiles of head h from its column d0 (a multiple of 16) on (products taken with the columns as rows): a lane's accumulators are 4 consecutive columns of one
 // token; fragment 4 * (token >> 5) + (d >> 4) wants, in lane (token & 31) + 32 * x, the columns 8 x .. + 8 of its 16.
-template <typename T, int MT> __device__ __forceinline__ void store_k(const f32x4 (&acc)[MT][4], const Params& p, int seq_end, int m0, int h) {
+template <typename T, int MT, int NT>
+__device__ __forceinline__ void store_k(const f32x4 (&acc)[MT][NT], const Params& p, int seq_end, int m0, int h, int d0 = 0) {
 #pragma unroll
   for (int i = 0; i < MT; i += 2) {
     const int row = m0 + 16 * i;
     if (row >= p.m) break;
-    T* const t = half_tile<T>(p.kt, p, seq_end, row, h) + ((row >> 5) & 1) * 2048;
+    T* const t = half_tile<T>(p.kt, p, seq_end, row, h) + ((row >> 5) & 1) * 2048 + d0 * 32;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
+    for (int j = 0; j < NT; ++j) {
       const f32x4 &c = acc[i][j], &d = acc[i + 1][j];
       uint32_t x0 = Mma<T>::two(c[0], c[1]), x1 = Mma<T>::two(c[2], c[3]);
       uint32_t y0 = Mma<T>::two(d[0], d[1]), y1 = Mma<T>::two(d[2], d[3]);
@@ -522,13 +524,13 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       if (EPI == EPI_QKV && v_tile) {
         asm volatile("; V tile");
         main_loop<T, TM, MT, EPI, true>(acc, c0, bias, next_bias, lda, ldb, st, p, sa, sb, smem, lds0, w, lane, offa, offb);
-        if (n0 < p.n) store_v<T, MT>(acc, p, bias.seq_end, m0, (n0 - 2 * dm) >> 6);
+        if (n0 < p.n) store_v<T>(acc, p, bias.seq_end, m0, (n0 - 2 * dm) >> 6);
         asm volatile("; V tile done");
         continue;
       }
       main_loop<T, TM, MT, EPI, false>(acc, c0, bias, next_bias, lda, ldb, st, p, sa, sb, smem, lds0, w, lane, offa, offb);
       if (EPI == EPI_QKV && n0 >= dm) {
-        store_k<T, MT>(acc, p, bias.seq_end, m0, (n0 - dm) >> 6);
+        store_k<T>(acc, p, bias.seq_end, m0, (n0 - dm) >> 6);
         asm volatile("; K tile done");
         continue;
       }
@@ -543,35 +545,119 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 }
 
 // ---- smaller products ------------------------------------------------------------------------------------------------
-// One workgroup of NW (4 or 8) waves per tile of TM x TC outputs and per slice of the reduction; a wave owns MT row blocks of 16
-// and 64 columns.  Where the kernel above would give too few CUs a tile each, what bounds a product is the latency of a
-// workgroup's chain of steps: STAGES of both operands are in flight, up to two workgroups share a CU, and a long
-// reduction is cut into slices (EPI_PART: the fp32 sums of slice s go to c[s][M][N] and the kernel that reads
-// them, the layer's LayerNorm, adds the slices).
-//   A step: fragments of half 1 requested, products of half 0; the own loads of the next step and the own reads of this
-//   one have arrived, barrier; fragments of the next step's half 0 and the loads of the step STAGES ahead requested,
-//   products of half 1.
-template <typename T, int TM, int TC, int NW, int STAGES, int EPI>
-__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) void gemm_bt_small_kernel(Params p) {
+// One workgroup per tile of TM x TC outputs and per slice of the reduction, WM x WN waves of MT x NT blocks of 16 x 16.
+// Where the kernel above would give too few CUs a tile each, what bounds a product is the latency of a workgroup's chain
+// of steps, and a wave issues in order: a memory instruction that has to wait for its unit holds up the matrix
+// instructions behind it.  So every step is laid out by hand, one product, then at most two fragment reads and a load:
+//   DEEP (small tiles)   both halves' fragments of step s+1 are read, into a second set of registers, between the products
+//                        of step s: one barrier per step, no LDS latency in the chain
+//   otherwise            fragments of half 1 are read between the products of half 0 (a row's in place, when its last product
+//                        has been issued), and those of the next step's half 0 behind the barrier in half 1
+// Between a step's barrier and the next the loads of the step STAGES ahead go to the stage that the barrier has freed.
+// The bias and the ends of the batch's sequences come to LDS ahead of the first stage, so the epilogue waits for no memory.
+// Slices (EPI_PART): the fp32 sums of slice s go to c[s][M][N] and the kernel that reads them, the layer's LayerNorm, adds
+// them.
+// Measured (us, one launch among others, fp16; before: the fragments of a half read in one burst, the loads in another, bias
+// and sequence ends loaded behind the loop): 512 x 2304 x 768 7.6 -> 5.1, 512 x 768 x 3072 15.1 -> 9.4, 2048 x 768 x 768
+// 7.9 -> 5.7, 4096 x 768 x 3072 25.4 -> 21.5, 5568 x 768 x 3072 33.9 -> 27.5, 8192 x 768 x 3072 42.6 -> 35.9.  A 64 x 64 step
+// takes 330 cycles (matrix instructions 140), a 128 x 128 one 700 (560), a 192 x 192 one 1450 (1260).
+template <typename T> struct Product;        // the instruction as a builtin: these accumulators leave registers to spare
+template <> struct Product<_Float16> {
+  __device__ static f32x4 run(f16x8 a, f16x8 b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0); }
+};
+template <> struct Product<__bf16> {
+  __device__ static f32x4 run(bf16x8 a, bf16x8 b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0); }
+};
+
+// 64 lanes x 4 bytes from srd[voff] to LDS bytes [lds, lds + 256), as load_to_lds
+__device__ inline void load_words_to_lds(i32x4 srd, int voff, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dword %0, %1, 0 offen lds" :: "v"(voff), "s"(srd), "s"(lds) : "memory");
+}
+
+// Rows of C (EPI_PART: of a slice, in fp32) as store_rows writes them, for any even NT: rows of the room lie 16 bytes further
+// apart than they are long, which puts the 16 rows of a write on different banks.
+template <int NT, int EPI> constexpr int block_pitch() { return NT * (EPI == EPI_PART ? 64 : 32) + 16; }
+template <typename T, int MT, int NT, int EPI>
+__device__ __forceinline__ void store_block(const f32x4 (&acc)[MT][NT], __amdgpu_buffer_rsrc_t sc, int n, int m0, int n0, char* room) {
+  static_assert(NT % 2 == 0, "whole stores");
+  constexpr int SIZE = EPI == EPI_PART ? 4 : 2, PER = 16 / SIZE;
+  constexpr int CH = NT * SIZE, PITCH = block_pitch<NT, EPI>(), ST = CH / 4;      // 16-byte chunks of a row, stores per 16 rows
+  const int lane = threadIdx.x & 63, l16 = lane & 15, g4 = lane >> 4;
+  uint32_t voff[ST], rows16[ST];
+  int rd[ST];
+#pragma unroll
+  for (int k = 0; k < ST; ++k) {
+    const int c = k * 64 + lane, row = c / CH, ch = c - row * CH;
+    const bool ok = n0 + ch * PER < n;
+    voff[k] = ok ? (uint32_t(m0 + row) * uint32_t(n) + uint32_t(n0 + ch * PER)) * uint32_t(SIZE) : 0xfffffff0u;
+    rows16[k] = ok ? uint32_t(n) * uint32_t(16 * SIZE) : 0u;
+    rd[k] = row * PITCH + ch * 16;
+  }
+  const int wr = l16 * PITCH + g4 * 4 * SIZE;
+#pragma unroll
+  for (int i = 0; i <= MT; ++i) {
+    u32x4 o[ST];
+    if (i > 0) {
+#pragma unroll
+      for (int k = 0; k < ST; ++k) o[k] = *reinterpret_cast<const u32x4*>(room + ((i - 1) & 1) * 16 * PITCH + rd[k]);
+    }
+    if (i < MT) {
+#pragma unroll
+      for (int j = 0; j < NT; ++j) {
+        f32x4 v = acc[i][j];
+        char* const to = room + (i & 1) * 16 * PITCH + wr + j * 16 * SIZE;
+        if constexpr (EPI == EPI_PART) {
+          *reinterpret_cast<f32x4*>(to) = v;
+        } else {
+          if (EPI == EPI_GELU) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = gelu_tanh(v[e]);
+          }
+          *reinterpret_cast<u32x2*>(to) = u32x2{Mma<T>::two(v[0], v[1]), Mma<T>::two(v[2], v[3])};
+        }
+      }
+    }
+    if (i > 0) {
+#pragma unroll
+      for (int k = 0; k < ST; ++k) {
+        __builtin_amdgcn_raw_buffer_store_b128(o[k], sc, int(voff[k]), 0, 0);
+        voff[k] += rows16[k];
+      }
+    }
+    SB();
+  }
+}
+
+constexpr int SMALL_EXTRA = 1024 + 256;       // LDS behind the stages: the tile's bias, the ends of the first 64 sequences
+
+template <typename T, int MT, int NT, int WM, int WN, int STAGES, int EPI>
+__global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_bt_small_kernel(Params p) {
   typedef typename Mma<T>::v8 v8;
   extern __shared__ __align__(16) char smem[];
-  constexpr int WN = TC / 64, WM = NW / WN, MT = TM / 16 / WM;
+  constexpr int NW = WM * WN, TM = 16 * MT * WM, TC = 16 * NT * WN;
   constexpr int NA = TM / 8 / NW, NB = TC / 8 / NW, LOADS = NA + NB;      // load instructions of a wave and step
-  constexpr uint32_t STAGE = (TM + TC) * ROW;
-  static_assert(MT >= 1 && STAGES * STAGE >= NW * EPI_BYTES && NA >= 1 && NB >= 1, "tile");
+  constexpr uint32_t STAGE = (TM + TC) * ROW, BIAS = STAGES * STAGE, ENDS = BIAS + 1024;
+  constexpr bool DEEP = MT * NT <= 8;
+  static_assert(TM % (8 * NW) == 0 && TC % (8 * NW) == 0 && STAGES >= 2 && STAGES <= 4, "tile");
+  static_assert(NW * 32 * block_pitch<NT, EPI>() <= BIAS && TC * 2 <= 1024, "room");
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, l16 = lane & 15, g4 = lane >> 4;
   // XCD x takes the x-th eighth of the list: slice, groups of 8 row panels, column, panel
   const int tiles = p.tiles_m * p.tiles_n, total = tiles * p.slices, per = gridDim.x >> 3;
   const int id = int(blockIdx.x & 7) * per + int(blockIdx.x >> 3);
   if (id >= total) return;
-  const int slice = id / tiles, tile = id - slice * tiles;
+  const int slice = EPI == EPI_PART ? id / tiles : 0, tile = id - slice * tiles;
   constexpr int G = 8;
   const int grp = tile / (G * p.tiles_n), in = tile - grp * G * p.tiles_n, h = min(G, p.tiles_m - grp * G);
   const int tn = in / h, tm = grp * G + (in - tn * h);
-  const int all = p.k / BK, first = all * slice / p.slices, steps = all * (slice + 1) / p.slices - first;
+  const int all = p.k / BK, first = EPI == EPI_PART ? all * slice / p.slices : 0;
+  const int steps = (EPI == EPI_PART ? all * (slice + 1) / p.slices : all) - first;       // at least 2
 
   const uint32_t lds0 = uint32_t(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) char*)smem));
   const i32x4 sa = make_srd(p.a, uint32_t(p.m) * uint32_t(p.k) * 2u), sb = make_srd(p.bt, uint32_t(p.n) * uint32_t(p.k) * 2u);
+  if (EPI != EPI_PART && w == 0) {             // past the end of the bias, and where there is none, the range check gives zeros
+    load_to_lds(make_srd(p.bias, p.bias ? uint32_t(p.n) * 2u : 0u), tn * TC * 2 + lane * 16, 0, lds0 + BIAS);
+    if (EPI == EPI_QKV) load_words_to_lds(make_srd(p.seq_blocks, uint32_t(p.batch + 1) * 4u), min(lane + 1, p.batch) * 4, lds0 + ENDS);
+  }
   int va[NA], vb[NB];
   {
     const int r = w * 8 + (lane >> 3), chunk = ((lane & 7) ^ ((r >> 1) & 7)) * 16;
@@ -594,116 +680,184 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) vo
   for (int q = 0; q < STAGES; ++q)
     if (q < steps) issue(q, q * STAGE, 0, LOADS);
 
-  const int m0 = tm * TM + (w / WN) * 16 * MT, n0 = tn * TC + (w % WN) * 64, dm = p.heads * 64;
+  const int wm = w / WN, wn = w % WN;
+  const int m0 = tm * TM + wm * 16 * MT, n0 = tn * TC + wn * 16 * NT, dm = p.heads * 64;
   const bool v_tile = EPI == EPI_QKV && n0 >= 2 * dm;
   int offa[2], offb[2];
 #pragma unroll
   for (int kk = 0; kk < 2; ++kk) {
     const int c = ((4 * kk + g4) ^ (l16 >> 1)) << 4;
-    offa[kk] = ((w / WN) * 16 * MT + l16) * ROW + c;
-    offb[kk] = (TM + (w % WN) * 64 + l16) * ROW + c;
+    offa[kk] = (wm * 16 * MT + l16) * ROW + c;
+    offb[kk] = (TM + wn * 16 * NT + l16) * ROW + c;
   }
-  v8 a[2][MT], b[2][4];
-  f32x4 acc[MT][4];
-  auto read = [&](int kk, uint32_t stage) __attribute__((always_inline)) {
-    const char *la = smem + stage + offa[kk], *lb = smem + stage + offb[kk];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) b[kk][j] = *reinterpret_cast<const v8*>(lb + j * 16 * ROW);
-#pragma unroll
-    for (int i = 0; i < MT; ++i) a[kk][i] = *reinterpret_cast<const v8*>(la + i * 16 * ROW);
+  // all loads but those of the last `left` steps have landed, and the own reads
+  auto wait = [&](int left) __attribute__((always_inline)) {
+    if (STAGES > 3 && left == 3) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" :: "n"(3 * LOADS) : "memory");
+    else if (STAGES > 2 && left == 2) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" :: "n"(2 * LOADS) : "memory");
+    else if (left == 1) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" :: "n"(LOADS) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
   };
+  constexpr int SETS = DEEP ? 2 : 1, HALVES = DEEP ? 2 : 1;
+  v8 a[SETS][HALVES][MT], b[SETS][2][NT];         // DEEP: [parity of the step][half]; else the row fragments in place
+  f32x4 acc[MT][NT], c0[NT];
   auto loop = [&](auto v_tag) __attribute__((always_inline)) {
     constexpr bool V_TILE = decltype(v_tag)::value;
-    auto products = [&](int kk, int i, auto init) __attribute__((always_inline)) {
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int c = i & 1 ? 3 - j : j;
-        const v8 &x = V_TILE ? a[kk][i] : b[kk][c], &y = V_TILE ? b[kk][c] : a[kk][i];
-        if (decltype(init)::value) Mma<T>::zero(x, y, acc[i][c]);
-        else Mma<T>::run(x, y, acc[i][c]);
-      }
+    uint32_t cur = 0;
+    // product t of a half, the columns in alternating direction (fewer operand bits toggle); the first half's start from c0
+    auto product = [&](int set, int kk, int t, auto init) __attribute__((always_inline)) {
+      const int i = t / NT, j = t % NT, c = i & 1 ? NT - 1 - j : j;
+      const v8 &fa = a[set][DEEP ? kk : 0][i], &fb = b[set][kk][c];
+      acc[i][c] = Product<T>::run(V_TILE ? fa : fb, V_TILE ? fb : fa, decltype(init)::value && kk == 0 ? c0[c] : acc[i][c]);
       SB();
     };
-    uint32_t cur = 0;
-    auto step = [&](int s, auto init) __attribute__((always_inline)) {
-      read(1, cur);
+    auto read_a = [&](int set, int kk, int i, uint32_t stage) __attribute__((always_inline)) {
+      a[set][DEEP ? kk : 0][i] = *reinterpret_cast<const v8*>(smem + stage + offa[kk] + i * 16 * ROW);
       SB();
-      asm volatile("s_nop 1");
+    };
+    auto read_b = [&](int set, int kk, int j, uint32_t stage) __attribute__((always_inline)) {
+      b[set][kk][j] = *reinterpret_cast<const v8*>(smem + stage + offb[kk] + j * 16 * ROW);
+      SB();
+    };
+    // MORE: the step STAGES ahead exists; else it is looked at.  LAST: nothing follows
+    auto deep_step = [&](int s, auto set_tag, auto init, auto more_tag, auto last_tag) __attribute__((always_inline)) {
+      constexpr int SET = decltype(set_tag)::value, PROD = MT * NT, READS = 2 * (MT + NT);
+      constexpr bool MORE = decltype(more_tag)::value, LAST = decltype(last_tag)::value;
+      constexpr int AHEAD = 2 * PROD >= 16 ? 4 : 0, REST = 2 * PROD - AHEAD;      // products ahead of the barrier, behind it
+      constexpr int EACH = READS > REST || PROD <= 4 ? 2 : 1;                     // reads behind a product
+      const uint32_t nxt = cur == (STAGES - 1) * STAGE ? 0u : cur + STAGE;
 #pragma unroll
-      for (int i = 0; i < MT; ++i) products(0, i, init);
-      if (s + STAGES <= steps) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" :: "n"((STAGES - 2) * LOADS) : "memory");
-      else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+      for (int t = 0; t < AHEAD; ++t) product(SET, 0, t, init);
+      if (LAST) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");                // the epilogue's room lies in the stages
+      else if (MORE) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" :: "n"((STAGES - 2) * LOADS) : "memory");
+      else wait(min(STAGES - 2, steps - 2 - s));
       __builtin_amdgcn_s_barrier();
       SB();
-      const uint32_t nxt = cur == (STAGES - 1) * STAGE ? 0u : cur + STAGE;
-      if (s + 1 < steps) read(0, nxt);
-      SB();
-      const bool more = s + STAGES < steps;
-      constexpr int PER_ROW = (LOADS + MT - 1) / MT;
+      const bool more = MORE || (!LAST && s + STAGES < steps);
 #pragma unroll
-      for (int i = 0; i < MT; ++i) {
-        products(1, i, std::false_type());
-        if (more) issue(s + STAGES, cur, i * PER_ROW, (i + 1) * PER_ROW);
+      for (int t = AHEAD; t < 2 * PROD; ++t) {
+        product(SET, t / PROD, t % PROD, init);
+        if (LAST) continue;
+        const int u = t - AHEAD;
+#pragma unroll
+        for (int r = u * EACH; r < min(READS, (u + 1) * EACH); ++r) {
+          const int kk = r / (MT + NT), q = r % (MT + NT);
+          if (q < NT) read_b(SET ^ 1, kk, q, nxt);
+          else read_a(SET ^ 1, kk, q - NT, nxt);
+        }
+        const int from = (u * LOADS + REST - 1) / REST, to = ((u + 1) * LOADS + REST - 1) / REST;
+        if (from < to && more) issue(s + STAGES, cur, from, to);
         SB();
       }
       cur = nxt;
     };
-    if (STAGES <= steps) asm volatile("s_waitcnt vmcnt(%0)" :: "n"((STAGES - 1) * LOADS) : "memory");
-    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    auto step = [&](int s, auto init, auto more_tag, auto last_tag) __attribute__((always_inline)) {
+      constexpr bool MORE = decltype(more_tag)::value, LAST = decltype(last_tag)::value;
+      constexpr int AHEAD = MT >= 4 ? 1 : 0, REST = (MT - AHEAD) * NT, EVERY = REST >= 2 * NT ? 2 : 1;     // rows, products, reads of b
+      const uint32_t nxt = cur == (STAGES - 1) * STAGE ? 0u : cur + STAGE;
+#pragma unroll
+      for (int t = 0; t < MT * NT; ++t) {
+        product(0, 0, t, init);
+        if (t % 2 == 0 && t / 2 < NT) read_b(0, 1, t / 2, cur);
+        if (t % NT == NT - 1) read_a(0, 1, t / NT, cur);
+      }
+#pragma unroll
+      for (int t = 0; t < AHEAD * NT; ++t) product(0, 1, t, std::false_type());
+      if (MORE) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" :: "n"((STAGES - 2) * LOADS) : "memory");
+      else wait(LAST ? 0 : min(STAGES - 2, steps - 2 - s));
+      __builtin_amdgcn_s_barrier();
+      SB();
+      const bool more = MORE || (!LAST && s + STAGES < steps);
+#pragma unroll
+      for (int t = 0; t < REST; ++t) {
+        const int i = AHEAD + t / NT;
+        product(0, 1, AHEAD * NT + t, std::false_type());
+        if (LAST) continue;
+        if (t % EVERY == 0 && t / EVERY < NT) read_b(0, 0, t / EVERY, nxt);
+        if (t % NT == 0 && t / NT < AHEAD) read_a(0, 0, t / NT, nxt);
+        if (t % NT == NT - 1) read_a(0, 0, i, nxt);
+        const int from = (t * LOADS + REST - 1) / REST, to = ((t + 1) * LOADS + REST - 1) / REST;
+        if (from < to && more) issue(s + STAGES, cur, from, to);
+        SB();
+      }
+      cur = nxt;
+    };
+    wait(min(STAGES, steps) - 1);
     __builtin_amdgcn_s_barrier();
     SB();
-    read(0, 0);
-    step(0, std::true_type());
-#pragma clang loop unroll(disable)
-    for (int s = 1; s < steps; ++s) step(s, std::false_type());
-    asm volatile("s_nop 15\n\ts_nop 7");
+#pragma unroll
+    for (int kk = 0; kk < HALVES; ++kk) {
+#pragma unroll
+      for (int j = 0; j < NT; ++j) read_b(0, kk, j, 0);
+#pragma unroll
+      for (int i = 0; i < MT; ++i) read_a(0, kk, i, 0);
+    }
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+      const char* const bl = smem + BIAS + (wn * 16 * NT + 16 * j) * 2;
+      if (EPI == EPI_PART) {
+        c0[j] = f32x4(0.f);
+      } else if (V_TILE) {
+        c0[j] = f32x4(Mma<T>::lo(*reinterpret_cast<const uint16_t*>(bl + l16 * 2)));
+      } else {
+        const u32x2 x = *reinterpret_cast<const u32x2*>(bl + g4 * 8);
+        c0[j] = f32x4{Mma<T>::lo(x.x), Mma<T>::hi(x.x), Mma<T>::lo(x.y), Mma<T>::hi(x.y)};
+      }
+    }
     SB();
+    const std::true_type yes;
+    const std::false_type no;
+    int s = 1;
+    if constexpr (DEEP) {
+      const std::integral_constant<int, 0> even;
+      const std::integral_constant<int, 1> odd;
+      deep_step(0, even, yes, no, no);
+#pragma clang loop unroll(disable)
+      for (; s + 1 < steps - STAGES; s += 2) {
+        deep_step(s, odd, no, yes, no);
+        deep_step(s + 1, even, no, yes, no);
+      }
+#pragma clang loop unroll(disable)
+      for (; s + 1 < steps - 1; s += 2) {
+        deep_step(s, odd, no, no, no);
+        deep_step(s + 1, even, no, no, no);
+      }
+      if (s + 1 < steps) {
+        deep_step(s, odd, no, no, no);
+        deep_step(s + 1, even, no, no, yes);
+      } else {
+        deep_step(s, odd, no, no, yes);
+      }
+    } else {
+      step(0, yes, no, no);
+#pragma clang loop unroll(disable)
+      for (; s < steps - STAGES; ++s) step(s, no, yes, no);
+#pragma clang loop unroll(disable)
+      for (; s < steps - 1; ++s) step(s, no, no, no);
+      step(s, no, no, yes);
+    }
   };
   if (v_tile) loop(std::true_type());
   else loop(std::false_type());
   if (n0 >= p.n) return;
 
-  if (EPI == EPI_PART) {
-    // whole 64-byte runs: 4 consecutive columns per lane
+  char* const room = smem + w * 32 * block_pitch<NT, EPI>();
+  if constexpr (EPI == EPI_PART) {
     const __amdgpu_buffer_rsrc_t sc =
         __builtin_amdgcn_make_buffer_rsrc(static_cast<float*>(p.c) + int64_t(slice) * p.m * p.n, 0, uint32_t(p.m) * uint32_t(p.n) * 4u, 0x00020000);
-#pragma unroll
-    for (int i = 0; i < MT; ++i)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int col = n0 + 16 * j + 4 * g4;
-        const uint32_t voff = col < p.n ? (uint32_t(m0 + 16 * i + l16) * uint32_t(p.n) + uint32_t(col)) * 4u : 0xfffffff0u;
-        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, acc[i][j]), sc, int(voff), 0, 0);
-      }
+    store_block<T, MT, NT, EPI>(acc, sc, p.n, m0, n0, room);
     return;
   }
-  if (p.bias) {
-    const T* bp = static_cast<const T*>(p.bias);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      f32x4 c;
-      if (v_tile) {
-        c = f32x4(Mma<T>::lo(reinterpret_cast<const uint16_t*>(bp)[min(n0 + 16 * j + l16, p.n - 1)]));
-      } else {
-        const u32x2 x = *reinterpret_cast<const u32x2*>(bp + min(n0 + 16 * j + 4 * g4, p.n - 4));
-        c = f32x4{Mma<T>::lo(x.x), Mma<T>::hi(x.x), Mma<T>::lo(x.y), Mma<T>::hi(x.y)};
-      }
-#pragma unroll
-      for (int i = 0; i < MT; ++i)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) acc[i][j][e] += c[e];
+  if constexpr (EPI == EPI_QKV) {
+    static_assert(MT % 2 == 0 && (NT == 2 || NT == 4), "a wave's columns lie in one head");
+    if (n0 >= dm) {
+      const int seq_end = *reinterpret_cast<const int*>(smem + ENDS + lane * 4), col = n0 - (v_tile ? 2 : 1) * dm;
+      if (v_tile) store_v<T>(acc, p, seq_end, m0, col >> 6, col & 63);
+      else store_k<T>(acc, p, seq_end, m0, col >> 6, col & 63);
+      return;
     }
-  }
-  if (EPI == EPI_QKV && n0 >= dm) {
-    const int seq_end = p.seq_blocks[min(lane + 1, p.batch)];
-    if constexpr (MT % 2 == 0) {
-      if (v_tile) store_v<T, MT>(acc, p, seq_end, m0, (n0 - 2 * dm) >> 6);
-      else store_k<T, MT>(acc, p, seq_end, m0, (n0 - dm) >> 6);
-    }
-    return;
   }
   const __amdgpu_buffer_rsrc_t sc = __builtin_amdgcn_make_buffer_rsrc(p.c, 0, uint32_t(p.m) * uint32_t(p.n) * 2u, 0x00020000);
-  store_rows<T, MT, EPI, 0>(acc, sc, p.n, m0, n0, smem + w * EPI_BYTES);
+  store_block<T, MT, NT, EPI>(acc, sc, p.n, m0, n0, room);
 }
 
 // More dynamic LDS than the default has to be asked for once per kernel and device.
@@ -735,47 +889,54 @@ template <typename T, int TM, int MT0, int MT1, int EPI> int launch(const Params
   return launched();
 }
 
-template <typename T, int TM, int TC, int NW, int STAGES, int EPI> int launch_small(const Params& base, hipStream_t st) {
+template <typename T, int MT, int NT, int WM, int WN, int STAGES, int EPI> int launch_small(const Params& base, hipStream_t st) {
+  constexpr int TM = 16 * MT * WM, TC = 16 * NT * WN, LDS = STAGES * (TM + TC) * ROW + SMALL_EXTRA;
   Params p = base;
   p.tiles_m = (p.m + TM - 1) / TM;
   p.tiles_n = (p.n + TC - 1) / TC;
-  constexpr int LDS = STAGES * (TM + TC) * ROW;
   static std::atomic<uint64_t> done{0};
-  if (int rc = allow_lds(&gemm_bt_small_kernel<T, TM, TC, NW, STAGES, EPI>, LDS, done)) return rc;
+  if (int rc = allow_lds(&gemm_bt_small_kernel<T, MT, NT, WM, WN, STAGES, EPI>, LDS, done)) return rc;
   const int total = p.tiles_m * p.tiles_n * p.slices;
-  RT_LAUNCH((gemm_bt_small_kernel<T, TM, TC, NW, STAGES, EPI>), dim3((total + 7) / 8 * 8), dim3(64 * NW), LDS, st, p);
+  RT_LAUNCH((gemm_bt_small_kernel<T, MT, NT, WM, WN, STAGES, EPI>), dim3((total + 7) / 8 * 8), dim3(64 * WM * WN), LDS, st, p);
   return launched();
 }
 
 // ---- which kernel ----------------------------------------------------------------------------------------------------
-// A product's time is estimated for every kernel and number of slices from a model with three measured figures
-// each (microseconds, random fp16 operands): one step of a workgroup that has its CU to itself, how much longer it
-// takes when every CU has one, and a step of two workgroups that share a CU; plus the launch, its first loads and its
-// epilogue.  Where the lines fall, with both sides measured (us, before: hipBLASLt):
-//   512 x 2304 x 768    128 x 64: 7.0, 192 x 256: 13.7 (15.8)     4096 x 2304 x 768  192 x 256: 17.1, 128 x 64: 23 (21)
-//   512 x 768 x 3072    64 x 64 in 4 slices: 8.1, uncut 15.3 (16) 5568 x 768 x 3072  192 x 128: 33.6, 128 x 128: 41 (36)
-//   4096 x 768 x 3072   128 x 128: 27.4, 64 x 64: 34 (28.6)       8192 x 768 x 3072  256 x 128: 43, 192 x 256: 46 (41)
-// Both sides again for every kernel at 13 shapes (512-37184 rows, N 768-3072, K 768 and 3072) in fp16 and in bf16: bf16 is 0-6 %
-// faster throughout and the kernels stand in the same order, but for pairs within 3 %; what the rule picks is the
-// fastest or within 5 % of it in both types.
+// A product's time is estimated for every kernel and number of slices from a model with measured figures for each
+// (microseconds, random fp16 operands, weights and activations in rotation through 180 MB and up to 340 MB, as a stack of
+// layers finds them: with one set of operands in the caches the long reductions run a quarter faster and slices do not pay):
+// one step of a workgroup that has its CU to itself, how much longer it takes when every CU has one, a step of two workgroups
+// that share a CU, the launch, and what each round of workgroups spends on its first loads and its epilogue; plus the GELU
+// by the outputs of a round, and the slices' way to memory and back.  The figures are a least-squares fit to 940 launches
+// (15 row counts from 64 to 37184 at hidden 768, five from 128 to 40768 at 1024, all four products of a layer, up to six
+// slices; root mean square of the error 7 %), over which the kernel that the model picks is 0.6 % slower than the fastest on
+// average; with the LayerNorm behind it (20 row counts, up to eight slices) 1.3 %.  Where the lines fall, both sides (us):
+//   512 x 3072 x 768 + GELU   128 x 64: 6.9, 64 x 64: 7.2, 128 x 128: 8.5    1024 x 2304 x 768 split   128 x 128: 8.3, 128 x 64: 9.1
+//   2816 x 2304 x 768 split   128 x 256: 14.6, 128 x 128: 16.1, 192 x 256: 18.2    4096 x 2304 x 768 split   192 x 256: 21.2, 128 x 256: 23.9
+//   2816 x 3072 x 768 + GELU  192 x 192: 17.5, 192 x 256: 18.0    8192 x 768 x 3072   128 x 192: 39.2, 192 x 192: 44.9, 192 x 256: 61.5
+//   with the LayerNorm: 512 x 768 x 3072   2 slices of 64 x 64: 11.7, uncut 14.3    2816 x 768 x 3072   2 slices of 192 x 128: 28.8,
+//   uncut 32.5    4096 x 768 x 3072   uncut 35.2, 2 slices 42.4
 struct Choice {
-  int tm, tc, waves, stages, slices;
+  int tm, tc, slices;
 };
 struct Kernel {
   Choice c;
   float step, crowd, pair;      // pair 0: one workgroup per CU
-  float fixed;                  // per round
-  bool qkv;                     // has the head split (which needs 32 rows per wave)
+  float launch, round;
+  bool qkv, part;               // has the head split (32 rows and half a head per wave); writes slices
 };
 const Kernel kKernels[] = {
-    {{256, 256, 8, 0, 1}, 1.05f, 0.20f, 0.f, 4.4f, true},
-    {{224, 256, 8, 0, 1}, 0.90f, 0.18f, 0.f, 4.2f, true},
-    {{192, 256, 8, 0, 1}, 0.78f, 0.16f, 0.f, 4.0f, true},
-    {{256, 128, 8, 3, 1}, 0.69f, 0.12f, 0.f, 3.4f, true},
-    {{192, 128, 8, 3, 1}, 0.58f, 0.11f, 0.f, 3.4f, false},
-    {{128, 128, 8, 4, 1}, 0.41f, 0.15f, 0.f, 3.4f, true},
-    {{128, 64, 4, 3, 1}, 0.35f, 0.02f, 0.54f, 3.4f, true},
-    {{64, 64, 4, 4, 1}, 0.27f, 0.02f, 0.37f, 3.4f, false},
+    {{256, 256, 1}, 1.072f, 0.467f, 0.f, 2.75f, 2.55f, true, false},
+    {{224, 256, 1}, 0.927f, 0.544f, 0.f, 3.55f, 1.30f, true, false},
+    {{192, 256, 1}, 0.830f, 0.559f, 0.f, 4.10f, 0.40f, true, false},
+    {{192, 192, 1}, 0.594f, 0.416f, 0.f, 1.75f, 2.30f, false, false},
+    {{128, 256, 1}, 0.605f, 0.394f, 0.f, 1.90f, 1.30f, true, false},
+    {{192, 128, 1}, 0.475f, 0.301f, 0.f, 1.95f, 1.20f, false, true},
+    {{128, 192, 1}, 0.463f, 0.328f, 0.f, 2.05f, 1.15f, false, false},
+    {{128, 128, 1}, 0.328f, 0.265f, 0.f, 2.45f, 0.85f, true, true},
+    {{128, 64, 1}, 0.267f, 0.150f, 0.631f, 1.60f, 0.90f, true, true},
+    {{96, 64, 1}, 0.243f, 0.104f, 0.532f, 1.70f, 0.65f, false, true},
+    {{64, 64, 1}, 0.162f, 0.081f, 0.404f, 2.05f, 0.55f, true, true},
 };
 
 // max_slices 1: the caller takes the product itself; more: fp32 slices will do, which the caller's next kernel reads.
@@ -785,14 +946,15 @@ Choice choose(int64_t m, int64_t n, int64_t k, int epi, int max_slices) {
   float best_us = 0.f;
   for (const Kernel& kn : kKernels) {
     if (epi == EPI_QKV && !kn.qkv) continue;
-    for (int s = 1; s <= (kn.c.stages == 0 ? 1 : max_slices); ++s) {
+    for (int s = 1; s <= (kn.part ? max_slices : 1); ++s) {
       if (s > 1 && steps / s < 6) break;
       const int64_t wgs = ((m + kn.c.tm - 1) / kn.c.tm) * ((n + kn.c.tc - 1) / kn.c.tc) * s;
-      const int64_t slots = kn.pair > 0.f ? 512 : 256, full = wgs / slots, rest = wgs % slots;
+      const int64_t slots = kn.pair > 0.f ? 512 : 256, full = wgs / slots, rest = wgs % slots, rounds = full + (rest ? 1 : 0);
       const float alone = kn.step + kn.crowd * float(rest < 256 ? rest : 256) / 256.f, both = kn.pair > 0.f ? kn.pair : kn.step + kn.crowd;
-      const float rounds = float(full) * both + (rest == 0 ? 0.f : rest <= 256 ? alone : both);
-      float us = rounds * float((steps + s - 1) / s) + kn.fixed * float(full + (rest ? 1 : 0));
-      if (s > 1) us += float(m) * float(n) * float(8 * s - 4) * 2e-7f;      // the slices' way to memory and back at 5 TB/s
+      const float stepping = float(full) * both + (rest == 0 ? 0.f : rest <= 256 ? alone : both);
+      float us = kn.launch + kn.round * float(rounds) + stepping * float((steps + s - 1) / s);
+      if (epi == EPI_GELU) us += 2.9e-5f * float(kn.c.tm * kn.c.tc) * float(rounds) * (kn.pair > 0.f && full ? 2.f : 1.f);
+      if (s > 1) us += 0.6f + float(m) * float(n) * (1.7e-6f * float(s) - 1.4e-6f);       // against 16 bits to the LayerNorm
       if (best_us == 0.f || us < best_us) { best_us = us; best = kn.c; best.slices = s; }
     }
   }
@@ -802,23 +964,24 @@ Choice choose(int64_t m, int64_t n, int64_t k, int epi, int max_slices) {
 template <typename T, int EPI> int dispatch(Params& p, const Choice& c, hipStream_t st) {
   p.slices = c.slices;
   if constexpr (EPI != EPI_PART) {
-    if (c.tc == TN) {
+    if (c.tc == TN && c.tm >= 192) {
       if (c.tm == 256) return launch<T, 256, 8, 8, EPI>(p, st);
       if (c.tm == 224) return launch<T, 224, 8, 6, EPI>(p, st);
       return launch<T, 192, 6, 6, EPI>(p, st);
     }
+    if (c.tc == 256) return launch_small<T, 4, 4, 2, 4, 3, EPI>(p, st);
   }
-  if (c.tc == 128) {
-    if (c.tm == 256) return launch_small<T, 256, 128, 8, 3, EPI>(p, st);
-    if constexpr (EPI != EPI_QKV) {
-      if (c.tm == 192) return launch_small<T, 192, 128, 8, 3, EPI>(p, st);
-    }
-    return launch_small<T, 128, 128, 8, 4, EPI>(p, st);
+  if constexpr (EPI == EPI_NONE || EPI == EPI_GELU) {
+    if (c.tc == 192 && c.tm == 192) return launch_small<T, 3, 6, 4, 2, 3, EPI>(p, st);
+    if (c.tc == 192) return launch_small<T, 2, 6, 4, 2, 3, EPI>(p, st);
   }
   if constexpr (EPI != EPI_QKV) {
-    if (c.tm == 64) return launch_small<T, 64, 64, 4, 4, EPI>(p, st);
+    if (c.tm == 192) return launch_small<T, 6, 2, 2, 4, 3, EPI>(p, st);
+    if (c.tm == 96) return launch_small<T, 3, 2, 2, 2, 3, EPI>(p, st);
   }
-  return launch_small<T, 128, 64, 4, 3, EPI>(p, st);
+  if (c.tc == 128) return launch_small<T, 2, 4, 4, 2, 4, EPI>(p, st);
+  if (c.tm == 128) return launch_small<T, 4, 2, 2, 2, 3, EPI>(p, st);
+  return launch_small<T, 2, 2, 2, 2, 4, EPI>(p, st);
 }
 
 }  // namespace

@@ -42,15 +42,15 @@ def check(got, a, b, bias, gelu, dtype):
 
 
 @pytest.mark.parametrize("m,n,k,dtype", [
-    (12288, 256, 128, torch.float16),       # 128 x 128, the shortest reduction
-    (12295, 264, 192, torch.bfloat16),      # 128 x 64, odd number of steps; 8 columns and 7 rows in tiles of their own
-    (9409, 520, 768, torch.float16),        # 192 x 128: one row in the last panel
-    (16384 + 33, 1000, 256, torch.bfloat16),        # 192 x 256
+    (12288, 256, 128, torch.float16),       # whole tiles, the shortest reduction
+    (12295, 264, 192, torch.bfloat16),      # odd number of steps; 8 columns and 7 rows in tiles of their own
+    (9409, 520, 768, torch.float16),        # 128 x 192
+    (16384 + 33, 1000, 256, torch.bfloat16),        # 192 x 128
     # More tiles than workgroups with the shortest reductions: a tile's first step is followed by its last (two steps, loads
     # reach into the tile after the next) or by one more (three); one row, 8 columns in the last tiles
     (8065, 2312, 128, torch.float16),       # 192 x 256
-    (16353, 2304, 128, torch.bfloat16),     # 224 x 256
-    (12289, 2312, 128, torch.float16),      # 256 x 256
+    (16353, 2304, 128, torch.bfloat16),     # 192 x 256, with GELU 224 x 256
+    (12289, 2312, 128, torch.float16),
     (8065, 2312, 192, torch.bfloat16),
     (12321, 3080, 192, torch.float16),
     (1, 8, 128, torch.float16),             # one row, one chunk of columns
@@ -58,8 +58,8 @@ def check(got, a, b, bias, gelu, dtype):
     (333, 776, 768, torch.float16),         # tiles of 64 x 64
     (64, 5120, 1280, torch.bfloat16),
     (700, 2312, 192, torch.float16),        # tiles of 128 x 64
-    (1500, 2304, 768, torch.bfloat16),      # 128 x 128
-    (2049, 3080, 320, torch.float16),       # 256 x 128
+    (1500, 2304, 768, torch.bfloat16),      # 128 x 128, with GELU 128 x 64
+    (2049, 3080, 320, torch.float16),       # 128 x 256
     (5600, 768, 1024, torch.bfloat16),      # 192 x 128
 ])
 @pytest.mark.parametrize("epilogue", [0, 1, 2])
@@ -70,6 +70,31 @@ def test_gemm_bt_edges(capi, m, n, k, dtype, epilogue):
     capi.Gemm().bt(a, b, c[:m], bias=bias if epilogue else None, epilogue=epilogue)
     check(c[:m], a, b, bias if epilogue else None, epilogue == 2, dtype)
     assert bool((c[m] == 7.0).all())                   # nothing past the last row
+
+
+# One row in the last panel and 8 columns in the last tile of every kernel (the model's choice for the shape), with as many
+# steps as its stages hold, fewer, and more, in odd and even number.
+@pytest.mark.parametrize("m,n,k", [
+    (1, 8, 192), (65, 72, 256), (65, 72, 320), (513, 520, 704),                                  # 64 x 64, four stages
+    (1, 8, 128), (97, 72, 128), (9217, 72, 192), (9217, 72, 256), (9217, 72, 320),               # 96 x 64, three
+    (12289, 72, 128), (12289, 72, 192), (12289, 72, 256), (12289, 72, 448),                      # 128 x 64, three
+    (1537, 1928, 768), (1537, 1928, 832),                                                        # 128 x 128
+    (2305, 1672, 128), (2305, 1672, 192), (2305, 1672, 256), (2305, 1672, 320),                  # 192 x 128, three
+    (7297, 520, 192), (7297, 520, 256), (7297, 520, 320),                                        # 128 x 192, three
+    (2049, 3080, 128), (2049, 3080, 192), (2049, 3080, 256), (2049, 3080, 448),                  # 128 x 256, three
+    (4609, 1736, 128), (4609, 1544, 192), (4609, 1544, 256), (4609, 1544, 320),                  # 192 x 192, three
+    (8193, 1544, 128), (16513, 1544, 192),                                                       # 256 x 256, one round and two
+    (3585, 3336, 128), (16513, 1288, 128),                                                       # 224 x 256
+])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_gemm_bt_every_tile(capi, m, n, k, dtype):
+    print("gemm_bt tile", m, n, k, dtype, flush=True)
+    a, b, bias = operands(m, n, k, dtype, seed=4)
+    c = torch.full((m + 1, n), 7.0, dtype=dtype, device="cuda")
+    gelu = dtype == torch.float16
+    capi.Gemm().bt(a, b, c[:m], bias=bias, epilogue=2 if gelu else 1)
+    check(c[:m], a, b, bias, gelu, dtype)
+    assert bool((c[m] == 7.0).all())
 
 
 @pytest.mark.parametrize("m,n,k,own", [
@@ -98,11 +123,16 @@ def test_long_reductions_with_few_outputs_go_to_the_library(capi, m, n, k, own, 
     (12, [832, 64, 3008, 1024], torch.float16),
     (5, [64] * 70 + [2048], torch.bfloat16),          # more sequences than one wave looks up at a time, K and V halves of a tile
     (16, [4096, 320], torch.float16),
-    (2, [64], torch.float16),                         # half a tile of 128 x 64
+    (2, [64], torch.float16),                         # 64 x 64
     (12, [192, 320], torch.bfloat16),
+    (2, [192], torch.bfloat16),                       # 64 x 64
+    (3, [64, 256], torch.float16),
+    (3, [2112], torch.bfloat16),                      # 128 x 64, the last panel half full
+    (9, [1216], torch.float16),                       # 128 x 128: the same, and columns past the end
+    (7, [3136], torch.bfloat16),                      # 128 x 256: the same
     (7, [960, 576], torch.float16),                   # 128 x 64, 252 of 256 workgroups
     (7, [960, 640], torch.float16),                   # 128 x 128
-    (12, [2048, 1088], torch.bfloat16),               # 256 x 128
+    (12, [2048, 1088], torch.bfloat16),               # 128 x 256
     # More tiles than workgroups, so that a tile is followed by another one, where some waves store nothing of it:
     (6, [14464], torch.float16),                      # tiles of 192: columns past the end, and a last panel with its lower half past the end
     (10, [4096, 4096, 4160], torch.bfloat16),         # 224: the same
@@ -132,6 +162,11 @@ def test_qkv_project_equals_gemm_and_split(capi, heads, seq_lens, dtype):
     (1500, 1024, 4096, torch.bfloat16),
     (2816, 768, 3072, torch.float16),
     (1000, 512, 448, torch.float16),                  # seven steps
+    (1, 256, 2048, torch.bfloat16),                   # 64 x 64: slices of six and seven steps
+    (1441, 512, 3136, torch.float16),                 # 96 x 64: 24 and 25
+    (1025, 512, 3136, torch.bfloat16),                # 128 x 64: 16 and 17, one row in the last panel
+    (1025, 1024, 3136, torch.float16),                # 128 x 128
+    (2881, 768, 3136, torch.bfloat16),                # 192 x 128
     (64, 320, 1280, torch.float16),                   # a width the slices' LayerNorm does not have
     (9000, 768, 768, torch.float16),                  # enough rows: not cut
 ])
