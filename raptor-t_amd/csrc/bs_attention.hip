@@ -1314,6 +1314,7 @@ __global__ __launch_bounds__(256, 2) void bs_attention_kernel(Args<T> a) {
 // (8 tiles, 13 us) or a global row's (a quarter of the sequence's blocks).  Here a unit's tiles are shared by several waves,
 // whose states merge through LDS: one workgroup of 8 waves (one per CU) takes one global row, or RPW other rows with
 // 8 / RPW waves each (rows_per_workgroup has the rule and the times of both kernels).  At most 64 sequences (a lane each).
+constexpr int FEW_CUS = 256;
 template <typename T, int NW> struct FewRoom {
   // four wave states in a merge; each wave's room for a query tile
   static constexpr int PARK = 4 * PARK_FLOATS > NW * Q_STAGE_BYTES / 4 ? 4 * PARK_FLOATS : NW * Q_STAGE_BYTES / 4;
@@ -1348,6 +1349,16 @@ template <typename T> struct FewBatch {
     }
     return u;
   }
+  // Shares of a global row: eight, one workgroup of eight waves per row; or four, the two global rows of a (sequence, head) in one
+  // workgroup, where that saves a round of workgroups, unless one would be a longer chain (16 tiles) than the other rows' two
+  // rounds.  Measured (us, eight shares / four, 12 heads): three sequences of 8704 tokens in all 31.8 / 26.3, four of 9344 30.8 /
+  // 27.3, six of 8512 27.0 / 21.8, bf16 padded 5 x 320-3000 31.6 / 27.8; where the rounds stay as many, six of 9600 28.4 / 33.6,
+  // five of 11008 31.3 / 34.7.
+  __device__ __forceinline__ int global_shares(const Args<T>& a, int n_sparse, int rows_per_wg) const {
+    const int pairs = n_sparse * a.heads, others = (a.nb_total * a.heads - 2 * pairs + rows_per_wg - 1) / rows_per_wg;
+    const bool fewer = (pairs + others - 1) / FEW_CUS < (2 * pairs + others - 1) / FEW_CUS;
+    return fewer && !__any(lane < a.batch && sb1 - sb0 > 64) ? 4 : 8;
+  }
   // sequence of a position in a per-lane ascending prefix (lane s: first position of sequence s)
   __device__ __forceinline__ int seq_of(const Args<T>& a, int prefix, int x) const {
     return __popcll(__ballot(lane < a.batch && prefix <= x)) - 1;
@@ -1364,13 +1375,13 @@ template <typename T> __device__ __forceinline__ Buffers<T> few_buffers(const Ar
   return b;
 }
 
-// The workgroup's NW waves on their rows, from the first tile to the output.  `whole`: unit u is the same in all
-// waves, which take its eight shares; else 8 / RPW waves (but no more than there are) take the shares of one row and u is
-// theirs.  `valid`: the wave has a row.
+// The workgroup's NW waves on their rows, from the first tile to the output: a row's tiles in `share` shares (the same number
+// in all waves; 8 where RPW is 1), taken by that many waves side by side, or by all NW if there are fewer.  u: the
+// wave's row; `valid`: it has one.
 template <typename T, bool MASKED, int RPW, int NW>
 __device__ __forceinline__ void share_rows(const Args<T>& a, const Buffers<T>& b, FewRoom<T, NW>& room, const QSide<T>& qbias,
-                                           const Unit& u, bool valid, bool whole, int lane, int wave) {
-  const int share = whole ? 8 : 8 / RPW, waves = share < NW ? share : NW, row = wave / waves, part = wave - row * waves;
+                                           const Unit& u, bool valid, int share, int lane, int wave) {
+  const int waves = share < NW ? share : NW, row = wave / waves, part = wave - row * waves;
   const Row r = describe<T>(a, u);
   State st;
   if (NW < 8 && share > NW) {
@@ -1408,7 +1419,7 @@ __device__ __forceinline__ void share_rows(const Args<T>& a, const Buffers<T>& b
   }
 #pragma unroll
   for (int half = NW / 2; half >= 1; half >>= 1) {
-    if (2 * half > 8 / RPW && !whole) continue;
+    if (2 * half > share) continue;
     __syncthreads();                                   // the park is free
     float* const place = room.park + (row * half + (part & (half - 1))) * PARK_FLOATS;
     if (part >= half && part < 2 * half) park_state(st, place, lane);
@@ -1442,14 +1453,15 @@ __global__ __launch_bounds__(512, 2) void bs_attention_few_kernel(Args<T> a) {
   Unit u;
   bool valid = true;
   const int n_pairs = n_sparse * a.heads;
-  const int p_lo = int(int64_t(n_pairs) * xcd / 8), p_hi = int(int64_t(n_pairs) * (xcd + 1) / 8), n_glob = 2 * (p_hi - p_lo);
-  const bool whole = slot < n_glob;
-  if (whole) {
-    const int pair = p_lo + (slot >> 1), h = pair / n_sparse, k = pair - h * n_sparse;
+  const int p_lo = int(int64_t(n_pairs) * xcd / 8), p_hi = int(int64_t(n_pairs) * (xcd + 1) / 8);
+  const int shares = batch.global_shares(a, n_sparse, RPW), n_glob = shares == 8 ? 2 * (p_hi - p_lo) : p_hi - p_lo;
+  const bool global = slot < n_glob;
+  if (global) {
+    const int pair = p_lo + (shares == 8 ? slot >> 1 : slot), h = pair / n_sparse, k = pair - h * n_sparse;
     // the k-th sparse sequence
     const int s = __builtin_ctzll(__ballot((sparse >> lane & 1ull) && __popcll(sparse & ((1ull << lane) - 1ull)) == k));
     u = batch.template unit_at<MASKED>(a, s, h, 0);
-    if (slot & 1) u.i = u.n - 1;
+    if (shares == 8 ? slot & 1 : wave >> 2) u.i = u.n - 1;
   } else {
     const int total = n_rows * a.heads;
     const int lo = int(int64_t(total) * xcd / 8), hi = int(int64_t(total) * (xcd + 1) / 8);
@@ -1464,7 +1476,7 @@ __global__ __launch_bounds__(512, 2) void bs_attention_few_kernel(Args<T> a) {
     u.i = j - __builtin_amdgcn_readlane(listed_before, s) + ((sparse >> s & 1ull) ? 1 : 0);
   }
   __syncthreads();
-  share_rows<T, MASKED, RPW, 8>(a, few_buffers(a), room, qbias, u, valid, whole, lane, wave);
+  share_rows<T, MASKED, RPW, 8>(a, few_buffers(a), room, qbias, u, valid, global ? shares : 8 / RPW, lane, wave);
 }
 
 // With a caller's plan workgroup c walks its slice, as in the persistent kernel: four waves, two workgroups per CU, a global
@@ -1486,6 +1498,8 @@ __global__ __launch_bounds__(256, 2) void bs_attention_few_plan_kernel(Args<T> a
   const FewBatch<T> batch(a, room);
   const QSide<T> qbias{room.qbias, reinterpret_cast<char*>(room.park) + wave * Q_STAGE_BYTES};
   const Buffers<T> b = few_buffers(a);
+  const int shares =
+      batch.global_shares(a, __popcll(__ballot(batch.lane < a.batch && batch.sb1 - batch.sb0 >= RT_MIN_SPARSE_BLOCKS)), RPW);
   auto unit_of_flat = [&](int id) {
     const int s = batch.seq_of(a, batch.sb0 * a.heads, id);
     const int g0 = __builtin_amdgcn_readlane(batch.sb0, s), n = __builtin_amdgcn_readlane(batch.sb1, s) - g0;
@@ -1519,7 +1533,7 @@ __global__ __launch_bounds__(256, 2) void bs_attention_few_plan_kernel(Args<T> a
     }
     if (threadIdx.x < 8) room.failed[threadIdx.x] = 0;           // (the last rows' flags were read several barriers ago)
     __syncthreads();
-    share_rows<T, MASKED, RPW, 4>(a, b, room, qbias, u, whole || SIDE * wave / 4 < run, whole, batch.lane, wave);
+    share_rows<T, MASKED, RPW, 4>(a, b, room, qbias, u, whole || SIDE * wave / 4 < run, whole ? shares : 8 / RPW, batch.lane, wave);
     p += run;
   }
 }

@@ -26,6 +26,9 @@ def capi():
     (5, [2048, 832, 64], 40.0),                       # scores beyond the pipelined loop's range
     (12, [256, 1024, 640, 896], 1.0),                 # 2 waves to a row
     (12, [2048, 3008, 384], 1.0),                     # a wave to a row, global rows by 8 waves
+    (12, [2944, 3008, 2752], 1.0),                    # the two global rows of a head in one workgroup, by 4 waves each
+    (12, [4096, 2624, 1984], 40.0),                   # the same at the longest sequence that takes them so
+    (12, [4160, 2560, 1984], 1.0),                    # one block longer: by 8 waves each, in two rounds
     (2, [64] * 64, 1.0),                              # as many sequences as lanes
     (2, [64] * 64 + [128], 1.0),                      # one more: the persistent kernel
     (8, [4096 * 4], 1.0),                             # global rows of 256 tiles
@@ -56,6 +59,7 @@ def test_few_units(capi, heads, lens, scale, padded):
     (12, [1024, 1088], 1.0),                          # 4
     (12, [256, 1024, 640, 896], 1.0),                 # 2: two units side by side
     (12, [2048, 3008, 384], 6.0),                     # 1: four
+    (12, [2944, 3008, 2752], 6.0),                    # 1, global rows in 4 shares: one to a wave
 ])
 @pytest.mark.parametrize("padded", [False, True])
 def test_few_units_walk_the_plan(capi, heads, lens, scale, padded):
@@ -91,6 +95,7 @@ def test_few_units_walk_the_plan(capi, heads, lens, scale, padded):
     (12, [1024, 256]),                                # 4 waves to a row, global rows by 8
     (12, [512, 1024, 1280]),                          # 2
     (12, [2048, 3008, 384]),                          # 1
+    (12, [2944, 3008, 2752]),                         # 1, global rows by 4
     (16, [2048] * 6),                                 # the persistent kernel
 ])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
