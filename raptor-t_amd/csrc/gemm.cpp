@@ -1,6 +1,6 @@
 // Dense GEMM of the layer: row-major C[M,N] = A[M,K] . B[K,N], inputs and output in fp16 / bf16 / fp32, accumulation
-// in fp32.  B[N,K]^T in a 16-bit type, which is what the layers run, goes to the kernels of gemm_mfma.hip; the
-// rest (fp32, B[K,N], shapes those kernels do not take, long reductions with few outputs) to hipBLASLt.
+// in fp32.  B[N,K]^T, which is what the layers run, goes to the kernels of gemm_mfma.hip (16-bit types) and gemm_f32.hip;
+// the rest (B[K,N], shapes those kernels do not take, products with few outputs) to hipBLASLt.
 //
 // Replaces kernels::MatMul (layers/kernels/mat_mul.cpp:9-96), which calls cublasGemmEx
 // with the operands swapped to express a row-major product in a column-major library and
@@ -357,6 +357,9 @@ int rt_gemm_bt(rt_gemm_ctx* ctx, const void* a, const void* bt, const void* bias
       rt::gemm_mfma_takes(a, bt, epilogue == RT_EPILOGUE_NONE ? nullptr : bias, c, m, n, k, dtype))
     return rt::gemm_mfma_bt(a, bt, epilogue == RT_EPILOGUE_NONE ? nullptr : bias, c, m, n, k,
                             epilogue == RT_EPILOGUE_BIAS_GELU, dtype, stream);
+  if (ctx && a && bt && c && m > 0 && n > 0 && k > 0 && dtype == RT_F32 && rt::gemm_f32_pays(m, n, k) &&
+      rt::gemm_f32_takes(a, bt, epilogue == RT_EPILOGUE_NONE ? nullptr : bias, c, m, n, k))
+    return rt::gemm_f32_bt(a, bt, epilogue == RT_EPILOGUE_NONE ? nullptr : bias, c, m, n, k, epilogue == RT_EPILOGUE_BIAS_GELU, stream);
   return run_gemm(ctx, a, bt, epilogue == RT_EPILOGUE_NONE ? nullptr : bias, c, m, n, k, epilogue, true, dtype, stream);
 }
 

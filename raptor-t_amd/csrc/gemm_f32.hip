@@ -1,0 +1,300 @@
+// Dense products of the fp32 layers: C[M,N] = A[M,K] . Bt[N,K]^T (+ bias, + tanh GELU), all operands fp32, on the bf16 matrix
+// instruction.  An operand is cut, exactly, into three bf16 parts (the first rounded to nearest) and the six largest of the nine
+// products of parts are added up in fp32; what is left out is at most 2^-24 of a product.  A 16x16x32 bf16 instruction takes 16
+// cycles where fp32 instructions take 256 for the same 32 reduction steps: six of them are 2.7 times as fast.
+//
+// A workgroup owns 64 x 64 outputs; each of its 4 or 8 waves takes every fourth or eighth run of 32 reduction steps of all of
+// them, and the waves' sums meet in LDS at the end.  So a wave needs its operands for itself: loads straight to its own
+// 16 KB of LDS (whole 128-byte rows; 16-byte pieces of 64 rows in the instruction's own layout would take four times as
+// long), from there to registers, where they are cut; the next run's loads follow at once and have the cutting and the
+// products ahead of them.  No barrier in the loop.  Two waves to a SIMD: one cuts (six vector instructions an element,
+// 384 a run) while the other multiplies (96 matrix instructions a run).
+//
+// Bound by the operands' way to the CU (16 KB for 96 matrix instructions: a wave's run takes 2 650 cycles of its SIMD where the
+// matrix instructions take 1 640) and, up to 256 tiles, by one workgroup's chain.  Measured (us, operands in rotation,
+// hipBLASLt's best suggestion for another row count as a batch of a new length meets it / this kernel): 512 x 3072 x 768 + GELU 37.7 /
+// 23.6, 1024 x 2304 x 768 50 / 32 (33 where the library was tuned for the shape), 1024 x 768 x 768 20.7 / 14.0, 1024 x 768 x
+// 3072 59 / 36, 4096 x 3072 x 768 + GELU 284 / 123, 8192 x 2304 x 768 390 / 184; relative error against 64 bits 2.4-5.0e-7 /
+// 1.0-4.2e-7.  A priority for one of a SIMD's two waves: no gain; all three parts rounded instead of the first: 3 % slower.
+//
+// Values that bf16 parts cannot hold: a part that overflows or is not finite makes a result that is not finite; a part below
+// 2^-126 counts as zero, which moves a result by at most 2^-125 * K * (max |a| + max |b|).  A workgroup that finds a result not
+// finite, or so small that this could show in its last bits, does its tile again on the fp32 instruction.
+#include <hip/hip_runtime.h>
+
+#include <atomic>
+#include <type_traits>
+
+#include "gemm_mfma.h"
+#include "lds_load.h"
+#include "rt_launch.h"
+
+namespace {
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+constexpr int TILE = 64, RUN = 32, BLOCKS = 4;                 // outputs of a tile each way, reduction steps of a run, blocks of 16
+constexpr int WAVE_BYTES = 2 * TILE * RUN * 4;
+
+struct Params {
+  const float *a, *bt, *bias;
+  float* c;
+  int m, n, k, tiles_m, tiles_n;
+};
+
+// A lane's eight consecutive steps of one row.
+struct Raw {
+  f32x4 lo, hi;
+};
+struct Parts {
+  bf16x8 p0, p1, p2;
+};
+
+__device__ inline uint32_t two(float x, float y) { return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{x, y}, bf16x2)); }
+
+// The three parts of a pair; peak collects the largest magnitude.  Only the first part is rounded: the rest is then at most a
+// 2^-9th, of 16 bits, and its upper and lower half are the other two parts as they are (conversions are the dear ones
+// among these instructions).
+__device__ inline uint32_t upper(float x, float y) { return __builtin_amdgcn_perm(__float_as_uint(y), __float_as_uint(x), 0x07060302u); }
+__device__ inline void cut(float x, float y, uint32_t (&w)[3], float& peak) {
+  peak = fmaxf(fmaxf(peak, fabsf(x)), fabsf(y));
+  w[0] = two(x, y);
+  x -= __uint_as_float(w[0] << 16);
+  y -= __uint_as_float(w[0] & 0xffff0000u);
+  w[1] = upper(x, y);
+  x -= __uint_as_float(__float_as_uint(x) & 0xffff0000u);
+  y -= __uint_as_float(__float_as_uint(y) & 0xffff0000u);
+  w[2] = upper(x, y);
+}
+__device__ inline Parts cut(const Raw& r, float& peak) {
+  uint32_t w[4][3];
+  cut(r.lo[0], r.lo[1], w[0], peak);
+  cut(r.lo[2], r.lo[3], w[1], peak);
+  cut(r.hi[0], r.hi[1], w[2], peak);
+  cut(r.hi[2], r.hi[3], w[3], peak);
+  return Parts{__builtin_bit_cast(bf16x8, u32x4{w[0][0], w[1][0], w[2][0], w[3][0]}),
+               __builtin_bit_cast(bf16x8, u32x4{w[0][1], w[1][1], w[2][1], w[3][1]}),
+               __builtin_bit_cast(bf16x8, u32x4{w[0][2], w[1][2], w[2][2], w[3][2]})};
+}
+
+__device__ inline float gelu_tanh(float x) {   // as the 16-bit products' epilogue
+  constexpr float K0 = -2.0f * 0.7978845608028654f * 1.4426950408889634f;
+  constexpr float K1 = K0 * 0.044715f;
+  return x * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(x * fmaf(K1, x * x, K0)));
+}
+
+template <int NW, bool GELU>
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_f32_kernel(Params p) {
+  // a run's operands of every wave, 128-byte rows, chunk c of row r at c ^ ((r >> 1) & 7); after the loop four waves' sums,
+  // [row block][wave][column block][lane]
+  extern __shared__ __align__(16) char smem[];
+  f32x4 (*const room)[4][BLOCKS][64] = reinterpret_cast<f32x4 (*)[4][BLOCKS][64]>(smem);
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, l16 = lane & 15, g4 = lane >> 4;
+  // XCD x takes the x-th eighth of the tiles, in groups of 8 row panels, the panel fastest
+  const int total = p.tiles_m * p.tiles_n, per = gridDim.x >> 3, id = int(blockIdx.x & 7) * per + int(blockIdx.x >> 3);
+  if (id >= total) return;
+  constexpr int G = 8;
+  const int grp = id / (G * p.tiles_n), in = id - grp * G * p.tiles_n, h = min(G, p.tiles_m - grp * G);
+  const int tn = in / h, tm = grp * G + (in - tn * h);
+
+  const i32x4 sa = make_srd(p.a, uint32_t(p.m) * uint32_t(p.k) * 4u), sb = make_srd(p.bt, uint32_t(p.n) * uint32_t(p.k) * 4u);
+  const uint32_t own = uint32_t(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) char*)smem)) + w * WAVE_BYTES;
+  int va[8], vb[8];                                            // rows past the end repeat the last one: nothing of them is stored
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const int r = 8 * i + (lane >> 3), chunk = ((lane & 7) ^ ((r >> 1) & 7)) * 16;
+    va[i] = min(tm * TILE + r, p.m - 1) * p.k * 4 + chunk;
+    vb[i] = min(tn * TILE + r, p.n - 1) * p.k * 4 + chunk;
+  }
+  const int runs = p.k / RUN;
+  auto request = [&](int run) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) load_to_lds(sb, vb[i], run * (RUN * 4), own + 8192 + i * 1024);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) load_to_lds(sa, va[i], run * (RUN * 4), own + i * 1024);
+  };
+  // rows 16 * i + l16 of an operand, steps 8 * g4 .. + 8
+  const int row_lo = l16 * 128 + (((2 * g4) ^ (l16 >> 1)) << 4), row_hi = l16 * 128 + (((2 * g4 + 1) ^ (l16 >> 1)) << 4);
+  auto read = [&](int at, int i) __attribute__((always_inline)) {
+    const char* const b = smem + w * WAVE_BYTES + at + i * 2048;
+    return Raw{*reinterpret_cast<const f32x4*>(b + row_lo), *reinterpret_cast<const f32x4*>(b + row_hi)};
+  };
+
+  f32x4 acc[BLOCKS][BLOCKS];
+  float peak_a = 0.f, peak_b = 0.f;
+  // the wave's runs; a run's rows are requested when the last run's have been cut
+  auto products = [&](auto plain) __attribute__((always_inline)) {
+    constexpr bool PLAIN = decltype(plain)::value;
+#pragma unroll
+    for (int i = 0; i < BLOCKS; ++i)
+#pragma unroll
+      for (int j = 0; j < BLOCKS; ++j) acc[i][j] = f32x4(0.f);
+    if (w >= runs) return;
+    request(w);
+#pragma clang loop unroll(disable)
+    for (int r = w; r < runs; r += NW) {
+      Raw ra[BLOCKS], rb[BLOCKS];
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#pragma unroll
+      for (int j = 0; j < BLOCKS; ++j) rb[j] = read(8192, j);
+#pragma unroll
+      for (int i = 0; i < BLOCKS; ++i) ra[i] = read(0, i);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      __builtin_amdgcn_sched_barrier(0);
+      if (r + NW < runs) request(r + NW);
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (PLAIN) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+#pragma unroll
+          for (int i = 0; i < BLOCKS; ++i)
+#pragma unroll
+            for (int j = 0; j < BLOCKS; ++j)
+              acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(e < 4 ? rb[j].lo[e & 3] : rb[j].hi[e & 3],
+                                                               e < 4 ? ra[i].lo[e & 3] : ra[i].hi[e & 3], acc[i][j], 0, 0, 0);
+      } else {
+        Parts b[BLOCKS], a[BLOCKS];
+#pragma unroll
+        for (int j = 0; j < BLOCKS; ++j) b[j] = cut(rb[j], peak_b);
+#pragma unroll
+        for (int i = 0; i < BLOCKS; ++i) a[i] = cut(ra[i], peak_a);
+        auto row = [&](int i, bf16x8 Parts::*pb, bf16x8 Parts::*pa) __attribute__((always_inline)) {
+#pragma unroll
+          for (int j = 0; j < BLOCKS; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[j].*pb, a[i].*pa, acc[i][j], 0, 0, 0);
+        };
+#pragma unroll
+        for (int i = 0; i < BLOCKS; ++i) {
+          row(i, &Parts::p0, &Parts::p2);                      // the smallest first
+          row(i, &Parts::p2, &Parts::p0);
+          row(i, &Parts::p1, &Parts::p1);
+          row(i, &Parts::p0, &Parts::p1);
+          row(i, &Parts::p1, &Parts::p0);
+          row(i, &Parts::p0, &Parts::p0);
+        }
+      }
+    }
+  };
+  // waves 0-3: all waves' sums of row block w
+  f32x4 sum[BLOCKS];
+  auto meet = [&]() __attribute__((always_inline)) {
+    __syncthreads();                                           // the operands of all waves are read
+    if (NW == 8) {                                             // a wave and its partner four further on first
+      if (w >= 4) {
+#pragma unroll
+        for (int i = 0; i < BLOCKS; ++i)
+#pragma unroll
+          for (int j = 0; j < BLOCKS; ++j) room[i][w - 4][j][lane] = acc[i][j];
+      }
+      __syncthreads();
+      if (w < 4) {
+#pragma unroll
+        for (int i = 0; i < BLOCKS; ++i)
+#pragma unroll
+          for (int j = 0; j < BLOCKS; ++j) acc[i][j] += room[i][w][j][lane];
+      }
+      __syncthreads();
+    }
+    if (w < 4) {
+#pragma unroll
+      for (int i = 0; i < BLOCKS; ++i)
+#pragma unroll
+        for (int j = 0; j < BLOCKS; ++j) room[i][w][j][lane] = acc[i][j];
+    }
+    __syncthreads();
+    if (w < 4) {
+#pragma unroll
+      for (int j = 0; j < BLOCKS; ++j) sum[j] = (room[w][0][j][lane] + room[w][1][j][lane]) + (room[w][2][j][lane] + room[w][3][j][lane]);
+    }
+  };
+  products(std::false_type());
+  meet();
+  // One bound for the tile's rows and columns, each wave's of what it has read; the waves' are joined below.
+#pragma unroll
+  for (int d = 32; d >= 1; d >>= 1) {
+    peak_a = fmaxf(peak_a, __shfl_xor(peak_a, d));
+    peak_b = fmaxf(peak_b, __shfl_xor(peak_b, d));
+  }
+  __shared__ float peaks[NW][2];
+  if (lane == 0) { peaks[w][0] = peak_a; peaks[w][1] = peak_b; }
+  __syncthreads();
+  float big_a = 0.f, big_b = 0.f;
+#pragma unroll
+  for (int q = 0; q < NW; ++q) {
+    big_a = fmaxf(big_a, peaks[q][0]);
+    big_b = fmaxf(big_b, peaks[q][1]);
+  }
+  // 2^-125 * K * (..) is less than a 2^-24th of what is at least `least`; products of zeros are zero either way
+  const float least = big_a == 0.f || big_b == 0.f ? 0.f : 0x1p-100f * float(p.k) * (big_a + big_b);
+  bool bad = !(least < __builtin_inff());
+  if (w < 4) {
+#pragma unroll
+    for (int j = 0; j < BLOCKS; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) bad = bad || !(fabsf(sum[j][e]) >= least && fabsf(sum[j][e]) < __builtin_inff());
+  }
+  if (__syncthreads_or(bad)) {                                 // also: the sums are read
+    products(std::true_type());
+    meet();
+  }
+
+  if (w >= 4) return;
+  const int row = tm * TILE + 16 * w + l16;
+  const __amdgpu_buffer_rsrc_t sc = __builtin_amdgcn_make_buffer_rsrc(p.c, 0, uint32_t(p.m) * uint32_t(p.n) * 4u, 0x00020000);
+#pragma unroll
+  for (int j = 0; j < BLOCKS; ++j) {
+    const int col = tn * TILE + 16 * j + 4 * g4;
+    f32x4 v = sum[j];
+    if (p.bias) v += *reinterpret_cast<const f32x4*>(p.bias + min(col, p.n - 4));
+    if (GELU) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = gelu_tanh(v[e]);
+    }
+    const uint32_t voff = col < p.n && row < p.m ? (uint32_t(row) * uint32_t(p.n) + uint32_t(col)) * 4u : 0xfffffff0u;
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), sc, int(voff), 0, 0);
+  }
+}
+
+}  // namespace
+
+namespace rt {
+
+bool gemm_f32_takes(const void* a, const void* bt, const void* bias, const void* c, int64_t m, int64_t n, int64_t k) {
+  auto aligned = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; };
+  return k % RUN == 0 && n % 4 == 0 && m * k < (int64_t(1) << 29) && n * k < (int64_t(1) << 29) && m * n < (int64_t(1) << 29) &&
+         aligned(a) && aligned(bt) && aligned(bias) && aligned(c);
+}
+
+// One workgroup's chain takes 6 us and 0.28 a run of every wave; the library's rate is 75 TFLOP/s or less.  Measured (us, library /
+// own): 256 x 3072 x 768 19.8 / 15.5, 512 x 2304 x 768 33 / 23, 1024 x 768 x 768 20.7 / 14.0 (18.8 when tuned for the shape), 1024 x
+// 768 x 3072 59 / 36 (39); on the other side 128 x 2304 x 768 12.5 / 14.6, 256 x 2304 x 768 17.6 / 14.9, 256 x 768 x 768 7.9 / 13.3,
+// 512 x 768 x 768 14.3 / 13.6, 512 x 768 x 3072 30.5 / 33.9, 64 x 768 x 3072 8.8 / 34.
+bool gemm_f32_pays(int64_t m, int64_t n, int64_t k) {
+  return 2e-6f / 75.f * float(m) * float(n) * float(k) > 6.f + 0.0088f * float(k);
+}
+
+int gemm_f32_bt(const void* a, const void* bt, const void* bias, void* c, int64_t m, int64_t n, int64_t k, bool gelu, void* stream) {
+  Params p{static_cast<const float*>(a), static_cast<const float*>(bt), static_cast<const float*>(bias), static_cast<float*>(c),
+           int(m), int(n), int(k), int((m + TILE - 1) / TILE), int((n + TILE - 1) / TILE)};
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  const int64_t tiles = int64_t(p.tiles_m) * p.tiles_n;
+  const dim3 grid(unsigned((tiles + 7) / 8 * 8));
+  auto go = [&](auto waves, auto act) {
+    constexpr int NW = decltype(waves)::value, LDS = NW * WAVE_BYTES;
+    constexpr bool GELU = decltype(act)::value;
+    static std::atomic<uint64_t> done{0};
+    if (int rc = allow_lds(reinterpret_cast<const void*>(&gemm_f32_kernel<NW, GELU>), LDS, done)) return rc;
+    RT_LAUNCH((gemm_f32_kernel<NW, GELU>), grid, dim3(64 * NW), LDS, st, p);
+    const hipError_t e = hipGetLastError();
+    return e == hipSuccess ? int(RT_OK) : rt::fail(RT_EIO, "fp32 gemm launch failed: %s", hipGetErrorString(e));
+  };
+  const std::integral_constant<int, 4> four;
+  const std::integral_constant<int, 8> eight;
+  if (tiles <= 256) return gelu ? go(eight, std::true_type()) : go(eight, std::false_type());
+  return gelu ? go(four, std::true_type()) : go(four, std::false_type());
+}
+
+}  // namespace rt

@@ -1,4 +1,4 @@
-// The library's own dense products (gemm_mfma.hip), called by the entry points in gemm.cpp.
+// The library's own dense products (gemm_mfma.hip, gemm_f32.hip), called by the entry points in gemm.cpp.
 #pragma once
 #include <cstdint>
 
@@ -21,5 +21,12 @@ int gemm_mfma_qkv(const void* a, const void* bt, const void* bias, void* rows, v
 int gemm_mfma_slices(int64_t m, int64_t n, int64_t k, int64_t max_bytes);
 // The slices; `slices` > 1 as gemm_mfma_slices gave it.
 int gemm_mfma_part(const void* a, const void* bt, float* parts, int64_t m, int64_t n, int64_t k, int slices, int dtype, void* stream);
+
+// gemm_f32.hip: the same product of fp32 operands on bf16 parts; K a multiple of 32, N of 4, 16-byte aligned operands whose
+// byte offsets fit 31 bits.
+bool gemm_f32_takes(const void* a, const void* bt, const void* bias, const void* c, int64_t m, int64_t n, int64_t k);
+// Whether it is also the faster way: not for few outputs, which hipBLASLt cuts.
+bool gemm_f32_pays(int64_t m, int64_t n, int64_t k);
+int gemm_f32_bt(const void* a, const void* bt, const void* bias, void* c, int64_t m, int64_t n, int64_t k, bool gelu, void* stream);
 
 }  // namespace rt

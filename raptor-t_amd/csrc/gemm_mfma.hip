@@ -45,6 +45,7 @@
 #include <type_traits>
 
 #include "gemm_mfma.h"
+#include "lds_load.h"
 #include "rt_launch.h"
 
 namespace {
@@ -57,7 +58,6 @@ typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-typedef int i32x4 __attribute__((ext_vector_type(4)));
 
 // The matrix instruction as assembly, so that its accumulators stay where they are: given the choice the compiler
 // writes them to other registers and runs out of them.  It cannot see the instruction's hazards then; the two that
@@ -96,18 +96,6 @@ template <int TM> constexpr int a_stage() { return TM * ROW > WAVES * EPI_BYTES 
 template <int TM> constexpr int lds_bytes() { return 3 * a_stage<TM>() + 2 * B_STAGE; }
 
 #define SB() __builtin_amdgcn_sched_barrier(0)
-
-// 64 lanes x 16 bytes from srd[voff + soff] to LDS bytes [lds, lds + 1024).  Hidden from the compiler's wait
-// counting on purpose (it would wait for every load before any LDS read); the waits stand in the loop.
-__device__ inline void load_to_lds(i32x4 srd, int voff, int soff, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds"
-               :: "v"(voff), "s"(srd), "s"(soff), "s"(lds) : "memory");
-}
-
-__device__ inline i32x4 make_srd(const void* p, uint32_t bytes) {
-  const uint64_t a = reinterpret_cast<uint64_t>(p);
-  return i32x4{int(uint32_t(a)), int(uint32_t(a >> 32) & 0xffffu), int(bytes), 0x00020000};
-}
 
 __device__ inline float gelu_tanh(float x) {   // x / (1 + 2^(x (k0 + k1 x^2))), as bias_gelu_kernel
   constexpr float K0 = -2.0f * 0.7978845608028654f * 1.4426950408889634f;
@@ -860,18 +848,6 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(2,
   store_block<T, MT, NT, EPI>(acc, sc, p.n, m0, n0, room);
 }
 
-// More dynamic LDS than the default has to be asked for once per kernel and device.
-template <typename K> int allow_lds(K kernel, int bytes, std::atomic<uint64_t>& done) {
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return rt::fail(RT_EIO, "hipGetDevice failed: no usable GPU");
-  const uint64_t bit = uint64_t(1) << (dev & 63);
-  if (done.load(std::memory_order_relaxed) & bit) return RT_OK;
-  const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-  if (e != hipSuccess) return rt::fail(RT_EIO, "gemm: %d bytes of LDS refused: %s", bytes, hipGetErrorString(e));
-  done.fetch_or(bit, std::memory_order_relaxed);
-  return RT_OK;
-}
-
 int launched() {
   const hipError_t e = hipGetLastError();
   return e == hipSuccess ? RT_OK : rt::fail(RT_EIO, "gemm launch failed: %s", hipGetErrorString(e));
@@ -882,7 +858,7 @@ template <typename T, int TM, int MT0, int MT1, int EPI> int launch(const Params
   p.tiles_m = (p.m + TM - 1) / TM;
   p.tiles_n = (p.n + TN - 1) / TN;
   static std::atomic<uint64_t> done{0};
-  if (int rc = allow_lds(&gemm_bt_kernel<T, TM, MT0, MT1, EPI>, lds_bytes<TM>(), done)) return rc;
+  if (int rc = allow_lds(reinterpret_cast<const void*>(&gemm_bt_kernel<T, TM, MT0, MT1, EPI>), lds_bytes<TM>(), done)) return rc;
   const int total = p.tiles_m * p.tiles_n;
   const int grid = total >= 256 ? 256 : (total + 7) / 8 * 8;
   RT_LAUNCH((gemm_bt_kernel<T, TM, MT0, MT1, EPI>), dim3(grid), dim3(512), lds_bytes<TM>(), st, p);
@@ -895,7 +871,7 @@ template <typename T, int MT, int NT, int WM, int WN, int STAGES, int EPI> int l
   p.tiles_m = (p.m + TM - 1) / TM;
   p.tiles_n = (p.n + TC - 1) / TC;
   static std::atomic<uint64_t> done{0};
-  if (int rc = allow_lds(&gemm_bt_small_kernel<T, MT, NT, WM, WN, STAGES, EPI>, LDS, done)) return rc;
+  if (int rc = allow_lds(reinterpret_cast<const void*>(&gemm_bt_small_kernel<T, MT, NT, WM, WN, STAGES, EPI>), LDS, done)) return rc;
   const int total = p.tiles_m * p.tiles_n * p.slices;
   RT_LAUNCH((gemm_bt_small_kernel<T, MT, NT, WM, WN, STAGES, EPI>), dim3((total + 7) / 8 * 8), dim3(64 * WM * WN), LDS, st, p);
   return launched();

@@ -248,3 +248,69 @@ def test_library_product_as_first_call_in_a_capture(capi, call, dtype):
         run(eager, want)
         torch.cuda.synchronize()
         assert torch.equal(out, want)
+
+
+def check_f32(got, a, b, bias, gelu):
+    """Per element against 64 bits: a sum of k terms in fp32 in any order (k * 2^-24 * sum |a| |b|) of products that miss at most a
+    2^-24th, bias and rounding; the GELU's slope (<= 1.13) and its fp32 exponential and reciprocal, as in check()."""
+    a, b = a.double(), b.double()
+    x = a @ b.t()
+    err = 2.0 ** -24 * (a.shape[1] + 2) * (a.abs() @ b.abs().t())
+    if bias is not None:
+        x = x + bias.double()
+        err = err + 2.0 ** -23 * x.abs()
+    want = torch.nn.functional.gelu(x, approximate="tanh") if gelu else x
+    over = ((got.double() - want).abs() - 1.13 * err - 2.0 ** -20 * x.abs() * gelu - 2.0 ** -24 * want.abs()).max().item()
+    assert over <= 0, over
+
+
+# Sizes that the own kernel takes (gemm_f32_pays): one row and one chunk of columns in the last tiles, fewer runs of 32 steps than
+# waves, runs that the waves share unevenly, eight waves (up to 256 tiles) and four.
+@pytest.mark.parametrize("m,n,k", [
+    (2945, 3076, 32), (2113, 3076, 96), (1025, 772, 768), (449, 3076, 736), (1025, 2308, 800), (961, 1028, 3104), (2049, 772, 1056),
+])
+@pytest.mark.parametrize("epilogue", [0, 1, 2])
+def test_f32_products(capi, m, n, k, epilogue):
+    print("gemm f32", m, n, k, epilogue, flush=True)
+    a, b, bias = operands(m, n, k, torch.float32, seed=5)
+    c = torch.full((m + 1, n), 7.0, device="cuda")
+    gemm = capi.Gemm()
+    start, stop = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+    for e in (start, stop):
+        e.record()
+    assert capi.time_next_launch(start.cuda_event, stop.cuda_event) == 0
+    gemm.bt(a, b, c[:m], bias=bias if epilogue else None, epilogue=epilogue)
+    assert capi.time_next_launch(None, None) == 0      # an own kernel has taken the pair
+    check_f32(c[:m], a, b, bias if epilogue else None, epilogue == 2)
+    assert bool((c[m] == 7.0).all())
+
+
+@pytest.mark.parametrize("case", ["ones", "tiny", "tiny and huge", "largest", "infinite", "zeros"])
+def test_f32_products_at_the_ends_of_the_range(capi, case):
+    """Operands that bf16 parts hold badly or not at all: as accurate as the fp32 instruction all the same."""
+    m, n, k = 1024, 832, 768
+    a, b, _ = operands(m, n, k, torch.float32, seed=6)
+    if case == "ones":                                 # every bit of the mantissa set: the parts that are left out are largest
+        a = torch.exp2(torch.floor(torch.log2(a.abs().clamp_min(1e-3)))) * (2 - 2.0 ** -23)
+        b = torch.exp2(torch.floor(torch.log2(b.abs().clamp_min(1e-3)))) * (2 - 2.0 ** -23)
+    elif case == "tiny":                               # third parts below 2^-126, results above it
+        a, b = a * 2.0 ** -112, b * 2.0 ** 4
+    elif case == "tiny and huge":
+        a, b = a * 2.0 ** -118, b * 2.0 ** 110
+    elif case == "largest":                            # a first part that rounds up to infinity
+        a[5, 7], b[:, 7] = torch.finfo(torch.float32).max, b[:, 7] * 2.0 ** -30
+    elif case == "infinite":
+        a[3, 1], a[70, 2], b[9, 4] = float("inf"), float("nan"), float("-inf")
+    else:
+        a[64:200] = 0
+    c = torch.empty(m, n, device="cuda")
+    capi.Gemm().bt(a, b, c, epilogue=0)
+    if case == "infinite":
+        want = a.double() @ b.double().t()
+        assert torch.equal(c.isnan(), want.isnan()) and torch.equal(c == float("inf"), want == float("inf"))
+        rows, cols = torch.ones(m, dtype=torch.bool), torch.ones(n, dtype=torch.bool)
+        rows[[3, 70]], cols[9] = False, False
+        c, a, b = c[rows.cuda()][:, cols.cuda()], a[rows.cuda()], b[cols.cuda()]
+    check_f32(c, a, b, None, False)
+    if case == "zeros":
+        assert bool((c[64:200] == 0).all())
