@@ -152,13 +152,19 @@ __device__ inline void state_init(State& st) {
   st.l[0] = st.l[1] = 0.f;
 }
 
-// Scores of padded keys become minus infinity: no weight.  s = 32 x 32 accumulator tile of key half kt; the key of
-// element e in this lane is 32 kt + 8 (e >> 2) + (e & 3) + 4 (lane >> 5), padding from `tail` on.
-__device__ inline void mask_padded(f32x16& s, int kt, int tail, int lane) {
+// Scores of padded keys become minus infinity: no weight.  The others gain log2(times), as if the tile were listed that
+// often.  s = 32 x 32 accumulator tile of key half kt; the key of element e in this lane is
+// 32 kt + 8 (e >> 2) + (e & 3) + 4 (lane >> 5), padding from `tail` on.
+__device__ inline void mask_padded(f32x16& s, int kt, int tail, int lane, int times = 1) {
   int lim = tail - 4 * (lane >> 5);
   asm volatile("" : "+v"(lim));       // the 16 comparisons are made here, not once per kernel and kept in 32 scalar pairs
 #pragma unroll
   for (int e = 0; e < 16; ++e) s[e] = (32 * kt + 8 * (e >> 2) + (e & 3) >= lim) ? -INFINITY : s[e];
+  if (times > 1) {
+    const float gain = __builtin_amdgcn_logf(float(times));
+#pragma unroll
+    for (int e = 0; e < 16; ++e) s[e] += gain;
+  }
 }
 
 template <typename T>
@@ -576,45 +582,43 @@ __device__ inline void request_first(const Buffers<T>& b, int so, int lane, Tile
 // sequence's first block that is padding as a whole: tiles from there on are taken off the wave's tile list.
 // pad_off = offset of the tile whose keys from `tail` on are padding, -1 if there is none.  The loop masks in its
 // last tile only, so a row's padded tile is moved to the end of the list (the order of a row's tiles does not matter
-// to the result beyond rounding; the reference comes from the first tile).
-struct Padding { int pad_off, drop_off, tail; bool last; };
+// to the result beyond rounding; the reference comes from the first tile).  A row that lists it several times (the plan of
+// 1024 tokens draws the last block once more for some rows) meets it once, with the binary logarithm of the number added to
+// its scores: such a row took the moving-maximum loop before.  Sequences 17 tokens short, f16, before / now in us: 6 of 8512 in
+// all 37.0 / 24.5, 10 x 1024 (16 heads) 64 / 42, 32 x 1024 168 / 109; others within 1 % but 40 of 150-1700 112 / 114.
+struct Padding { int pad_off, drop_off, tail, last; };
 __device__ inline Padding padding_of(const Unit& u, int goff) {
   Padding pd;
   pd.pad_off = u.tail < 64 ? goff + (u.nbv - 1) * 8192 : -1;
   pd.drop_off = goff + u.nbv * 8192;
   pd.tail = u.tail;
-  pd.last = false;
+  pd.last = 0;
   return pd;
 }
 // Lanes 0 .. my-1 of ids hold the tile offsets of the wave's entries.  Takes the tiles that are padding as a whole
-// off the list (my shrinks), moves the padded tile to the last lane in use and sets pd.last.  False: the pipelined
-// loop cannot run this list (the padded tile is listed more than once, or the list's first tile does not stay
+// off the list (my shrinks), moves the padded tile to the last lane in use, further entries of it behind that, and sets
+// pd.last to their number.  False: the pipelined loop cannot run this list (its first tile does not stay
 // first, which a hand-over from the previous row may already have requested).
 __device__ inline bool pad_to_end(int& ids, int& my, int lane, Padding& pd) {
-  pd.last = false;
-  const unsigned long long listed = __ballot(lane < my);
-  const unsigned long long keep = __ballot(lane < my && ids < pd.drop_off);
-  if (keep != listed) {
-    if (!(keep & 1ull)) return false;
-    // kept entries move up in order; the dropped ones go behind them, lanes beyond the list stay (a permutation)
-    const unsigned long long below = (1ull << lane) - 1ull;
-    const int kept = __popcll(keep);
-    const bool mine = (keep >> lane) & 1ull;
-    const int dest = lane >= my ? lane : (mine ? __popcll(keep & below) : kept + __popcll(listed & ~keep & below));
-    ids = __builtin_amdgcn_ds_permute(dest * 4, ids);
-    my = kept;
+  pd.last = 0;
+  const unsigned long long listed = __ballot(lane < my), dropped = __ballot(lane < my && ids >= pd.drop_off);
+  const unsigned long long pads = pd.pad_off < 0 ? 0 : __ballot(lane < my && ids == pd.pad_off) & ~dropped;
+  const unsigned long long front = listed & ~dropped & ~pads;
+  if ((dropped | pads) == 0) return true;
+  if ((dropped & 1ull) || ((pads & 1ull) && front)) return false;
+  if (dropped == 0 && pads == 1ull << (my - 1)) {            // in its place already: rows over a whole sequence
+    pd.last = 1;
+    return true;
   }
-  if (pd.pad_off < 0) return true;
-  const unsigned long long m = __ballot(lane < my && ids == pd.pad_off);
-  if (m == 0) return true;
-  if (__popcll(m) > 1) return false;
-  const int jp = __builtin_ctzll(m);
-  if (jp == 0 && my > 1) return false;
-  if (jp != my - 1) {
-    const int moved = __builtin_amdgcn_readlane(ids, my - 1);
-    ids = lane == jp ? moved : (lane == my - 1 ? pd.pad_off : ids);
-  }
-  pd.last = true;
+  // a permutation: the others in order, the padded tiles, the dropped ones; lanes beyond the list stay
+  auto below = [](unsigned long long m) { return int(__builtin_amdgcn_mbcnt_hi(unsigned(m >> 32), __builtin_amdgcn_mbcnt_lo(unsigned(m), 0))); };
+  const int n_front = __popcll(front), n_pads = __popcll(pads);
+  int dest = below(front);
+  if (!(front >> lane & 1ull)) dest = (pads >> lane & 1ull) ? n_front + below(pads) : n_front + n_pads + below(dropped);
+  if (lane >= my) dest = lane;
+  ids = __builtin_amdgcn_ds_permute(dest * 4, ids);
+  my = n_front + (n_pads > 0);
+  pd.last = n_pads;
   return true;
 }
 
@@ -704,7 +708,7 @@ __device__ inline void fast_loop(const Buffers<T>& b, int ids, int my, const int
       uint32_t t01 = 0, t23 = 0, t45 = 0, t67 = 0;
       float lacc = 0.f;
       // a row's padded tile is its last one (pad_to_end): its scores lose the padded keys before they are exponentiated
-      if (MASKED && LAST && pd.last) mask_padded(cur, S >> 1, pd.tail, lane);
+      if (MASKED && LAST && pd.last) mask_padded(cur, S >> 1, pd.tail, lane, pd.last);
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
         SB();
@@ -809,7 +813,7 @@ __device__ inline bool fast_share(const Args<T>& a, const Buffers<T>& b, const Q
   request_first<T>(b, __builtin_amdgcn_readlane(ids, 0), lane, t);
   if (!HAVE_Q) finish_q<T>(a, qbias, r.u, lane, t.qf);
   float mref;
-  if (!fast_reference<T, MASKED>(t, mref, pd.last && my == 1, pd.tail, lane)) return false;
+  if (!fast_reference<T, MASKED>(t, mref, pd.last > 0 && my == 1, pd.tail, lane)) return false;
   fast_loop<T, MASKED>(b, ids, my, -1, lane, mref, t, st, NoNextQ{}, pd);
   return sums_finite(st);
 }
@@ -1233,7 +1237,7 @@ __global__ __launch_bounds__(256, 2) void bs_attention_kernel(Args<T> a) {
           }
           if (ok) {
             finish_q<T>(a, qbias, cur.u, lane, t.qf);
-            ok = fast_reference<T, MASKED>(t, mref, pd.last && my == 1, pd.tail, lane);
+            ok = fast_reference<T, MASKED>(t, mref, pd.last > 0 && my == 1, pd.tail, lane);
           }
           // the next row's block ids: requested here, looked at in the loop's last tile
           bool nx_short = false;

@@ -1,6 +1,7 @@
 """Block-sparse attention of batches with few units (rows shared by several waves): every number of rows to a
 workgroup, the edges of the rule that picks it, padding, scores that outgrow the pipelined loop's reference, and
 the caller's plan, against the oracle."""
+import numpy as np
 import pytest
 import torch
 
@@ -125,3 +126,49 @@ def test_infinite_and_very_low_scores(capi, heads, lens, dtype):
     # weights and output rounded to the type (half a unit in the last place of values up to max |v| each)
     tol = 4 * (2.0 ** -11 if dtype == torch.float16 else 2.0 ** -8) * v[v.isfinite()].abs().max().item()
     assert (out - ref)[ok].abs().max().item() <= tol
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("heads,lens,short", [
+    (3, [1024, 768, 64], 17),                         # few units; 64 tokens: every entry is the padded tile
+    (4, [1024, 1600, 320], 63),                       # a tail of one key
+    (12, [1024] * 15, 40),                            # 2880 units: the persistent kernel
+    (12, [1024, 768] * 8, 150),                       # whole blocks of padding dropped in front of it
+])
+def test_padded_tile_listed_several_times(capi, heads, lens, short, dtype):
+    """Every third entry of the plan becomes the block the real tokens end in: rows that list it up to a dozen times,
+    first, last and as their only tile."""
+    print("padded tile listed several times", heads, lens[:3], short, dtype, flush=True)
+    g = torch.Generator().manual_seed(heads)
+    t = sum(lens)
+    tokens = [max(1, n - short) for n in lens]
+    q, k, v = (torch.randn(t, heads, 64, generator=g).to(dtype).cuda() for _ in range(3))
+    sb, idx, pos, ph, sb_d, _, pos_d = lh.device_plan(capi, lens, heads, 5, None)
+    idx = idx.copy()
+    rng = np.random.default_rng(heads)
+    row, seen = 0, 0
+    for h in range(ph):                               # rows of the index: head by head, sequence by sequence
+        for n, real in zip(lens, tokens):
+            for _ in range(n // 64):
+                a, b = int(pos[row]), int(pos[row + 1])
+                last = (real - 1) // 64
+                idx[a:b] = np.where(rng.random(b - a) < 1 / 3, last, idx[a:b])
+                if not (idx[a:b] <= last).any():
+                    idx[a] = last                     # a row of padding alone has no softmax
+                seen = max(seen, int((idx[a:b] == last).sum()))
+                row += 1
+    assert row == len(pos) - 1 and seen > 4
+    qs = (q.float() * (lh.LOG2E / 8.0)).to(dtype)
+    out = torch.empty(t, heads * 64, dtype=dtype, device="cuda")
+    capi.bs_attention_fwd(lh.pack_heads(qs, sb), lh.pack_heads(k, sb), lh.pack_heads(v, sb, transpose_v=True), out, sb_d,
+                          heads, torch.from_numpy(idx).cuda(), pos_d, ph, None, None,
+                          torch.tensor(tokens, dtype=torch.int32).cuda())
+    torch.cuda.synchronize()
+    ref = lh.oa.csr_attention(qs.cpu(), k.cpu(), v.cpu(), sb.tolist(), idx, pos, ph, scale=1.0 / lh.LOG2E, seq_tokens=tokens)
+    # as above, with the type's own unit roundoff
+    tol = 4 * 2.0 ** -(lh.MANTISSA_BITS[dtype] + 1) * v.float().abs().max().item()
+    start = 0
+    for n, real in zip(lens, tokens):                 # real query rows only
+        err = (out[start:start + real].float().cpu() - ref[start:start + real]).abs().max().item()
+        assert err <= tol, (n, real, err)
+        start += n

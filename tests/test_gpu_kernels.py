@@ -430,9 +430,8 @@ def test_attention_padded_tail_matches_oracle(capi, dtype, n_wg, reference_plan)
     """Sequences whose last block ends in padding: the keys past the true length get no weight.  Covers a
     sparse sequence, a full-attention one (below 12 blocks), a tail of a single token, no padding at all, a
     sequence of one block (its only tile is the padded one: the pipelined loop's reference has to leave the
-    padded keys out too) and one of two; 768 tokens are 12 blocks, where rows list the last block twice (those
-    take the moving-maximum loop), and the reference's head-shared plan keeps more duplicates still.  The padded
-    rows hold large values so that a missed mask shows."""
+    padded keys out too) and one of two; 768 tokens are 12 blocks, where rows list the last block twice,
+    and the reference's head-shared plan keeps more duplicates still.  The padded rows hold large values so that a missed mask shows."""
     say("attention padded", dtype, n_wg, reference_plan)
     heads = 4
     seq_lens = [1024, 320, 832, 768, 64, 128]
