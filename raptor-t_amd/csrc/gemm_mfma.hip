@@ -970,11 +970,11 @@ bool gemm_mfma_takes(const void* a, const void* bt, const void* bias, const void
          n * k < (int64_t(1) << 29) && (m + 256) * n < (int64_t(1) << 31) && aligned(a) && aligned(bt) && aligned(bias) && aligned(c);
 }
 
-// An uncut product is one chain of steps, 0.25 us each; with at most 64 of the smallest tiles most CUs have none and a
-// library that cuts the reduction is ahead.  Measured (us in a graph, hipBLASLt / here): 64 x 768 x 1280 4.8 / 7.6, x 3072 5.8 /
-// 14.9, x 16384 14.8 / 65; 256 x 1024 (64 tiles) x 1280 5.8 / 7.8, x 4096 10.5 / 19.1; on the other side 64 x 768 x 768
-// 5.9 / 5.6, 256 x 768 x 1024 8.7 / 6.7, 512 x 768 (96 tiles) x 2048 13.5 / 10.9, 512 x 1024 x 4096 19.2 / 19.1; 65-128
-// tiles go either way (0.8 to 1.3).
+// An uncut product is one chain of steps, 0.16 us each; with at most 64 of the smallest tiles most CUs have none and a
+// library that cuts the reduction is ahead on long ones.  Measured (us in a graph, operands in rotation, hipBLASLt / here): 64 x
+// 768 x 1280 6.0 / 5.7, x 3072 7.2 / 10.9, x 16384 14.9 / 41; 256 x 1024 (64 tiles) x 1280 6.8 / 6.4, x 4096 10.8 / 13.4.  The
+// line at 1280 dates from slower steps; moved to where the two cross (about 1500) it would give at most 0.4 us.  On the
+// other side, here: 256 x 768 x 1024 5.3, 512 x 768 (96 tiles) x 2048 8.6, 512 x 1024 x 4096 13.9.
 bool gemm_mfma_pays(int64_t m, int64_t n, int64_t k) {
   return k < 20 * BK || ((m + 63) / 64) * ((n + 63) / 64) > 64;
 }
