@@ -305,8 +305,9 @@ int rt_gemm_bt(rt_gemm_ctx* ctx, const void* a, const void* bt, const void* bias
                int64_t m, int64_t n, int64_t k, int epilogue, int dtype, void* stream);
 
 /* The product of rt_gemm_bt (RT_EPILOGUE_NONE, fp16 / bf16) as fp32 slices of its reduction, for a caller whose next
- * step is rt_slices_residual_layernorm: with few rows, cutting a long reduction is what gives every CU a share.
- * *n_parts = 0: the product is better not cut (or cannot be: hidden sizes other than 256 / 512 / 768 / 1024), nothing
+ * step is rt_slices_residual_layernorm: with few rows, cutting a long reduction is what gives every CU a share, and the
+ * sums of a product of few outputs reach the LayerNorm unrounded (*n_parts = 1: not cut).
+ * *n_parts = 0: the product is better taken in 16 bits (or has a hidden size other than 256 / 512 / 768 / 1024), nothing
  * was launched, use rt_gemm_bt + rt_bias_residual_layernorm.  Otherwise the slices parts[n_parts][m][n] are being
  * written on `stream`, in a workspace of the context (32 MiB): they are valid until the next call on the context. */
 int rt_gemm_bt_slices(rt_gemm_ctx* ctx, const void* a, const void* bt, int64_t m, int64_t n, int64_t k, int dtype,

@@ -431,7 +431,7 @@ class Gemm:
         return c
 
     def bt_layernorm(self, a, bt, bias, residual, gamma, beta, out, eps):
-        """out = LN(a @ bt.T + bias + residual) * gamma + beta.  Returns the number of slices the product was cut into
+        """out = LN(a @ bt.T + bias + residual) * gamma + beta.  Returns the number of fp32 slices of the product
         (0: rt_gemm_bt and rt_bias_residual_layernorm)."""
         m, k = a.shape
         n = bt.shape[0]

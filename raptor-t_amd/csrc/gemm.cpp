@@ -328,7 +328,7 @@ int rt_gemm_bt_slices(rt_gemm_ctx* ctx, const void* a, const void* bt, int64_t m
   *n_parts = 0;
   if (m == 0 || n % 256 != 0 || n > 1024 || !rt::gemm_mfma_takes(a, bt, nullptr, nullptr, m, n, k, dtype)) return RT_OK;
   const int slices = rt::gemm_mfma_slices(m, n, k, SLICES_BYTES);
-  if (slices < 2) return RT_OK;
+  if (slices == 0) return RT_OK;
   std::lock_guard<std::mutex> lk(ctx->m);
   const int rc = rt::gemm_mfma_part(a, bt, ctx->slices, m, n, k, slices, dtype, stream);
   if (rc) return rc;

@@ -17,9 +17,9 @@ int gemm_mfma_qkv(const void* a, const void* bt, const void* bias, void* rows, v
                   int batch, int64_t m, int heads, int64_t k, int dtype, void* stream);
 
 // Into how many slices of the reduction this product should be cut if the caller can take fp32 slices [slices][M][N] of
-// up to max_bytes and add them up itself (1: not at all, use gemm_mfma_bt).
+// up to max_bytes and add them up itself (1: uncut, but in fp32; 0: uncut and in 16 bits, use gemm_mfma_bt).
 int gemm_mfma_slices(int64_t m, int64_t n, int64_t k, int64_t max_bytes);
-// The slices; `slices` > 1 as gemm_mfma_slices gave it.
+// The slices; `slices` >= 1 as gemm_mfma_slices gave it.
 int gemm_mfma_part(const void* a, const void* bt, float* parts, int64_t m, int64_t n, int64_t k, int slices, int dtype, void* stream);
 
 // gemm_f32.hip: the same product of fp32 operands on bf16 parts; K a multiple of 32, N of 4, 16-byte aligned operands whose

@@ -915,14 +915,26 @@ const Kernel kKernels[] = {
     {{64, 64, 1}, 0.162f, 0.081f, 0.404f, 2.05f, 0.55f, true, true},
 };
 
-// max_slices 1: the caller takes the product itself; more: fp32 slices will do, which the caller's next kernel reads.
+// Products of few outputs hand their sums to the LayerNorm behind them in fp32, cut or not: rounded to 16 bits on the way they
+// add 12 % (K = 768) to 18 % (K = 3072) to the error of its output against 64 bits (fp16 2.07e-4 -> 2.31e-4 and 2.48e-4, bf16
+// 1.65e-3 -> 1.85e-3 and 1.96e-3), and one fp32 slice takes 0.2-0.4 us more than 16 bits (512 x 768 x 768 with the LayerNorm
+// 8.6 -> 8.8).  The range is that of the products which pay for slices on operands in the caches; with more outputs
+// the fp32 rows' way to memory and back would cost up to 6 us.
+bool keeps_sums(int64_t m, int64_t n, int64_t k) {
+  const int64_t rows = k <= 3072 ? 192 : 256;      // tiles of rows x 128 whose two slices are one round of workgroups
+  return k >= 768 && m * n <= (k < 1344 ? 684 : k < 2048 ? 768 : 1160) * k && ((m + rows - 1) / rows) * ((n + 127) / 128) <= 128;
+}
+
+// max_slices 0: the caller takes the product itself; more: fp32 slices will do, which the caller's next kernel reads, and one
+// slice is an uncut product in 16 bits, or in fp32 where keeps_sums.
 Choice choose(int64_t m, int64_t n, int64_t k, int epi, int max_slices) {
   const int steps = int(k / BK);
+  const bool sums = max_slices > 0 && keeps_sums(m, n, k);
   Choice best = kKernels[0].c;
   float best_us = 0.f;
   for (const Kernel& kn : kKernels) {
-    if (epi == EPI_QKV && !kn.qkv) continue;
-    for (int s = 1; s <= (kn.part ? max_slices : 1); ++s) {
+    if ((epi == EPI_QKV && !kn.qkv) || (sums && !kn.part)) continue;
+    for (int s = 1; s <= (kn.part && max_slices > 1 ? max_slices : 1); ++s) {
       if (s > 1 && steps / s < 6) break;
       const int64_t wgs = ((m + kn.c.tm - 1) / kn.c.tm) * ((n + kn.c.tc - 1) / kn.c.tc) * s;
       const int64_t slots = kn.pair > 0.f ? 512 : 256, full = wgs / slots, rest = wgs % slots, rounds = full + (rest ? 1 : 0);
@@ -930,7 +942,7 @@ Choice choose(int64_t m, int64_t n, int64_t k, int epi, int max_slices) {
       const float stepping = float(full) * both + (rest == 0 ? 0.f : rest <= 256 ? alone : both);
       float us = kn.launch + kn.round * float(rounds) + stepping * float((steps + s - 1) / s);
       if (epi == EPI_GELU) us += 2.9e-5f * float(kn.c.tm * kn.c.tc) * float(rounds) * (kn.pair > 0.f && full ? 2.f : 1.f);
-      if (s > 1) us += 0.6f + float(m) * float(n) * (1.7e-6f * float(s) - 1.4e-6f);       // against 16 bits to the LayerNorm
+      if (s > 1 || sums) us += 0.6f + float(m) * float(n) * (1.7e-6f * float(s) - 1.4e-6f);       // against 16 bits to the LayerNorm
       if (best_us == 0.f || us < best_us) { best_us = us; best = kn.c; best.slices = s; }
     }
   }
@@ -985,7 +997,7 @@ int gemm_mfma_bt(const void* a, const void* bt, const void* bias, void* c, int64
   p.a = a; p.bt = bt; p.bias = bias; p.c = c;
   p.m = int(m); p.n = int(n); p.k = int(k);
   hipStream_t st = static_cast<hipStream_t>(stream);
-  const Choice ch = choose(m, n, k, gelu ? EPI_GELU : EPI_NONE, 1);
+  const Choice ch = choose(m, n, k, gelu ? EPI_GELU : EPI_NONE, 0);
   if (dtype == RT_F16) return gelu ? dispatch<_Float16, EPI_GELU>(p, ch, st) : dispatch<_Float16, EPI_NONE>(p, ch, st);
   return gelu ? dispatch<__bf16, EPI_GELU>(p, ch, st) : dispatch<__bf16, EPI_NONE>(p, ch, st);
 }
@@ -997,14 +1009,16 @@ int gemm_mfma_qkv(const void* a, const void* bt, const void* bias, void* rows, v
   p.m = int(m); p.n = 3 * heads * 64; p.k = int(k);
   p.kt = kt; p.vt = vt; p.seq_blocks = seq_blocks_dev; p.batch = batch; p.heads = heads;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  const Choice ch = choose(m, p.n, k, EPI_QKV, 1);
+  const Choice ch = choose(m, p.n, k, EPI_QKV, 0);
   return dtype == RT_F16 ? dispatch<_Float16, EPI_QKV>(p, ch, st) : dispatch<__bf16, EPI_QKV>(p, ch, st);
 }
 
 int gemm_mfma_slices(int64_t m, int64_t n, int64_t k, int64_t max_bytes) {
-  if ((m + 256) * n * 4 >= (int64_t(1) << 32)) return 1;
+  if ((m + 256) * n * 4 >= (int64_t(1) << 32)) return 0;
   const int64_t fit = max_bytes / (m * n * 4);
-  return choose(m, n, k, EPI_PART, int(fit < 1 ? 1 : fit > 8 ? 8 : fit)).slices;
+  if (fit < 1) return 0;
+  const int slices = choose(m, n, k, EPI_PART, int(fit > 8 ? 8 : fit)).slices;
+  return slices > 1 || keeps_sums(m, n, k) ? slices : 0;
 }
 
 int gemm_mfma_part(const void* a, const void* bt, float* parts, int64_t m, int64_t n, int64_t k, int slices, int dtype, void* stream) {

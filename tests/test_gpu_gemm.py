@@ -201,6 +201,29 @@ def test_gemm_bt_layernorm(capi, m, n, k, dtype):
     assert bool((out[m] == 7.0).all())
 
 
+@pytest.mark.parametrize("m,n,k", [
+    (256, 768, 768), (512, 768, 768), (649, 768, 768), (659, 1024, 1024), (2048, 256, 768),      # uncut
+    (1024, 768, 3072), (1000, 1024, 3072), (5646, 256, 2048), (4096, 1024, 5120),
+    (64, 768, 3072), (2816, 768, 3072),                                                          # in slices
+])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_sums_reach_the_layernorm_in_fp32(capi, m, n, k, dtype):
+    """Cut or not, a product of few outputs is not rounded to 16 bits on its way to the LayerNorm: the output is as far from
+    64 bits as its own rounding (fp32 sums and the LayerNorm add less than 1e-2 of that: k * 2^-24 against 2^-9 or 2^-12 of
+    the root mean square); one more rounding on the way would make it 1.11 to 1.2 times as far."""
+    print("sums in fp32", m, n, k, dtype, flush=True)
+    a, b, bias = operands(m, n, k, dtype, seed=7)
+    g = torch.Generator(device="cuda").manual_seed(8)
+    res, gamma, beta = (torch.randn(*s, generator=g, device="cuda").to(dtype) for s in ((m, n), (n,), (n,)))
+    out = torch.empty(m, n, dtype=dtype, device="cuda")
+    assert capi.Gemm().bt_layernorm(a, b, bias, res, gamma, beta, out, 1e-5) >= 1
+    x = a.double() @ b.double().t() + bias.double() + res.double()
+    want = torch.nn.functional.layer_norm(x, (n,), gamma.double(), beta.double(), 1e-5)
+    far = (out.double() - want).norm().item()
+    rounding = (want.to(dtype).double() - want).norm().item()
+    assert far <= 1.02 * rounding, far / rounding
+
+
 def test_cut_product_as_first_call_in_a_capture(capi):
     """A context's first product that is cut may be met inside a capture, which allows no allocation."""
     m, n, k = 512, 768, 3072
