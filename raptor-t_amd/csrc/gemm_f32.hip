@@ -1,7 +1,8 @@
 // Dense products of the fp32 layers: C[M,N] = A[M,K] . Bt[N,K]^T (+ bias, + tanh GELU), all operands fp32, on the bf16 matrix
-// instruction.  An operand is cut, exactly, into three bf16 parts (the first rounded to nearest) and the six largest of the nine
-// products of parts are added up in fp32; what is left out is at most 2^-24 of a product.  A 16x16x32 bf16 instruction takes 16
-// cycles where fp32 instructions take 256 for the same 32 reduction steps: six of them are 2.7 times as fast.
+// instruction.  An operand is cut, exactly, into three bf16 parts, each rounded to nearest, and the six largest of the nine
+// products of parts are added up in fp32; what is left out (second by third part twice, third by third) is at most 2^-24 of a
+// product, of either sign.  A 16x16x32 bf16 instruction takes 16 cycles where fp32 instructions take 256 for the same 32
+// reduction steps: six of them are 2.7 times as fast.
 //
 // A workgroup owns 64 x 64 outputs; each of its 4 or 8 waves takes every fourth or eighth run of 32 reduction steps of all of
 // them, and the waves' sums meet in LDS at the end.  So a wave needs its operands for itself: loads straight to its own
@@ -15,7 +16,7 @@
 // hipBLASLt's best suggestion for another row count as a batch of a new length meets it / this kernel): 512 x 3072 x 768 + GELU 37.7 /
 // 23.6, 1024 x 2304 x 768 50 / 32 (33 where the library was tuned for the shape), 1024 x 768 x 768 20.7 / 14.0, 1024 x 768 x
 // 3072 59 / 36, 4096 x 3072 x 768 + GELU 284 / 123, 8192 x 2304 x 768 390 / 184; relative error against 64 bits 2.4-5.0e-7 /
-// 1.0-4.2e-7.  A priority for one of a SIMD's two waves: no gain; all three parts rounded instead of the first: 3 % slower.
+// 1.0-4.2e-7.  A priority for one of a SIMD's two waves: no gain.
 //
 // Values that bf16 parts cannot hold: a part that overflows or is not finite makes a result that is not finite; a part below
 // 2^-126 counts as zero, which moves a result by at most 2^-125 * K * (max |a| + max |b|).  A workgroup that finds a result not
@@ -56,18 +57,20 @@ struct Parts {
 
 __device__ inline uint32_t two(float x, float y) { return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{x, y}, bf16x2)); }
 
-// The three parts of a pair; peak collects the largest magnitude.  Only the first part is rounded: the rest is then at most a
-// 2^-9th, of 16 bits, and its upper and lower half are the other two parts as they are (conversions are the dear ones
-// among these instructions).
+// The three parts of a pair; peak collects the largest magnitude.  For a number in [1, 2) the first rest is at most 2^-8, the second at
+// most 2^-17 and a multiple of 2^-23, so the third part is exact without a conversion, the upper half of the rest.  With the second part
+// truncated, its rest is up to 2^-16 and what is left out 2^-23 of a product, always towards zero: a single product of 1 + 2^-8 + 2^-7 -
+// d 2^-23 and 1 + 2^-8 - e 2^-23 was up to 1.95 * 2^-23 off, now 1.47 (2^-23 of it the instruction's sums, which are cut off), a sum of
+// 768 such terms of either sign 1.6e-7, now 1.4e-7 (on the fp32 instruction 5.0e-7).  The conversion takes 1.5 % of a launch.
 __device__ inline uint32_t upper(float x, float y) { return __builtin_amdgcn_perm(__float_as_uint(y), __float_as_uint(x), 0x07060302u); }
 __device__ inline void cut(float x, float y, uint32_t (&w)[3], float& peak) {
   peak = fmaxf(fmaxf(peak, fabsf(x)), fabsf(y));
   w[0] = two(x, y);
   x -= __uint_as_float(w[0] << 16);
   y -= __uint_as_float(w[0] & 0xffff0000u);
-  w[1] = upper(x, y);
-  x -= __uint_as_float(__float_as_uint(x) & 0xffff0000u);
-  y -= __uint_as_float(__float_as_uint(y) & 0xffff0000u);
+  w[1] = two(x, y);
+  x -= __uint_as_float(w[1] << 16);
+  y -= __uint_as_float(w[1] & 0xffff0000u);
   w[2] = upper(x, y);
 }
 __device__ inline Parts cut(const Raw& r, float& peak) {

@@ -308,6 +308,35 @@ def test_f32_products(capi, m, n, k, epilogue):
     assert bool((c[m] == 7.0).all())
 
 
+def on_own_kernel(capi, call):
+    """Runs the call and asserts that it launched a kernel of the library's own, which takes a waiting pair of events."""
+    start, stop = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+    for e in (start, stop):
+        e.record()
+    assert capi.time_next_launch(start.cuda_event, stop.cuda_event) == 0
+    call()
+    assert capi.time_next_launch(None, None) == 0
+
+
+# eight waves (up to 256 tiles), four
+@pytest.mark.parametrize("m,n,k", [(1025, 772, 800), (2113, 3076, 96)])
+def test_f32_products_of_single_terms(capi, m, n, k):
+    """Sums of one term and zeros: nothing but the parts of two numbers.  What is left out is at most 2^-24 (1 + 2^-10) of the term; of
+    the six sums of parts, which the instruction cuts off, the last costs up to 2^-23 and the others, at most 2^-7 of the
+    term, 2^-28.  The mantissas leave out the most: a first part short by almost 2^-8, a second one by almost 2^-17."""
+    print("gemm f32 single terms", m, n, k, flush=True)
+    i, j = torch.arange(m, device="cuda"), torch.arange(n, device="cuda")
+    x = (1 + 2.0 ** -8 + 2.0 ** -7 - (1 + i % 397) * 2.0 ** -23) * torch.exp2(i % 5 - 2.0)
+    y = (1 + 2.0 ** -8 - (1 + j % 389) * 2.0 ** -23) * torch.exp2(j % 3 - 1.0) * (1 - 2 * (j % 2))
+    a, b = torch.zeros(m, k, device="cuda"), y.float()[:, None].repeat(1, k).contiguous()
+    a[i, i * 37 % k] = x.float()
+    c = torch.empty(m, n, device="cuda")
+    on_own_kernel(capi, lambda: capi.Gemm().bt(a, b, c))
+    want = a.double().sum(1)[:, None] * y.float().double()
+    over = ((c.double() - want).abs() / want.abs()).max().item()
+    assert over <= 1.5 * 2.0 ** -23 * (1 + 2.0 ** -5), over * 2.0 ** 23
+
+
 @pytest.mark.parametrize("case", ["ones", "tiny", "tiny and huge", "largest", "infinite", "zeros"])
 def test_f32_products_at_the_ends_of_the_range(capi, case):
     """Operands that bf16 parts hold badly or not at all: as accurate as the fp32 instruction all the same."""
