@@ -320,49 +320,87 @@ def on_own_kernel(capi, call):
 
 # eight waves (up to 256 tiles), four
 @pytest.mark.parametrize("m,n,k", [(1025, 772, 800), (2113, 3076, 96)])
-def test_f32_products_of_single_terms(capi, m, n, k):
+@pytest.mark.parametrize("scale_a,scale_b", [
+    (0, 0), (50, 60),
+    (-105, 0), (0, -115), (-118, 110),                               # parts below 2^-126
+    (-42, -50), (-55, -60), (-60, -60), (-30, -90),                  # products of parts and their sums below it
+])
+def test_f32_products_of_single_terms(capi, m, n, k, scale_a, scale_b):
     """Sums of one term and zeros: nothing but the parts of two numbers.  What is left out is at most 2^-24 (1 + 2^-10) of the term; of
     the six sums of parts, which the instruction cuts off, the last costs up to 2^-23 and the others, at most 2^-7 of the
     term, 2^-28.  The mantissas leave out the most: a first part short by almost 2^-8, a second one by almost 2^-17."""
-    print("gemm f32 single terms", m, n, k, flush=True)
+    print("gemm f32 single terms", m, n, k, scale_a, scale_b, flush=True)
     i, j = torch.arange(m, device="cuda"), torch.arange(n, device="cuda")
-    x = (1 + 2.0 ** -8 + 2.0 ** -7 - (1 + i % 397) * 2.0 ** -23) * torch.exp2(i % 5 - 2.0)
-    y = (1 + 2.0 ** -8 - (1 + j % 389) * 2.0 ** -23) * torch.exp2(j % 3 - 1.0) * (1 - 2 * (j % 2))
+    x = (1 + 2.0 ** -8 + 2.0 ** -7 - (1 + i % 397) * 2.0 ** -23) * torch.exp2(i % 5 - 2.0) * 2.0 ** scale_a
+    y = (1 + 2.0 ** -8 - (1 + j % 389) * 2.0 ** -23) * torch.exp2(j % 3 - 1.0) * (1 - 2 * (j % 2)) * 2.0 ** scale_b
     a, b = torch.zeros(m, k, device="cuda"), y.float()[:, None].repeat(1, k).contiguous()
     a[i, i * 37 % k] = x.float()
     c = torch.empty(m, n, device="cuda")
     on_own_kernel(capi, lambda: capi.Gemm().bt(a, b, c))
     want = a.double().sum(1)[:, None] * y.float().double()
-    over = ((c.double() - want).abs() / want.abs()).max().item()
+    # (a sum below 2^-126 is cut off at 2^-149)
+    over = (((c.double() - want).abs() - 6 * 2.0 ** -149).clamp_min(0) / want.abs()).max().item()
     assert over <= 1.5 * 2.0 ** -23 * (1 + 2.0 ** -5), over * 2.0 ** 23
 
 
-@pytest.mark.parametrize("case", ["ones", "tiny", "tiny and huge", "largest", "infinite", "zeros"])
-def test_f32_products_at_the_ends_of_the_range(capi, case):
+RANGE_CASES = ["ones", "tiny", "both tiny", "tiny and huge", "largest", "infinite", "zeros", "zero column"]
+
+
+# whole tiles on eight waves; on eight and on four waves one row and 4 columns in the last tiles, runs of 32 steps that the
+# waves share unevenly, waves without one, and the other epilogues behind the second pass
+@pytest.mark.parametrize("m,n,k,epilogue", [(1024, 832, 768, 0), (1025, 772, 800, 1), (2113, 3076, 96, 2), (2113, 1028, 1056, 1)])
+@pytest.mark.parametrize("case", RANGE_CASES)
+def test_f32_products_at_the_ends_of_the_range(capi, case, m, n, k, epilogue):
     """Operands that bf16 parts hold badly or not at all: as accurate as the fp32 instruction all the same."""
-    m, n, k = 1024, 832, 768
-    a, b, _ = operands(m, n, k, torch.float32, seed=6)
-    if case == "ones":                                 # every bit of the mantissa set: the parts that are left out are largest
+    print("gemm f32 range", case, m, n, k, epilogue, flush=True)
+    a, b, bias = operands(m, n, k, torch.float32, seed=6)
+    if case == "ones":                                 # every bit of the mantissa set
         a = torch.exp2(torch.floor(torch.log2(a.abs().clamp_min(1e-3)))) * (2 - 2.0 ** -23)
         b = torch.exp2(torch.floor(torch.log2(b.abs().clamp_min(1e-3)))) * (2 - 2.0 ** -23)
     elif case == "tiny":                               # third parts below 2^-126, results above it
         a, b = a * 2.0 ** -112, b * 2.0 ** 4
+    elif case == "both tiny":                          # all parts above 2^-126, products of parts below
+        a, b = a * 2.0 ** -55, b * 2.0 ** -60
     elif case == "tiny and huge":
         a, b = a * 2.0 ** -118, b * 2.0 ** 110
     elif case == "largest":                            # a first part that rounds up to infinity
         a[5, 7], b[:, 7] = torch.finfo(torch.float32).max, b[:, 7] * 2.0 ** -30
     elif case == "infinite":
         a[3, 1], a[70, 2], b[9, 4] = float("inf"), float("nan"), float("-inf")
-    else:
+    elif case == "zeros":
         a[64:200] = 0
-    c = torch.empty(m, n, device="cuda")
-    capi.Gemm().bt(a, b, c, epilogue=0)
+    else:
+        b[70] = 0
+    c = torch.full((m + 1, n), 7.0, device="cuda")
+    bias = bias if epilogue else None
+    on_own_kernel(capi, lambda: capi.Gemm().bt(a, b, c[:m], bias=bias, epilogue=epilogue))
+    assert bool((c[m] == 7.0).all())
+    c = c[:m]
     if case == "infinite":
-        want = a.double() @ b.double().t()
+        want = a.double() @ b.double().t() + (bias.double() if epilogue else 0)
+        want = torch.nn.functional.gelu(want, approximate="tanh") if epilogue == 2 else want
         assert torch.equal(c.isnan(), want.isnan()) and torch.equal(c == float("inf"), want == float("inf"))
         rows, cols = torch.ones(m, dtype=torch.bool), torch.ones(n, dtype=torch.bool)
         rows[[3, 70]], cols[9] = False, False
         c, a, b = c[rows.cuda()][:, cols.cuda()], a[rows.cuda()], b[cols.cuda()]
-    check_f32(c, a, b, None, False)
-    if case == "zeros":
-        assert bool((c[64:200] == 0).all())
+        bias = bias[cols.cuda()] if epilogue else None
+    check_f32(c, a, b, bias, epilogue == 2)
+    if epilogue == 0 and case in ("zeros", "zero column"):
+        assert bool(((c[64:200] if case == "zeros" else c[:, 70]) == 0).all())
+
+
+@pytest.mark.parametrize("m,n,k", [(1025, 772, 800), (2113, 3076, 96)])
+def test_f32_rows_and_columns_stand_alone(capi, m, n, k):
+    """A row's or column's bits do not depend on what else lies in its tile, whichever of the two instructions that takes."""
+    print("gemm f32 alone", m, n, k, flush=True)
+    a, b, _ = operands(m, n, k, torch.float32, seed=9)
+    want = torch.empty(m, n, device="cuda")
+    capi.Gemm().bt(a, b, want)
+    rows, cols = torch.ones(m, dtype=torch.bool, device="cuda"), torch.ones(n, dtype=torch.bool, device="cuda")
+    rows[[2, 20, 70, 90, 130, m - 1]], cols[[5, 40, 75, n - 1]] = False, False
+    a[2], a[20], a[70, 3], a[90] = 0, a[20] * 2.0 ** -120, float("inf"), a[90] * 2.0 ** 100
+    a[130, 1:], a[m - 1, 7] = 0, float("nan")
+    b[5], b[40, 1], b[75], b[n - 1] = 0, float("nan"), b[75] * 2.0 ** -100, b[n - 1] * 2.0 ** 90
+    got = torch.empty(m, n, device="cuda")
+    on_own_kernel(capi, lambda: capi.Gemm().bt(a, b, got))
+    assert torch.equal(got[rows][:, cols], want[rows][:, cols])
