@@ -1316,8 +1316,9 @@ __global__ __launch_bounds__(256, 2) void bs_attention_kernel(Args<T> a) {
 // ---- batches with few units --------------------------------------------------------------------------------------------
 // Where the persistent kernel would leave most waves of the chip without a unit, its time is one unit's chain of tiles
 // (8 tiles, 13 us) or a global row's (a quarter of the sequence's blocks).  Here a unit's tiles are shared by several waves,
-// whose states merge through LDS: one workgroup of 8 waves (one per CU) takes one global row, or RPW other rows with
-// 8 / RPW waves each (rows_per_workgroup has the rule and the times of both kernels).  At most 64 sequences (a lane each).
+// whose states merge through LDS: one workgroup of 8 waves (one per CU) takes one global row, the two of a head with 4 waves
+// each (global_shares), or RPW other rows with 8 / RPW waves each (rows_per_workgroup has the rule and the times of both
+// kernels).  At most 64 sequences (a lane each).
 constexpr int FEW_CUS = 256;
 template <typename T, int NW> struct FewRoom {
   // four wave states in a merge; each wave's room for a query tile
@@ -1358,8 +1359,10 @@ template <typename T> struct FewBatch {
   // rounds.  Measured (us, eight shares / four, 12 heads): three sequences of 8704 tokens in all 31.8 / 26.3, four of 9344 30.8 /
   // 27.3, six of 8512 27.0 / 21.8, bf16 padded 5 x 320-3000 31.6 / 27.8; where the rounds stay as many, six of 9600 28.4 / 33.6,
   // five of 11008 31.3 / 34.7.
-  __device__ __forceinline__ int global_shares(const Args<T>& a, int n_sparse, int rows_per_wg) const {
-    const int pairs = n_sparse * a.heads, others = (a.nb_total * a.heads - 2 * pairs + rows_per_wg - 1) / rows_per_wg;
+  // Only with 8 other rows to a workgroup, the least of them, are there more than one round (rows_per_workgroup).
+  template <int RPW> __device__ __forceinline__ int global_shares(const Args<T>& a, int n_sparse) const {
+    if (RPW < 8 || n_sparse == 0) return 8;
+    const int pairs = n_sparse * a.heads, others = (a.nb_total * a.heads - 2 * pairs + RPW - 1) / RPW;
     const bool fewer = (pairs + others - 1) / FEW_CUS < (2 * pairs + others - 1) / FEW_CUS;
     return fewer && !__any(lane < a.batch && sb1 - sb0 > 64) ? 4 : 8;
   }
@@ -1385,7 +1388,7 @@ template <typename T> __device__ __forceinline__ Buffers<T> few_buffers(const Ar
 template <typename T, bool MASKED, int RPW, int NW>
 __device__ __forceinline__ void share_rows(const Args<T>& a, const Buffers<T>& b, FewRoom<T, NW>& room, const QSide<T>& qbias,
                                            const Unit& u, bool valid, int share, int lane, int wave) {
-  const int waves = share < NW ? share : NW, row = wave / waves, part = wave - row * waves;
+  const int waves = share < NW ? share : NW, row = wave >> __builtin_ctz(waves), part = wave & (waves - 1);      // powers of two
   const Row r = describe<T>(a, u);
   State st;
   if (NW < 8 && share > NW) {
@@ -1458,7 +1461,7 @@ __global__ __launch_bounds__(512, 2) void bs_attention_few_kernel(Args<T> a) {
   bool valid = true;
   const int n_pairs = n_sparse * a.heads;
   const int p_lo = int(int64_t(n_pairs) * xcd / 8), p_hi = int(int64_t(n_pairs) * (xcd + 1) / 8);
-  const int shares = batch.global_shares(a, n_sparse, RPW), n_glob = shares == 8 ? 2 * (p_hi - p_lo) : p_hi - p_lo;
+  const int shares = batch.template global_shares<RPW>(a, n_sparse), n_glob = shares == 8 ? 2 * (p_hi - p_lo) : p_hi - p_lo;
   const bool global = slot < n_glob;
   if (global) {
     const int pair = p_lo + (shares == 8 ? slot >> 1 : slot), h = pair / n_sparse, k = pair - h * n_sparse;
@@ -1485,11 +1488,12 @@ __global__ __launch_bounds__(512, 2) void bs_attention_few_kernel(Args<T> a) {
 
 // With a caller's plan workgroup c walks its slice, as in the persistent kernel: four waves, two workgroups per CU, a global
 // row by all of them, other entries side by side as far as there are waves for them.  A unit's tiles are cut into as many
-// shares as without a plan, so the bits are the same; a wave takes two of eight.  The slice is clamped to the list, ids
-// outside it are skipped.  Measured (us a call, 12 heads, rt_meta_partition_lpt into 512 and 256; persistent kernel / this one):
-// 1 x 4096 tokens 22.7, 21.1 / 23.7, 21.1; 8 x 150-1700 28.8, 35.6 / 28.7, 32.1; 2 x 4096 31.9, 34.7 / 32.7, 32.0;
-// 6 x 2048 44.5, 50.4 / 42.1, 41.9; 7 x 2048 50.7, 60.6 / 46.8, 52.1 (one workgroup of 8 waves per unit: 96).  Behind it: plans
-// of fewer workgroups than CUs for few units (1 x 2048 into 64: 21.7 / 41.8), whose rows are cut finer than they need.
+// shares as without a plan, so the bits are the same; a wave takes two of a global row's eight, or one of its four.  The slice
+// is clamped to the list, ids outside it are skipped.  Measured (us a call, 12 heads, rt_meta_partition_lpt into 512 and 256;
+// persistent kernel / this one): 1 x 4096 tokens 22.7, 21.1 / 23.7, 21.1; 8 x 150-1700 28.8, 35.6 / 28.7, 32.1; 2 x 4096 31.9,
+// 34.7 / 32.7, 32.0; 6 x 2048 44.5, 50.4 / 42.1, 41.9; 7 x 2048 50.7, 60.6 / 46.8, 52.1 (one workgroup of 8 waves per unit: 96).
+// Behind it: plans of fewer workgroups than CUs for few units (1 x 2048 into 64: 21.7 / 41.8), whose rows are cut finer than
+// they need.
 template <typename T, bool MASKED, int RPW>
 __global__ __launch_bounds__(256, 2) void bs_attention_few_plan_kernel(Args<T> a) {
   constexpr int SIDE = RPW > 2 ? RPW / 2 : 1;          // rows side by side
@@ -1503,7 +1507,7 @@ __global__ __launch_bounds__(256, 2) void bs_attention_few_plan_kernel(Args<T> a
   const QSide<T> qbias{room.qbias, reinterpret_cast<char*>(room.park) + wave * Q_STAGE_BYTES};
   const Buffers<T> b = few_buffers(a);
   const int shares =
-      batch.global_shares(a, __popcll(__ballot(batch.lane < a.batch && batch.sb1 - batch.sb0 >= RT_MIN_SPARSE_BLOCKS)), RPW);
+      batch.template global_shares<RPW>(a, __popcll(__ballot(batch.lane < a.batch && batch.sb1 - batch.sb0 >= RT_MIN_SPARSE_BLOCKS)));
   auto unit_of_flat = [&](int id) {
     const int s = batch.seq_of(a, batch.sb0 * a.heads, id);
     const int g0 = __builtin_amdgcn_readlane(batch.sb0, s), n = __builtin_amdgcn_readlane(batch.sb1, s) - g0;
