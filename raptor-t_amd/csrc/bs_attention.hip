@@ -155,12 +155,16 @@ __device__ inline void state_init(State& st) {
 // Scores of padded keys become minus infinity: no weight.  The others gain log2(times), as if the tile were listed that
 // often.  s = 32 x 32 accumulator tile of key half kt; the key of element e in this lane is
 // 32 kt + 8 (e >> 2) + (e & 3) + 4 (lane >> 5), padding from `tail` on.
+// BRANCH: the gain is passed by where there is none.  With few units that saves 0.15 us; in the persistent fp16 kernel the
+// branch costs registers (124 spilled instead of 116; 20 x 883 tokens 68.9 us instead of 67.3), so a gain of zero is added.
+template <bool BRANCH = true>
 __device__ inline void mask_padded(f32x16& s, int kt, int tail, int lane, int times = 1) {
   int lim = tail - 4 * (lane >> 5);
   asm volatile("" : "+v"(lim));       // the 16 comparisons are made here, not once per kernel and kept in 32 scalar pairs
 #pragma unroll
   for (int e = 0; e < 16; ++e) s[e] = (32 * kt + 8 * (e >> 2) + (e & 3) >= lim) ? -INFINITY : s[e];
-  if (times > 1) {
+  if (!BRANCH) asm volatile("" : "+s"(times));
+  if (!BRANCH || times > 1) {
     const float gain = __builtin_amdgcn_logf(float(times));
 #pragma unroll
     for (int e = 0; e < 16; ++e) s[e] += gain;
@@ -585,7 +589,8 @@ __device__ inline void request_first(const Buffers<T>& b, int so, int lane, Tile
 // to the result beyond rounding; the reference comes from the first tile).  A row that lists it several times (the plan of
 // 1024 tokens draws the last block once more for some rows) meets it once, with the binary logarithm of the number added to
 // its scores: such a row took the moving-maximum loop before.  Sequences 17 tokens short, f16, before / now in us: 6 of 8512 in
-// all 37.0 / 24.5, 10 x 1024 (16 heads) 64 / 42, 32 x 1024 168 / 109; others within 1 % but 40 of 150-1700 112 / 114.
+// all 37.0 / 24.5, 10 x 1024 (16 heads) 64 / 42, 32 x 1024 168 / 109.  Where no row lists it twice: 30 x 1193-1483 123.1 / 123.2,
+// 24 x 1563-2483 139.7 / 139.7, 14 x 77-376 13.15 / 13.22.
 struct Padding { int pad_off, drop_off, tail, last; };
 __device__ inline Padding padding_of(const Unit& u, int goff) {
   Padding pd;
@@ -606,7 +611,12 @@ __device__ inline bool pad_to_end(int& ids, int& my, int lane, Padding& pd) {
   const unsigned long long front = listed & ~dropped & ~pads;
   if ((dropped | pads) == 0) return true;
   if ((dropped & 1ull) || ((pads & 1ull) && front)) return false;
-  if (dropped == 0 && pads == 1ull << (my - 1)) {            // in its place already: rows over a whole sequence
+  if (dropped == 0 && (pads & (pads - 1)) == 0) {            // one: it and the last entry change places
+    const int jp = __builtin_ctzll(pads);
+    if (jp != my - 1) {
+      const int moved = __builtin_amdgcn_readlane(ids, my - 1);
+      ids = lane == jp ? moved : (lane == my - 1 ? pd.pad_off : ids);
+    }
     pd.last = 1;
     return true;
   }
@@ -653,7 +663,7 @@ __device__ inline bool fast_reference(const Tiles<T>& t, float& mref, bool pad_f
 // fragment k of the next row's queries into t.qf; called in the last tile's last two steps, once
 // the score products have read the fragment it replaces.
 struct NoNextQ { __device__ void operator()(int) const {} };
-template <typename T, bool MASKED, typename NextQ>
+template <typename T, bool MASKED, bool FEW, typename NextQ>
 __device__ inline void fast_loop(const Buffers<T>& b, int ids, int my, const int& so_after, int lane, float mref,
                                  Tiles<T>& t, State& st, NextQ next_q, const Padding& pd) {
   typedef typename Mma<T>::v8 v8;
@@ -708,7 +718,7 @@ __device__ inline void fast_loop(const Buffers<T>& b, int ids, int my, const int
       uint32_t t01 = 0, t23 = 0, t45 = 0, t67 = 0;
       float lacc = 0.f;
       // a row's padded tile is its last one (pad_to_end): its scores lose the padded keys before they are exponentiated
-      if (MASKED && LAST && pd.last) mask_padded(cur, S >> 1, pd.tail, lane, pd.last);
+      if (MASKED && LAST && pd.last) mask_padded<FEW>(cur, S >> 1, pd.tail, lane, pd.last);
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
         SB();
@@ -795,7 +805,7 @@ __device__ inline void slow_row(const Args<T>& a, const Buffers<T>& b, const QSi
 // from or to another row.  False: the row has to be run with the moving-maximum loop instead (more
 // than 64 entries for this wave, or scores that outgrew the reference); the state is then undefined.
 // HAVE_Q: the queries are in t.qf already; they are there afterwards too.
-template <typename T, bool MASKED, bool HAVE_Q>
+template <typename T, bool MASKED, bool HAVE_Q, bool FEW>
 __device__ inline bool fast_share(const Args<T>& a, const Buffers<T>& b, const QSide<T>& qbias, const Row& r, int first, int step,
                                   int lane, Tiles<T>& t, State& st) {
   state_init(st);
@@ -814,14 +824,14 @@ __device__ inline bool fast_share(const Args<T>& a, const Buffers<T>& b, const Q
   if (!HAVE_Q) finish_q<T>(a, qbias, r.u, lane, t.qf);
   float mref;
   if (!fast_reference<T, MASKED>(t, mref, pd.last > 0 && my == 1, pd.tail, lane)) return false;
-  fast_loop<T, MASKED>(b, ids, my, -1, lane, mref, t, st, NoNextQ{}, pd);
+  fast_loop<T, MASKED, FEW>(b, ids, my, -1, lane, mref, t, st, NoNextQ{}, pd);
   return sums_finite(st);
 }
-template <typename T, bool MASKED>
+template <typename T, bool MASKED, bool FEW = false>
 __device__ inline bool fast_row(const Args<T>& a, const Buffers<T>& b, const QSide<T>& qbias, const Row& r, int first, int step,
                                 int lane, State& st) {
   Tiles<T> t;
-  return fast_share<T, MASKED, false>(a, b, qbias, r, first, step, lane, t, st);
+  return fast_share<T, MASKED, false, FEW>(a, b, qbias, r, first, step, lane, t, st);
 }
 
 // One over a row's whole sum.  A row that has met nothing but padding writes zeros; one whose keys all have a score
@@ -1255,7 +1265,7 @@ __global__ __launch_bounds__(256, 2) void bs_attention_kernel(Args<T> a) {
           primed = false;
           if (ok) {
             const QPlan qn = q_plan<T>(a, nx.u, lane);      // without a next unit: this unit's queries again
-            fast_loop<T, MASKED>(b, ids, my, nx.first_off, lane, mref, t, st,
+            fast_loop<T, MASKED, false>(b, ids, my, nx.first_off, lane, mref, t, st,
                                  [&](int k) { t.qf[k >> 2][k & 3] = fetch_q<T>(b, qn, k); }, pd);
             lane = lane_id;
             asm volatile("" : "+v"(lane));
@@ -1409,13 +1419,13 @@ __device__ __forceinline__ void share_rows(const Args<T>& a, const Buffers<T>& b
       for (int nt = 0; nt < 2; ++nt) st.l[nt] = pair_sum(st.l[nt]);
       return ok;
     };
-    const bool ok = two_shares([&](int p) { return fast_share<T, MASKED, true>(a, b, qbias, r, p, 8, lane, t, st); });
+    const bool ok = two_shares([&](int p) { return fast_share<T, MASKED, true, true>(a, b, qbias, r, p, 8, lane, t, st); });
     if (__syncthreads_or(!ok))
       two_shares([&](int p) { slow_row<T, MASKED>(a, b, qbias, r, p, 8, lane, true, t.qf, st); return true; });
     absorb_state(st, own, lane);
   } else {
     state_init(st);
-    if (valid && !fast_row<T, MASKED>(a, b, qbias, r, part, share, lane, st) && lane == 0) room.failed[row] = 1;
+    if (valid && !fast_row<T, MASKED, true>(a, b, qbias, r, part, share, lane, st) && lane == 0) room.failed[row] = 1;
     __syncthreads();                                   // the query rooms are read
     if (valid && room.failed[row]) {
       typename Mma<T>::v8 qf[2][4];
