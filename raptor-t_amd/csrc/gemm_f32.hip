@@ -11,12 +11,12 @@
 // products ahead of them.  No barrier in the loop.  Two waves to a SIMD: one cuts (six vector instructions an element,
 // 384 a run) while the other multiplies (96 matrix instructions a run).
 //
-// Bound by the operands' way to the CU (16 KB for 96 matrix instructions: a wave's run takes 2 650 cycles of its SIMD where the
-// matrix instructions take 1 640) and, up to 256 tiles, by one workgroup's chain.  Measured (us, operands in rotation,
-// hipBLASLt's best suggestion for another row count as a batch of a new length meets it / this kernel): 512 x 3072 x 768 + GELU 37.7 /
-// 23.6, 1024 x 2304 x 768 50 / 32 (33 where the library was tuned for the shape), 1024 x 768 x 768 20.7 / 14.0, 1024 x 768 x
-// 3072 59 / 36, 4096 x 3072 x 768 + GELU 284 / 123, 8192 x 2304 x 768 390 / 184; relative error against 64 bits 2.4-5.0e-7 /
-// 1.0-4.2e-7.  A priority for one of a SIMD's two waves: no gain.
+// Bound by what a SIMD issues, the products of parts and the cutting (what-if builds: without two of the six products
+// -36 %, without the loads -10 %), and, up to 256 tiles, by one workgroup's chain.  Measured (us, operands in rotation,
+// hipBLASLt tuned for the shape, the same on a solution picked for another row count, as a batch of a new length meets it / this
+// kernel): 1024 x 2304 x 768 33.5, 47.9 / 33.0, 1024 x 3072 x 768 + GELU 40.6, 43.4 / 36.0, 1024 x 768 x 3072 39.5, 47.8 / 36.5,
+// 4096 x 3072 x 768 + GELU 142, 158 / 124, 8192 x 2304 x 768 207, 215 / 178; relative error against 64 bits 4.0-9.9e-7 / 1.3-4.3e-7
+// (K = 768 to 3072).  A priority for one of a SIMD's two waves: no gain.
 //
 // Values that bf16 parts cannot hold: a part that overflows or is not finite makes a result that is not finite; a part below
 // 2^-126 counts as zero, which moves a result by at most 2^-125 * K * (max |a| + max |b|) (products and sums of parts below it
@@ -62,11 +62,12 @@ struct Parts {
 
 __device__ inline uint32_t two(float x, float y) { return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{x, y}, bf16x2)); }
 
-// The three parts of a pair; peak collects the largest magnitude.  For a number in [1, 2) the first rest is at most 2^-8, the second at
-// most 2^-17 and a multiple of 2^-23, so the third part is exact without a conversion, the upper half of the rest.  With the second part
-// truncated, its rest is up to 2^-16 and what is left out 2^-23 of a product, always towards zero: a single product of 1 + 2^-8 + 2^-7 -
-// d 2^-23 and 1 + 2^-8 - e 2^-23 was up to 1.95 * 2^-23 off, now 1.47 (2^-23 of it the instruction's sums, which are cut off), a sum of
-// 768 such terms of either sign 1.6e-7, now 1.4e-7 (on the fp32 instruction 5.0e-7).  The conversion takes 1.5 % of a launch.
+// The three parts of a pair; peak collects the largest magnitude.  For a number in [1, 2) the first rest is at most 2^-8, the
+// second at most 2^-17 and a multiple of 2^-23, so the third part is exact without a conversion, the upper half of the rest.
+// With the second part truncated, its rest is up to 2^-16 and what is left out 2^-23 of a product, always towards zero: a
+// single product of 1 + 2^-8 + 2^-7 - d 2^-23 and 1 + 2^-8 - e 2^-23 was up to 1.95 * 2^-23 off, now 1.47 (2^-23 of it the
+// instruction's sums, which are cut off), a sum of 768 such terms of either sign 1.6e-7, now 1.4e-7 (on the fp32 instruction
+// 5.0e-7).  The conversion takes 1.5 % of a launch.
 __device__ inline uint32_t upper(float x, float y) { return __builtin_amdgcn_perm(__float_as_uint(y), __float_as_uint(x), 0x07060302u); }
 __device__ inline void cut(float x, float y, uint32_t (&w)[3], float& peak) {
   peak = fmaxf(fmaxf(peak, fabsf(x)), fabsf(y));
@@ -290,12 +291,21 @@ bool gemm_f32_takes(const void* a, const void* bt, const void* bias, const void*
          aligned(a) && aligned(bt) && aligned(bias) && aligned(c);
 }
 
-// One workgroup's chain takes 6 us and 0.28 a run of every wave; the library's rate is 75 TFLOP/s or less.  Measured (us, library /
-// own): 256 x 3072 x 768 19.8 / 15.5, 512 x 2304 x 768 33 / 23, 1024 x 768 x 768 20.7 / 14.0 (18.8 when tuned for the shape), 1024 x
-// 768 x 3072 59 / 36 (39); on the other side 128 x 2304 x 768 12.5 / 14.6, 256 x 2304 x 768 17.6 / 14.9, 256 x 768 x 768 7.9 / 13.3,
-// 512 x 768 x 768 14.3 / 13.6, 512 x 768 x 3072 30.5 / 33.9, 64 x 768 x 3072 8.8 / 34.
+// Where this kernel is faster than the library on a solution that was tuned for the very shape (the first M of a context; on one
+// picked for another M the library takes up to three times as long).  The library: 5.35 us and 137 TFLOP/s, which
+// it meets or stays behind.  This kernel: a workgroup's chain on eight waves (up to 256 tiles), slower when nearly every CU has
+// one, or rounds of two workgroups of four waves per CU, a round that leaves half of them out at 0.55.  Of 372 products
+// (hidden 512, 768 and 1024, 31 row counts from 64 to 8192) three of those that go here are more than 1 % slower than there, by
+// 5 % at most, and of the others 0.15 % could be gained.  Both sides (us, library / own): here 1024 x 1024 x 1536 27.5 / 25.0,
+// 704 x 2304 x 768 26.4 / 23.2, 1024 x 768 x 3072 39.5 / 36.5, 4096 x 3072 x 384 75.6 / 71.7; there 512 x 2304 x 768 20.1 /
+// 22.8, 1024 x 768 x 768 14.3 / 15.9, 640 x 768 x 3072 28.1 / 36.2, 2048 x 2304 x 256 26.0 / 29.1, 2113 x 3076 x 96 22.8 /
+// 28.1.
 bool gemm_f32_pays(int64_t m, int64_t n, int64_t k) {
-  return 2e-6f / 75.f * float(m) * float(n) * float(k) > 6.f + 0.0088f * float(k);
+  const int64_t tiles = ((m + TILE - 1) / TILE) * ((n + TILE - 1) / TILE), full = tiles / 512, rest = tiles % 512;
+  const float steps = float(k), round = 2.9f + 0.0211f * steps;
+  const float own = tiles <= 256 ? 8.5f + steps * (0.0088f + 0.0019f * float(tiles > 192 ? tiles - 192 : 0) / 64.f)
+                                 : 4.4f + round * (float(full) + (rest == 0 ? 0.f : rest <= 256 ? 0.55f : 1.f));
+  return own < 5.35f + 2e-6f / 136.8f * float(m) * float(n) * steps;
 }
 
 int gemm_f32_bt(const void* a, const void* bt, const void* bias, void* c, int64_t m, int64_t n, int64_t k, bool gelu, void* stream) {

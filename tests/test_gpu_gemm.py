@@ -273,6 +273,35 @@ def test_library_product_as_first_call_in_a_capture(capi, call, dtype):
         assert torch.equal(out, want)
 
 
+def on_own_kernel(capi, call):
+    """Runs the call and asserts that it launched a kernel of the library's own, which takes a waiting pair of events."""
+    start, stop = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+    for e in (start, stop):
+        e.record()
+    assert capi.time_next_launch(start.cuda_event, stop.cuda_event) == 0
+    call()
+    assert capi.time_next_launch(None, None) == 0
+
+
+# Both sides of the line between the own kernel and the library, each where it is the faster one by 3 % or more
+@pytest.mark.parametrize("m,n,k,own", [
+    (1024, 768, 3072, True), (704, 2304, 768, True), (1024, 1024, 1536, True), (4096, 768, 768, True),
+    (640, 768, 3072, False), (512, 2304, 768, False), (1024, 768, 768, False), (384, 1024, 4096, False), (256, 3072, 768, False),
+    (2113, 3076, 96, False), (2048, 2304, 256, False),                   # short reductions
+])
+def test_f32_products_run_on_the_faster_of_kernel_and_library(capi, m, n, k, own):
+    a, b, _ = operands(m, n, k, torch.float32, seed=10)
+    c, gemm = torch.empty(m, n, device="cuda"), capi.Gemm()
+    gemm.set_tuning(1)
+    start, stop = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+    for e in (start, stop):
+        e.record()
+    assert capi.time_next_launch(start.cuda_event, stop.cuda_event) == 0
+    gemm.bt(a, b, c)
+    assert capi.time_next_launch(None, None) == (0 if own else 1)        # an own kernel takes the pair, the library leaves it
+    check_f32(c, a, b, None, False)
+
+
 def check_f32(got, a, b, bias, gelu):
     """Per element against 64 bits: a sum of k terms in fp32 in any order (k * 2^-24 * sum |a| |b|) of products that miss at most a
     2^-24th, bias and rounding; the GELU's slope (<= 1.13) and its fp32 exponential and reciprocal, as in check()."""
@@ -287,39 +316,23 @@ def check_f32(got, a, b, bias, gelu):
     assert over <= 0, over
 
 
-# Sizes that the own kernel takes (gemm_f32_pays): one row and one chunk of columns in the last tiles, fewer runs of 32 steps than
-# waves, runs that the waves share unevenly, eight waves (up to 256 tiles) and four.
-@pytest.mark.parametrize("m,n,k", [
-    (2945, 3076, 32), (2113, 3076, 96), (1025, 772, 768), (449, 3076, 736), (1025, 2308, 800), (961, 1028, 3104), (2049, 772, 1056),
-])
+# Sizes that the own kernel takes (gemm_f32_pays): one row and one chunk of columns in the last tiles, runs of 32 steps that the
+# waves share unevenly, eight waves (up to 256 tiles) and four.
+F32_SIZES = [(1025, 900, 3104), (961, 964, 2080), (1857, 1028, 1056), (4097, 3076, 480)]
+
+
+@pytest.mark.parametrize("m,n,k", F32_SIZES + [(1024, 960, 1536), (2049, 772, 1056)])
 @pytest.mark.parametrize("epilogue", [0, 1, 2])
 def test_f32_products(capi, m, n, k, epilogue):
     print("gemm f32", m, n, k, epilogue, flush=True)
     a, b, bias = operands(m, n, k, torch.float32, seed=5)
     c = torch.full((m + 1, n), 7.0, device="cuda")
-    gemm = capi.Gemm()
-    start, stop = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
-    for e in (start, stop):
-        e.record()
-    assert capi.time_next_launch(start.cuda_event, stop.cuda_event) == 0
-    gemm.bt(a, b, c[:m], bias=bias if epilogue else None, epilogue=epilogue)
-    assert capi.time_next_launch(None, None) == 0      # an own kernel has taken the pair
+    on_own_kernel(capi, lambda: capi.Gemm().bt(a, b, c[:m], bias=bias if epilogue else None, epilogue=epilogue))
     check_f32(c[:m], a, b, bias if epilogue else None, epilogue == 2)
     assert bool((c[m] == 7.0).all())
 
 
-def on_own_kernel(capi, call):
-    """Runs the call and asserts that it launched a kernel of the library's own, which takes a waiting pair of events."""
-    start, stop = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
-    for e in (start, stop):
-        e.record()
-    assert capi.time_next_launch(start.cuda_event, stop.cuda_event) == 0
-    call()
-    assert capi.time_next_launch(None, None) == 0
-
-
-# eight waves (up to 256 tiles), four
-@pytest.mark.parametrize("m,n,k", [(1025, 772, 800), (2113, 3076, 96)])
+@pytest.mark.parametrize("m,n,k", [F32_SIZES[0], F32_SIZES[2]])
 @pytest.mark.parametrize("scale_a,scale_b", [
     (0, 0), (50, 60),
     (-105, 0), (0, -115), (-118, 110),                               # parts below 2^-126
@@ -347,8 +360,8 @@ RANGE_CASES = ["ones", "tiny", "both tiny", "tiny and huge", "largest", "infinit
 
 
 # whole tiles on eight waves; on eight and on four waves one row and 4 columns in the last tiles, runs of 32 steps that the
-# waves share unevenly, waves without one, and the other epilogues behind the second pass
-@pytest.mark.parametrize("m,n,k,epilogue", [(1024, 832, 768, 0), (1025, 772, 800, 1), (2113, 3076, 96, 2), (2113, 1028, 1056, 1)])
+# waves share unevenly, and the other epilogues behind the second pass
+@pytest.mark.parametrize("m,n,k,epilogue", [(1024, 960, 1536, 0)] + [size + (e,) for size, e in zip(F32_SIZES, (1, 2, 1, 2))])
 @pytest.mark.parametrize("case", RANGE_CASES)
 def test_f32_products_at_the_ends_of_the_range(capi, case, m, n, k, epilogue):
     """Operands that bf16 parts hold badly or not at all: as accurate as the fp32 instruction all the same."""
@@ -389,7 +402,7 @@ def test_f32_products_at_the_ends_of_the_range(capi, case, m, n, k, epilogue):
         assert bool(((c[64:200] if case == "zeros" else c[:, 70]) == 0).all())
 
 
-@pytest.mark.parametrize("m,n,k", [(1025, 772, 800), (2113, 3076, 96)])
+@pytest.mark.parametrize("m,n,k", [F32_SIZES[0], F32_SIZES[2]])
 def test_f32_rows_and_columns_stand_alone(capi, m, n, k):
     """A row's or column's bits do not depend on what else lies in its tile, whichever of the two instructions that takes."""
     print("gemm f32 alone", m, n, k, flush=True)
