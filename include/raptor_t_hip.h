@@ -300,7 +300,13 @@ int rt_gemm_bias_act(rt_gemm_ctx* ctx, const void* a, const void* b, const void*
  * RT_EPILOGUE_NONE): the b_trans = true form of kernels::MatMul
  * (layers/kernels/mat_mul.cpp:9-96, which passes CUBLAS_OP_T for it).  Both operands are then
  * contiguous along K, the layout the library's kernels for these shapes are fastest on, so the
- * layer objects keep their weights as [out, in] and call this. */
+ * layer objects keep their weights as [out, in] and call this.
+ * 16-bit types with K a multiple of 64 run on kernels of the library's own, but for long reductions of few outputs
+ * (rt_gemm_bt_tile); so does RT_F32 with K a multiple of 32, N of 4 and enough outputs; the rest on hipBLASLt, which is the only
+ * one that rt_gemm_set_tuning and rt_gemm_set_retuning concern.  The fp32 kernel multiplies operands as three bf16 parts, six of
+ * nine products of parts, added up in fp32: at most 2^-24 (1 + 2^-10) of a product is left out, and the sums are no further
+ * from 64 bits than fp32 instructions'.  Results that are not finite, or so small beside their row and column that parts below
+ * 2^-126 could show, come from fp32 instructions; which ones depends on no other row or column. */
 int rt_gemm_bt(rt_gemm_ctx* ctx, const void* a, const void* bt, const void* bias, void* c,
                int64_t m, int64_t n, int64_t k, int epilogue, int dtype, void* stream);
 
@@ -316,6 +322,13 @@ int rt_gemm_bt_slices(rt_gemm_ctx* ctx, const void* a, const void* bt, int64_t m
 int rt_slices_residual_layernorm(void* out, const float* parts, int n_parts, const void* residual, const void* bias,
                                  const void* gamma, const void* beta, int64_t rows, int hidden, float eps, int dtype,
                                  void* stream);
+
+/* Which kernel a 16-bit product of these sizes (16-byte aligned operands) runs on: rt_gemm_bt (kind = its epilogue),
+ * rt_qkv_project (n = 3 * heads * 64) or rt_gemm_bt_slices.  *rows x *cols outputs of a workgroup's tile and the number of
+ * slices of the reduction; *rows = 0: none of the library's own (rt_gemm_bt: hipBLASLt, rt_gemm_bt_slices: *n_parts = 0).
+ * Launches nothing and needs no GPU. */
+enum { RT_PRODUCT_QKV = 3, RT_PRODUCT_SLICES = 4 };
+int rt_gemm_bt_tile(int64_t m, int64_t n, int64_t k, int kind, int* rows, int* cols, int* slices);
 
 /* ------------------------------------------------------------------ pooling + pooler head */
 

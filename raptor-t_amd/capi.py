@@ -17,6 +17,7 @@ RT_PLAN_HF, RT_PLAN_REFERENCE, RT_PLAN_EXPLICIT = 0, 1, 2
 RT_POLICY_REFERENCE_PATCHED, RT_POLICY_HF_UPSTREAM = 0, 1
 RT_EINVAL, RT_ENOMEM, RT_EIO, RT_ENOSYS, RT_ECANCELED = -22, -12, -5, -38, -125
 RT_EPILOGUE_NONE, RT_EPILOGUE_BIAS, RT_EPILOGUE_BIAS_GELU = 0, 1, 2
+RT_PRODUCT_QKV, RT_PRODUCT_SLICES = 3, 4
 RT_GEMM_TUNE_ALL = -1
 
 EXPORTS = [
@@ -25,7 +26,7 @@ EXPORTS = [
     "rt_meta_partition_lpt", "rt_meta_check_partition", "rt_meta_check_to_index", "rt_qkv_bias_split", "rt_qkv_project", "rt_unpack_head_tiles", "rt_bs_attention_fwd",
     "rt_bs_attention_fwd_masked", "rt_bs_attention_fwd_qrows", "rt_bs_attention_fwd_no_alloc",
     "rt_bias_residual_layernorm", "rt_bias_gelu", "rt_embed_layernorm", "rt_gemm_create", "rt_gemm_destroy", "rt_gemm_set_tuning", "rt_gemm_set_retuning", "rt_gemm",
-    "rt_gemm_bias_act", "rt_gemm_bt", "rt_gemm_bt_slices", "rt_slices_residual_layernorm", "rt_sequence_pool", "rt_pooler_dense_tanh",
+    "rt_gemm_bias_act", "rt_gemm_bt", "rt_gemm_bt_slices", "rt_gemm_bt_tile", "rt_slices_residual_layernorm", "rt_sequence_pool", "rt_pooler_dense_tanh",
     "rt_pipeline_create", "rt_pipeline_publish", "rt_pipeline_acquire", "rt_pipeline_release",
     "rt_pipeline_destroy", "rt_pipeline_set_index_check",
 ]
@@ -79,6 +80,7 @@ def lib():
         L.rt_gemm_bias_act.argtypes = [vp, vp, vp, vp, vp, L64, L64, L64, I, I, vp]
         L.rt_gemm_bt.argtypes = [vp, vp, vp, vp, vp, L64, L64, L64, I, I, vp]
         L.rt_gemm_bt_slices.argtypes = [vp, vp, vp, L64, L64, L64, I, ctypes.POINTER(vp), i32p, vp]
+        L.rt_gemm_bt_tile.argtypes = [L64, L64, L64, I, i32p, i32p, i32p]
         L.rt_slices_residual_layernorm.argtypes = [vp, vp, I, vp, vp, vp, vp, L64, I, F, I, vp]
         L.rt_sequence_pool.argtypes = [vp, vp, vp, I, I, I, vp, I, vp]
         L.rt_pooler_dense_tanh.argtypes = [vp, vp, vp, vp, I, I, I, I, vp]
@@ -385,6 +387,15 @@ def embed_layernorm(input_ids, position_ids, token_type_ids, word, position, tok
                                    position.shape[0], token_type.shape[0], eps, _dtype_code(word), _dtype_code(out),
                                    _stream()))
     return out
+
+
+def gemm_bt_tile(m, n, k, kind):
+    """(rows, columns, slices) of the tile that a 16-bit product runs on, None where no kernel of the library's own takes
+    it; kind = an epilogue of rt_gemm_bt, RT_PRODUCT_QKV or RT_PRODUCT_SLICES."""
+    tile = (ctypes.c_int * 3)()
+    at = [ctypes.cast(ctypes.byref(tile, 4 * i), ctypes.POINTER(ctypes.c_int)) for i in range(3)]
+    check(lib().rt_gemm_bt_tile(m, n, k, kind, *at))
+    return tuple(tile) if tile[0] else None
 
 
 class Gemm:

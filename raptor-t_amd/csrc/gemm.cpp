@@ -304,6 +304,12 @@ int run_gemm(rt_gemm_ctx* ctx, const void* a, const void* b, const void* bias, v
   return RT_OK;
 }
 
+// How many fp32 slices rt_gemm_bt_slices leaves; 0: none
+int slices_of(const void* a, const void* bt, int64_t m, int64_t n, int64_t k, int dtype) {
+  if (m == 0 || n % 256 != 0 || n > 1024 || !rt::gemm_mfma_takes(a, bt, nullptr, nullptr, m, n, k, dtype)) return 0;
+  return rt::gemm_mfma_slices(m, n, k, SLICES_BYTES);
+}
+
 }  // namespace
 
 extern "C" {
@@ -326,14 +332,31 @@ int rt_gemm_bt_slices(rt_gemm_ctx* ctx, const void* a, const void* bt, int64_t m
   RT_REQUIRE(m >= 0 && n > 0 && k > 0, RT_EINVAL, "bad shape M=%lld N=%lld K=%lld", (long long)m, (long long)n, (long long)k);
   *parts = nullptr;
   *n_parts = 0;
-  if (m == 0 || n % 256 != 0 || n > 1024 || !rt::gemm_mfma_takes(a, bt, nullptr, nullptr, m, n, k, dtype)) return RT_OK;
-  const int slices = rt::gemm_mfma_slices(m, n, k, SLICES_BYTES);
+  const int slices = slices_of(a, bt, m, n, k, dtype);
   if (slices == 0) return RT_OK;
   std::lock_guard<std::mutex> lk(ctx->m);
   const int rc = rt::gemm_mfma_part(a, bt, ctx->slices, m, n, k, slices, dtype, stream);
   if (rc) return rc;
   *parts = ctx->slices;
   *n_parts = slices;
+  return RT_OK;
+}
+
+int rt_gemm_bt_tile(int64_t m, int64_t n, int64_t k, int kind, int* rows, int* cols, int* slices) {
+  RT_REQUIRE(rows && cols && slices, RT_EINVAL, "NULL argument");
+  RT_REQUIRE(kind >= RT_EPILOGUE_NONE && kind <= RT_PRODUCT_SLICES, RT_EINVAL, "unknown kind of product %d", kind);
+  RT_REQUIRE(m > 0 && n > 0 && k > 0, RT_EINVAL, "bad shape M=%lld N=%lld K=%lld", (long long)m, (long long)n, (long long)k);
+  *rows = *cols = *slices = 0;
+  const int parts = kind == RT_PRODUCT_SLICES ? slices_of(nullptr, nullptr, m, n, k, RT_F16) : 0;
+  const bool own = kind == RT_PRODUCT_SLICES ? parts > 0
+                                             : rt::gemm_mfma_takes(nullptr, nullptr, nullptr, nullptr, m, n, k, RT_F16) &&
+                                                   (kind == RT_PRODUCT_QKV || rt::gemm_mfma_pays(m, n, k));
+  if (!own) return RT_OK;
+  int tile[3];
+  rt::gemm_mfma_tile(m, n, k, kind == RT_EPILOGUE_BIAS_GELU, kind == RT_PRODUCT_QKV, parts, tile);
+  *rows = tile[0];
+  *cols = tile[1];
+  *slices = tile[2];
   return RT_OK;
 }
 

@@ -21,6 +21,8 @@ int gemm_mfma_qkv(const void* a, const void* bt, const void* bias, void* rows, v
 int gemm_mfma_slices(int64_t m, int64_t n, int64_t k, int64_t max_bytes);
 // The slices; `slices` >= 1 as gemm_mfma_slices gave it.
 int gemm_mfma_part(const void* a, const void* bt, float* parts, int64_t m, int64_t n, int64_t k, int slices, int dtype, void* stream);
+// The tile [rows, columns, slices] that the three above take; max_slices as gemm_mfma_slices gives it, 0 for the other two.
+void gemm_mfma_tile(int64_t m, int64_t n, int64_t k, bool gelu, bool qkv, int max_slices, int* tile);
 
 // gemm_f32.hip: the same product of fp32 operands on bf16 parts; K a multiple of 32, N of 4, 16-byte aligned operands whose
 // byte offsets fit 31 bits.

@@ -1031,4 +1031,11 @@ int gemm_mfma_part(const void* a, const void* bt, float* parts, int64_t m, int64
   return dtype == RT_F16 ? dispatch<_Float16, EPI_PART>(p, ch, st) : dispatch<__bf16, EPI_PART>(p, ch, st);
 }
 
+void gemm_mfma_tile(int64_t m, int64_t n, int64_t k, bool gelu, bool qkv, int max_slices, int* tile) {
+  const Choice ch = choose(m, n, k, max_slices ? EPI_PART : qkv ? EPI_QKV : gelu ? EPI_GELU : EPI_NONE, max_slices);
+  tile[0] = ch.tm;
+  tile[1] = ch.tc;
+  tile[2] = ch.slices;
+}
+
 }  // namespace rt

@@ -41,30 +41,42 @@ def check(got, a, b, bias, gelu, dtype):
     assert over <= 0, over
 
 
-@pytest.mark.parametrize("m,n,k,dtype", [
-    (12288, 256, 128, torch.float16),       # whole tiles, the shortest reduction
-    (12295, 264, 192, torch.bfloat16),      # odd number of steps; 8 columns and 7 rows in tiles of their own
-    (9409, 520, 768, torch.float16),        # 128 x 192
-    (16384 + 33, 1000, 256, torch.bfloat16),        # 192 x 128
+# Tiles that rt_gemm_bt runs these on without and with GELU (None: the library)
+EDGES = [
+    (12288, 256, 128, torch.float16, "96x64 96x64"),        # whole tiles, the shortest reduction
+    (12295, 264, 192, torch.bfloat16, "128x64 128x64"),     # odd number of steps; 8 columns and 7 rows in tiles of their own
+    (9409, 520, 768, torch.float16, "128x192 128x192"),
+    (16384 + 33, 1000, 256, torch.bfloat16, "192x128 192x128"),
     # More tiles than workgroups with the shortest reductions: a tile's first step is followed by its last (two steps, loads
     # reach into the tile after the next) or by one more (three); one row, 8 columns in the last tiles
-    (8065, 2312, 128, torch.float16),       # 192 x 256
-    (16353, 2304, 128, torch.bfloat16),     # 192 x 256, with GELU 224 x 256
-    (12289, 2312, 128, torch.float16),
-    (8065, 2312, 192, torch.bfloat16),
-    (12321, 3080, 192, torch.float16),
-    (1, 8, 128, torch.float16),             # one row, one chunk of columns
-    (64, 768, 3072, torch.bfloat16),        # a long reduction with few outputs: the library
-    (333, 776, 768, torch.float16),         # tiles of 64 x 64
-    (64, 5120, 1280, torch.bfloat16),
-    (700, 2312, 192, torch.float16),        # tiles of 128 x 64
-    (1500, 2304, 768, torch.bfloat16),      # 128 x 128, with GELU 128 x 64
-    (2049, 3080, 320, torch.float16),       # 128 x 256
-    (5600, 768, 1024, torch.bfloat16),      # 192 x 128
-])
+    (8065, 2312, 128, torch.float16, "192x256 192x256"),
+    (16353, 2304, 128, torch.bfloat16, "192x256 224x256"),
+    (12289, 2312, 128, torch.float16, "192x256 192x256"),
+    (8065, 2312, 192, torch.bfloat16, "192x256 192x256"),
+    (12321, 3080, 192, torch.float16, "224x256 224x256"),
+    (32641, 1288, 128, torch.float16, "192x256 256x256"),   # the last panel's lower half has one row
+    (19969, 1288, 192, torch.bfloat16, "256x256 256x256"),
+    (1, 8, 128, torch.float16, "96x64 96x64"),              # one row, one chunk of columns
+    (64, 768, 3072, torch.bfloat16, "None None"),           # a long reduction with few outputs
+    (333, 776, 768, torch.float16, "64x64 64x64"),
+    (64, 5120, 1280, torch.bfloat16, "64x64 64x64"),
+    (700, 2312, 192, torch.float16, "128x64 128x64"),
+    (1500, 2304, 768, torch.bfloat16, "128x128 128x64"),
+    (2049, 3080, 320, torch.float16, "128x256 128x256"),
+    (5600, 768, 1024, torch.bfloat16, "192x128 192x128"),
+]
+
+
+def tile_name(capi, m, n, k, kind):
+    tile = capi.gemm_bt_tile(m, n, k, kind)
+    return "None" if tile is None else "%dx%d" % tile[:2]
+
+
+@pytest.mark.parametrize("m,n,k,dtype,tiles", EDGES)
 @pytest.mark.parametrize("epilogue", [0, 1, 2])
-def test_gemm_bt_edges(capi, m, n, k, dtype, epilogue):
+def test_gemm_bt_edges(capi, m, n, k, dtype, tiles, epilogue):
     print("gemm_bt", m, n, k, dtype, epilogue, flush=True)
+    assert tile_name(capi, m, n, k, epilogue) == tiles.split()[epilogue == 2]
     a, b, bias = operands(m, n, k, dtype)
     c = torch.full((m + 1, n), 7.0, dtype=dtype, device="cuda")
     capi.Gemm().bt(a, b, c[:m], bias=bias if epilogue else None, epilogue=epilogue)
@@ -74,21 +86,26 @@ def test_gemm_bt_edges(capi, m, n, k, dtype, epilogue):
 
 # One row in the last panel and 8 columns in the last tile of every kernel (the model's choice for the shape), with as many
 # steps as its stages hold, fewer, and more, in odd and even number.
-@pytest.mark.parametrize("m,n,k", [
-    (1, 8, 192), (65, 72, 256), (65, 72, 320), (513, 520, 704),                                  # 64 x 64, four stages
-    (1, 8, 128), (97, 72, 128), (9217, 72, 192), (9217, 72, 256), (9217, 72, 320),               # 96 x 64, three
-    (12289, 72, 128), (12289, 72, 192), (12289, 72, 256), (12289, 72, 448),                      # 128 x 64, three
-    (1537, 1928, 768), (1537, 1928, 832),                                                        # 128 x 128
-    (2305, 1672, 128), (2305, 1672, 192), (2305, 1672, 256), (2305, 1672, 320),                  # 192 x 128, three
-    (7297, 520, 192), (7297, 520, 256), (7297, 520, 320),                                        # 128 x 192, three
-    (2049, 3080, 128), (2049, 3080, 192), (2049, 3080, 256), (2049, 3080, 448),                  # 128 x 256, three
-    (4609, 1736, 128), (4609, 1544, 192), (4609, 1544, 256), (4609, 1544, 320),                  # 192 x 192, three
-    (8193, 1544, 128), (16513, 1544, 192),                                                       # 256 x 256, one round and two
-    (3585, 3336, 128), (16513, 1288, 128),                                                       # 224 x 256
-])
+TILES = {
+    "64x64": [(2433, 776, 128), (2433, 776, 192), (65, 72, 256), (65, 72, 320), (513, 520, 704)],            # four stages
+    "96x64": [(1, 8, 128), (97, 72, 128), (9217, 72, 192), (9217, 72, 256), (9217, 72, 320)],                # three
+    "128x64": [(12289, 72, 128), (12289, 72, 192), (12289, 72, 256), (12289, 72, 448)],                      # three
+    "128x128": [(1537, 1928, 768), (1537, 1928, 832)],                                                       # four
+    "192x128": [(2305, 1672, 128), (2305, 1672, 192), (2305, 1672, 256), (2305, 1672, 320)],                 # three
+    "128x192": [(7297, 520, 192), (7297, 520, 256), (7297, 520, 320)],                                       # three
+    "128x256": [(2049, 3080, 128), (2049, 3080, 192), (2049, 3080, 256), (2049, 3080, 448)],                 # three
+    "192x192": [(4609, 1736, 128), (4609, 1544, 192), (4609, 1544, 256), (4609, 1544, 320)],                 # three
+    "192x256": [(8065, 2312, 128)],                                                                          # two rounds
+    "224x256": [(3585, 3336, 128), (16577, 1288, 128)],                                                      # one round and two
+    "256x256": [(8193, 1544, 128), (19969, 1288, 192)],                                                      # one round and two
+}
+
+
+@pytest.mark.parametrize("m,n,k,tile", [shape + (tile,) for tile, shapes in TILES.items() for shape in shapes])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
-def test_gemm_bt_every_tile(capi, m, n, k, dtype):
-    print("gemm_bt tile", m, n, k, dtype, flush=True)
+def test_gemm_bt_every_tile(capi, m, n, k, tile, dtype):
+    print("gemm_bt tile", m, n, k, tile, dtype, flush=True)
+    assert tile_name(capi, m, n, k, 2 if dtype == torch.float16 else 1) == tile
     a, b, bias = operands(m, n, k, dtype, seed=4)
     c = torch.full((m + 1, n), 7.0, dtype=dtype, device="cuda")
     gelu = dtype == torch.float16
@@ -119,30 +136,34 @@ def test_long_reductions_with_few_outputs_go_to_the_library(capi, m, n, k, own, 
     check(c, a, b, bias if epilogue else None, epilogue == 2, torch.float16)
 
 
-@pytest.mark.parametrize("heads,seq_lens,dtype", [
-    (12, [832, 64, 3008, 1024], torch.float16),
-    (5, [64] * 70 + [2048], torch.bfloat16),          # more sequences than one wave looks up at a time, K and V halves of a tile
-    (16, [4096, 320], torch.float16),
-    (2, [64], torch.float16),                         # 64 x 64
-    (12, [192, 320], torch.bfloat16),
-    (2, [192], torch.bfloat16),                       # 64 x 64
-    (3, [64, 256], torch.float16),
-    (3, [2112], torch.bfloat16),                      # 128 x 64, the last panel half full
-    (9, [1216], torch.float16),                       # 128 x 128: the same, and columns past the end
-    (7, [3136], torch.bfloat16),                      # 128 x 256: the same
-    (7, [960, 576], torch.float16),                   # 128 x 64, 252 of 256 workgroups
-    (7, [960, 640], torch.float16),                   # 128 x 128
-    (12, [2048, 1088], torch.bfloat16),               # 128 x 256
+QKV_CASES = [
+    (12, [832, 64, 3008, 1024], torch.float16, "192x256"),
+    (5, [64] * 70 + [2048], torch.bfloat16, "128x256"),     # more sequences than one wave looks up at a time, K and V halves of a tile
+    (16, [4096, 320], torch.float16, "224x256"),
+    (2, [64], torch.float16, "64x64"),
+    (12, [192, 320], torch.bfloat16, "128x64"),
+    (2, [192], torch.bfloat16, "64x64"),
+    (3, [64, 256], torch.float16, "64x64"),
+    (3, [2112], torch.bfloat16, "128x64"),                  # the last panel half full
+    (9, [1216], torch.float16, "128x128"),                  # the same, and columns past the end
+    (7, [3136], torch.bfloat16, "128x256"),                 # the same
+    (7, [960, 576], torch.float16, "128x64"),               # 252 of 256 workgroups
+    (7, [960, 640], torch.float16, "128x128"),
+    (12, [2048, 1088], torch.bfloat16, "128x256"),
     # More tiles than workgroups, so that a tile is followed by another one, where some waves store nothing of it:
-    (6, [14464], torch.float16),                      # tiles of 192: columns past the end, and a last panel with its lower half past the end
-    (10, [4096, 4096, 4160], torch.bfloat16),         # 224: the same
-    (6, [22976], torch.bfloat16),                     # 256: columns past the end
-    (24, [3712], torch.float16),                      # 192: rows past the end only
-    (24, [4096, 2368], torch.bfloat16),               # 256: the same
-])
-def test_qkv_project_equals_gemm_and_split(capi, heads, seq_lens, dtype):
+    (6, [14464], torch.float16, "192x256"),                 # columns past the end, and a last panel with its lower half past the end
+    (10, [4096, 4096, 4160], torch.bfloat16, "224x256"),    # the same
+    (6, [22976], torch.bfloat16, "256x256"),                # columns past the end
+    (24, [3712], torch.float16, "192x256"),                 # rows past the end only
+    (24, [4096, 2368], torch.bfloat16, "256x256"),          # the same
+]
+
+
+@pytest.mark.parametrize("heads,seq_lens,dtype,tile", QKV_CASES)
+def test_qkv_project_equals_gemm_and_split(capi, heads, seq_lens, dtype, tile):
     print("qkv_project", heads, len(seq_lens), dtype, flush=True)
     t, d = sum(seq_lens), heads * 64
+    assert tile_name(capi, t, 3 * d, d, capi.RT_PRODUCT_QKV) == tile
     x, w, bias = operands(t, 3 * d, d, dtype, seed=1)
     sb = torch.from_numpy(capi.seq_prefix_blocks(seq_lens)).cuda()
     rows, k, vt = torch.full((t, 3 * d), 7.0, dtype=dtype, device="cuda"), *(torch.zeros(t * d, dtype=dtype, device="cuda") for _ in "kv")
@@ -155,22 +176,25 @@ def test_qkv_project_equals_gemm_and_split(capi, heads, seq_lens, dtype):
     assert bool((rows[:, d:] == 7.0).all())            # only the queries' columns are written
 
 
-@pytest.mark.parametrize("m,n,k,dtype", [
-    (1, 256, 768, torch.float16),
-    (64, 768, 3072, torch.bfloat16),                  # eight slices
-    (515, 768, 3072, torch.float16),
-    (1500, 1024, 4096, torch.bfloat16),
-    (2816, 768, 3072, torch.float16),
-    (1000, 512, 448, torch.float16),                  # seven steps
-    (1, 256, 2048, torch.bfloat16),                   # 64 x 64: slices of six and seven steps
-    (1441, 512, 3136, torch.float16),                 # 96 x 64: 24 and 25
-    (1025, 512, 3136, torch.bfloat16),                # 128 x 64: 16 and 17, one row in the last panel
-    (1025, 1024, 3136, torch.float16),                # 128 x 128
-    (2881, 768, 3136, torch.bfloat16),                # 192 x 128
-    (64, 320, 1280, torch.float16),                   # a width the slices' LayerNorm does not have
-    (9000, 768, 768, torch.float16),                  # enough rows: not cut
-])
-def test_gemm_bt_layernorm(capi, m, n, k, dtype):
+SLICED = [
+    (1, 256, 768, torch.float16, (64, 64, 2)),
+    (64, 768, 3072, torch.bfloat16, (64, 64, 8)),
+    (515, 768, 3072, torch.float16, (64, 64, 2)),
+    (1500, 1024, 4096, torch.bfloat16, (96, 64, 2)),
+    (2816, 768, 3072, torch.float16, (192, 128, 2)),
+    (1000, 512, 448, torch.float16, None),                  # seven steps: not cut
+    (1, 256, 2048, torch.bfloat16, (64, 64, 5)),            # slices of six and seven steps
+    (1441, 512, 3136, torch.float16, (96, 64, 2)),          # 24 and 25
+    (1025, 512, 3136, torch.bfloat16, (128, 64, 3)),        # 16 and 17, one row in the last panel
+    (1025, 1024, 3136, torch.float16, (128, 128, 3)),
+    (2881, 768, 3136, torch.bfloat16, (192, 128, 2)),
+    (64, 320, 1280, torch.float16, None),                   # a width the slices' LayerNorm does not have
+    (9000, 768, 768, torch.float16, None),                  # enough rows: not cut
+]
+
+
+@pytest.mark.parametrize("m,n,k,dtype,tile", SLICED)
+def test_gemm_bt_layernorm(capi, m, n, k, dtype, tile):
     """rt_gemm_bt_slices + rt_slices_residual_layernorm against fp32.  The LayerNorm's input x is a sum of the product
     (error of an fp32 sum as in check(); uncut, the product is also rounded to the stored type), bias and residual; an
     error e of an element moves the output by at most e * gamma / std plus the shift of mean and variance by the row's
@@ -181,11 +205,7 @@ def test_gemm_bt_layernorm(capi, m, n, k, dtype):
     res, gamma, beta = (torch.randn(*s, generator=g, device="cuda").to(dtype) for s in ((m, n), (n,), (n,)))
     out = torch.full((m + 1, n), 7.0, dtype=dtype, device="cuda")
     slices = capi.Gemm().bt_layernorm(a, b, bias, res, gamma, beta, out[:m], 1e-5)
-    print("  slices", slices, flush=True)
-    if n == 320 or m == 9000:
-        assert slices == 0
-    elif k >= 3072:
-        assert slices > 1
+    assert capi.gemm_bt_tile(m, n, k, capi.RT_PRODUCT_SLICES) == tile and slices == (tile[2] if tile else 0)
     prod = a.float() @ b.float().t()
     err = 2.0 ** -23 * k * (a.float().abs() @ b.float().abs().t())
     if slices == 0:
@@ -199,6 +219,21 @@ def test_gemm_bt_layernorm(capi, m, n, k, dtype):
     over = ((out[:m].float() - want).abs() - bound).max().item()
     assert over <= 0, over
     assert bool((out[m] == 7.0).all())
+
+
+def test_every_tile_of_the_selection_is_met(capi):
+    """The shapes above reach every tile that a product of up to 40 000 rows can run on, in each of its forms."""
+    rows = [64 * r for r in range(1, 64)] + [1024 * r for r in range(4, 40)]
+    def chosen(kind, shapes):
+        return {capi.gemm_bt_tile(m, n, k, kind)[:2] for n, k in shapes for m in rows if capi.gemm_bt_tile(m, n, k, kind)}
+    def name(tiles):
+        return {"%dx%d" % t for t in tiles}
+    wide = [(n, k) for n in (8, 72, 264, 520, 776, 1288, 1672, 2056, 2304, 3072, 3336, 4096) for k in (128, 192, 768, 1024, 3072)]
+    assert name(chosen(capi.RT_EPILOGUE_NONE, wide) | chosen(capi.RT_EPILOGUE_BIAS_GELU, wide)) == set(TILES)
+    heads = [(192 * h, 64 * h) for h in range(2, 25)]
+    assert name(chosen(capi.RT_PRODUCT_QKV, heads)) == {c[3] for c in QKV_CASES}
+    ends = [(n, k) for n in (256, 512, 768, 1024) for k in (256, 768, 1024, 3072, 4096)]
+    assert chosen(capi.RT_PRODUCT_SLICES, ends) == {c[4][:2] for c in SLICED if c[4]}
 
 
 @pytest.mark.parametrize("m,n,k", [
