@@ -547,8 +547,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 // them.
 // Measured (us, one launch among others, fp16; before: the fragments of a half read in one burst, the loads in another, bias
 // and sequence ends loaded behind the loop): 512 x 2304 x 768 7.6 -> 5.1, 512 x 768 x 3072 15.1 -> 9.4, 2048 x 768 x 768
-// 7.9 -> 5.7, 4096 x 768 x 3072 25.4 -> 21.5, 5568 x 768 x 3072 33.9 -> 27.5, 8192 x 768 x 3072 42.6 -> 35.9.  A 64 x 64 step
-// takes 330 cycles (matrix instructions 140), a 128 x 128 one 700 (560), a 192 x 192 one 1450 (1260).
+// 7.9 -> 5.7, 4096 x 768 x 3072 25.4 -> 21.5, 5568 x 768 x 3072 33.9 -> 27.5, 8192 x 768 x 3072 42.6 -> 35.9.  Counters over
+// two lengths of the reduction: a 64 x 64 step takes 365 cycles (its SIMD's matrix instructions 128), a 128 x 128 one 663 (512), a
+// 192 x 192 one 1414 (1152).
 template <typename T> struct Product;        // the instruction as a builtin: these accumulators leave registers to spare
 template <> struct Product<_Float16> {
   __device__ static f32x4 run(f16x8 a, f16x8 b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0); }
@@ -983,12 +984,13 @@ bool gemm_mfma_takes(const void* a, const void* bt, const void* bias, const void
 }
 
 // An uncut product is one chain of steps, 0.16 us each; with at most 64 of the smallest tiles most CUs have none and a
-// library that cuts the reduction is ahead on long ones.  Measured (us in a graph, operands in rotation, hipBLASLt / here): 64 x
-// 768 x 1280 6.0 / 5.7, x 3072 7.2 / 10.9, x 16384 14.9 / 41; 256 x 1024 (64 tiles) x 1280 6.8 / 6.4, x 4096 10.8 / 13.4.  The
-// line at 1280 dates from slower steps; moved to where the two cross (about 1500) it would give at most 0.4 us.  On the
-// other side, here: 256 x 768 x 1024 5.3, 512 x 768 (96 tiles) x 2048 8.6, 512 x 1024 x 4096 13.9.
+// library that cuts the reduction is ahead on long ones.  Measured (us in a graph, operands in rotation, hipBLASLt tuned for the
+// shape / here): 64 x 768 x 1280 6.3 / 6.3, x 1536 7.0 / 6.7, x 2048 5.5-8.3 / 7.8, x 3072 7.4-10.7 / 10.7, x 8192 10.3 / 23.0;
+// 256 x 1024 (64 tiles) x 1280 7.0 / 6.5, x 1536 7.6 / 7.0, x 2560 8.4-10.1 / 10.2, x 4096 11.1 / 13.5; 1 x 4096 x 1536
+// 7.8 / 6.8, x 3072 8.8-10.7 / 11.1.  Between 1536 and 2560 it depends on which solution the library's timing has found.  More
+// outputs, here: 512 x 768 (96 tiles) x 2048 8.6, 512 x 1024 x 4096 13.9.
 bool gemm_mfma_pays(int64_t m, int64_t n, int64_t k) {
-  return k < 20 * BK || ((m + 63) / 64) * ((n + 63) / 64) > 64;
+  return k <= 24 * BK || ((m + 63) / 64) * ((n + 63) / 64) > 64;
 }
 
 int gemm_mfma_bt(const void* a, const void* bt, const void* bias, void* c, int64_t m, int64_t n, int64_t k, bool gelu, int dtype,

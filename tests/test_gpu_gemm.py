@@ -115,8 +115,8 @@ def test_gemm_bt_every_tile(capi, m, n, k, tile, dtype):
 
 
 @pytest.mark.parametrize("m,n,k,own", [
-    (64, 768, 1216, True), (64, 768, 1280, False), (1, 256, 16384, False), (1, 4096, 4096, False), (1, 4104, 4096, True),
-    (512, 512, 3072, False), (513, 512, 3072, True),
+    (64, 768, 1536, True), (64, 768, 1600, False), (1, 256, 16384, False), (1, 4096, 4096, False), (1, 4104, 4096, True),
+    (512, 512, 1536, True), (512, 512, 3072, False), (513, 512, 3072, True),
 ])
 @pytest.mark.parametrize("epilogue", [0, 2])
 def test_long_reductions_with_few_outputs_go_to_the_library(capi, m, n, k, own, epilogue):
