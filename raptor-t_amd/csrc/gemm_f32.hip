@@ -12,11 +12,12 @@
 // 384 a run) while the other multiplies (96 matrix instructions a run).
 //
 // Bound by what a SIMD issues, the products of parts and the cutting (what-if builds: without two of the six products
-// -36 %, without the loads -10 %), and, up to 256 tiles, by one workgroup's chain.  Measured (us, operands in rotation,
-// hipBLASLt tuned for the shape, the same on a solution picked for another row count, as a batch of a new length meets it / this
-// kernel): 1024 x 2304 x 768 33.5, 47.9 / 33.0, 1024 x 3072 x 768 + GELU 40.6, 43.4 / 36.0, 1024 x 768 x 3072 39.5, 47.8 / 36.5,
-// 4096 x 3072 x 768 + GELU 142, 158 / 124, 8192 x 2304 x 768 207, 215 / 178; relative error against 64 bits 4.0-9.9e-7 / 1.3-4.3e-7
-// (K = 768 to 3072).  A priority for one of a SIMD's two waves: no gain.
+// -36 %, without the loads -10 %; counters: 2440-2650 cycles a run, 1536 of them matrix instructions), and, up to 256 tiles, by
+// one workgroup's chain.  Measured (us, operands in rotation, hipBLASLt tuned for the shape, the same on a solution picked for
+// another row count, as a batch of a new length meets it / this kernel): 1024 x 2304 x 768 33.5, 47.9 / 33.0, 1024 x 3072 x 768 +
+// GELU 40.6, 43.4 / 36.0, 1024 x 768 x 3072 39.5, 47.8 / 36.5, 4096 x 3072 x 768 + GELU 142, 158 / 124, 8192 x 2304 x 768 207,
+// 215 / 178; relative error against 64 bits 4.0-9.9e-7 / 1.3-4.3e-7 (K = 768 to 3072).  A priority for one of a SIMD's two
+// waves: no gain.
 //
 // Values that bf16 parts cannot hold: a part that overflows or is not finite makes a result that is not finite; a part below
 // 2^-126 counts as zero, which moves a result by at most 2^-125 * K * (max |a| + max |b|) (products and sums of parts below it
