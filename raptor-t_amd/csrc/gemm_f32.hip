@@ -91,12 +91,6 @@ __device__ inline Parts cut(const Raw& r, float& peak) {
                __builtin_bit_cast(bf16x8, u32x4{w[0][2], w[1][2], w[2][2], w[3][2]})};
 }
 
-__device__ inline float gelu_tanh(float x) {   // as the 16-bit products' epilogue
-  constexpr float K0 = -2.0f * 0.7978845608028654f * 1.4426950408889634f;
-  constexpr float K1 = K0 * 0.044715f;
-  return x * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(x * fmaf(K1, x * x, K0)));
-}
-
 template <int NW, bool GELU>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_f32_kernel(Params p) {
   // a run's operands of every wave, 128-byte rows, chunk c of row r at c ^ ((r >> 1) & 7); after the loop four waves' sums,

@@ -97,13 +97,6 @@ template <int TM> constexpr int lds_bytes() { return 3 * a_stage<TM>() + 2 * B_S
 
 #define SB() __builtin_amdgcn_sched_barrier(0)
 
-__device__ inline float gelu_tanh(float x) {   // x / (1 + 2^(x (k0 + k1 x^2))), as bias_gelu_kernel
-  constexpr float K0 = -2.0f * 0.7978845608028654f * 1.4426950408889634f;
-  constexpr float K1 = K0 * 0.044715f;
-  const float t = x * fmaf(K1, x * x, K0);
-  return x * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(t));
-}
-
 // v_permlane32_swap: the upper 32 lanes of a change places with the lower 32 of b; v_permlane16_swap: lanes 16-31 and
 // 48-63 of a with lanes 0-15 and 32-47 of b.
 __device__ inline void permlane32_swap(uint32_t& a, uint32_t& b) {

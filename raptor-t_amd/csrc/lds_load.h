@@ -1,4 +1,4 @@
-// What the kernels of the dense products share: loads from memory straight to LDS, and leave to use much of it.
+// What the kernels of the dense products share: loads from memory straight to LDS, leave to use much of it, the GELU.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -20,6 +20,13 @@ __device__ inline void load_to_lds(i32x4 srd, int voff, int soff, uint32_t lds) 
 __device__ inline i32x4 make_srd(const void* p, uint32_t bytes) {
   const uint64_t a = reinterpret_cast<uint64_t>(p);
   return i32x4{int(uint32_t(a)), int(uint32_t(a >> 32) & 0xffffu), int(bytes), 0x00020000};
+}
+
+__device__ inline float gelu_tanh(float x) {   // x / (1 + 2^(x (k0 + k1 x^2))), as bias_gelu_kernel
+  constexpr float K0 = -2.0f * 0.7978845608028654f * 1.4426950408889634f;
+  constexpr float K1 = K0 * 0.044715f;
+  const float t = x * fmaf(K1, x * x, K0);
+  return x * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(t));
 }
 
 // More dynamic LDS than the default has to be asked for once per kernel and device.
