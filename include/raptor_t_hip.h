@@ -303,10 +303,11 @@ int rt_gemm_bias_act(rt_gemm_ctx* ctx, const void* a, const void* b, const void*
  * layer objects keep their weights as [out, in] and call this.
  * 16-bit types with K a multiple of 64 run on kernels of the library's own, but for long reductions of few outputs
  * (rt_gemm_bt_tile); so does RT_F32 with K a multiple of 32, N of 4 and enough outputs; the rest on hipBLASLt, which is the only
- * one that rt_gemm_set_tuning and rt_gemm_set_retuning concern.  The fp32 kernel multiplies operands as three bf16 parts, six of
- * nine products of parts, added up in fp32: at most 2^-24 (1 + 2^-10) of a product is left out, and the sums are no further
- * from 64 bits than fp32 instructions'.  Results that are not finite, or so small beside their row and column that parts below
- * 2^-126 could show, come from fp32 instructions; which ones depends on no other row or column. */
+ * one that rt_gemm_set_tuning and rt_gemm_set_retuning concern.  The fp32 kernel multiplies operands as three bf16 parts and adds
+ * up the six largest of nine products of parts in fp32: at most 2^-24 (1 + 2^-10) of a product is left out.  A product by itself is
+ * off by up to 1.5 * 2^-23; sums of hundreds are nearer to 64 bits than those of fp32 instructions (1.3-4.3e-7 against 4.0-9.9e-7,
+ * relative, at K = 768 to 3072).  Results that are not finite, or so small beside their row and column that parts below 2^-126
+ * could show, come from fp32 instructions; which ones depends on no other row or column. */
 int rt_gemm_bt(rt_gemm_ctx* ctx, const void* a, const void* bt, const void* bias, void* c,
                int64_t m, int64_t n, int64_t k, int epilogue, int dtype, void* stream);
 
