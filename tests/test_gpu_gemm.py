@@ -318,9 +318,9 @@ def on_own_kernel(capi, call):
     assert capi.time_next_launch(None, None) == 0
 
 
-# Both sides of the line between the own kernel and the library, each where it is the faster one by 3 % or more
+# Both sides of the line between the own kernel and the library at its best (tuned for the shape): own up to 7 % behind it
 @pytest.mark.parametrize("m,n,k,own", [
-    (1024, 768, 3072, True), (704, 2304, 768, True), (1024, 1024, 1536, True), (4096, 768, 768, True),
+    (1024, 768, 3072, True), (704, 2304, 768, True), (1024, 2304, 768, True), (2048, 768, 768, True), (1024, 1024, 1536, True), (4096, 768, 768, True),
     (640, 768, 3072, False), (512, 2304, 768, False), (1024, 768, 768, False), (384, 1024, 4096, False), (256, 3072, 768, False),
     (2113, 3076, 96, False), (2048, 2304, 256, False),                   # short reductions
 ])
