@@ -346,6 +346,25 @@ int rt_sequence_pool(const void* hidden, const int* seq_blocks_dev, const int* s
 int rt_pooler_dense_tanh(const void* pooled, const void* weight_t, const void* bias, void* out,
                          int batch, int d_in, int d_out, int dtype, void* stream);
 
+/* ------------------------------------------------------------- padded <-> packed batches */
+
+/* tokens_dev[s] = the number of ones of row s of an attention mask [batch, width] (integer entries of 1, 4 or 8 bytes,
+ * rows row_stride entries apart), or -1 where they are not a prefix of the row or other nonzero values occur. */
+int rt_padded_tokens(const void* mask, int elem_bytes, int64_t row_stride, int batch, int64_t width, int* tokens_dev,
+                     void* stream);
+
+/* The packed ids of a padded batch [batch, width] (int32 or int64, rows *_stride entries apart; types may be NULL: zeros).
+ * Sequence s takes tokens_dev[s] places rounded up to `block`, or fixed_length where that is not 0; `longest` is the
+ * largest of these lengths and `total` their sum, the entries of each output.  Places past the padded width hold zeros. */
+int rt_pack_tokens(const void* ids, int ids_bytes, int64_t ids_stride, const void* types, int types_bytes,
+                   int64_t types_stride, int batch, int64_t width, const int* tokens_dev, int block, int fixed_length,
+                   int64_t longest, int64_t total, int* out_ids, int* out_positions, int* out_types, void* stream);
+
+/* out[s, j] = packed[starts[s] + j] for j < tokens[s], zeros for the other rows of out[batch, width] (rows of row_bytes
+ * bytes, a multiple of 16).  starts and tokens are host arrays. */
+int rt_unpack_rows(const void* packed, int64_t packed_rows, int64_t row_bytes, const int64_t* starts,
+                   const int64_t* tokens, int batch, int64_t width, void* out, void* stream);
+
 /* ------------------------------------------------------- metadata / stream pipeline */
 
 /* Replaces Semaphore + MetaData + the per-layer std::async index workers

@@ -27,6 +27,7 @@ EXPORTS = [
     "rt_bs_attention_fwd_masked", "rt_bs_attention_fwd_qrows", "rt_bs_attention_fwd_no_alloc",
     "rt_bias_residual_layernorm", "rt_bias_gelu", "rt_embed_layernorm", "rt_gemm_create", "rt_gemm_destroy", "rt_gemm_set_tuning", "rt_gemm_set_retuning", "rt_gemm",
     "rt_gemm_bias_act", "rt_gemm_bt", "rt_gemm_bt_slices", "rt_gemm_bt_tile", "rt_slices_residual_layernorm", "rt_sequence_pool", "rt_pooler_dense_tanh",
+    "rt_padded_tokens", "rt_pack_tokens", "rt_unpack_rows",
     "rt_pipeline_create", "rt_pipeline_publish", "rt_pipeline_acquire", "rt_pipeline_release",
     "rt_pipeline_destroy", "rt_pipeline_set_index_check",
 ]
@@ -84,6 +85,9 @@ def lib():
         L.rt_slices_residual_layernorm.argtypes = [vp, vp, I, vp, vp, vp, vp, L64, I, F, I, vp]
         L.rt_sequence_pool.argtypes = [vp, vp, vp, I, I, I, vp, I, vp]
         L.rt_pooler_dense_tanh.argtypes = [vp, vp, vp, vp, I, I, I, I, vp]
+        L.rt_padded_tokens.argtypes = [vp, I, L64, I, L64, vp, vp]
+        L.rt_pack_tokens.argtypes = [vp, I, L64, vp, I, L64, I, L64, vp, I, I, L64, L64, vp, vp, vp, vp]
+        L.rt_unpack_rows.argtypes = [vp, L64, L64, i64p, i64p, I, L64, vp, vp]
         L.rt_pipeline_create.argtypes = [ctypes.POINTER(vp), I, I, I, I, I, I, I]
         L.rt_pipeline_publish.argtypes = [vp, i32p, I]
         L.rt_pipeline_acquire.argtypes = [vp, I, vp, ctypes.POINTER(vp), ctypes.POINTER(vp), i32p,
@@ -368,6 +372,44 @@ def pooler_dense_tanh(pooled, weight_t, bias, out):
         _dp(t, pooled.dtype, None, name)
     check(lib().rt_pooler_dense_tanh(_dp(pooled), _dp(weight_t), _dp(bias), _dp(out), batch, d_in, d_out,
                                      _dtype_code(pooled), _stream()))
+    return out
+
+
+def _rows_of(t, sizes, name):
+    """(device pointer, bytes of an entry, entries between rows) of an integer [batch, length] GPU tensor whose rows are runs."""
+    if not t.is_cuda or t.dim() != 2 or t.dtype.is_floating_point or t.element_size() not in sizes or t.stride(1) != 1:
+        raise ValueError("%s must be a [batch, length] GPU tensor of integers with contiguous rows" % name)
+    return ctypes.c_void_p(t.data_ptr()), t.element_size(), t.stride(0)
+
+
+def padded_tokens(mask, tokens):
+    """tokens[s] (int32) = ones of row s of the mask, -1 where they are not a prefix of the row."""
+    p, size, stride = _rows_of(mask, (1, 4, 8), "mask")
+    check(lib().rt_padded_tokens(p, size, stride, mask.shape[0], mask.shape[1], _ip(tokens, mask.shape[0], "tokens"), _stream()))
+    return tokens
+
+
+def pack_tokens(ids, types, tokens, block, fixed_length, longest, out_ids, out_positions, out_types):
+    """Packed ids, positions and token types (types may be None: zeros) of a padded batch; see rt_pack_tokens."""
+    total = out_ids.numel()
+    p, size, stride = _rows_of(ids, (4, 8), "ids")
+    tp, tsize, tstride = (ctypes.c_void_p(0), 4, 0) if types is None else _rows_of(types, (4, 8), "types")
+    if types is not None and types.shape != ids.shape:
+        raise ValueError("types must have the shape of ids")
+    check(lib().rt_pack_tokens(p, size, stride, tp, tsize, tstride, ids.shape[0], ids.shape[1],
+                               _ip(tokens, ids.shape[0], "tokens"), block, fixed_length, longest, total,
+                               _ip(out_ids, total, "out_ids"), _ip(out_positions, total, "out_positions"),
+                               _ip(out_types, total, "out_types"), _stream()))
+
+
+def unpack_rows(packed, starts, tokens, out):
+    """out[s, j] = packed[starts[s] + j] for j < tokens[s], zeros elsewhere; starts and tokens are sequences of ints."""
+    batch = len(starts)
+    if packed.dim() != 2 or out.dim() != 3 or out.shape[0] != batch or out.shape[2] != packed.shape[1] or len(tokens) != batch:
+        raise ValueError("packed must be [rows, width] and out [sequences, length, width]")
+    arr = ctypes.c_int64 * batch
+    check(lib().rt_unpack_rows(_dp(packed, out.dtype, None, "packed"), packed.shape[0], packed.shape[1] * packed.element_size(),
+                               arr(*starts), arr(*tokens), batch, out.shape[1], _dp(out, name="out"), _stream()))
     return out
 
 

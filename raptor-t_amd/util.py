@@ -7,10 +7,12 @@ count is an argument instead of the literal 12.  `generate_array_with_avg` (:78-
 `generate_input_data` (:114-123) produce the synthetic variable-length batches of the
 reference's benchmarks.
 """
+import itertools
 import random
 
 import numpy as np
 import torch
+from torch.autograd import forward_ad
 
 from . import capi
 
@@ -101,6 +103,9 @@ def pack_padded_batch(input_ids, attention_mask, token_type_ids=None, block_size
     """
     if input_ids.dim() != 2 or attention_mask.shape != input_ids.shape:
         raise ValueError("input_ids and attention_mask must both be [batch, length]")
+    packed = _pack_on_gpu(input_ids, attention_mask, token_type_ids, block_size, keep_width)
+    if packed is not None:
+        return packed
     mask = attention_mask.to(torch.int64)
     tokens = mask.sum(dim=1)
     b, length = input_ids.shape
@@ -130,9 +135,63 @@ def pack_padded_batch(input_ids, attention_mask, token_type_ids=None, block_size
             "seq_tokens_tensor": torch.tensor(seq_tokens, dtype=torch.int32, device=input_ids.device)}
 
 
+def _ordinary(t):
+    """A tensor whose memory a kernel may read as it is: on the current GPU, no subclass, nothing that traces, batches or
+    differentiates the operators applied to it."""
+    return (type(t) is torch.Tensor and t.is_cuda and t.device.index == torch.cuda.current_device() and not t.requires_grad and
+            not torch._C._functorch.is_functorch_wrapped_tensor(t) and forward_ad._current_level < 0 and not torch.jit.is_tracing())
+
+
+def _rows(t, dtypes):
+    return _ordinary(t) and t.dtype in dtypes and t.stride(1) == 1 and t.stride(0) >= 0
+
+
+def _pack_on_gpu(input_ids, attention_mask, token_type_ids, block_size, keep_width):
+    """pack_padded_batch by two kernels; None where the batch has to take the general way: other types or strides, no entries,
+    and every mask that is not plain ones and zeros with the ones in front, which the general way refuses or counts."""
+    ints = (torch.int32, torch.int64)
+    if not (type(block_size) is int and block_size >= 1 and 1 <= input_ids.shape[0] <= 65535 and input_ids.shape[1] >= 1 and
+            _rows(input_ids, ints) and _rows(attention_mask, ints + (torch.bool, torch.uint8))):
+        return None
+    if token_type_ids is not None and not (isinstance(token_type_ids, torch.Tensor) and token_type_ids.shape == input_ids.shape and
+                                           _rows(token_type_ids, ints)):
+        return None
+    length = input_ids.shape[1]
+    tokens = torch.empty(input_ids.shape[0], dtype=torch.int32, device=input_ids.device)
+    seq_tokens = capi.padded_tokens(attention_mask, tokens).tolist()
+    if min(seq_tokens) < 1:
+        return None
+    up = lambda n: (n + block_size - 1) // block_size * block_size
+    fixed = up(length) if keep_width else 0
+    seq_lens = [fixed] * len(seq_tokens) if keep_width else [up(n) for n in seq_tokens]
+    total = sum(seq_lens)
+    if total >= 1 << 31 or fixed >= 1 << 31:
+        return None
+    ids, pos, typ = (torch.empty(total, dtype=torch.int32, device=input_ids.device) for _ in range(3))
+    capi.pack_tokens(input_ids, token_type_ids, tokens, block_size, fixed, max(seq_lens), ids, pos, typ)
+    return {"input_ids": ids, "position_ids": pos, "token_type_ids": typ, "seq_lens": seq_lens, "seq_tokens": seq_tokens,
+            "seq_tokens_tensor": tokens}
+
+
+def _unpacks_on_gpu(packed, starts, seq_lens, seq_tokens, length):
+    """Whether the unpacking kernel takes these rows: ordinary ones of whole 16-byte vectors on the current GPU, every
+    sequence inside of them and of the padded length.  (The general way has the words for what is wrong otherwise.)"""
+    if not (_ordinary(packed) and packed.dim() == 2 and packed.is_contiguous() and packed.data_ptr() % 16 == 0):
+        return False
+    row = packed.shape[1] * packed.element_size()
+    if row == 0 or row % 16 or row >= 1 << 24 or type(length) is not int or not 1 <= length < 1 << 24 or length * row >= 1 << 37:
+        return False
+    return (len(starts) >= 1 and len(seq_lens) == len(seq_tokens) and all(type(n) is int for n in (*seq_lens, *seq_tokens)) and
+            all(n >= 0 and 0 <= t <= length and s + t <= packed.shape[0] for s, n, t in zip(starts, seq_lens, seq_tokens)))
+
+
 def unpack_to_padded(packed, seq_lens, seq_tokens, length):
     """[T, D] packed encoder output -> [B, length, D] with zeros on the padded positions (the padded rows of
     the packed output are whatever the layers computed for padding tokens and are dropped here)."""
+    starts = list(itertools.accumulate(seq_lens, initial=0))[:-1]
+    if _unpacks_on_gpu(packed, starts, seq_lens, seq_tokens, length):
+        out = torch.empty(len(seq_lens), length, packed.shape[1], dtype=packed.dtype, device=packed.device)
+        return capi.unpack_rows(packed, starts, seq_tokens, out)
     out = packed.new_zeros(len(seq_lens), length, packed.shape[1])
     start = 0
     for s, (n, real) in enumerate(zip(seq_lens, seq_tokens)):

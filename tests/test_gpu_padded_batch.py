@@ -1,0 +1,91 @@
+"""Packing a padded batch and unpacking its rows on the GPU: the kernels against the same call on host tensors, which takes
+the general way."""
+import importlib
+
+import pytest
+import torch
+
+import __graft_entry__ as graft
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ut():
+    graft.load_package()
+    return importlib.import_module("raptor_t_amd.util")
+
+
+def mask_of(lens, width, dtype):
+    return (torch.arange(width)[None, :] < torch.tensor(lens)[:, None]).to(dtype)
+
+
+@pytest.mark.parametrize("lens,width", [([1], 1), ([64, 1, 63, 65], 65), ([130, 64, 1], 150), ([300, 256, 257, 1024], 1024),
+                                        ([(7 * i) % 300 + 1 for i in range(300)], 301)])
+@pytest.mark.parametrize("ids_dtype,mask_dtype,types_dtype", [(torch.int64, torch.int64, None), (torch.int32, torch.bool, torch.int64),
+                                                              (torch.int64, torch.uint8, torch.int32), (torch.int32, torch.int32, torch.int32)])
+@pytest.mark.parametrize("keep_width", [False, True])
+def test_pack_equals_the_general_way(ut, lens, width, ids_dtype, mask_dtype, types_dtype, keep_width):
+    gen = torch.Generator().manual_seed(width)
+    wide = torch.randint(1, 50000, (len(lens), 2 * width), generator=gen).to(ids_dtype)
+    ids = wide[:, width // 2:width // 2 + width]                     # rows further apart than they are long
+    types = None if types_dtype is None else torch.randint(0, 2, (len(lens), width), generator=gen).to(types_dtype)
+    mask = mask_of(lens, width, mask_dtype)
+    want = ut.pack_padded_batch(ids, mask, types, keep_width=keep_width)
+    got = ut.pack_padded_batch(wide.cuda()[:, width // 2:width // 2 + width], mask.cuda(), None if types is None else types.cuda(),
+                               keep_width=keep_width)
+    assert got["seq_lens"] == want["seq_lens"] and got["seq_tokens"] == want["seq_tokens"]
+    for name in ("input_ids", "position_ids", "token_type_ids", "seq_tokens_tensor"):
+        assert got[name].is_cuda and got[name].dtype == want[name].dtype and got[name].is_contiguous()
+        assert torch.equal(got[name].cpu(), want[name]), name
+
+
+@pytest.mark.parametrize("change", ["hole", "empty", "left", "values", "float", "transposed"])
+def test_pack_odd_masks_as_the_general_way(ut, change):
+    """What the general way refuses is refused, what it accepts gives the same batch."""
+    ids = torch.arange(3 * 200).view(3, 200) + 1
+    mask = mask_of([200, 100, 7], 200, torch.int64)
+    if change == "hole":
+        mask[1, 50] = 0
+    elif change == "empty":
+        mask[2] = 0
+    elif change == "left":
+        mask = mask.flip(1)
+    elif change == "values":                        # the sum of the entries counts: 100 places hold a token, 2 more are claimed
+        mask[1, :2] = 2
+    elif change == "float":
+        mask = mask.float()
+    elif change == "transposed":
+        ids = ids.t().contiguous().t()
+
+    def call(i, m):
+        try:
+            return ut.pack_padded_batch(i, m)
+        except ValueError as e:
+            return str(e)
+    want, got = call(ids, mask), call(ids.cuda() if change != "transposed" else ids.t().cuda().t(), mask.cuda())
+    if isinstance(want, str):
+        assert got == want
+    else:
+        assert got["seq_tokens"] == want["seq_tokens"] and torch.equal(got["input_ids"].cpu(), want["input_ids"])
+
+
+@pytest.mark.parametrize("lens,width", [([1], 1), ([64, 1, 63, 65], 65), ([130, 64, 1], 150), ([0, 5, 0], 9), ([700, 3], 1100),
+                                        ([(7 * i) % 30 + 1 for i in range(300)], 31)])
+@pytest.mark.parametrize("cols,dtype", [(8, torch.float16), (768, torch.bfloat16), (12, torch.float32), (3, torch.float32), (1024, torch.float32)])
+def test_unpack_equals_the_general_way(ut, lens, width, cols, dtype):
+    """Rows of one vector and of many, of whole vectors and not (3 columns: the general way), several launches (300 sequences),
+    sequences without a row."""
+    seq_lens = [-(-n // 64) * 64 for n in lens]
+    packed = torch.randn(max(1, sum(seq_lens)), cols, generator=torch.Generator().manual_seed(cols)).to(dtype)
+    want = ut.unpack_to_padded(packed, seq_lens, lens, width)
+    torch.empty(want.shape, dtype=dtype, device="cuda").fill_(float("nan"))      # what the allocator hands out next is not zeros
+    got = ut.unpack_to_padded(packed.cuda(), seq_lens, lens, width)
+    assert got.dtype == dtype and torch.equal(got.cpu(), want)
+
+
+@pytest.mark.parametrize("seq_lens,tokens,width", [([64, 64], [64, 65], 100), ([64, 64], [64, 64], 60), ([64], [64], 64.0)])
+def test_unpack_refuses_what_the_general_way_refuses(ut, seq_lens, tokens, width):
+    packed = torch.zeros(128 if len(seq_lens) > 1 else 64, 8, dtype=torch.float16, device="cuda")
+    with pytest.raises((RuntimeError, TypeError)):
+        ut.unpack_to_padded(packed, seq_lens, tokens, width)
