@@ -472,19 +472,8 @@ template <typename T> struct QSide { const T* bias; char* stage; };
 // Rows -> fragments through the wave's own LDS room (no other wave touches it: LDS operations of one wave
 // execute in order), then (x + bias) * scale in fp32, rounded once: the arithmetic of the split kernel.
 template <typename T>
-__device__ inline void finish_q(const Args<T>& a, const QSide<T>& qs, const Unit& u, int lane,
-                                typename Mma<T>::v8 (&qf)[2][4]) {
+__device__ inline void scale_q(const Args<T>& a, const T* qbias, const Unit& u, int lane, typename Mma<T>::v8 (&qf)[2][4]) {
   typedef typename Mma<T>::v8 v8;
-  if (!a.q_rows) return;
-  const T* qbias = qs.bias;
-  {
-    char* wr = qs.stage + (lane >> 3) * Q_STAGE_PITCH + (lane & 7) * 16;
-#pragma unroll
-    for (int k = 0; k < 8; ++k) *reinterpret_cast<v8*>(wr + k * 8 * Q_STAGE_PITCH) = qf[k >> 2][k & 3];
-    const char* rd = qs.stage + (lane & 31) * Q_STAGE_PITCH + (lane >> 5) * 16;
-#pragma unroll
-    for (int k = 0; k < 8; ++k) qf[k >> 2][k & 3] = *reinterpret_cast<const v8*>(rd + (k >> 2) * 32 * Q_STAGE_PITCH + (k & 3) * 32);
-  }
 #pragma unroll
   for (int c = 0; c < 4; ++c) {
     const v8 bb = *reinterpret_cast<const v8*>(qbias + u.h * 64 + c * 16 + (lane >> 5) * 8);
@@ -498,6 +487,21 @@ __device__ inline void finish_q(const Args<T>& a, const QSide<T>& qs, const Unit
         qf[nt][c][e] = static_cast<T>(y);
       }
   }
+}
+template <typename T>
+__device__ inline void finish_q(const Args<T>& a, const QSide<T>& qs, const Unit& u, int lane,
+                                typename Mma<T>::v8 (&qf)[2][4]) {
+  typedef typename Mma<T>::v8 v8;
+  if (!a.q_rows) return;
+  {
+    char* wr = qs.stage + (lane >> 3) * Q_STAGE_PITCH + (lane & 7) * 16;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) *reinterpret_cast<v8*>(wr + k * 8 * Q_STAGE_PITCH) = qf[k >> 2][k & 3];
+    const char* rd = qs.stage + (lane & 31) * Q_STAGE_PITCH + (lane >> 5) * 16;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) qf[k >> 2][k & 3] = *reinterpret_cast<const v8*>(rd + (k >> 2) * 32 * Q_STAGE_PITCH + (k & 3) * 32);
+  }
+  scale_q<T>(a, qs.bias, u, lane, qf);
 }
 
 // lane j: byte offset inside K / V^T of the tile of the row's entry first + j * step (the first 64 of them)
@@ -801,10 +805,36 @@ __device__ inline void slow_row(const Args<T>& a, const Buffers<T>& b, const QSi
   stream_tiles<T, MASKED>(a.k + gbase, a.vt + gbase, a.to_idx + r.p0, first, step, r.cnt, r.u.n, r.u.tail, r.u.nbv, lane, qf, st);
 }
 
-// Entries first, first + step, ... of row r through the state with the pipelined loop, no hand-over
-// from or to another row.  False: the row has to be run with the moving-maximum loop instead (more
-// than 64 entries for this wave, or scores that outgrew the reference); the state is then undefined.
-// HAVE_Q: the queries are in t.qf already; they are there afterwards too.
+// Entries first, first + step, ... of row r for the pipelined loop, no hand-over from or to another row: the tiles the wave
+// has (ids, my, pd), the first of them requested, behind the queries if WITH_Q.
+enum { SHARE_SLOW, SHARE_EMPTY, SHARE_RUNS };      // for the moving-maximum loop (more than 64 entries); no tile that counts
+template <typename T, bool MASKED, bool WITH_Q>
+__device__ inline int begin_share(const Args<T>& a, const Buffers<T>& b, const Row& r, int first, int step, int lane, Tiles<T>& t,
+                                  int& ids, int& my, Padding& pd) {
+  first = __builtin_amdgcn_readfirstlane(first);
+  my = __builtin_amdgcn_readfirstlane((r.cnt - first + step - 1) / step);           // this wave's entries
+  if (my <= 0) return SHARE_EMPTY;
+  if (my > 64) return SHARE_SLOW;
+  ids = row_offsets<T>(a, r, first, step, lane);
+  pd = padding_of(r.u, r.goff);
+  if (MASKED) {
+    if (!pad_to_end(ids, my, lane, pd)) return SHARE_SLOW;
+    if (my == 0) return SHARE_EMPTY;                   // every tile of this wave's share is padding
+  }
+  if (WITH_Q) request_q<T>(a, b, r.u, lane, t.qf);
+  request_first<T>(b, __builtin_amdgcn_readlane(ids, 0), lane, t);
+  return SHARE_RUNS;
+}
+// The share through the state, its queries in t.qf (they are there afterwards too).  False: the row has to be run with the
+// moving-maximum loop instead (scores that outgrew the reference); the state is then undefined.
+template <typename T, bool MASKED, bool FEW>
+__device__ inline bool end_share(const Buffers<T>& b, int ids, int my, const Padding& pd, int lane, Tiles<T>& t, State& st) {
+  float mref;
+  if (!fast_reference<T, MASKED>(t, mref, pd.last > 0 && my == 1, pd.tail, lane)) return false;
+  fast_loop<T, MASKED, FEW>(b, ids, my, -1, lane, mref, t, st, NoNextQ{}, pd);
+  return sums_finite(st);
+}
+// Both, by one wave for itself.  HAVE_Q: the queries are in t.qf already.
 template <typename T, bool MASKED, bool HAVE_Q, bool FEW>
 __device__ inline bool fast_share(const Args<T>& a, const Buffers<T>& b, const QSide<T>& qbias, const Row& r, int first, int step,
                                   int lane, Tiles<T>& t, State& st) {
@@ -1330,12 +1360,19 @@ __global__ __launch_bounds__(256, 2) void bs_attention_kernel(Args<T> a) {
 // each (global_shares), or RPW other rows with 8 / RPW waves each (rows_per_workgroup has the rule and the times of both
 // kernels).  At most 64 sequences (a lane each).
 constexpr int FEW_CUS = 256;
+// A share's outputs in LDS: 64 queries x 64 fp32 in rows 272 bytes apart, which puts the 16 lanes of an access on different
+// banks both for the writes (16 rows, 16 bytes of each) and for the reads (2 rows, every second 16 bytes).
+constexpr int SLOT_PITCH = 68, SLOT_FLOATS = 64 * SLOT_PITCH;
 template <typename T, int NW> struct FewRoom {
-  // four wave states in a merge; each wave's room for a query tile
-  static constexpr int PARK = 4 * PARK_FLOATS > NW * Q_STAGE_BYTES / 4 ? 4 * PARK_FLOATS : NW * Q_STAGE_BYTES / 4;
-  __attribute__((aligned(16))) float park[PARK];
+  // a slot per wave; ahead of the merge, query tiles (wave w's own at stage(w), a shared row's at that of its number)
+  __attribute__((aligned(16))) float slots[NW][SLOT_FLOATS];
+  float m[8][64], l[8][64];                            // per share and query: reference and sum
   __attribute__((aligned(16))) T qbias[MAX_HEADS_QROWS * 64];
-  int failed[8];                                       // per row: a wave's pipelined loop handed it back
+  __device__ __forceinline__ char* stage(int w) { return reinterpret_cast<char*>(slots) + w * Q_STAGE_BYTES; }
+  // Per row: a wave's pipelined loop handed it back.  Between the rows of the last slot, behind the query tiles.  (With four
+  // waves the room is half of a CU's LDS to the byte.)
+  static_assert(NW * Q_STAGE_BYTES <= (NW - 1) * SLOT_FLOATS * 4, "the flags lie behind the query tiles");
+  __device__ __forceinline__ int& failed(int row) { return reinterpret_cast<int&>(slots[NW - 1][row * SLOT_PITCH + 64]); }
 };
 
 // Lane l: where sequence l begins and ends.  Also fills the bias copy; the caller's barrier follows.
@@ -1347,7 +1384,7 @@ template <typename T> struct FewBatch {
     sb1 = a.seq_blocks[min(lane + 1, a.batch)];
     if (a.q_rows)
       for (int i = threadIdx.x; i < a.heads * 64; i += 64 * NW) room.qbias[i] = a.q_bias ? a.q_bias[i] : static_cast<T>(0.f);
-    if (threadIdx.x < 8) room.failed[threadIdx.x] = 0;
+    if (threadIdx.x < 8) room.failed(threadIdx.x) = 0;
   }
   template <bool MASKED> __device__ __forceinline__ Unit unit_at(const Args<T>& a, int s, int h, int i) const {
     Unit u;
@@ -1366,9 +1403,9 @@ template <typename T> struct FewBatch {
   }
   // Shares of a global row: eight, one workgroup of eight waves per row; or four, the two global rows of a (sequence, head) in one
   // workgroup, where that saves a round of workgroups, unless one would be a longer chain (16 tiles) than the other rows' two
-  // rounds.  Measured (us, eight shares / four, 12 heads): three sequences of 8704 tokens in all 31.8 / 26.3, four of 9344 30.8 /
-  // 27.3, six of 8512 27.0 / 21.8, bf16 padded 5 x 320-3000 31.6 / 27.8; where the rounds stay as many, six of 9600 28.4 / 33.6,
-  // five of 11008 31.3 / 34.7.
+  // rounds.  Measured (us, eight shares / four, 12 heads): three sequences of 8704 tokens in all 32.7 / 28.1, four of 9344 32.5 /
+  // 27.1, six of 8512 29.2 / 22.8, bf16 padded 5 x 320-3000 32.0 / 28.2; where the rounds stay as many, six of 9600 31.5 / 36.3,
+  // five of 11008 34.3 / 38.3.
   // Only with 8 other rows to a workgroup, the least of them, are there more than one round (rows_per_workgroup).
   template <int RPW> __device__ __forceinline__ int global_shares(const Args<T>& a, int n_sparse) const {
     if (RPW < 8 || n_sparse == 0) return 8;
@@ -1392,64 +1429,204 @@ template <typename T> __device__ __forceinline__ Buffers<T> few_buffers(const Ar
   return b;
 }
 
-// The workgroup's NW waves on their rows, from the first tile to the output: a row's tiles in `share` shares (the same number
-// in all waves; 8 where RPW is 1), taken by that many waves side by side, or by all NW if there are fewer.  u: the
-// wave's row; `valid`: it has one.
-template <typename T, bool MASKED, int RPW, int NW>
-__device__ __forceinline__ void share_rows(const Args<T>& a, const Buffers<T>& b, FewRoom<T, NW>& room, const QSide<T>& qbias,
-                                           const Unit& u, bool valid, int share, int lane, int wave) {
-  const int waves = share < NW ? share : NW, row = wave >> __builtin_ctz(waves), part = wave & (waves - 1);      // powers of two
-  const Row r = describe<T>(a, u);
-  State st;
-  if (NW < 8 && share > NW) {
-    // two shares per wave: the later one first, whose state waits in the wave's own park place (u is valid in all waves)
-    static_assert(NW == 8 || NW == 4, "eight shares are one or two per wave");
-    Tiles<T> t;
-    request_q<T>(a, b, u, lane, t.qf);
-    finish_q<T>(a, qbias, u, lane, t.qf);
-    __syncthreads();                                   // the query rooms are read
-    float* const own = room.park + wave * PARK_FLOATS;
-    auto two_shares = [&](auto one) {
-      bool ok = one(wave + 4);
+// The queries of a row in t.qf of all its WAVES waves: wave `part` fetches its part of the eight requests, all read the tile
+// from LDS.  fetch_queries requests, share_queries ends behind the workgroup's barrier (none if a row has one wave).
+template <int WAVES, typename T>
+__device__ __forceinline__ void fetch_queries(const Args<T>& a, const Buffers<T>& b, const Unit& u, int part, int lane, Tiles<T>& t) {
+  const QPlan q = q_plan<T>(a, u, lane);
 #pragma unroll
-      for (int nt = 0; nt < 2; ++nt) st.l[nt] = pair_sum(st.l[nt]);
-      park_state(st, own, lane);
-      ok = one(wave) && ok;
+  for (int j = 0; j < 8 / WAVES; ++j) t.qf[j >> 2][j & 3] = fetch_q<T>(b, q, part + j * WAVES);
+}
+template <int WAVES, typename T>
+__device__ __forceinline__ void share_queries(const Args<T>& a, const T* qbias, const Unit& u, bool valid, char* stage, int part, int lane, Tiles<T>& t) {
+  typedef typename Mma<T>::v8 v8;
+  // rows, read as fragments; or the fragments as they are
+  const int wr = a.q_rows ? (lane >> 3) * Q_STAGE_PITCH + (lane & 7) * 16 : lane * 16, wr_k = a.q_rows ? 8 * Q_STAGE_PITCH : 1024;
+  const int rd = a.q_rows ? (lane & 31) * Q_STAGE_PITCH + (lane >> 5) * 16 : lane * 16;
+  const int rd_nt = a.q_rows ? 32 * Q_STAGE_PITCH : 4096, rd_c = a.q_rows ? 32 : 1024;
+  if (valid) {
 #pragma unroll
-      for (int nt = 0; nt < 2; ++nt) st.l[nt] = pair_sum(st.l[nt]);
-      return ok;
-    };
-    const bool ok = two_shares([&](int p) { return fast_share<T, MASKED, true, true>(a, b, qbias, r, p, 8, lane, t, st); });
-    if (__syncthreads_or(!ok))
-      two_shares([&](int p) { slow_row<T, MASKED>(a, b, qbias, r, p, 8, lane, true, t.qf, st); return true; });
-    absorb_state(st, own, lane);
-  } else {
-    state_init(st);
-    if (valid && !fast_row<T, MASKED, true>(a, b, qbias, r, part, share, lane, st) && lane == 0) room.failed[row] = 1;
-    __syncthreads();                                   // the query rooms are read
-    if (valid && room.failed[row]) {
-      typename Mma<T>::v8 qf[2][4];
-      slow_row<T, MASKED>(a, b, qbias, r, part, share, lane, false, qf, st);
-    }
-#pragma unroll
-    for (int nt = 0; nt < 2; ++nt) st.l[nt] = pair_sum(st.l[nt]);
+    for (int j = 0; j < 8 / WAVES; ++j) *reinterpret_cast<v8*>(stage + wr + (part + j * WAVES) * wr_k) = t.qf[j >> 2][j & 3];
   }
+  if (WAVES > 1) __syncthreads();
+  if (!valid) return;
 #pragma unroll
-  for (int half = NW / 2; half >= 1; half >>= 1) {
-    if (2 * half > share) continue;
-    __syncthreads();                                   // the park is free
-    float* const place = room.park + (row * half + (part & (half - 1))) * PARK_FLOATS;
-    if (part >= half && part < 2 * half) park_state(st, place, lane);
-    __syncthreads();
-    if (part < half) absorb_state(st, place, lane);
+  for (int k = 0; k < 8; ++k) t.qf[k >> 2][k & 3] = *reinterpret_cast<const v8*>(stage + rd + (k >> 2) * rd_nt + (k & 3) * rd_c);
+  if (a.q_rows) scale_q<T>(a, qbias, u, lane, t.qf);
+}
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+// The state's outputs times w in the wave's slot, 16 runs of 4 per lane; ADD: plus what stands there times w4.
+template <bool ADD> __device__ __forceinline__ void to_slot(float* slot, const State& st, const float (&w)[2], const float (&w4)[2], int lane) {
+#pragma clang fp contract(off)
+#pragma unroll
+  for (int nt = 0; nt < 2; ++nt)
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        f32x4* const at = reinterpret_cast<f32x4*>(slot + (32 * nt + (lane & 31)) * SLOT_PITCH + 32 * t + 8 * q + 4 * (lane >> 5));
+        f32x4 x;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x[e] = st.o[t][nt][4 * q + e] * w[nt];
+        if (ADD) {
+          const f32x4 kept = *at;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) x[e] = x[e] + kept[e] * w4[nt];
+        }
+        *at = x;
+      }
+}
+
+// The SHARES shares of a row, one or two per wave, to its output, in two steps: every wave scales its outputs to the largest of
+// the shares' references and leaves them in its slot; then every wave adds up its part of the queries, over all of the row's
+// slots, and stores it.  Sums are formed in the order ((0 + 4) + (2 + 6)) + ((1 + 5) + (3 + 7)), or its part for fewer shares,
+// whoever forms them.
+template <typename T, int NW, int SHARES>
+__device__ __forceinline__ void merge_shares(FewRoom<T, NW>& room, const State& st, T* out_unit, int64_t stride, bool valid, int row,
+                                             int part, int lane, int wave) {
+#pragma clang fp contract(off)
+  constexpr int WAVES = SHARES < NW ? SHARES : NW;
+  constexpr bool TWO = SHARES > NW;
+  const int base = row * WAVES;                        // the row's first share
+  auto reference = [&](int query) {                    // of the whole row; finite even if no share has met a key
+    float m[SHARES];
+#pragma unroll
+    for (int s = 0; s < SHARES; ++s) m[s] = room.m[base + s][query];
+#pragma unroll
+    for (int s = 1; s < SHARES; ++s) m[0] = fmaxf(m[0], m[s]);
+    return m[0];
+  };
+  {
+    float w[2], w4[2];
+#pragma unroll
+    for (int nt = 0; nt < 2; ++nt) {
+      const int query = 32 * nt + (lane & 31);
+      const float m = fmaxf(reference(query), LOWEST);
+      w[nt] = __builtin_amdgcn_exp2f(st.m[nt] - m);
+      w4[nt] = TWO ? __builtin_amdgcn_exp2f(room.m[part + 4][query] - m) : 0.f;
+      if (lane < 32) {
+        room.l[base + part][query] = st.l[nt] * w[nt];
+        if (TWO) room.l[part + 4][query] *= w4[nt];
+      }
+    }
+    to_slot<TWO>(room.slots[wave], st, w, w4, lane);
   }
   __syncthreads();
-  if (valid && part == 0) {
+  if (!valid) return;
+  // eight queries at a time, eight outputs per lane
+  constexpr int TIMES = 8 / WAVES;
+  const int first = part * (64 / WAVES) + (lane >> 3);
+  float l[TIMES][SHARES];
+  f32x4 x[TIMES][WAVES][2];
+#pragma unroll
+  for (int i = 0; i < TIMES; ++i) {
+#pragma unroll
+    for (int s = 0; s < SHARES; ++s) l[i][s] = room.l[base + s][first + 8 * i];
+#pragma unroll
+    for (int s = 0; s < WAVES; ++s) {
+      const f32x4* const from = reinterpret_cast<const f32x4*>(room.slots[base + s] + (first + 8 * i) * SLOT_PITCH + (lane & 7) * 8);
+      x[i][s][0] = from[0];
+      x[i][s][1] = from[1];
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < TIMES; ++i) {
+#pragma unroll
+    for (int half = SHARES / 2; half >= 1; half /= 2)
+#pragma unroll
+      for (int s = 0; s < half; ++s) {
+        l[i][s] = l[i][s] + l[i][s + half];
+        if (half < WAVES) {
+          x[i][s][0] = x[i][s][0] + x[i][s + half][0];
+          x[i][s][1] = x[i][s][1] + x[i][s + half][1];
+        }
+      }
+    float w = __builtin_amdgcn_rcpf(fmaxf(l[i][0], 1e-30f));
+    if (__any(l[i][0] == 0.f)) w = row_weight(l[i][0], reference(first + 8 * i));       // no key, or none with a finite score
+    u32x4 o;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[e] = Mma<T>::two(x[i][0][e >> 1][2 * (e & 1)] * w, x[i][0][e >> 1][2 * (e & 1) + 1] * w);
+    *reinterpret_cast<u32x4*>(out_unit + int64_t(first + 8 * i) * stride + (lane & 7) * 8) = o;
+  }
+}
+
+// The workgroup's NW waves on their rows, from the first tile to the output: a row's tiles in SHARES shares, taken by that many
+// waves side by side, or by all NW, two each, if there are fewer.  u: the wave's row; `valid`: it has one.
+template <typename T, bool MASKED, int SHARES, int NW>
+__device__ __forceinline__ void share_rows(const Args<T>& a, const Buffers<T>& b, FewRoom<T, NW>& room, const QSide<T>& qbias,
+                                           const Unit& u, bool valid, int lane, int wave) {
+  constexpr int WAVES = SHARES < NW ? SHARES : NW;
+  constexpr bool TWO = SHARES > NW;                    // part and part + 4 (u is valid in all waves)
+  static_assert(SHARES <= 2 * NW && (!TWO || NW == 4), "one or two shares per wave");
+  const int row = wave / WAVES, part = wave % WAVES;
+  float* const slot = room.slots[wave];
+  const float ones[2] = {1.f, 1.f};
+  const int64_t stride = int64_t(a.heads) * 64;
+  T* const out_unit = a.out + int64_t(u.g0 + u.i) * 64 * stride + u.h * 64;
+  State st;
+  Row r;
+  bool redo;                                           // by the moving-maximum loop
+  describe_bounds<T>(a, u, r);
+  auto publish = [&](int s) {                          // what the row's other waves have to know of share s
+#pragma unroll
+    for (int nt = 0; nt < 2; ++nt) {
+      st.l[nt] = pair_sum(st.l[nt]);
+      if (lane < 32) {
+        room.m[s][32 * nt + lane] = st.m[nt];
+        room.l[s][32 * nt + lane] = st.l[nt];
+      }
+    }
+  };
+  {
+    Tiles<T> t;
+    int ids = 0, my = 0, what = SHARE_EMPTY;
+    Padding pd;
+    if (valid) {
+      fetch_queries<WAVES, T>(a, b, u, part, lane, t);
+      what = begin_share<T, MASKED, false>(a, b, r, TWO ? part + 4 : part, SHARES, lane, t, ids, my, pd);
+    }
+    share_queries<WAVES, T>(a, room.qbias, u, valid, room.stage(row), part, lane, t);
+    if (TWO) __syncthreads();                          // the query tile is read: its place is a slot's
+    state_init(st);
+    bool ok = what == SHARE_RUNS ? end_share<T, MASKED, true>(b, ids, my, pd, lane, t, st) : what == SHARE_EMPTY;
+    if (TWO) {
+      publish(part + 4);
+      to_slot<false>(slot, st, ones, ones, lane);
+      ok = fast_share<T, MASKED, true, true>(a, b, qbias, r, part, SHARES, lane, t, st) && ok;
+    }
+    redo = !ok;
+    if (SHARES > 1 && redo && lane == 0) room.failed(row) = 1;
+  }
+  int any_failed = 0;                                  // the same in all waves
+  if (SHARES > 1) {
+    publish(row * WAVES + part);
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < NW / WAVES; ++i) any_failed |= room.failed(i);
+    any_failed = __builtin_amdgcn_readfirstlane(any_failed);
+    redo = any_failed && __builtin_amdgcn_readfirstlane(room.failed(row)) != 0;
+  }
+  if (valid && redo) {
+    typename Mma<T>::v8 qf[2][4];
+    if (TWO) {                                         // (one row: all waves are here)
+      slow_row<T, MASKED>(a, b, qbias, r, part + 4, SHARES, lane, false, qf, st);
+      __syncthreads();                                 // the query tiles are read
+      publish(part + 4);
+      to_slot<false>(slot, st, ones, ones, lane);
+    }
+    slow_row<T, MASKED>(a, b, qbias, r, part, SHARES, lane, TWO, qf, st);
+    if (SHARES > 1) publish(row * WAVES + part);
+  }
+  if constexpr (SHARES == 1) {
+    if (!valid) return;
     float w[2];
 #pragma unroll
-    for (int nt = 0; nt < 2; ++nt) w[nt] = row_weight(st.l[nt], st.m[nt]);
-    const int64_t stride = int64_t(a.heads) * 64;
-    store_output<T>(a.out + int64_t(u.g0 + u.i) * 64 * stride + u.h * 64, stride, lane, st, w, qbias.stage);
+    for (int nt = 0; nt < 2; ++nt) w[nt] = row_weight(pair_sum(st.l[nt]), st.m[nt]);
+    store_output<T>(out_unit, stride, lane, st, w, qbias.stage);
+  } else {
+    if (any_failed) __syncthreads();
+    merge_shares<T, NW, SHARES>(room, st, out_unit, stride, valid, row, part, lane, wave);
   }
 }
 
@@ -1462,7 +1639,7 @@ __global__ __launch_bounds__(512, 2) void bs_attention_few_kernel(Args<T> a) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const FewBatch<T> batch(a, room);
   const int lane = batch.lane, sb0 = batch.sb0, sb1 = batch.sb1;
-  const QSide<T> qbias{room.qbias, reinterpret_cast<char*>(room.park) + wave * Q_STAGE_BYTES};
+  const QSide<T> qbias{room.qbias, room.stage(wave)};
   const unsigned long long sparse = __ballot(lane < a.batch && sb1 - sb0 >= RT_MIN_SPARSE_BLOCKS);
   const int n_sparse = __popcll(sparse), n_rows = a.nb_total - 2 * n_sparse;
   const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
@@ -1493,15 +1670,18 @@ __global__ __launch_bounds__(512, 2) void bs_attention_few_kernel(Args<T> a) {
     u.i = j - __builtin_amdgcn_readlane(listed_before, s) + ((sparse >> s & 1ull) ? 1 : 0);
   }
   __syncthreads();
-  share_rows<T, MASKED, RPW, 8>(a, few_buffers(a), room, qbias, u, valid, global ? shares : 8 / RPW, lane, wave);
+  const Buffers<T> b = few_buffers(a);
+  if (RPW > 1 && !global) share_rows<T, MASKED, 8 / RPW, 8>(a, b, room, qbias, u, valid, lane, wave);
+  else if (RPW < 8 || shares == 8) share_rows<T, MASKED, 8, 8>(a, b, room, qbias, u, valid, lane, wave);
+  else share_rows<T, MASKED, 4, 8>(a, b, room, qbias, u, valid, lane, wave);
 }
 
 // With a caller's plan workgroup c walks its slice, as in the persistent kernel: four waves, two workgroups per CU, a global
 // row by all of them, other entries side by side as far as there are waves for them.  A unit's tiles are cut into as many
 // shares as without a plan, so the bits are the same; a wave takes two of a global row's eight, or one of its four.  The slice
 // is clamped to the list, ids outside it are skipped.  Measured (us a call, 12 heads, rt_meta_partition_lpt into 512 and 256;
-// persistent kernel / this one): 1 x 4096 tokens 22.7, 21.1 / 23.7, 21.1; 8 x 150-1700 28.8, 35.6 / 28.7, 32.1; 2 x 4096 31.9,
-// 34.7 / 32.7, 32.0; 6 x 2048 44.5, 50.4 / 42.1, 41.9; 7 x 2048 50.7, 60.6 / 46.8, 52.1 (one workgroup of 8 waves per unit: 96).
+// persistent kernel / this one): 1 x 4096 tokens 22.7, 21.1 / 22.5, 21; 8 x 150-1700 28.8, 35.6 / 28.7, 32.1; 2 x 4096 31.9,
+// 34.7 / 32.7, 32.0; 6 x 2048 44.5, 50.4 / 40.8, 41; 7 x 2048 50.7, 60.6 / 46.8, 52.1 (one workgroup of 8 waves per unit: 96).
 // Behind it: plans of fewer workgroups than CUs for few units (1 x 2048 into 64: 21.7 / 41.8), whose rows are cut finer than
 // they need.
 template <typename T, bool MASKED, int RPW>
@@ -1514,7 +1694,7 @@ __global__ __launch_bounds__(256, 2) void bs_attention_few_plan_kernel(Args<T> a
   const int end = min(max(a.from_pos[blockIdx.x + 1], begin), n_units);
   if (begin == end) return;
   const FewBatch<T> batch(a, room);
-  const QSide<T> qbias{room.qbias, reinterpret_cast<char*>(room.park) + wave * Q_STAGE_BYTES};
+  const QSide<T> qbias{room.qbias, room.stage(wave)};
   const Buffers<T> b = few_buffers(a);
   const int shares =
       batch.template global_shares<RPW>(a, __popcll(__ballot(batch.lane < a.batch && batch.sb1 - batch.sb0 >= RT_MIN_SPARSE_BLOCKS)));
@@ -1549,9 +1729,14 @@ __global__ __launch_bounds__(256, 2) void bs_attention_few_plan_kernel(Args<T> a
         }
       }
     }
-    if (threadIdx.x < 8) room.failed[threadIdx.x] = 0;           // (the last rows' flags were read several barriers ago)
+    // what the code below derives from the lane number is derived again for every unit, not kept in registers
+    int lane = batch.lane;
+    asm volatile("" : "+v"(lane));
+    if (threadIdx.x < 8) room.failed(threadIdx.x) = 0;           // (the last rows' flags were read several barriers ago)
     __syncthreads();
-    share_rows<T, MASKED, RPW, 4>(a, b, room, qbias, u, whole || SIDE * wave / 4 < run, whole ? shares : 8 / RPW, batch.lane, wave);
+    if (RPW > 1 && !whole) share_rows<T, MASKED, 8 / RPW, 4>(a, b, room, qbias, u, SIDE * wave / 4 < run, lane, wave);
+    else if (RPW < 8 || shares == 8) share_rows<T, MASKED, 8, 4>(a, b, room, qbias, u, true, lane, wave);
+    else share_rows<T, MASKED, 4, 4>(a, b, room, qbias, u, true, lane, wave);
     p += run;
   }
 }
@@ -1602,12 +1787,11 @@ int64_t most_pairs(int batch, int total_blocks, int heads) {
 }
 
 // Rows that share a workgroup of bs_attention_few_kernel, as few as still give every workgroup a CU of its own and every
-// wave a tile (1 x 64 tokens: 6.7, 7.1, 5.7, 4.3 us with 1, 2, 4, 8; persistent kernel 13.2); 0: the persistent kernel.
-// Measured (us, 12 heads, persistent kernel / this one with 1, 2, 4, 8 rows to a workgroup): 1 x 512
-// tokens 18.2 / 8.1, 9.0, 10.5, 13.3; 1 x 2048 19.7 / 16.0, 12.3, 12.3, 14.0; 4 x 256-1024 22.5 / 23.1, 18.3, 13.1,
-// 16.7; 1 x 4096 25.6 / 29.5, 18.5, 17.7, 17.2; 8 x 150-1700 27.5 / 34.7, 26.8, 23.1, 16.8; 2 x 4096 35.4 / -, -, 25.9,
-// 22.7; 6 x 2048 42.0 / -, -, 40.9, 35.9.  From 3072 units on (16 heads, 6 x 2048: 50.9 / 51.5) a row is no longer the
-// shorter chain, and the persistent kernel's schedule is the better one.
+// wave a tile (1 x 64 tokens: 6.6, 7.7, 6.5, 5.3 us with 1, 2, 4, 8; persistent kernel 12.8); 0: the persistent kernel.
+// Measured (us in a graph, 12 heads, persistent kernel / this one with 1, 2, 4, 8 rows to a workgroup): 1 x 512
+// tokens 18.8 / 8.4, 9.5, 11.9, 14.8; 1 x 2048 20.1 / 16.5, 12.6, 13.0, 15.9; 4 x 256-1024 22.2 / 22.8, 20.0, 14.5,
+// 18.0; 1 x 4096 26.5 / 30.9, 20.3, 18.4, 18.3; 8 x 150-1700 28.9 / 37.3, 29.3, 24.4, 19.9; 2 x 4096 36.1 / 52.4, 39.1, 29.2,
+// 23.0; 6 x 2048 43.7 / 73.8, 52.9, 43.8, 37.8.
 int rows_per_workgroup(int batch, int total_blocks, int heads) {
   const int64_t units = int64_t(total_blocks) * heads;
   if (batch > 64 || units > 2816) return 0;
