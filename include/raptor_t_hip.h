@@ -73,7 +73,7 @@ int rt_abi_version(void);
  * launch (layers/kernels/add_bias_act.cu:109-131, the `info` map of every launcher); a pair of events recorded
  * around a launch also counts the gaps to the neighbouring kernels.  After this call the next kernel that one
  * of this library's kernel entry points (every one below, but not a product that goes to hipBLASLt; each launches one
- * kernel, rt_bs_attention_fwd_no_alloc a small clearing kernel before it that does not count) launches from the calling
+ * kernel) launches from the calling
  * thread writes the start and end timestamps of its dispatch into the two hipEvent_t (created by the caller,
  * either may be NULL); hipEventElapsedTime between them is the kernel's duration as a profiler reports it.
  * One launch consumes the pair; (NULL, NULL) withdraws a pair no launch has taken.  Returns 1 if the call
@@ -174,19 +174,15 @@ int rt_unpack_head_tiles(const void* packed, void* dst, const int* seq_blocks_de
  * out[T, H*64] token-major = softmax over the listed key blocks of (q . k) @ v, evaluated
  * as 2^(q.k) / sum 2^(q.k): the scale log2(e)/sqrt(d) is already folded into q.  to_idx/to_pos: device CSR from rt_meta_build_to_index
  * (plan_heads = 1 or heads).  If from_idx/from_pos are non-NULL the launch is
- * `n_wg` persistent workgroups each walking its slice of the LPT plan (balanced);
- * otherwise the kernel hands the units out itself: two persistent workgroups per CU draw
- * tickets from per-XCD counters, the two rows of each sparse (sequence, head) that list every
- * block first (four waves share such a row), then one unit per wave.
+ * `n_wg` workgroups each walking its slice of the LPT plan (balanced);
+ * otherwise the launch enumerates the units itself: the two rows of each sparse (sequence, head) that list every
+ * block first (four waves or more share such a row), then the others.
  * dtype RT_F16 / RT_BF16: fp32 accumulation, probabilities rounded to the tensor type for the
  * second product.  RT_F32 (the reference's fp32-output dispatch, sparse_attention.cu:1582-1599):
  * every tensor fp32, fp32 matrix instructions; an accuracy mode, about ten times slower.
  * Limits of one launch (RT_EINVAL beyond them): batch <= 1024 sequences, total_blocks <= 4096
- * (262144 tokens), total_blocks * heads * 24576 < 2^31 (byte offsets are 32-bit).  The first launch
- * on a device without from_idx/from_pos allocates 384 KiB of counters that the library keeps
- * (rt_bs_attention_fwd_no_alloc does not): a ring of 64 sets, one per launch, each left zeroed by the
- * launch that used it.  Launches may overlap on any number of streams and threads, in any order, as
- * long as no more than 64 of them are in flight on one device at a time. */
+ * (262144 tokens), total_blocks * heads * 24576 < 2^31 (byte offsets are 32-bit).  A launch uses no
+ * memory but its arguments: launches may overlap on any number of streams and threads, in any order. */
 int rt_bs_attention_fwd(const void* q, const void* k, const void* vt, void* out,
                         const int* seq_blocks_dev, int batch, int total_blocks, int heads,
                         const int* to_idx, const int* to_pos, int plan_heads,
@@ -225,17 +221,10 @@ int rt_bs_attention_fwd_qrows(const void* qkv, const void* qkv_bias, float q_sca
 
 /* rt_bs_attention_fwd_masked for callers that cannot allocate device memory (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc).  It has no counterpart in the
- * reference.  The other attention entry points take the kernel's queue counters from a ring that the
- * library allocates on a device's first launch; this one keeps them in a static device array of
- * RT_NO_ALLOC_SCRATCH_BYTES that every GPU the library runs on holds until the process ends, and calls
- * no hipMalloc, hipFree or other allocating routine.  It always runs the kernel's own enumeration (no
- * from_idx/from_pos plan; that launch uses no counters and allocates nothing in any entry point).
- * Limits: batch <= RT_NO_ALLOC_MAX_BATCH and total_blocks <= RT_NO_ALLOC_MAX_BLOCKS, else RT_EINVAL.
- * Every call on one GPU uses the same counters, cleared by a small kernel ahead of the launch: calls
- * that overlap on one GPU (two streams, two threads) race and give wrong results; calls on one stream,
- * or otherwise ordered, are fine.  The first call on a device looks the array's address up
- * (hipGetSymbolAddress): make that call outside a graph capture. */
-#define RT_NO_ALLOC_SCRATCH_BYTES 8192
+ * reference.  Its limits are stated as constants; it takes no from_idx/from_pos plan.  (None of the attention entry points
+ * allocates in the 16-bit types; this one and its scratch size date from a kernel that kept queue counters.)
+ * Limits: batch <= RT_NO_ALLOC_MAX_BATCH and total_blocks <= RT_NO_ALLOC_MAX_BLOCKS, else RT_EINVAL. */
+#define RT_NO_ALLOC_SCRATCH_BYTES 0
 #define RT_NO_ALLOC_MAX_BATCH 1024
 #define RT_NO_ALLOC_MAX_BLOCKS 4096
 int rt_bs_attention_fwd_no_alloc(const void* q, const void* k, const void* vt, void* out,

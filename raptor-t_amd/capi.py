@@ -301,7 +301,7 @@ def bs_attention_fwd(q, k, vt, out, seq_blocks_dev, heads, to_idx, to_pos, plan_
 
 
 def bs_attention_fwd_no_alloc(q, k, vt, out, seq_blocks_dev, heads, to_idx, to_pos, plan_heads, seq_tokens_dev=None):
-    """bs_attention_fwd through the entry point that allocates no device memory (static queue counters)."""
+    """bs_attention_fwd through the entry point that allocates no device memory."""
     batch, nb, _ = _attention_args(out, k, vt, seq_blocks_dev, heads, to_idx, to_pos, plan_heads, None, None, seq_tokens_dev)
     _dp(q, out.dtype, out.numel(), "q")
     check(lib().rt_bs_attention_fwd_no_alloc(_dp(q), _dp(k), _dp(vt), _dp(out), _dp(seq_blocks_dev), _dp(seq_tokens_dev),

@@ -24,32 +24,26 @@
 //       (maximum over the row's first 32 keys, shared by a lane's two queries) and enters the
 //       score product as the MFMA's C operand.  Nothing is tested inside the loop: a row whose
 //       scores outgrow the reference shows up as a row sum that is not finite.
-//   moving maximum (fallback) such rows, rows of more than 64 entries per wave and launches with
-//       padded sequences are put aside and run afterwards by the loop that tracks the maximum
-//       tile by tile.  The two loops never share a loop nest: the register allocator treats
-//       them apart, and the pipelined one stays free of scratch-memory traffic.
+//   moving maximum (fallback) such rows and rows of more than 64 entries per wave are run by the loop that tracks the
+//       maximum tile by tile.  The two loops never share a loop nest: the register allocator treats them apart, and the
+//       pipelined one stays free of scratch-memory traffic.
 //
-// Schedule: persistent workgroups (two per CU) that draw work from ticket counters in device
-// memory, one pair of counters per XCD (workgroups are dealt round-robin to the 8 XCDs, and each
-// XCD has its own L2): XCD x owns the x-th eighth of the (head, row) items, so the K / V^T tiles
-// of a (sequence, head) are fetched into one L2.
-//   phase 1  global rows (the first and last block of a sparse sequence): one workgroup per row,
-//            its 4 waves take every 4th key block and merge their softmax states through LDS;
-//            the two rows of a (sequence, head) are consecutive tickets, so they stream the
-//            same tiles at the same time;
-//   phase 2  all other rows: every wave draws single units.  While it computes unit u it knows
-//            unit u+1 (ticket, CSR row bounds and block ids through scalar loads), requests
-//            u+1's first K / V^T tile in u's last tile steps and u+1's queries in the same
-//            steps, and draws the ticket of unit u+2: a tile loop ahead while the queue is long,
-//            only after the loop near its end (a wave never holds two waiting units then).
-// With an LPT plan (from_idx / from_pos) n_wg workgroups walk their unit lists instead.
+// Schedule: one workgroup of four waves per global row (the first and the last block of a sparse sequence), whose tiles the waves
+// share and whose results meet in LDS, then one per four other rows, a wave each; two workgroups to a CU, started by the
+// hardware as earlier ones end.  Workgroups are dealt round-robin to the 8 XCDs, each of which has its own L2: XCD x owns the x-th
+// eighth of the rows, head-major.  Few rows are cut finer (cut_rows).  With an LPT plan (from_idx / from_pos) n_wg
+// workgroups walk their unit lists instead.
+//
+// Bound by the tile loop, where a wave alone on its SIMD takes 0.97 us a tile and two together 0.77 (matrix and vector
+// pipe at the clock they leave each other, K / V^T requests on the CU's path from the L2), and by 4 us ahead of a row's first tile
+// (geometry, block list, queries, tile: four dependent round trips), in which the SIMD's other wave runs alone.
+// 8 x 4096 tokens, 12 heads, fp16, 62.6 GFLOP: 74 us.
 //
 // Replaces, from the reference: layers/kernels/sparse_attention.cu:2953-3190 (balanced,
 // persistent workgroups over the LPT plan), :2111-2403 (one workgroup per unit) and the
 // dispatcher :3192-3228.
 #include <hip/hip_runtime.h>
 
-#include <mutex>
 #include <type_traits>
 
 #include "rt_launch.h"
@@ -155,16 +149,12 @@ __device__ inline void state_init(State& st) {
 // Scores of padded keys become minus infinity: no weight.  The others gain log2(times), as if the tile were listed that
 // often.  s = 32 x 32 accumulator tile of key half kt; the key of element e in this lane is
 // 32 kt + 8 (e >> 2) + (e & 3) + 4 (lane >> 5), padding from `tail` on.
-// BRANCH: the gain is passed by where there is none.  With few units that saves 0.15 us; in the persistent fp16 kernel the
-// branch costs registers (124 spilled instead of 116; 20 x 883 tokens 68.9 us instead of 67.3), so a gain of zero is added.
-template <bool BRANCH = true>
 __device__ inline void mask_padded(f32x16& s, int kt, int tail, int lane, int times = 1) {
   int lim = tail - 4 * (lane >> 5);
   asm volatile("" : "+v"(lim));       // the 16 comparisons are made here, not once per kernel and kept in 32 scalar pairs
 #pragma unroll
   for (int e = 0; e < 16; ++e) s[e] = (32 * kt + 8 * (e >> 2) + (e & 3) >= lim) ? -INFINITY : s[e];
-  if (!BRANCH) asm volatile("" : "+s"(times));
-  if (!BRANCH || times > 1) {
+  if (times > 1) {
     const float gain = __builtin_amdgcn_logf(float(times));
 #pragma unroll
     for (int e = 0; e < 16; ++e) s[e] += gain;
@@ -363,7 +353,6 @@ struct Row {
   Unit u;
   int p0, cnt;            // the row is to_idx[p0 .. p0 + cnt)
   int goff;               // byte offset of the unit's (sequence, head) group inside K and V^T
-  int first_off;          // byte offset of the row's first tile inside K and V^T
 };
 
 template <typename T> struct Args {
@@ -375,41 +364,11 @@ template <typename T> struct Args {
   // optional: Q taken from the QKV projection's own output rows [tokens, 3 * heads * 64] (columns
   // 0 .. heads*64-1), bias added and scale applied while loading; q is then unused
   const T* q_rows; const T* q_bias; float q_scale;
-  int* queues;                           // QUEUE_INTS ints of device memory, all zero when the kernel starts and when it ends
 };
 
-constexpr int MAX_BATCH = 1024;         // sequences per launch (geometry is kept in LDS)
-constexpr int MAX_BLOCKS = 4096;        // 64-token blocks per launch (the row table is kept in LDS)
+constexpr int MAX_BATCH = 1024;         // sequences per launch (16 to a lane)
+constexpr int MAX_BLOCKS = 4096;        // 64-token blocks per launch
 constexpr int MAX_HEADS_QROWS = 64;     // heads whose query bias fits the LDS copy
-// Queue counters of one launch: 24 of them (tickets of the 8 global-row queues, tickets of the 8 unit
-// queues, then per XCD the number of its workgroups that have finished), each alone in a 256-byte line:
-// tickets of one line are served one after the other.  Every counter is only ever touched by the
-// workgroups of one XCD, through atomics that its L2 executes; the last workgroup of an XCD to finish
-// puts that XCD's three counters back to zero, so a launch leaves its counters as it found them.
-constexpr int QUEUE_STRIDE = 64;                    // ints between two counters
-constexpr int QUEUE_COUNTERS = 24;
-constexpr int QUEUE_INTS = QUEUE_COUNTERS * QUEUE_STRIDE;
-constexpr int REDO_SLOTS = 32;          // units a wave may put aside for the moving-maximum loop before it runs them
-constexpr int REDO_ENTRIES = 2048;      // LPT plan: entries per workgroup whose pipelined attempt is tracked
-
-// Geometry of the batch in LDS.
-struct Geometry {
-  int sb[MAX_BATCH + 1];                // prefix blocks
-  uint32_t rows[MAX_BLOCKS];            // j-th row that is not a global row: sequence << 16 | block inside the sequence
-  uint16_t sparse_seq[MAX_BATCH];       // k-th sequence that has global rows
-  uint8_t tail[MAX_BATCH];              // real tokens in each sequence's last block that holds any (64 without padding)
-  uint16_t nbv[MAX_BATCH];              // blocks of each sequence that hold real tokens
-  int n_rows, n_sparse;
-};
-
-__device__ inline int upper_seq(const int* __restrict__ prefix, int batch, int x) {
-  int lo = 0, hi = batch;               // prefix[lo] <= x < prefix[hi]
-  while (hi - lo > 1) {
-    const int mid = (lo + hi) >> 1;
-    if (prefix[mid] <= x) lo = mid; else hi = mid;
-  }
-  return lo;
-}
 
 __device__ inline bool is_global_row(const Unit& u) { return u.n >= RT_MIN_SPARSE_BLOCKS && (u.i == 0 || u.i == u.n - 1); }
 
@@ -515,46 +474,13 @@ __device__ inline int row_offsets(const Args<T>& a, const Row& r, int first, int
 
 // CSR row bounds through scalar loads
 template <typename T>
-__device__ inline void describe_bounds(const Args<T>& a, const Unit& u, Row& r) {
+__device__ inline void describe(const Args<T>& a, const Unit& u, Row& r) {
   r.u = u;
   const int row = __builtin_amdgcn_readfirstlane((a.plan_heads > 1 ? u.h : 0) * a.nb_total + u.g0 + u.i);
   const_int* pos = (const_int*)(uintptr_t)(a.to_pos);
   r.p0 = pos[row];
   r.cnt = pos[row + 1] - r.p0;
   r.goff = (u.g0 * a.heads + u.h * u.n) * 8192;
-}
-// the row's first block, through a scalar load
-template <typename T>
-__device__ inline void describe_first(const Args<T>& a, Row& r) {
-  const_int* idx = (const_int*)(uintptr_t)(a.to_idx);
-  int blk = r.cnt > 0 ? idx[r.p0] : 0;
-  blk = blk < 0 ? 0 : (blk >= r.u.n ? r.u.n - 1 : blk);
-  r.first_off = r.goff + blk * 8192;
-}
-
-// A short row's block ids through scalar loads (they do not queue behind the tile requests, and
-// what they return is not a pending vector load inside the tile loop): 16 entries starting at the
-// row's first.  The caller has checked that p0 + 16 does not pass the end of to_idx.
-constexpr int SHORT_ROW = 16;
-typedef int i32x8 __attribute__((ext_vector_type(8), aligned(4)));
-typedef const i32x8 __attribute__((address_space(4))) const_ids8;
-template <typename T>
-__device__ inline void request_short_row(const Args<T>& a, const Row& r, int (&blk)[SHORT_ROW]) {
-  const_ids8* p = (const_ids8*)(uintptr_t)(a.to_idx + r.p0);
-  const i32x8 lo = p[0], hi = p[1];
-#pragma unroll
-  for (int j = 0; j < 8; ++j) { blk[j] = lo[j]; blk[8 + j] = hi[j]; }
-}
-// lane j (< 16): byte offset inside K / V^T of the tile of the row's entry j
-__device__ inline int short_row_offsets(const Row& r, const int (&blk)[SHORT_ROW], int lane) {
-  int ids = 0;
-#pragma unroll
-  for (int j = 0; j < SHORT_ROW; ++j) {
-    int bj = blk[j];
-    bj = bj < 0 ? 0 : (bj >= r.u.n ? r.u.n - 1 : bj);
-    ids = lane == j ? r.goff + bj * 8192 : ids;
-  }
-  return ids;
 }
 
 #define SB() __builtin_amdgcn_sched_barrier(0)
@@ -606,15 +532,13 @@ __device__ inline Padding padding_of(const Unit& u, int goff) {
 }
 // Lanes 0 .. my-1 of ids hold the tile offsets of the wave's entries.  Takes the tiles that are padding as a whole
 // off the list (my shrinks), moves the padded tile to the last lane in use, further entries of it behind that, and sets
-// pd.last to their number.  False: the pipelined loop cannot run this list (its first tile does not stay
-// first, which a hand-over from the previous row may already have requested).
-__device__ inline bool pad_to_end(int& ids, int& my, int lane, Padding& pd) {
+// pd.last to their number.
+__device__ inline void pad_to_end(int& ids, int& my, int lane, Padding& pd) {
   pd.last = 0;
   const unsigned long long listed = __ballot(lane < my), dropped = __ballot(lane < my && ids >= pd.drop_off);
   const unsigned long long pads = pd.pad_off < 0 ? 0 : __ballot(lane < my && ids == pd.pad_off) & ~dropped;
   const unsigned long long front = listed & ~dropped & ~pads;
-  if ((dropped | pads) == 0) return true;
-  if ((dropped & 1ull) || ((pads & 1ull) && front)) return false;
+  if ((dropped | pads) == 0) return;
   if (dropped == 0 && (pads & (pads - 1)) == 0) {            // one: it and the last entry change places
     const int jp = __builtin_ctzll(pads);
     if (jp != my - 1) {
@@ -622,7 +546,7 @@ __device__ inline bool pad_to_end(int& ids, int& my, int lane, Padding& pd) {
       ids = lane == jp ? moved : (lane == my - 1 ? pd.pad_off : ids);
     }
     pd.last = 1;
-    return true;
+    return;
   }
   // a permutation: the others in order, the padded tiles, the dropped ones; lanes beyond the list stay
   auto below = [](unsigned long long m) { return int(__builtin_amdgcn_mbcnt_hi(unsigned(m >> 32), __builtin_amdgcn_mbcnt_lo(unsigned(m), 0))); };
@@ -633,7 +557,6 @@ __device__ inline bool pad_to_end(int& ids, int& my, int lane, Padding& pd) {
   ids = __builtin_amdgcn_ds_permute(dest * 4, ids);
   my = n_front + (n_pads > 0);
   pd.last = n_pads;
-  return true;
 }
 
 // reference of the pipelined loop: maximum over the row's first 32 keys, shared by the lane's two
@@ -661,15 +584,10 @@ __device__ inline bool fast_reference(const Tiles<T>& t, float& mref, bool pad_f
   return !__any(!(fabsf(m0 - m1) <= MAX_REFERENCE_GAP));           // false also for NaN / infinite scores
 }
 
-// The pipelined tile loop over `my` (1..64) tiles whose byte offsets sit in the lanes of `ids`; the
-// first tile is in flight or there (request_first).  so_after >= 0: the last tile's steps request that
-// tile (the first one of the wave's next row) instead of a dummy.  next_q(k), k = 0..7: requests
-// fragment k of the next row's queries into t.qf; called in the last tile's last two steps, once
-// the score products have read the fragment it replaces.
-struct NoNextQ { __device__ void operator()(int) const {} };
-template <typename T, bool MASKED, bool FEW, typename NextQ>
-__device__ inline void fast_loop(const Buffers<T>& b, int ids, int my, const int& so_after, int lane, float mref,
-                                 Tiles<T>& t, State& st, NextQ next_q, const Padding& pd) {
+// The pipelined tile loop over `my` (1..64) tiles whose byte offsets sit in the lanes of `ids`; the first tile is in flight
+// or there (request_first).
+template <typename T, bool MASKED>
+__device__ inline void fast_loop(const Buffers<T>& b, int ids, int my, int lane, float mref, Tiles<T>& t, State& st, const Padding& pd) {
   typedef typename Mma<T>::v8 v8;
   typedef Mma<T> P;
   state_init(st);
@@ -690,8 +608,7 @@ __device__ inline void fast_loop(const Buffers<T>& b, int ids, int my, const int
   // anything still pending there turns them into waits for all requests.
   __builtin_amdgcn_s_waitcnt(0x0F70);                 // vmcnt(0)
   // Inside the loop a wave yields to the other wave of its SIMD whenever that one is between two loops (queries,
-  // reference, output, the next row's description): that code is a chain of short latencies, the loop always has
-  // matrix work in flight.  Worth 2 % where rows are long (8 x 4096 tokens), nothing elsewhere.
+  // reference, output): that code is a chain of short latencies, the loop always has matrix work in flight.
   __builtin_amdgcn_s_setprio(0);
   SB();
   // pipeline prologue: scores of the first accumulator tile; an all-zero P for the first step's PV slot
@@ -722,25 +639,23 @@ __device__ inline void fast_loop(const Buffers<T>& b, int ids, int my, const int
       uint32_t t01 = 0, t23 = 0, t45 = 0, t67 = 0;
       float lacc = 0.f;
       // a row's padded tile is its last one (pad_to_end): its scores lose the padded keys before they are exponentiated
-      if (MASKED && LAST && pd.last) mask_padded<FEW>(cur, S >> 1, pd.tail, lane, pd.last);
+      if (MASKED && LAST && pd.last) mask_padded(cur, S >> 1, pd.tail, lane, pd.last);
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
         SB();
         // matrix slot
         if ((i & 1) == 0) {
           const int c = i >> 1;
-          // the last tile's last step has no following scores to start: its slots request the next row's queries
+          // the last tile's last step has no following scores to start
           if (!(LAST && S == 3)) nxt = P::run(t.kf[ktn * 4 + c], t.qf[ntn][c], c == 0 ? negm : nxt);
         } else {
           const int tt = (i >> 1) & 1, s = i >> 2;
           st.o[tt][ntp] = P::run(t.vf[tt * 4 + 2 * ktp + s], pprev[s], st.o[tt][ntp]);
         }
         // tile requests: one per slot in the steps whose registers are free
-        if (S == 1) { if (i < 4) ldk(i, so_next); else { const int f = (i & 1) + 2 + 4 * ((i >> 1) & 1); ldv(f, so_cur); } }
-        if (S == 3) { if (i < 4) ldk(4 + i, so_next); else { const int f = (i & 1) + 4 * ((i >> 1) & 1); ldv(f, so_next); } }
-        // the next row's queries: first query half after this row's last use of it (step 1), second after step 2's
-        if (LAST && S == 2 && (i & 1) == 1) next_q(i >> 1);
-        if (LAST && S == 3 && (i & 1) == 0) next_q(4 + (i >> 1));
+        if (S == 1 && i >= 4) { const int f = (i & 1) + 2 + 4 * ((i >> 1) & 1); ldv(f, so_cur); }
+        if (S == 1 && i < 4 && !LAST) ldk(i, so_next);
+        if (S == 3 && !LAST) { if (i < 4) ldk(4 + i, so_next); else { const int f = (i & 1) + 4 * ((i >> 1) & 1); ldv(f, so_next); } }
         SB();
         // vector slot: two exponentials, rounding and sums of the previous slot's pair
         p[2 * i] = __builtin_amdgcn_exp2f(cur[2 * i]);
@@ -779,7 +694,7 @@ __device__ inline void fast_loop(const Buffers<T>& b, int ids, int my, const int
     tile(so_next, std::false_type{});
     so_cur = so_next;
   }
-  tile(so_after >= 0 ? so_after : so_cur, std::true_type{});
+  tile(so_cur, std::true_type{});
   // pipeline epilogue: the last tile's a[3] (second key half, second query half)
 #pragma unroll
   for (int tt = 0; tt < 2; ++tt)
@@ -805,10 +720,10 @@ __device__ inline void slow_row(const Args<T>& a, const Buffers<T>& b, const QSi
   stream_tiles<T, MASKED>(a.k + gbase, a.vt + gbase, a.to_idx + r.p0, first, step, r.cnt, r.u.n, r.u.tail, r.u.nbv, lane, qf, st);
 }
 
-// Entries first, first + step, ... of row r for the pipelined loop, no hand-over from or to another row: the tiles the wave
-// has (ids, my, pd), the first of them requested, behind the queries if WITH_Q.
+// Entries first, first + step, ... of row r for the pipelined loop: the tiles the wave has (ids, my, pd), the first of them
+// requested.
 enum { SHARE_SLOW, SHARE_EMPTY, SHARE_RUNS };      // for the moving-maximum loop (more than 64 entries); no tile that counts
-template <typename T, bool MASKED, bool WITH_Q>
+template <typename T, bool MASKED>
 __device__ inline int begin_share(const Args<T>& a, const Buffers<T>& b, const Row& r, int first, int step, int lane, Tiles<T>& t,
                                   int& ids, int& my, Padding& pd) {
   first = __builtin_amdgcn_readfirstlane(first);
@@ -818,50 +733,20 @@ __device__ inline int begin_share(const Args<T>& a, const Buffers<T>& b, const R
   ids = row_offsets<T>(a, r, first, step, lane);
   pd = padding_of(r.u, r.goff);
   if (MASKED) {
-    if (!pad_to_end(ids, my, lane, pd)) return SHARE_SLOW;
+    pad_to_end(ids, my, lane, pd);
     if (my == 0) return SHARE_EMPTY;                   // every tile of this wave's share is padding
   }
-  if (WITH_Q) request_q<T>(a, b, r.u, lane, t.qf);
   request_first<T>(b, __builtin_amdgcn_readlane(ids, 0), lane, t);
   return SHARE_RUNS;
 }
 // The share through the state, its queries in t.qf (they are there afterwards too).  False: the row has to be run with the
 // moving-maximum loop instead (scores that outgrew the reference); the state is then undefined.
-template <typename T, bool MASKED, bool FEW>
+template <typename T, bool MASKED>
 __device__ inline bool end_share(const Buffers<T>& b, int ids, int my, const Padding& pd, int lane, Tiles<T>& t, State& st) {
   float mref;
   if (!fast_reference<T, MASKED>(t, mref, pd.last > 0 && my == 1, pd.tail, lane)) return false;
-  fast_loop<T, MASKED, FEW>(b, ids, my, -1, lane, mref, t, st, NoNextQ{}, pd);
+  fast_loop<T, MASKED>(b, ids, my, lane, mref, t, st, pd);
   return sums_finite(st);
-}
-// Both, by one wave for itself.  HAVE_Q: the queries are in t.qf already.
-template <typename T, bool MASKED, bool HAVE_Q, bool FEW>
-__device__ inline bool fast_share(const Args<T>& a, const Buffers<T>& b, const QSide<T>& qbias, const Row& r, int first, int step,
-                                  int lane, Tiles<T>& t, State& st) {
-  state_init(st);
-  first = __builtin_amdgcn_readfirstlane(first);
-  int my = __builtin_amdgcn_readfirstlane((r.cnt - first + step - 1) / step);           // this wave's entries
-  if (my <= 0) return true;
-  if (my > 64) return false;
-  int ids = row_offsets<T>(a, r, first, step, lane);
-  Padding pd = padding_of(r.u, r.goff);
-  if (MASKED) {
-    if (!pad_to_end(ids, my, lane, pd)) return false;
-    if (my == 0) return true;                          // every tile of this wave's share is padding
-  }
-  if (!HAVE_Q) request_q<T>(a, b, r.u, lane, t.qf);
-  request_first<T>(b, __builtin_amdgcn_readlane(ids, 0), lane, t);
-  if (!HAVE_Q) finish_q<T>(a, qbias, r.u, lane, t.qf);
-  float mref;
-  if (!fast_reference<T, MASKED>(t, mref, pd.last > 0 && my == 1, pd.tail, lane)) return false;
-  fast_loop<T, MASKED, FEW>(b, ids, my, -1, lane, mref, t, st, NoNextQ{}, pd);
-  return sums_finite(st);
-}
-template <typename T, bool MASKED, bool FEW = false>
-__device__ inline bool fast_row(const Args<T>& a, const Buffers<T>& b, const QSide<T>& qbias, const Row& r, int first, int step,
-                                int lane, State& st) {
-  Tiles<T> t;
-  return fast_share<T, MASKED, false, FEW>(a, b, qbias, r, first, step, lane, t, st);
 }
 
 // One over a row's whole sum.  A row that has met nothing but padding writes zeros; one whose keys all have a score
@@ -870,500 +755,11 @@ __device__ inline float row_weight(float l, float m) {
   return l == 0.f && m == LOWEST ? __builtin_nanf("") : __builtin_amdgcn_rcpf(fmaxf(l, 1e-30f));
 }
 
-// normalises the state and writes the unit's output tile; FAST: the state comes from the pipelined loop
-template <typename T, bool FAST>
-__device__ inline void finish_unit(const Args<T>& a, const QSide<T>& qs, const Unit& u, int lane, State& st) {
-  float w[2];
-#pragma unroll
-  for (int nt = 0; nt < 2; ++nt) {
-    const float l = pair_sum(st.l[nt]);
-    w[nt] = FAST ? __builtin_amdgcn_rcpf(fmaxf(l, 1e-30f)) : row_weight(l, st.m[nt]);
-  }
-  const int64_t stride = int64_t(a.heads) * 64;
-  store_output<T>(a.out + int64_t(u.g0 + u.i) * 64 * stride + u.h * 64, stride, lane, st, w, qs.stage);
-}
-
-template <typename T>
-__device__ inline Row describe(const Args<T>& a, const Unit& u) {
-  Row r;
-  describe_bounds<T>(a, u, r);
-  describe_first<T>(a, r);
-  return r;
-}
-
-// One wave, one unit, all of its key blocks.  FAST: pipelined loop; false = the unit has to be run
-// again with FAST = false (nothing was written).
-template <typename T, bool MASKED, bool FAST>
-__device__ inline bool run_solo(const Args<T>& a, const Buffers<T>& b, const QSide<T>& qbias, const Unit& u, int lane) {
-  const Row r = describe<T>(a, u);
-  State st;
-  if (FAST) {
-    if (!fast_row<T, MASKED>(a, b, qbias, r, 0, 1, lane, st)) return false;
-  } else {
-    typename Mma<T>::v8 qf[2][4];
-    slow_row<T, MASKED>(a, b, qbias, r, 0, 1, lane, false, qf, st);
-  }
-  finish_unit<T, FAST>(a, qbias, u, lane, st);
-  return true;
-}
-
-// A wave's softmax state in LDS, and the merge of a parked state into the wave's own.
-constexpr int PARK_FLOATS = 68 * 64;
-__device__ inline void park_state(const State& st, float* slot, int lane) {
-#pragma unroll
-  for (int t = 0; t < 2; ++t)
-#pragma unroll
-    for (int nt = 0; nt < 2; ++nt)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) slot[((t * 2 + nt) * 16 + e) * 64 + lane] = st.o[t][nt][e];
-#pragma unroll
-  for (int nt = 0; nt < 2; ++nt) {
-    slot[(64 + nt) * 64 + lane] = st.m[nt];
-    slot[(66 + nt) * 64 + lane] = st.l[nt];
-  }
-}
-__device__ inline void absorb_state(State& st, const float* slot, int lane) {
-#pragma unroll
-  for (int nt = 0; nt < 2; ++nt) {
-    const float m1 = slot[(64 + nt) * 64 + lane], l1 = slot[(66 + nt) * 64 + lane];
-    const float m = fmaxf(st.m[nt], m1), mt = fmaxf(m, LOWEST);        // mt: finite even if both are empty
-    const float a0 = __builtin_amdgcn_exp2f(st.m[nt] - mt), a1 = __builtin_amdgcn_exp2f(m1 - mt);
-    st.m[nt] = m;
-    st.l[nt] = st.l[nt] * a0 + l1 * a1;
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-      for (int e = 0; e < 16; ++e)
-        st.o[t][nt][e] = st.o[t][nt][e] * a0 + slot[((t * 2 + nt) * 16 + e) * 64 + lane] * a1;
-  }
-}
-
-// Four waves, one unit: wave w streams key blocks w, w+4, ...; tree merge through LDS.  FAST:
-// pipelined loop; false (the same in all four waves) = the unit has to be run again with FAST = false.
-template <typename T, bool MASKED, bool FAST>
-__device__ inline bool run_split4(const Args<T>& a, const Buffers<T>& b, const QSide<T>& qbias, const Unit& u, int lane,
-                                  int wave, float* park) {
-  const Row r = describe<T>(a, u);
-  State st;
-  if (FAST) {
-    const bool ok = fast_row<T, MASKED>(a, b, qbias, r, wave, 4, lane, st);
-    if (__syncthreads_or(!ok)) return false;          // also: the park is free (previous item is over)
-  } else {
-    typename Mma<T>::v8 qf[2][4];
-    slow_row<T, MASKED>(a, b, qbias, r, wave, 4, lane, false, qf, st);
-    __syncthreads();                                  // the park is free (previous item is over)
-  }
-#pragma unroll
-  for (int nt = 0; nt < 2; ++nt) st.l[nt] = pair_sum(st.l[nt]);
-
-  if (wave >= 2) park_state(st, park + (wave - 2) * PARK_FLOATS, lane);
-  __syncthreads();
-  if (wave < 2) absorb_state(st, park + wave * PARK_FLOATS, lane);
-  __syncthreads();
-  if (wave == 1) park_state(st, park, lane);
-  __syncthreads();
-  if (wave == 0) {
-    absorb_state(st, park, lane);
-    float w[2];
-#pragma unroll
-    for (int nt = 0; nt < 2; ++nt) w[nt] = row_weight(st.l[nt], st.m[nt]);
-    const int64_t stride = int64_t(a.heads) * 64;
-    // wave 0's room is the start of the park, which it has just finished reading
-    store_output<T>(a.out + int64_t(u.g0 + u.i) * 64 * stride + u.h * 64, stride, lane, st, w, qbias.stage);
-  }
-  __syncthreads();                                    // the park is read: the next item may stage its queries there
-  return true;
-}
-
-// One ticket of a queue counter, in lane 0: a request, not yet waited for.  A buffer atomic whose
-// resource covers just the counter: every lane executes it, lanes 1..63 address past the end and
-// are dropped by the hardware, so no branch (and no wait at the end of one) surrounds the request.
-__device__ inline __amdgpu_buffer_rsrc_t ticket_counter(int* p) { return __builtin_amdgcn_make_buffer_rsrc(p, 0, 4, 0x00020000); }
-__device__ inline int request_ticket(__amdgpu_buffer_rsrc_t counter, int lane) {
-  return __builtin_amdgcn_raw_ptr_buffer_atomic_add_i32(1, counter, lane * 4, 0, 1);
-}
-// the same instruction; if `really` (wave-uniform) is false all lanes address past the end: nothing is drawn
-__device__ inline int request_ticket_if(__amdgpu_buffer_rsrc_t counter, int lane, bool really) {
-  return __builtin_amdgcn_raw_ptr_buffer_atomic_add_i32(1, counter, lane * 4 + (really ? 0 : 4), 0, 1);
-}
-
-// Persistent workgroups (two per CU).
-template <typename T, bool MASKED>
-__global__ __launch_bounds__(256, 2) void bs_attention_kernel(Args<T> a) {
-  // 36864 bytes with two uses that never overlap in time: two parked wave states (2 x 17408 bytes) of the merge
-  // that ends a row shared by the four waves, and each wave's room for a query tile in row order (finish_q)
-  static_assert(4 * Q_STAGE_BYTES >= 2 * PARK_FLOATS * int(sizeof(float)), "the park must hold two wave states");
-  __shared__ __attribute__((aligned(16))) float park[4 * Q_STAGE_BYTES / 4];
-  __shared__ Geometry geo;
-  __shared__ __attribute__((aligned(16))) T qbias_lds[MAX_HEADS_QROWS * 64];
-  __shared__ int s_item;
-  __shared__ int redo[4][REDO_SLOTS];                 // per wave: units put aside for the moving-maximum loop
-  __shared__ int redo_rows[REDO_SLOTS];               // per workgroup: global rows put aside
-  __shared__ uint8_t s_redo[REDO_ENTRIES];            // LPT plan: entries of the workgroup's slice to run again
-  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const QSide<T> qbias{qbias_lds, reinterpret_cast<char*>(park) + wave * Q_STAGE_BYTES};
-
-  // Geometry: prefix blocks, the sequences that have global rows, the list of rows that are not global rows.  Every
-  // one of the 512 workgroups builds it for itself, so it is built by all 256 threads: sequence s's place in both
-  // lists follows from the number of sparse sequences before it (a ballot per wave, the waves' counts through LDS),
-  // since rows before s = blocks before s - 2 * (sparse sequences before s).
-  int* const row_base = reinterpret_cast<int*>(park);            // per sequence: rows listed before it (scratch use of the park)
-  int* const wave_sparse = row_base + MAX_BATCH;                 // [round][wave]: sparse sequences among the wave's 64
-  for (int i = threadIdx.x; i <= a.batch; i += 256) geo.sb[i] = a.seq_blocks[i];
-  if (a.q_rows)                                                  // without a bias (the rows carry it already): zeros
-    for (int i = threadIdx.x; i < a.heads * 64; i += 256) qbias_lds[i] = a.q_bias ? a.q_bias[i] : static_cast<T>(0.f);
-  __syncthreads();
-  const int rounds = (a.batch + 255) >> 8;                       // at most MAX_BATCH / 256 = 4
-  int before_in_wave[MAX_BATCH / 256];
-  bool is_sparse[MAX_BATCH / 256];
-#pragma unroll
-  for (int r = 0; r < MAX_BATCH / 256; ++r) {
-    before_in_wave[r] = 0;
-    is_sparse[r] = false;
-    if (r < rounds) {
-      const int sq = r * 256 + int(threadIdx.x);
-      is_sparse[r] = sq < a.batch && geo.sb[sq + 1] - geo.sb[sq] >= RT_MIN_SPARSE_BLOCKS;
-      const unsigned long long votes = __ballot(is_sparse[r]);
-      before_in_wave[r] = __popcll(votes & ((1ull << lane) - 1ull));
-      if (lane == 0) wave_sparse[r * 4 + wave] = __popcll(votes);
-      if (sq < a.batch) {
-        const int nblk = geo.sb[sq + 1] - geo.sb[sq];
-        int t = 64, nv = nblk;
-        if (MASKED) {                                                // at least one real token, at most the sequence
-          const int tokens = min(max(a.seq_tokens[sq], 1), 64 * nblk);
-          nv = (tokens + 63) >> 6;
-          t = tokens - 64 * (nv - 1);
-        }
-        geo.nbv[sq] = uint16_t(nv);
-        geo.tail[sq] = uint8_t(t);
-      }
-    }
-  }
-  __syncthreads();
-  {
-    int running = 0;                                             // sparse sequences before this wave's 64 of round r
-#pragma unroll
-    for (int r = 0; r < MAX_BATCH / 256; ++r)
-      if (r < rounds) {
-        int before = running;
-        for (int w = 0; w < 4; ++w) {
-          const int c = wave_sparse[r * 4 + w];
-          if (w < wave) before += c;
-          running += c;
-        }
-        const int sq = r * 256 + int(threadIdx.x);
-        if (sq < a.batch) {
-          const int k = before + before_in_wave[r];
-          row_base[sq] = geo.sb[sq] - 2 * k;
-          if (is_sparse[r]) geo.sparse_seq[k] = uint16_t(sq);
-        }
-      }
-    if (threadIdx.x == 0) {
-      geo.n_sparse = running;
-      geo.n_rows = geo.sb[a.batch] - 2 * running;
-    }
-  }
-  __syncthreads();
-  for (int sq = wave; sq < a.batch; sq += 4) {                   // a wave per sequence, a lane per row
-    const int n = geo.sb[sq + 1] - geo.sb[sq];
-    const int skip = n >= RT_MIN_SPARSE_BLOCKS ? 1 : 0;          // a sparse sequence's rows 0 and n - 1 are global rows
-    for (int i = skip + lane; i < n - skip; i += 64) geo.rows[row_base[sq] + i - skip] = uint32_t(sq) << 16 | uint32_t(i);
-  }
-  __syncthreads();
-
-  Buffers<T> b;
-  {
-    const uint32_t kv_bytes = uint32_t(a.nb_total) * uint32_t(a.heads) * 8192u;
-    b.k = __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(a.k), 0, kv_bytes, 0x00020000);
-    b.v = __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(a.vt), 0, kv_bytes, 0x00020000);
-    b.q = a.q_rows ? __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(a.q_rows), 0, kv_bytes * 3u, 0x00020000)
-                   : __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(a.q), 0, kv_bytes, 0x00020000);
-  }
-
-  auto unit_of_flat = [&](int unit) {               // flat id = blk + head * n_s + seq_start * heads
-    int lo = 0, hi = a.batch;
-    while (hi - lo > 1) {
-      const int mid = (lo + hi) >> 1;
-      if (geo.sb[mid] * a.heads <= unit) lo = mid; else hi = mid;
-    }
-    Unit u;
-    u.g0 = geo.sb[lo];
-    u.n = geo.sb[lo + 1] - u.g0;
-    u.tail = geo.tail[lo];
-    u.nbv = MASKED ? int(geo.nbv[lo]) : u.n;
-    const int rem = unit - u.g0 * a.heads;
-    u.h = rem / u.n;
-    u.i = rem - u.h * u.n;
-    return u;
-  };
-
-  if (a.from_pos) {
-    // LPT plan: global rows are shared by the workgroup's four waves, runs of up to four other units go
-    // one per wave.  Two passes over the workgroup's slice: the pipelined loop first, then, for what
-    // it handed back (s_redo: one flag per plan entry of the slice, at most REDO_ENTRIES), the
-    // moving-maximum loop.
-    // A plan the host has not checked (rt_meta_check_partition) must not make this kernel read outside
-    // from_idx: the slice is clamped to its n_units entries, ids outside [0, n_units) are skipped.
-    const int n_units = a.nb_total * a.heads;
-    const int begin = min(max(a.from_pos[blockIdx.x], 0), n_units);
-    const int end = min(max(a.from_pos[blockIdx.x + 1], begin), n_units);
-    auto walk = [&](auto fast) {
-      constexpr bool FAST = decltype(fast)::value;
-      int p = begin;
-      while (p < end) {
-        // the next four plan entries in one round trip
-        const int mine_id = (p + wave < end) ? a.from_idx[p + wave] : -1;
-        int ids4[4];
-#pragma unroll
-        for (int w = 0; w < 4; ++w) ids4[w] = (p + w < end) ? a.from_idx[p + w] : -1;
-        if (ids4[0] < 0 || ids4[0] >= n_units) { ++p; continue; }
-        const Unit first = unit_of_flat(ids4[0]);
-        const bool tracked = p - begin < REDO_ENTRIES;         // entries past the flags take the moving-maximum loop
-        if (is_global_row(first)) {
-          const bool todo = FAST ? tracked : (!tracked || s_redo[p - begin] != 0);
-          if (todo) {
-            const bool ok = run_split4<T, MASKED, FAST>(a, b, qbias, first, lane, wave, park);
-            if (FAST && threadIdx.x == 0) s_redo[p - begin] = ok ? 0 : 1;
-          }
-          ++p;
-          continue;
-        }
-        int run = 1;
-        while (run < 4 && ids4[run] >= 0 && ids4[run] < n_units && !is_global_row(unit_of_flat(ids4[run]))) ++run;
-        if (wave < run) {
-          const int e = p + wave - begin;
-          const bool trk = e < REDO_ENTRIES;
-          const bool todo = FAST ? trk : (!trk || s_redo[e] != 0);
-          if (todo) {
-            const bool ok = run_solo<T, MASKED, FAST>(a, b, qbias, unit_of_flat(mine_id), lane);
-            if (FAST && lane == 0) s_redo[e] = ok ? 0 : 1;
-          }
-        }
-        p += run;
-      }
-    };
-    walk(std::true_type{});
-    __syncthreads();
-    walk(std::false_type{});
-    return;
-  }
-
-  const int xcd = blockIdx.x & 7;
-  const __amdgpu_buffer_rsrc_t gq = ticket_counter(a.queues + xcd * QUEUE_STRIDE);          // this XCD's global-row queue
-  const __amdgpu_buffer_rsrc_t uq = ticket_counter(a.queues + (8 + xcd) * QUEUE_STRIDE);    // this XCD's unit queue
-
-  // phase 1: global rows, one per workgroup.  A pair = the first and the last row of one (sequence,
-  // head): both stream the same K / V^T tiles, so they are consecutive tickets of the same XCD.
-  // Pairs are numbered head-major and XCD x owns the x-th eighth of them: the same heads whose
-  // other rows it runs in phase 2.
-  {
-    const int n_pairs = geo.n_sparse * a.heads;
-    const int p_lo = int(int64_t(n_pairs) * xcd / 8), p_hi = int(int64_t(n_pairs) * (xcd + 1) / 8);
-    const int n_glob = 2 * (p_hi - p_lo);             // tickets of this XCD that are rows
-    auto unit_of_row = [&](int ticket) {
-      const int pair = p_lo + (ticket >> 1);
-      const int h = pair / geo.n_sparse;
-      const int s = geo.sparse_seq[pair - h * geo.n_sparse];
-      Unit u;
-      u.g0 = geo.sb[s];
-      u.n = geo.sb[s + 1] - u.g0;
-      u.tail = geo.tail[s];
-      u.nbv = MASKED ? int(geo.nbv[s]) : u.n;
-      u.h = h;
-      u.i = (ticket & 1) ? u.n - 1 : 0;
-      return u;
-    };
-    // The XCD's workgroup number w takes row w without asking; rows beyond the XCD's workgroups are drawn from the
-    // counter (ticket k = row wgs + k).  A batch with no more rows than workgroups touches no counter in this phase.
-    const int wgs = int(gridDim.x >> 3), wg_local = int(blockIdx.x >> 3);
-    const bool drawn_rows = n_glob > wgs;
-    int item = wg_local < n_glob ? wg_local : -1;
-    bool drained = item < 0 && !drawn_rows;
-    while (!drained) {
-      int n_rows_redo = 0;
-      while (n_rows_redo < REDO_SLOTS) {
-        if (item < 0) {
-          if (!drawn_rows) { drained = true; break; }
-          if (wave == 0) {
-            const int k = __builtin_amdgcn_readfirstlane(request_ticket(gq, lane));
-            if (lane == 0) s_item = k;
-          }
-          __syncthreads();
-          item = wgs + s_item;
-          __syncthreads();
-          if (item >= n_glob) { drained = true; break; }
-        }
-        const bool ok = run_split4<T, MASKED, true>(a, b, qbias, unit_of_row(item), lane, wave, park);
-        if (!ok) {
-          if (threadIdx.x == 0) redo_rows[n_rows_redo] = item;
-          ++n_rows_redo;
-        }
-        item = -1;
-      }
-      __syncthreads();
-      for (int r = 0; r < n_rows_redo; ++r)
-        run_split4<T, MASKED, false>(a, b, qbias, unit_of_row(redo_rows[r]), lane, wave, park);
-      __syncthreads();
-    }
-  }
-
-  // phase 2: all other rows; every wave draws single units.  Item = head * n_rows + j (j-th listed
-  // row), XCD x owns the x-th eighth of the items.
-  {
-    const int lane_id = lane;
-    const int n_rows = geo.n_rows;
-    const int total = n_rows * a.heads;
-    const int lo = int(int64_t(total) * xcd / 8), hi = int(int64_t(total) * (xcd + 1) / 8);
-    const float inv_rows = 1.0f / float(n_rows > 0 ? n_rows : 1);
-    auto unit_of = [&](int item) {
-      int h = int((float(item) + 0.5f) * inv_rows);
-      int j = item - h * n_rows;
-      if (j < 0) { --h; j += n_rows; }
-      if (j >= n_rows) { ++h; j -= n_rows; }
-      const uint32_t e = geo.rows[j];
-      const int s = int(e >> 16);
-      Unit u;
-      u.g0 = geo.sb[s];
-      u.n = geo.sb[s + 1] - u.g0;
-      u.tail = geo.tail[s];
-      u.nbv = MASKED ? int(geo.nbv[s]) : u.n;
-      u.h = h;
-      u.i = int(e & 0xffffu);
-      return u;
-    };
-    auto item_of = [&](int ticket) {                  // -1: the queue is drained
-      const int k = __builtin_amdgcn_readfirstlane(ticket);
-      return lo + k < hi ? lo + k : -1;
-    };
-    const_int* pos_all = (const_int*)(uintptr_t)(a.to_pos);
-    const int idx_total = pos_all[a.plan_heads * a.nb_total];       // entries in to_idx
-    int n_redo = 0;
-    int item = item_of(request_ticket(uq, lane));
-    int item_nx = item >= 0 ? item_of(request_ticket(uq, lane)) : -1;
-    while (item >= 0 || n_redo > 0) {
-      // pipelined loop on one unit after the other, each handing the next one its first tile.  A wave
-      // holds the unit it runs and the next one; the one after that is drawn when the tile loop ends.
-      if (item >= 0) {
-        Tiles<T> t;
-        Row cur;
-        int blk[SHORT_ROW];
-        describe_bounds<T>(a, unit_of(item), cur);
-        bool cur_short = cur.cnt >= 1 && cur.cnt <= SHORT_ROW && cur.p0 + SHORT_ROW <= idx_total;
-        int ids = 0;
-        cur.first_off = 0;
-        if (cur_short) {
-          request_short_row<T>(a, cur, blk);
-          ids = short_row_offsets(cur, blk, lane_id);
-          cur.first_off = __builtin_amdgcn_readlane(ids, 0);
-        }
-        bool primed = false;
-        while (item >= 0 && n_redo < REDO_SLOTS) {
-          // what the code below derives from the lane number is derived again for every unit, not
-          // kept in registers across the tile loop
-          int lane = lane_id;
-          asm volatile("" : "+v"(lane));
-          const bool has_next = item_nx >= 0;
-          Row nx = cur;
-          if (has_next) describe_bounds<T>(a, unit_of(item_nx), nx);        // scalar loads, waited for below
-          State st;
-          bool ok = cur_short;
-          float mref = 0.f;
-          Padding pd = padding_of(cur.u, cur.goff);
-          int my = cur.cnt;                                 // tiles of the row that the loop runs
-          if (MASKED && ok) ok = pad_to_end(ids, my, lane, pd);
-          if (ok && !primed) {
-            request_q<T>(a, b, cur.u, lane, t.qf);
-            request_first<T>(b, cur.first_off, lane, t);
-          }
-          if (ok) {
-            finish_q<T>(a, qbias, cur.u, lane, t.qf);
-            ok = fast_reference<T, MASKED>(t, mref, pd.last > 0 && my == 1, pd.tail, lane);
-          }
-          // the next row's block ids: requested here, looked at in the loop's last tile
-          bool nx_short = false;
-          nx.first_off = -1;
-          if (has_next) {
-            nx_short = nx.cnt >= 1 && nx.cnt <= SHORT_ROW && nx.p0 + SHORT_ROW <= idx_total;
-            if (nx_short) {
-              request_short_row<T>(a, nx, blk);
-              int b0 = blk[0];
-              b0 = b0 < 0 ? 0 : (b0 >= nx.u.n ? nx.u.n - 1 : b0);
-              nx.first_off = nx.goff + b0 * 8192;
-            }
-          }
-          int item_after = -1;
-          primed = false;
-          if (ok) {
-            const QPlan qn = q_plan<T>(a, nx.u, lane);      // without a next unit: this unit's queries again
-            fast_loop<T, MASKED, false>(b, ids, my, nx.first_off, lane, mref, t, st,
-                                 [&](int k) { t.qf[k >> 2][k & 3] = fetch_q<T>(b, qn, k); }, pd);
-            lane = lane_id;
-            asm volatile("" : "+v"(lane));
-            // The unit after the next one: its ticket is drawn here, behind the tile loop, and looked at once this
-            // unit's output is on its way.  (Drawn ahead of the loop, the request was still in flight at the loop's
-            // entry, where everything requested must have arrived: a device round trip of waiting per unit.)  The
-            // request is always issued (without a next unit it addresses nothing): no branch around it.
-            const int t_next = request_ticket_if(uq, lane, has_next);
-            SB();
-            primed = nx_short;
-            if (sums_finite(st)) {
-              finish_unit<T, true>(a, qbias, cur.u, lane, st);
-              SB();
-            } else {
-              if (lane == 0) redo[wave][n_redo] = item;
-              ++n_redo;
-            }
-            item_after = has_next ? item_of(t_next) : -1;
-          } else {
-            if (lane == 0) redo[wave][n_redo] = item;
-            ++n_redo;
-            const int t_next = request_ticket_if(uq, lane, has_next);
-            item_after = has_next ? item_of(t_next) : -1;
-          }
-          item = item_nx;
-          item_nx = item_after;
-          cur = nx;
-          cur_short = nx_short;
-          if (nx_short) ids = short_row_offsets(nx, blk, lane);
-        }
-      }
-      // the units put aside: moving-maximum loop
-      for (int r = 0; r < n_redo; ++r) {
-        const int it = __builtin_amdgcn_readfirstlane(redo[wave][r]);
-        run_solo<T, MASKED, false>(a, b, qbias, unit_of(it), lane_id);
-      }
-      n_redo = 0;
-    }
-  }
-
-  // This workgroup draws no more tickets.  The last workgroup of the XCD to get here puts the XCD's counters
-  // back to zero for the next launch that is handed them (same L2, same kind of access as the tickets).
-  __syncthreads();
-  if (wave == 0) {
-    const __amdgpu_buffer_rsrc_t done = ticket_counter(a.queues + (16 + xcd) * QUEUE_STRIDE);
-    const int finished = __builtin_amdgcn_readfirstlane(request_ticket(done, lane));
-    if (finished == int(gridDim.x >> 3) - 1) {
-      // nobody else touches them any more: read each (an addition of nothing) and take that much away
-      const int g = __builtin_amdgcn_raw_ptr_buffer_atomic_add_i32(0, gq, lane * 4, 0, 1);
-      const int u = __builtin_amdgcn_raw_ptr_buffer_atomic_add_i32(0, uq, lane * 4, 0, 1);
-      (void)__builtin_amdgcn_raw_ptr_buffer_atomic_add_i32(-g, gq, lane * 4, 0, 0);
-      (void)__builtin_amdgcn_raw_ptr_buffer_atomic_add_i32(-u, uq, lane * 4, 0, 0);
-      (void)__builtin_amdgcn_raw_ptr_buffer_atomic_add_i32(-(finished + 1), done, lane * 4, 0, 0);
-    }
-  }
-}
-
-// ---- batches with few units --------------------------------------------------------------------------------------------
-// Where the persistent kernel would leave most waves of the chip without a unit, its time is one unit's chain of tiles
-// (8 tiles, 13 us) or a global row's (a quarter of the sequence's blocks).  Here a unit's tiles are shared by several waves,
-// whose states merge through LDS: one workgroup of 8 waves (one per CU) takes one global row, the two of a head with 4 waves
-// each (global_shares), or RPW other rows with 8 / RPW waves each (rows_per_workgroup has the rule and the times of both
-// kernels).  At most 64 sequences (a lane each).
-constexpr int FEW_CUS = 256;
+// ---- rows of a workgroup ----------------------------------------------------------------------------------------------
 // A share's outputs in LDS: 64 queries x 64 fp32 in rows 272 bytes apart, which puts the 16 lanes of an access on different
 // banks both for the writes (16 rows, 16 bytes of each) and for the reads (2 rows, every second 16 bytes).
 constexpr int SLOT_PITCH = 68, SLOT_FLOATS = 64 * SLOT_PITCH;
-template <typename T, int NW> struct FewRoom {
+template <typename T, int NW> struct Room {
   // a slot per wave; ahead of the merge, query tiles (wave w's own at stage(w), a shared row's at that of its number)
   __attribute__((aligned(16))) float slots[NW][SLOT_FLOATS];
   float m[8][64], l[8][64];                            // per share and query: reference and sum
@@ -1375,51 +771,97 @@ template <typename T, int NW> struct FewRoom {
   __device__ __forceinline__ int& failed(int row) { return reinterpret_cast<int&>(slots[NW - 1][row * SLOT_PITCH + 64]); }
 };
 
-// Lane l: where sequence l begins and ends.  Also fills the bias copy; the caller's barrier follows.
-template <typename T> struct FewBatch {
-  int lane, sb0, sb1;
-  template <int NW> __device__ __forceinline__ FewBatch(const Args<T>& a, FewRoom<T, NW>& room) {
+// Lane l: where sequences l, l + 64, ... of the batch begin and end (CHUNKS of them).  Also fills the bias copy and clears the
+// flags; the caller's barrier follows.
+template <typename T, int CHUNKS> struct Batch {
+  int lane, sb0[CHUNKS], sb1[CHUNKS];
+  template <int NW> __device__ __forceinline__ Batch(const Args<T>& a, Room<T, NW>& room) {
     lane = threadIdx.x & 63;
-    sb0 = a.seq_blocks[min(lane, a.batch)];
-    sb1 = a.seq_blocks[min(lane + 1, a.batch)];
+#pragma unroll
+    for (int c = 0; c < CHUNKS; ++c) {
+      sb0[c] = a.seq_blocks[min(64 * c + lane, a.batch)];
+      sb1[c] = a.seq_blocks[min(64 * c + lane + 1, a.batch)];
+    }
     if (a.q_rows)
       for (int i = threadIdx.x; i < a.heads * 64; i += 64 * NW) room.qbias[i] = a.q_bias ? a.q_bias[i] : static_cast<T>(0.f);
     if (threadIdx.x < 8) room.failed(threadIdx.x) = 0;
   }
-  template <bool MASKED> __device__ __forceinline__ Unit unit_at(const Args<T>& a, int s, int h, int i) const {
+  // which sequences of chunk c there are, and which have global rows
+  __device__ __forceinline__ unsigned long long there(const Args<T>& a, int c) const { return __ballot(64 * c + lane < a.batch); }
+  __device__ __forceinline__ unsigned long long sparse(const Args<T>& a, int c) const {
+    return __ballot(64 * c + lane < a.batch && sb1[c] - sb0[c] >= RT_MIN_SPARSE_BLOCKS);
+  }
+  __device__ __forceinline__ int sparse_count(const Args<T>& a) const {
+    int n = 0;
+#pragma unroll
+    for (int c = 0; c < CHUNKS; ++c) n += __popcll(sparse(a, c));
+    return n;
+  }
+  // row i of sequence l of chunk c
+  template <bool MASKED> __device__ __forceinline__ Unit unit_at(const Args<T>& a, int c, int l, int h, int i) const {
     Unit u;
-    u.g0 = __builtin_amdgcn_readlane(sb0, s);
-    u.n = __builtin_amdgcn_readlane(sb1, s) - u.g0;
+    u.g0 = __builtin_amdgcn_readlane(sb0[c], l);
+    u.n = __builtin_amdgcn_readlane(sb1[c], l) - u.g0;
     u.h = h;
     u.i = i;
     u.tail = 64;
     u.nbv = u.n;
     if (MASKED) {
-      const int tokens = min(max(__builtin_amdgcn_readfirstlane(a.seq_tokens[s]), 1), 64 * u.n);
+      const int tokens = min(max(__builtin_amdgcn_readfirstlane(a.seq_tokens[64 * c + l]), 1), 64 * u.n);
       u.nbv = (tokens + 63) >> 6;
       u.tail = tokens - 64 * (u.nbv - 1);
     }
     return u;
   }
-  // Shares of a global row: eight, one workgroup of eight waves per row; or four, the two global rows of a (sequence, head) in one
-  // workgroup, where that saves a round of workgroups, unless one would be a longer chain (16 tiles) than the other rows' two
-  // rounds.  Measured (us, eight shares / four, 12 heads): three sequences of 8704 tokens in all 32.7 / 28.1, four of 9344 32.5 /
-  // 27.1, six of 8512 29.2 / 22.8, bf16 padded 5 x 320-3000 32.0 / 28.2; where the rounds stay as many, six of 9600 31.5 / 36.3,
-  // five of 11008 34.3 / 38.3.
-  // Only with 8 other rows to a workgroup, the least of them, are there more than one round (rows_per_workgroup).
-  template <int RPW> __device__ __forceinline__ int global_shares(const Args<T>& a, int n_sparse) const {
-    if (RPW < 8 || n_sparse == 0) return 8;
-    const int pairs = n_sparse * a.heads, others = (a.nb_total * a.heads - 2 * pairs + RPW - 1) / RPW;
-    const bool fewer = (pairs + others - 1) / FEW_CUS < (2 * pairs + others - 1) / FEW_CUS;
-    return fewer && !__any(lane < a.batch && sb1 - sb0 > 64) ? 4 : 8;
+  // the first row of the k-th sequence that has global rows
+  template <bool MASKED> __device__ __forceinline__ Unit global_row(const Args<T>& a, int h, int k) const {
+    Unit u{};
+#pragma unroll
+    for (int c = 0; c < CHUNKS; ++c) {
+      const unsigned long long mask = sparse(a, c);
+      const int here = __popcll(mask);
+      if (k >= 0 && k < here)
+        u = unit_at<MASKED>(a, c, __builtin_ctzll(__ballot((mask >> lane & 1ull) && __popcll(mask & ((1ull << lane) - 1ull)) == k)), h, 0);
+      k -= here;
+    }
+    return u;
   }
-  // sequence of a position in a per-lane ascending prefix (lane s: first position of sequence s)
-  __device__ __forceinline__ int seq_of(const Args<T>& a, int prefix, int x) const {
-    return __popcll(__ballot(lane < a.batch && prefix <= x)) - 1;
+  // the j-th of the rows that are not global ones
+  template <bool MASKED> __device__ __forceinline__ Unit other_row(const Args<T>& a, int h, int j) const {
+    Unit u{};
+    int before = 0;                                    // sequences with global rows in earlier chunks
+    bool found = false;
+#pragma unroll
+    for (int c = 0; c < CHUNKS; ++c) {
+      const unsigned long long mask = sparse(a, c);
+      const int listed = sb0[c] - 2 * (before + __popcll(mask & ((1ull << lane) - 1ull)));       // rows of earlier sequences
+      before += __popcll(mask);
+      if (!found && j < __builtin_amdgcn_readlane(sb1[c], 63) - 2 * before) {
+        const int l = __popcll(there(a, c) & __ballot(listed <= j)) - 1;
+        u = unit_at<MASKED>(a, c, l, h, j - __builtin_amdgcn_readlane(listed, l) + int(mask >> l & 1ull));
+        found = true;
+      }
+    }
+    return u;
+  }
+  // the unit with the plan's id blk + head * n + first block * heads
+  template <bool MASKED> __device__ __forceinline__ Unit flat_unit(const Args<T>& a, int id) const {
+    Unit u{};
+    bool found = false;
+#pragma unroll
+    for (int c = 0; c < CHUNKS; ++c)
+      if (!found && id < __builtin_amdgcn_readlane(sb1[c], 63) * a.heads) {
+        const int l = __popcll(there(a, c) & __ballot(sb0[c] * a.heads <= id)) - 1;
+        const int g0 = __builtin_amdgcn_readlane(sb0[c], l), n = __builtin_amdgcn_readlane(sb1[c], l) - g0;
+        const int rem = id - g0 * a.heads, h = rem / n;
+        u = unit_at<MASKED>(a, c, l, h, rem - h * n);
+        found = true;
+      }
+    return u;
   }
 };
 
-template <typename T> __device__ __forceinline__ Buffers<T> few_buffers(const Args<T>& a) {
+template <typename T> __device__ __forceinline__ Buffers<T> buffers_of(const Args<T>& a) {
   Buffers<T> b;
   const uint32_t kv_bytes = uint32_t(a.nb_total) * uint32_t(a.heads) * 8192u;
   b.k = __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(a.k), 0, kv_bytes, 0x00020000);
@@ -1483,7 +925,7 @@ template <bool ADD> __device__ __forceinline__ void to_slot(float* slot, const S
 // slots, and stores it.  Sums are formed in the order ((0 + 4) + (2 + 6)) + ((1 + 5) + (3 + 7)), or its part for fewer shares,
 // whoever forms them.
 template <typename T, int NW, int SHARES>
-__device__ __forceinline__ void merge_shares(FewRoom<T, NW>& room, const State& st, T* out_unit, int64_t stride, bool valid, int row,
+__device__ __forceinline__ void merge_shares(Room<T, NW>& room, const State& st, T* out_unit, int64_t stride, bool valid, int row,
                                              int part, int lane, int wave) {
 #pragma clang fp contract(off)
   constexpr int WAVES = SHARES < NW ? SHARES : NW;
@@ -1554,7 +996,7 @@ __device__ __forceinline__ void merge_shares(FewRoom<T, NW>& room, const State& 
 // The workgroup's NW waves on their rows, from the first tile to the output: a row's tiles in SHARES shares, taken by that many
 // waves side by side, or by all NW, two each, if there are fewer.  u: the wave's row; `valid`: it has one.
 template <typename T, bool MASKED, int SHARES, int NW>
-__device__ __forceinline__ void share_rows(const Args<T>& a, const Buffers<T>& b, FewRoom<T, NW>& room, const QSide<T>& qbias,
+__device__ __forceinline__ void share_rows(const Args<T>& a, const Buffers<T>& b, Room<T, NW>& room, const QSide<T>& qbias,
                                            const Unit& u, bool valid, int lane, int wave) {
   constexpr int WAVES = SHARES < NW ? SHARES : NW;
   constexpr bool TWO = SHARES > NW;                    // part and part + 4 (u is valid in all waves)
@@ -1567,7 +1009,7 @@ __device__ __forceinline__ void share_rows(const Args<T>& a, const Buffers<T>& b
   State st;
   Row r;
   bool redo;                                           // by the moving-maximum loop
-  describe_bounds<T>(a, u, r);
+  describe<T>(a, u, r);
   auto publish = [&](int s) {                          // what the row's other waves have to know of share s
 #pragma unroll
     for (int nt = 0; nt < 2; ++nt) {
@@ -1584,16 +1026,18 @@ __device__ __forceinline__ void share_rows(const Args<T>& a, const Buffers<T>& b
     Padding pd;
     if (valid) {
       fetch_queries<WAVES, T>(a, b, u, part, lane, t);
-      what = begin_share<T, MASKED, false>(a, b, r, TWO ? part + 4 : part, SHARES, lane, t, ids, my, pd);
+      what = begin_share<T, MASKED>(a, b, r, TWO ? part + 4 : part, SHARES, lane, t, ids, my, pd);
     }
     share_queries<WAVES, T>(a, room.qbias, u, valid, room.stage(row), part, lane, t);
     if (TWO) __syncthreads();                          // the query tile is read: its place is a slot's
     state_init(st);
-    bool ok = what == SHARE_RUNS ? end_share<T, MASKED, true>(b, ids, my, pd, lane, t, st) : what == SHARE_EMPTY;
+    bool ok = what == SHARE_RUNS ? end_share<T, MASKED>(b, ids, my, pd, lane, t, st) : what == SHARE_EMPTY;
     if (TWO) {
       publish(part + 4);
       to_slot<false>(slot, st, ones, ones, lane);
-      ok = fast_share<T, MASKED, true, true>(a, b, qbias, r, part, SHARES, lane, t, st) && ok;
+      state_init(st);
+      what = begin_share<T, MASKED>(a, b, r, part, SHARES, lane, t, ids, my, pd);
+      ok = (what == SHARE_RUNS ? end_share<T, MASKED>(b, ids, my, pd, lane, t, st) : what == SHARE_EMPTY) && ok;
     }
     redo = !ok;
     if (SHARES > 1 && redo && lane == 0) room.failed(row) = 1;
@@ -1630,80 +1074,66 @@ __device__ __forceinline__ void share_rows(const Args<T>& a, const Buffers<T>& b
   }
 }
 
-// Without a plan nothing persists and nothing is drawn: workgroup b looks its rows up from the batch's prefix, XCD x
-// taking the x-th eighth of the global rows and of the rest, both head-major, as the persistent kernel does.
-template <typename T, bool MASKED, int RPW>
-__global__ __launch_bounds__(512, 2) void bs_attention_few_kernel(Args<T> a) {
-  constexpr int WAVES_PER_ROW = 8 / RPW;
-  __shared__ FewRoom<T, 8> room;
+// Workgroup b looks its rows up from the batch's prefix, XCD x taking the x-th eighth of the global rows and then of the rest, both
+// head-major: the K / V^T tiles of a (sequence, head) are fetched into one L2.  A global row is a workgroup's, its tiles in
+// GLOBAL shares; of the others it takes NW / OTHERS, each in OTHERS shares.  Nothing persists and nothing is drawn: as its waves
+// end, the CU starts the next workgroup.  The rows of a workgroup are neighbours and run in step, so they find most of the
+// window's tiles in the CU's cache.
+// (Persistent workgroups whose waves drew single rows from ticket counters and requested the next row's queries and first tile
+// inside the last one's steps took 85-90 us where this takes 74 at 8 x 4096 tokens, 12 heads; 92 / 84 at 16 x 512-4096, 28.6 /
+// 24.9 at 5 x 320-3000, 14.7 / 10.9 at 20 x 100-300, 16 heads 139 / 127 at 13120 + 5184 + 10240 + 12224.)
+template <typename T, bool MASKED, int OTHERS, int GLOBAL, int NW, int CHUNKS>
+__global__ __launch_bounds__(64 * NW, 2) void bs_attention_kernel(Args<T> a) {
+  constexpr int ROWS = NW / OTHERS;
+  __shared__ Room<T, NW> room;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const FewBatch<T> batch(a, room);
-  const int lane = batch.lane, sb0 = batch.sb0, sb1 = batch.sb1;
+  const Batch<T, CHUNKS> batch(a, room);
   const QSide<T> qbias{room.qbias, room.stage(wave)};
-  const unsigned long long sparse = __ballot(lane < a.batch && sb1 - sb0 >= RT_MIN_SPARSE_BLOCKS);
-  const int n_sparse = __popcll(sparse), n_rows = a.nb_total - 2 * n_sparse;
+  const int n_sparse = batch.sparse_count(a), n_rows = a.nb_total - 2 * n_sparse;
   const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
 
+  const int n_pairs = n_sparse * a.heads;
+  const int p_lo = int(int64_t(n_pairs) * xcd / 8), p_hi = int(int64_t(n_pairs) * (xcd + 1) / 8), n_glob = 2 * (p_hi - p_lo);
+  const bool global = slot < n_glob;
   Unit u;
   bool valid = true;
-  const int n_pairs = n_sparse * a.heads;
-  const int p_lo = int(int64_t(n_pairs) * xcd / 8), p_hi = int(int64_t(n_pairs) * (xcd + 1) / 8);
-  const int shares = batch.template global_shares<RPW>(a, n_sparse), n_glob = shares == 8 ? 2 * (p_hi - p_lo) : p_hi - p_lo;
-  const bool global = slot < n_glob;
   if (global) {
-    const int pair = p_lo + (shares == 8 ? slot >> 1 : slot), h = pair / n_sparse, k = pair - h * n_sparse;
-    // the k-th sparse sequence
-    const int s = __builtin_ctzll(__ballot((sparse >> lane & 1ull) && __popcll(sparse & ((1ull << lane) - 1ull)) == k));
-    u = batch.template unit_at<MASKED>(a, s, h, 0);
-    if (shares == 8 ? slot & 1 : wave >> 2) u.i = u.n - 1;
+    const int pair = p_lo + (slot >> 1), h = pair / n_sparse;
+    u = batch.template global_row<MASKED>(a, h, pair - h * n_sparse);
+    if (slot & 1) u.i = u.n - 1;
   } else {
     const int total = n_rows * a.heads;
     const int lo = int(int64_t(total) * xcd / 8), hi = int(int64_t(total) * (xcd + 1) / 8);
-    const int first = lo + (slot - n_glob) * RPW;
+    const int first = lo + (slot - n_glob) * ROWS;
     if (first >= hi) return;
-    const int item = first + wave / WAVES_PER_ROW;
+    const int item = first + wave / OTHERS;
     valid = item < hi;
-    const int it = valid ? item : first, h = it / n_rows, j = it - h * n_rows;
-    const int listed_before = sb0 - 2 * __popcll(sparse & ((1ull << lane) - 1ull));       // rows of earlier sequences
-    const int s = batch.seq_of(a, listed_before, j);
-    u = batch.template unit_at<MASKED>(a, s, h, 0);
-    u.i = j - __builtin_amdgcn_readlane(listed_before, s) + ((sparse >> s & 1ull) ? 1 : 0);
+    const int it = valid ? item : first, h = it / n_rows;
+    u = batch.template other_row<MASKED>(a, h, it - h * n_rows);
   }
   __syncthreads();
-  const Buffers<T> b = few_buffers(a);
-  if (RPW > 1 && !global) share_rows<T, MASKED, 8 / RPW, 8>(a, b, room, qbias, u, valid, lane, wave);
-  else if (RPW < 8 || shares == 8) share_rows<T, MASKED, 8, 8>(a, b, room, qbias, u, valid, lane, wave);
-  else share_rows<T, MASKED, 4, 8>(a, b, room, qbias, u, valid, lane, wave);
+  const Buffers<T> b = buffers_of(a);
+  if (OTHERS < GLOBAL && !global) share_rows<T, MASKED, OTHERS, NW>(a, b, room, qbias, u, valid, batch.lane, wave);
+  else share_rows<T, MASKED, GLOBAL, NW>(a, b, room, qbias, u, valid, batch.lane, wave);
 }
 
-// With a caller's plan workgroup c walks its slice, as in the persistent kernel: four waves, two workgroups per CU, a global
-// row by all of them, other entries side by side as far as there are waves for them.  A unit's tiles are cut into as many
-// shares as without a plan, so the bits are the same; a wave takes two of a global row's eight, or one of its four.  The slice
-// is clamped to the list, ids outside it are skipped.  Measured (us a call, 12 heads, rt_meta_partition_lpt into 512 and 256;
-// persistent kernel / this one): 1 x 4096 tokens 22.7, 21.1 / 22.5, 21; 8 x 150-1700 28.8, 35.6 / 28.7, 32.1; 2 x 4096 31.9,
-// 34.7 / 32.7, 32.0; 6 x 2048 44.5, 50.4 / 40.8, 41; 7 x 2048 50.7, 60.6 / 46.8, 52.1 (one workgroup of 8 waves per unit: 96).
-// Behind it: plans of fewer workgroups than CUs for few units (1 x 2048 into 64: 21.7 / 41.8), whose rows are cut finer than
-// they need.
-template <typename T, bool MASKED, int RPW>
-__global__ __launch_bounds__(256, 2) void bs_attention_few_plan_kernel(Args<T> a) {
-  constexpr int SIDE = RPW > 2 ? RPW / 2 : 1;          // rows side by side
-  __shared__ FewRoom<T, 4> room;
+// With a caller's plan workgroup c walks its slice: four waves, two workgroups per CU, a global row by all of them, other
+// entries side by side as far as there are waves for them.  A unit's tiles are cut into as many shares as without a plan, so
+// the bits are the same; a wave takes two of a global row's eight, or one of its four.  The slice is clamped to the list, ids
+// outside it are skipped.  An LPT plan spreads each (sequence, head) over many XCDs: 8 x 4096 tokens into 512 95 us, without a plan
+// 74; 16 x 512-4096 into 1024 116 / 84.
+template <typename T, bool MASKED, int OTHERS, int GLOBAL, int CHUNKS>
+__global__ __launch_bounds__(256, 2) void bs_attention_plan_kernel(Args<T> a) {
+  constexpr int SIDE = OTHERS < 4 ? 4 / OTHERS : 1;    // rows side by side
+  __shared__ Room<T, 4> room;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int n_units = a.nb_total * a.heads;
   const int begin = min(max(a.from_pos[blockIdx.x], 0), n_units);
   const int end = min(max(a.from_pos[blockIdx.x + 1], begin), n_units);
   if (begin == end) return;
-  const FewBatch<T> batch(a, room);
+  const Batch<T, CHUNKS> batch(a, room);
   const QSide<T> qbias{room.qbias, room.stage(wave)};
-  const Buffers<T> b = few_buffers(a);
-  const int shares =
-      batch.template global_shares<RPW>(a, __popcll(__ballot(batch.lane < a.batch && batch.sb1 - batch.sb0 >= RT_MIN_SPARSE_BLOCKS)));
-  auto unit_of_flat = [&](int id) {
-    const int s = batch.seq_of(a, batch.sb0 * a.heads, id);
-    const int g0 = __builtin_amdgcn_readlane(batch.sb0, s), n = __builtin_amdgcn_readlane(batch.sb1, s) - g0;
-    const int rem = id - g0 * a.heads, h = rem / n;
-    return batch.template unit_at<MASKED>(a, s, h, rem - h * n);
-  };
+  const Buffers<T> b = buffers_of(a);
   for (int p = begin; p < end;) {
     int ids[SIDE];                                     // the next entries in one round trip
 #pragma unroll
@@ -1712,7 +1142,7 @@ __global__ __launch_bounds__(256, 2) void bs_attention_few_plan_kernel(Args<T> a
       if (ids[w] >= n_units) ids[w] = -1;
     }
     if (ids[0] < 0) { ++p; continue; }
-    Unit u = unit_of_flat(ids[0]);
+    Unit u = batch.template flat_unit<MASKED>(a, ids[0]);
     const bool whole = is_global_row(u);
     int run = 1;
     if (!whole) {
@@ -1722,7 +1152,7 @@ __global__ __launch_bounds__(256, 2) void bs_attention_few_plan_kernel(Args<T> a
       for (int w = 1; w < SIDE; ++w) {
         more = more && ids[w] >= 0;
         if (more) {
-          const Unit v = unit_of_flat(ids[w]);
+          const Unit v = batch.template flat_unit<MASKED>(a, ids[w]);
           more = !is_global_row(v);
           if (more) ++run;
           if (more && w == mine) u = v;
@@ -1734,51 +1164,11 @@ __global__ __launch_bounds__(256, 2) void bs_attention_few_plan_kernel(Args<T> a
     asm volatile("" : "+v"(lane));
     if (threadIdx.x < 8) room.failed(threadIdx.x) = 0;           // (the last rows' flags were read several barriers ago)
     __syncthreads();
-    if (RPW > 1 && !whole) share_rows<T, MASKED, 8 / RPW, 4>(a, b, room, qbias, u, SIDE * wave / 4 < run, lane, wave);
-    else if (RPW < 8 || shares == 8) share_rows<T, MASKED, 8, 4>(a, b, room, qbias, u, true, lane, wave);
-    else share_rows<T, MASKED, 4, 4>(a, b, room, qbias, u, true, lane, wave);
+    if (OTHERS < GLOBAL && !whole) share_rows<T, MASKED, OTHERS, 4>(a, b, room, qbias, u, SIDE * wave / 4 < run, lane, wave);
+    else share_rows<T, MASKED, GLOBAL, 4>(a, b, room, qbias, u, true, lane, wave);
     p += run;
   }
 }
-
-// Two persistent workgroups per CU, a multiple of 8 so that every XCD gets the same number.
-unsigned plan_free_workgroups() {
-  static unsigned cached = 0;
-  if (cached == 0) {
-    int dev = 0, cus = 0;
-    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
-      cus = 256;
-    cached = unsigned((2 * cus + 7) / 8 * 8);
-  }
-  return cached;
-}
-
-// Queue counters of the library's own launches: a ring of slots, so that launches which overlap on
-// different streams do not share counters.  A launch leaves its slot zeroed (the kernel's last
-// workgroups do that), so the slots need no order among the launches that use them; what the ring cannot
-// cover is more than QUEUE_SLOTS attention launches of the library in flight on one device at the same time.
-constexpr int QUEUE_SLOTS = 64;
-int* library_queues(int* err) {
-  static int* base[64] = {};
-  static unsigned next[64] = {};
-  static std::mutex mu;
-  int dev = 0;
-  *err = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) { *err = 1; return nullptr; }
-  std::lock_guard<std::mutex> lock(mu);
-  if (!base[dev]) {
-    int* p = nullptr;
-    if (hipMalloc(&p, sizeof(int) * QUEUE_INTS * QUEUE_SLOTS) != hipSuccess) { *err = 2; return nullptr; }
-    if (hipMemset(p, 0, sizeof(int) * QUEUE_INTS * QUEUE_SLOTS) != hipSuccess) { *err = 3; return nullptr; }
-    base[dev] = p;
-  }
-  const unsigned slot = next[dev]++ % QUEUE_SLOTS;
-  return base[dev] + slot * QUEUE_INTS;
-}
-
-}  // namespace
-
-namespace {
 
 // Pairs of global rows the batch can have at most: the host knows the block count, not the sequences' lengths.
 int64_t most_pairs(int batch, int total_blocks, int heads) {
@@ -1786,40 +1176,54 @@ int64_t most_pairs(int batch, int total_blocks, int heads) {
   return int64_t(sparse < batch ? sparse : batch) * heads;
 }
 
-// Rows that share a workgroup of bs_attention_few_kernel, as few as still give every workgroup a CU of its own and every
-// wave a tile (1 x 64 tokens: 6.6, 7.7, 6.5, 5.3 us with 1, 2, 4, 8; persistent kernel 12.8); 0: the persistent kernel.
-// Measured (us in a graph, 12 heads, persistent kernel / this one with 1, 2, 4, 8 rows to a workgroup): 1 x 512
-// tokens 18.8 / 8.4, 9.5, 11.9, 14.8; 1 x 2048 20.1 / 16.5, 12.6, 13.0, 15.9; 4 x 256-1024 22.2 / 22.8, 20.0, 14.5,
-// 18.0; 1 x 4096 26.5 / 30.9, 20.3, 18.4, 18.3; 8 x 150-1700 28.9 / 37.3, 29.3, 24.4, 19.9; 2 x 4096 36.1 / 52.4, 39.1, 29.2,
-// 23.0; 6 x 2048 43.7 / 73.8, 52.9, 43.8, 37.8.
-int rows_per_workgroup(int batch, int total_blocks, int heads) {
-  const int64_t units = int64_t(total_blocks) * heads;
-  if (batch > 64 || units > 2816) return 0;
-  const int64_t global = 2 * most_pairs(batch, total_blocks, heads);
+// How a launch cuts its rows: shares of a row that is not global and of one that is, waves of a workgroup.  With few rows a
+// row's chain of tiles is the time of the launch, so its tiles are spread over 4 or 2 waves while the workgroups, two to a CU
+// at most, leave every wave a SIMD mostly to itself.  A global row's chain, a quarter of the sequence's blocks, is halved
+// by workgroups of 8 waves where it would outlast the others' work; they fill a CU one at a time, which costs up to 15 % where
+// there is work enough.  The longest sequence is not known here: half as long again as the average is taken for it.
+// Measured (us in a graph, 12 heads, bf16; others, global, waves 4 4 4 / 2 4 4 / 1 4 4 / 1 8 8): 1 x 64 tokens 5.8 / 6.1 / 5.2 / 5.4,
+// 1 x 192 6.0 / 7.0 / 6.9 / 9.1, 1 x 512 6.9 / 8.5 / 10.3 / 15.4, 1 x 1024 8.4 / 8.6 / 10.4 / 15.7, 1 x 1536 11.5 / 9.8 / 10.8 / 16.1,
+// 2 x 1024 10.7 / 9.3 / 11.0 / 16.0, 1 x 2048 13.1 / 11.5 / 11.7 / 16.3, 1 x 2560 14.6 / 15.3 / 13.6 / 16.8, 2 x 2048 17.8 / 15.5 / 13.0 /
+// 17.3, 1 x 4096 19.4 / 19.8 / 18.8 / 17.9, 2 x 4096 31.7 / 26.4 / 25.2 / 22.4, 4 x 4096 55.0 / 45.8 / 41.4 / 44.8, 16 heads 1 x 8192 39.1 /
+// 37.2 / 37.6 / 37.6, 1 x 12288 55.7 / 50.8 / 52.0 / 48.0.
+struct Cut { int others, global, waves; };
+Cut cut_rows(int batch, int total_blocks, int heads) {
+  if (batch > 64) return {1, 4, 4};
+  const int64_t units = int64_t(total_blocks) * heads, global = 2 * most_pairs(batch, total_blocks, heads);
   const int longest = total_blocks - batch + 1;         // tiles that a row can have at most
-  for (int rows = 1; rows <= 4; rows *= 2)
-    if (8 / rows <= longest && global + (units - global + rows - 1) / rows <= 256) return rows;
-  return 8;
+  if (longest >= 3 && units <= 256) return {4, 4, 4};
+  if (longest >= 2 && global + (units - global) / 2 <= 220) return {2, 4, 4};
+  const int likely = batch == 1 ? total_blocks : 3 * total_blocks / (2 * batch);
+  // one round of workgroups, or a single sequence whose chain, 5 us and 0.25 a tile, outlasts the units' 17 ns each
+  if (likely >= 60 && (global + (units - global) / 8 <= 256 || (batch == 1 && 5 + 0.25 * longest > 0.0167 * double(units))))
+    return {1, 8, 8};
+  return {1, 4, 4};
 }
 
-template <typename T> int launch_few(const Args<T>& a, int rpw, int n_wg, hipStream_t st) {
-  auto go = [&](auto masked, auto rows) {
+template <typename T> int launch_rows(const Args<T>& a, int n_wg, hipStream_t st) {
+  const Cut cut = cut_rows(a.batch, a.nb_total, a.heads);
+  auto go = [&](auto masked, auto others, auto global, auto waves, auto chunks) {
     constexpr bool MASKED = decltype(masked)::value;
-    constexpr int RPW = decltype(rows)::value;
+    constexpr int OTHERS = decltype(others)::value, GLOBAL = decltype(global)::value, NW = decltype(waves)::value, CHUNKS = decltype(chunks)::value;
     if (a.from_pos) {
-      RT_LAUNCH((bs_attention_few_plan_kernel<T, MASKED, RPW>), dim3(unsigned(n_wg)), dim3(256), 0, st, a);
+      RT_LAUNCH((bs_attention_plan_kernel<T, MASKED, OTHERS, GLOBAL, CHUNKS>), dim3(unsigned(n_wg)), dim3(256), 0, st, a);
       return;
     }
     // every XCD's share of the global rows (two per head of each sequence that may have them) and of the others
     const int64_t units = int64_t(a.nb_total) * a.heads, pairs = most_pairs(a.batch, a.nb_total, a.heads);
-    const int64_t per_xcd = 2 * ((pairs + 7) / 8) + ((units + 7) / 8 + rpw - 1) / rpw;
-    RT_LAUNCH((bs_attention_few_kernel<T, MASKED, RPW>), dim3(unsigned(8 * per_xcd)), dim3(512), 0, st, a);
+    const int64_t per_xcd = 2 * ((pairs + 7) / 8) + ((units + 7) / 8 + NW / OTHERS - 1) / (NW / OTHERS);
+    RT_LAUNCH((bs_attention_kernel<T, MASKED, OTHERS, GLOBAL, NW, CHUNKS>), dim3(unsigned(8 * per_xcd)), dim3(64 * NW), 0, st, a);
   };
   auto pick = [&](auto masked) {
-    if (rpw == 1) go(masked, std::integral_constant<int, 1>());
-    else if (rpw == 2) go(masked, std::integral_constant<int, 2>());
-    else if (rpw == 4) go(masked, std::integral_constant<int, 4>());
-    else go(masked, std::integral_constant<int, 8>());
+    const std::integral_constant<int, 1> one;
+    const std::integral_constant<int, 2> two;
+    const std::integral_constant<int, 4> four;
+    const std::integral_constant<int, 8> eight;
+    if (a.batch > 64) go(masked, one, four, four, std::integral_constant<int, MAX_BATCH / 64>());
+    else if (cut.others == 4) go(masked, four, four, four, one);
+    else if (cut.others == 2) go(masked, two, four, four, one);
+    else if (cut.global == 8) go(masked, one, eight, eight, one);
+    else go(masked, one, four, four, one);
   };
   if (a.seq_tokens) pick(std::true_type());
   else pick(std::false_type());
@@ -1830,7 +1234,7 @@ template <typename T> int launch_few(const Args<T>& a, int rpw, int n_wg, hipStr
 int launch_attention(const void* q, const void* q_rows, const void* q_bias, float q_scale, const void* k, const void* vt,
                      void* out, const int* seq_blocks_dev, const int* seq_tokens_dev, int batch, int total_blocks,
                      int heads, const int* to_idx, const int* to_pos, int plan_heads, const int* from_idx,
-                     const int* from_pos, int n_wg, int dtype, void* stream, int* own_queues = nullptr) {
+                     const int* from_pos, int n_wg, int dtype, void* stream) {
   RT_REQUIRE((q || q_rows) && k && vt && out && seq_blocks_dev && to_idx && to_pos, RT_EINVAL, "NULL pointer");
   RT_REQUIRE(batch >= 1 && total_blocks >= batch && heads >= 1, RT_EINVAL, "bad geometry: batch=%d total_blocks=%d heads=%d",
              batch, total_blocks, heads);
@@ -1854,46 +1258,13 @@ int launch_attention(const void* q, const void* q_rows, const void* q_bias, floa
   }
   RT_REQUIRE(!from_idx || n_wg >= 1, RT_EINVAL, "balanced launch needs n_wg >= 1, got %d", n_wg);
   hipStream_t st = static_cast<hipStream_t>(stream);
-  if (const int rpw = rows_per_workgroup(batch, total_blocks, heads)) {
-    auto few = [&](auto tag) {
-      typedef decltype(tag) T;
-      return launch_few(Args<T>{(const T*)q, (const T*)k, (const T*)vt, (T*)out, seq_blocks_dev, batch, heads, total_blocks, to_idx,
-                                to_pos, plan_heads, from_idx, from_pos, seq_tokens_dev, (const T*)q_rows, (const T*)q_bias,
-                                q_scale, nullptr},
-                        rpw, n_wg, st);
-    };
-    return dtype == RT_F16 ? few(_Float16()) : few(__bf16());
-  }
-  unsigned grid;
-  int* queues = nullptr;
-  if (from_idx) {
-    grid = unsigned(n_wg);
-  } else {
-    grid = plan_free_workgroups();
-    if (own_queues) {
-      queues = own_queues;
-    } else {
-      int err = 0;
-      queues = library_queues(&err);
-      if (!queues) return rt::fail(RT_ENOMEM, "no device memory for the work queues (step %d)", err);
-    }
-  }
-  if (dtype == RT_F16) {
-    Args<_Float16> a{(const _Float16*)q, (const _Float16*)k, (const _Float16*)vt, (_Float16*)out, seq_blocks_dev, batch,
-                     heads, total_blocks, to_idx, to_pos, plan_heads, from_idx, from_pos, seq_tokens_dev,
-                     (const _Float16*)q_rows, (const _Float16*)q_bias, q_scale, queues};
-    if (seq_tokens_dev) RT_LAUNCH((bs_attention_kernel<_Float16, true>), dim3(grid), dim3(256), 0, st, a);
-    else RT_LAUNCH((bs_attention_kernel<_Float16, false>), dim3(grid), dim3(256), 0, st, a);
-  } else {
-    Args<__bf16> a{(const __bf16*)q, (const __bf16*)k, (const __bf16*)vt, (__bf16*)out, seq_blocks_dev, batch, heads,
-                   total_blocks, to_idx, to_pos, plan_heads, from_idx, from_pos, seq_tokens_dev,
-                   (const __bf16*)q_rows, (const __bf16*)q_bias, q_scale, queues};
-    if (seq_tokens_dev) RT_LAUNCH((bs_attention_kernel<__bf16, true>), dim3(grid), dim3(256), 0, st, a);
-    else RT_LAUNCH((bs_attention_kernel<__bf16, false>), dim3(grid), dim3(256), 0, st, a);
-  }
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return rt::fail(RT_EIO, "bs_attention launch failed: %s", hipGetErrorString(e));
-  return RT_OK;
+  auto rows = [&](auto tag) {
+    typedef decltype(tag) T;
+    return launch_rows(Args<T>{(const T*)q, (const T*)k, (const T*)vt, (T*)out, seq_blocks_dev, batch, heads, total_blocks, to_idx,
+                               to_pos, plan_heads, from_idx, from_pos, seq_tokens_dev, (const T*)q_rows, (const T*)q_bias, q_scale},
+                       n_wg, st);
+  };
+  return dtype == RT_F16 ? rows(_Float16()) : rows(__bf16());
 }
 
 }  // namespace
@@ -1926,35 +1297,7 @@ extern "C" int rt_bs_attention_fwd(const void* q, const void* k, const void* vt,
                                     plan_heads, from_idx, from_pos, n_wg, dtype, stream);
 }
 
-// ---- the entry point that allocates nothing -------------------------------------------------------
-// Its queue counters live in this array instead of the library's allocated ring, zeroed by a fill kernel
-// ahead of every launch (whatever an earlier launch that was cut short may have left there).  In host code
-// the array's name is only a stand-in: its address on a device comes from hipGetSymbolAddress, once per device.
-constexpr int NO_ALLOC_SCRATCH_INTS = RT_NO_ALLOC_SCRATCH_BYTES / int(sizeof(int));
-static_assert(NO_ALLOC_SCRATCH_INTS >= QUEUE_INTS, "the scratch array must hold one launch's counters");
 static_assert(RT_NO_ALLOC_MAX_BATCH <= MAX_BATCH && RT_NO_ALLOC_MAX_BLOCKS <= MAX_BLOCKS, "header limits exceed the kernel's");
-static __device__ __align__(256) int scratch[NO_ALLOC_SCRATCH_INTS];
-
-namespace {
-
-__global__ void clear_queue_counters(int* counters) { counters[threadIdx.x * QUEUE_STRIDE] = 0; }
-
-int* no_alloc_scratch() {
-  static int* ptr[64] = {};
-  static std::mutex mu;
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return nullptr;
-  std::lock_guard<std::mutex> lock(mu);
-  if (!ptr[dev]) {
-    void* p = nullptr;
-    if (hipGetSymbolAddress(&p, HIP_SYMBOL(scratch)) != hipSuccess || !p) return nullptr;
-    ptr[dev] = static_cast<int*>(p);
-  }
-  return ptr[dev];
-}
-
-}  // namespace
-
 extern "C" int rt_bs_attention_fwd_no_alloc(const void* q, const void* k, const void* vt, void* out,
                                             const int* seq_blocks_dev, const int* seq_tokens_dev, int batch,
                                             int total_blocks, int heads, const int* to_idx, const int* to_pos,
@@ -1963,11 +1306,6 @@ extern "C" int rt_bs_attention_fwd_no_alloc(const void* q, const void* k, const 
   RT_REQUIRE(batch >= 1 && batch <= RT_NO_ALLOC_MAX_BATCH && total_blocks >= batch && total_blocks <= RT_NO_ALLOC_MAX_BLOCKS,
              RT_EINVAL, "rt_bs_attention_fwd_no_alloc takes at most %d sequences and %d blocks (%d tokens), got %d and %d",
              RT_NO_ALLOC_MAX_BATCH, RT_NO_ALLOC_MAX_BLOCKS, RT_NO_ALLOC_MAX_BLOCKS * 64, batch, total_blocks);
-  int* counters = no_alloc_scratch();
-  if (!counters) return rt::fail(RT_EIO, "the address of the static scratch array is not available on this device");
-  hipLaunchKernelGGL(clear_queue_counters, dim3(1), dim3(QUEUE_COUNTERS), 0, static_cast<hipStream_t>(stream), counters);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return rt::fail(RT_EIO, "clearing the queue counters failed: %s", hipGetErrorString(e));
   return launch_attention(q, nullptr, nullptr, 1.0f, k, vt, out, seq_blocks_dev, seq_tokens_dev, batch, total_blocks, heads,
-                          to_idx, to_pos, plan_heads, nullptr, nullptr, 0, dtype, stream, counters);
+                          to_idx, to_pos, plan_heads, nullptr, nullptr, 0, dtype, stream);
 }

@@ -31,7 +31,7 @@ def capi():
     (12, [4096, 2624, 1984], 40.0),                   # the same at the longest sequence that takes them so
     (12, [4160, 2560, 1984], 1.0),                    # one block longer: by 8 waves each, in two rounds
     (2, [64] * 64, 1.0),                              # as many sequences as lanes
-    (2, [64] * 64 + [128], 1.0),                      # one more: the persistent kernel
+    (2, [64] * 64 + [128], 1.0),                      # one more
     (8, [4096 * 4], 1.0),                             # global rows of 256 tiles
     (11, [64 * 128, 64 * 128], 6.0),                  # 2816 units, the most the rule takes
 ])
@@ -97,7 +97,7 @@ def test_few_units_walk_the_plan(capi, heads, lens, scale, padded):
     (12, [512, 1024, 1280]),                          # 2
     (12, [2048, 3008, 384]),                          # 1
     (12, [2944, 3008, 2752]),                         # 1, global rows by 4
-    (16, [2048] * 6),                                 # the persistent kernel
+    (16, [2048] * 6),                                 # 3072 units
 ])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_infinite_and_very_low_scores(capi, heads, lens, dtype):
@@ -132,7 +132,7 @@ def test_infinite_and_very_low_scores(capi, heads, lens, dtype):
 @pytest.mark.parametrize("heads,lens,short", [
     (3, [1024, 768, 64], 17),                         # few units; 64 tokens: every entry is the padded tile
     (4, [1024, 1600, 320], 63),                       # a tail of one key
-    (12, [1024] * 15, 40),                            # 2880 units: the persistent kernel
+    (12, [1024] * 15, 40),                            # 2880 units
     (12, [1024, 768] * 8, 150),                       # whole blocks of padding dropped in front of it
 ])
 def test_padded_tile_listed_several_times(capi, heads, lens, short, dtype):
