@@ -307,6 +307,11 @@ __device__ inline float pair_sum(float x) {
   return __builtin_bit_cast(float, a) + __builtin_bit_cast(float, b);
 }
 
+// the 64 rows of a unit's outputs
+template <typename T> __device__ __forceinline__ __amdgpu_buffer_rsrc_t unit_rows(T* out_unit, int64_t row_stride) {
+  return __builtin_amdgcn_make_buffer_rsrc(out_unit, 0, uint32_t(row_stride) * 128u, 0x00020000);
+}
+
 // Writes the wave's 64x64 output tile, O^T[d = 32t + 8*(e>>2) + 4*(lane>>5) + (e&3)]
 // [query 32nt + (lane&31)] * w, to out[token][h*64 + d], through the wave's own LDS room (64 rows, OUT_PITCH bytes
 // apart; no other wave touches it, and the LDS operations of one wave execute in order).  A lane holds 4
@@ -333,11 +338,12 @@ __device__ inline void store_output(T* __restrict__ out_unit, int64_t row_stride
       }
   }
   const char* rd = stage + (lane >> 3) * OUT_PITCH + (lane & 7) * 16;
-  T* dst = out_unit + int64_t(lane >> 3) * row_stride + (lane & 7) * 8;
+  const __amdgpu_buffer_rsrc_t dst = unit_rows(out_unit, row_stride);
+  const uint32_t at = uint32_t(lane >> 3) * uint32_t(row_stride) * 2u + uint32_t(lane & 7) * 16u;
 #pragma unroll
   for (int k = 0; k < 8; ++k) {
     const u32x4 v = *reinterpret_cast<const u32x4*>(rd + k * 8 * OUT_PITCH);
-    *reinterpret_cast<u32x4*>(dst + int64_t(8 * k) * row_stride) = v;
+    __builtin_amdgcn_raw_buffer_store_b128(v, dst, int(at + uint32_t(8 * k) * uint32_t(row_stride) * 2u), 0, rt::WRITE_THROUGH);
   }
 }
 
@@ -989,7 +995,8 @@ __device__ __forceinline__ void merge_shares(Room<T, NW>& room, const State& st,
     u32x4 o;
 #pragma unroll
     for (int e = 0; e < 4; ++e) o[e] = Mma<T>::two(x[i][0][e >> 1][2 * (e & 1)] * w, x[i][0][e >> 1][2 * (e & 1) + 1] * w);
-    *reinterpret_cast<u32x4*>(out_unit + int64_t(first + 8 * i) * stride + (lane & 7) * 8) = o;
+    __builtin_amdgcn_raw_buffer_store_b128(o, unit_rows(out_unit, stride), int((uint32_t(first + 8 * i) * uint32_t(stride) + uint32_t(lane & 7) * 8u) * 2u),
+                                           0, rt::WRITE_THROUGH);
   }
 }
 

@@ -230,9 +230,11 @@ __device__ __forceinline__ void store_rows(const f32x4 (&acc)[MT][4], __amdgpu_b
   }
 }
 
-// K and V^T tiles: where the half tile of the 32 tokens from `row` on begins (lane's part), for head h.  seq_end: lane
-// l holds the end of sequence l (batches of up to 64 sequences).
-template <typename T> __device__ __forceinline__ T* half_tile(void* base, const Params& p, int seq_end, int row, int h) {
+// K and V^T tiles: the byte at which the tile of token `row` begins (lane's part), for head h; past the tensors' end where
+// there is no such row or head, so the stores' range check drops what is written there.  seq_end: lane l holds the end of
+// sequence l (batches of up to 64 sequences).
+__device__ __forceinline__ uint32_t tile_offset(const Params& p, int seq_end, int row, int h) {
+  if (row >= p.m || h >= p.heads) return 0xfffc0000u;
   const int g = row >> 6, lane = again(threadIdx.x & 63);
   int s, g0, end;                                          // the sequence block g belongs to
   if (p.batch <= 64) {
@@ -246,7 +248,7 @@ template <typename T> __device__ __forceinline__ T* half_tile(void* base, const 
     g0 = p.seq_blocks[s];
     end = p.seq_blocks[s + 1];
   }
-  return static_cast<T*>(base) + (int64_t(g0) * p.heads + int64_t(h) * (end - g0) + (g - g0)) * 4096 + lane * 8;
+  return uint32_t(g0 * p.heads + h * (end - g0) + (g - g0)) * 8192u + uint32_t(lane) * 16u;
 }
 
 // V^T tiles of head h from its column d0 (a multiple of 32) on (products taken with the tokens as rows): a lane's accumulators are 4 consecutive tokens of one
@@ -254,11 +256,11 @@ template <typename T> __device__ __forceinline__ T* half_tile(void* base, const 
 // of its 16.
 template <typename T, int MT, int NT>
 __device__ __forceinline__ void store_v(const f32x4 (&acc)[MT][NT], const Params& p, int seq_end, int m0, int h, int d0 = 0) {
+  const __amdgpu_buffer_rsrc_t sv = __builtin_amdgcn_make_buffer_rsrc(p.vt, 0, uint32_t(p.m) * uint32_t(p.heads) * 128u, 0x00020000);
 #pragma unroll
   for (int i = 0; i < MT; i += 2) {
     const int row = m0 + 16 * i;
-    if (row >= p.m) break;
-    T* const t = half_tile<T>(p.vt, p, seq_end, row, h) + ((row >> 5) & 1) * 1024 + d0 * 64;
+    const uint32_t t = tile_offset(p, seq_end, row, h) + uint32_t(((row >> 5) & 1) * 2048 + d0 * 128);
 #pragma unroll
     for (int q = 0; q < 2; ++q)
 #pragma unroll
@@ -270,7 +272,7 @@ __device__ __forceinline__ void store_v(const f32x4 (&acc)[MT][NT], const Params
         permlane16_swap(x1, y1);
         permlane32_swap(x0, y0);
         permlane32_swap(x1, y1);
-        *reinterpret_cast<u32x4*>(t + (2 * j + q) * 512) = u32x4{x0, x1, y0, y1};
+        __builtin_amdgcn_raw_buffer_store_b128(u32x4{x0, x1, y0, y1}, sv, int(t + (2 * j + q) * 1024), 0, rt::WRITE_THROUGH);
       }
   }
 }
@@ -279,11 +281,11 @@ __device__ __forceinline__ void store_v(const f32x4 (&acc)[MT][NT], const Params
 // token; fragment 4 * (token >> 5) + (d >> 4) wants, in lane (token & 31) + 32 * x, the columns 8 x .. + 8 of its 16.
 template <typename T, int MT, int NT>
 __device__ __forceinline__ void store_k(const f32x4 (&acc)[MT][NT], const Params& p, int seq_end, int m0, int h, int d0 = 0) {
+  const __amdgpu_buffer_rsrc_t sk = __builtin_amdgcn_make_buffer_rsrc(p.kt, 0, uint32_t(p.m) * uint32_t(p.heads) * 128u, 0x00020000);
 #pragma unroll
   for (int i = 0; i < MT; i += 2) {
     const int row = m0 + 16 * i;
-    if (row >= p.m) break;
-    T* const t = half_tile<T>(p.kt, p, seq_end, row, h) + ((row >> 5) & 1) * 2048 + d0 * 32;
+    const uint32_t t = tile_offset(p, seq_end, row, h) + uint32_t(((row >> 5) & 1) * 4096 + d0 * 64);
 #pragma unroll
     for (int j = 0; j < NT; ++j) {
       const f32x4 &c = acc[i][j], &d = acc[i + 1][j];
@@ -291,7 +293,7 @@ __device__ __forceinline__ void store_k(const f32x4 (&acc)[MT][NT], const Params
       uint32_t y0 = Mma<T>::two(d[0], d[1]), y1 = Mma<T>::two(d[2], d[3]);
       permlane16_swap(x0, y0);
       permlane16_swap(x1, y1);
-      *reinterpret_cast<u32x4*>(t + j * 512) = u32x4{x0, x1, y0, y1};
+      __builtin_amdgcn_raw_buffer_store_b128(u32x4{x0, x1, y0, y1}, sk, int(t + j * 1024), 0, rt::WRITE_THROUGH);
     }
   }
 }
@@ -602,7 +604,7 @@ __device__ __forceinline__ void store_block(const f32x4 (&acc)[MT][NT], __amdgpu
     if (i > 0) {
 #pragma unroll
       for (int k = 0; k < ST; ++k) {
-        __builtin_amdgcn_raw_buffer_store_b128(o[k], sc, int(voff[k]), 0, 0);
+        __builtin_amdgcn_raw_buffer_store_b128(o[k], sc, int(voff[k]), 0, rt::WRITE_THROUGH);
         voff[k] += rows16[k];
       }
     }

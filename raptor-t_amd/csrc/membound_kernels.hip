@@ -70,6 +70,19 @@ template <> struct Vec<float> {
   }
 };
 
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+// `count` elements from p on, the same p in all lanes
+template <typename T> __device__ __forceinline__ __amdgpu_buffer_rsrc_t run_of(T* p, int count) {
+  return __builtin_amdgcn_make_buffer_rsrc(p, 0, uint32_t(count) * uint32_t(sizeof(T)), 0x00020000);
+}
+__device__ __forceinline__ void store_through(u32x2 v, __amdgpu_buffer_rsrc_t to, uint32_t at) {
+  __builtin_amdgcn_raw_buffer_store_b64(v, to, int(at), 0, rt::WRITE_THROUGH);
+}
+__device__ __forceinline__ void store_through(u32x4 v, __amdgpu_buffer_rsrc_t to, uint32_t at) {
+  __builtin_amdgcn_raw_buffer_store_b128(v, to, int(at), 0, rt::WRITE_THROUGH);
+}
+
 // Sum over G (32 or 64) consecutive lanes, in all of them.  The lanes' values change places inside the vector unit: through
 // LDS (__shfl_xor) the two sums of a LayerNorm are chains of up to 12 LDS latencies: bias + residual + LayerNorm in fp16 512 x 768
 // 2.51 -> 2.20 us, 2816 x 768 3.45 -> 3.22, 32768 x 768 22.7 -> 22.4.  Pairs are added in the same order, so the bits are the same.
@@ -102,6 +115,7 @@ __global__ __launch_bounds__(256) void bias_residual_layernorm_kernel(
   if (row >= rows) return;
   T* o = out + row * HIDDEN;
   const T* r = residual + row * HIDDEN;
+  const __amdgpu_buffer_rsrc_t dst = run_of(out + int64_t(blockIdx.x) * (256 / G) * HIDDEN, 256 / G * HIDDEN);
   float x[CHUNKS][N];
   float sum = 0.f;
   // every request of the row goes out before the first conversion waits for one (left to itself
@@ -138,7 +152,9 @@ __global__ __launch_bounds__(256) void bias_residual_layernorm_kernel(
     Vec<T>::load(beta + col, b);
 #pragma unroll
     for (int i = 0; i < N; ++i) y[i] = (x[c][i] - mean) * rstd * g[i] + b[i];
-    Vec<T>::store(o + col, y);
+    u32x4 packed;
+    Vec<T>::store(reinterpret_cast<T*>(&packed), y);
+    store_through(packed, dst, uint32_t(int(threadIdx.x / G) * HIDDEN + col) * uint32_t(sizeof(T)));
   }
 }
 
@@ -259,6 +275,8 @@ __global__ __launch_bounds__(256) void slices_residual_layernorm_kernel(T* __res
   const int64_t row = int64_t(blockIdx.x) * 4 + (threadIdx.x >> 6);
   if (row >= rows) return;
   const int64_t slice = rows * HIDDEN;
+  const int in_wg = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const __amdgpu_buffer_rsrc_t dst = run_of(out + (int64_t(blockIdx.x) * 4 + in_wg) * HIDDEN, HIDDEN);
   const float* src = parts + row * HIDDEN + lane * 4;
   float x[CH][4];
   uint2 res[CH], bi[CH], ga[CH], be[CH];
@@ -329,7 +347,9 @@ __global__ __launch_bounds__(256) void slices_residual_layernorm_kernel(T* __res
     Quad<T>::load(reinterpret_cast<const T*>(&be[c]), b);
 #pragma unroll
     for (int i = 0; i < 4; ++i) y[i] = (x[c][i] - mean) * rstd * g[i] + b[i];
-    Quad<T>::store(out + row * HIDDEN + c * 256 + lane * 4, y);
+    uint2 packed;
+    Quad<T>::store(reinterpret_cast<T*>(&packed), y);
+    store_through(u32x2{packed.x, packed.y}, dst, uint32_t(c * 256 + lane * 4) * uint32_t(sizeof(T)));
   }
 }
 
