@@ -13,6 +13,8 @@ import random
 import numpy as np
 import torch
 from torch.autograd import forward_ad
+from torch.overrides import _get_current_function_mode_stack
+from torch.utils._device import DeviceContext
 
 from . import capi
 
@@ -135,11 +137,18 @@ def pack_padded_batch(input_ids, attention_mask, token_type_ids=None, block_size
             "seq_tokens_tensor": torch.tensor(seq_tokens, dtype=torch.int32, device=input_ids.device)}
 
 
+def _watched():
+    """Whether something sees the operators that run now and would miss a kernel: a tracer or compiler, a transform, a dispatch or
+    function mode (a default device is a function mode too, and not meant)."""
+    return (torch.compiler.is_compiling() or torch.jit.is_tracing() or forward_ad._current_level >= 0 or
+            torch._C._len_torch_dispatch_stack() > 0 or any(type(m) is not DeviceContext for m in _get_current_function_mode_stack()))
+
+
 def _ordinary(t):
-    """A tensor whose memory a kernel may read as it is: on the current GPU, no subclass, nothing that traces, batches or
-    differentiates the operators applied to it."""
+    """A tensor whose memory a kernel may read as it is: on the current GPU, no subclass, not batched or differentiated, no
+    conjugation, sign or zeros that only its flags hold."""
     return (type(t) is torch.Tensor and t.is_cuda and t.device.index == torch.cuda.current_device() and not t.requires_grad and
-            not torch._C._functorch.is_functorch_wrapped_tensor(t) and forward_ad._current_level < 0 and not torch.jit.is_tracing())
+            not torch._C._functorch.is_functorch_wrapped_tensor(t) and not (t.is_conj() or t.is_neg() or t._is_zerotensor()))
 
 
 def _rows(t, dtypes):
@@ -149,6 +158,8 @@ def _rows(t, dtypes):
 def _pack_on_gpu(input_ids, attention_mask, token_type_ids, block_size, keep_width):
     """pack_padded_batch by two kernels; None where the batch has to take the general way: other types or strides, no entries,
     and every mask that is not plain ones and zeros with the ones in front, which the general way refuses or counts."""
+    if _watched():
+        return None
     ints = (torch.int32, torch.int64)
     if not (type(block_size) is int and block_size >= 1 and 1 <= input_ids.shape[0] <= 65535 and input_ids.shape[1] >= 1 and
             _rows(input_ids, ints) and _rows(attention_mask, ints + (torch.bool, torch.uint8))):
@@ -176,7 +187,7 @@ def _pack_on_gpu(input_ids, attention_mask, token_type_ids, block_size, keep_wid
 def _unpacks_on_gpu(packed, starts, seq_lens, seq_tokens, length):
     """Whether the unpacking kernel takes these rows: ordinary ones of whole 16-byte vectors on the current GPU, every
     sequence inside of them and of the padded length.  (The general way has the words for what is wrong otherwise.)"""
-    if not (_ordinary(packed) and packed.dim() == 2 and packed.is_contiguous() and packed.data_ptr() % 16 == 0):
+    if _watched() or not (_ordinary(packed) and packed.dim() == 2 and packed.is_contiguous() and packed.data_ptr() % 16 == 0):
         return False
     row = packed.shape[1] * packed.element_size()
     if row == 0 or row % 16 or row >= 1 << 24 or type(length) is not int or not 1 <= length < 1 << 24 or length * row >= 1 << 37:

@@ -4,6 +4,9 @@ import importlib
 
 import pytest
 import torch
+from torch.fx.experimental.proxy_tensor import make_fx
+from torch.overrides import TorchFunctionMode
+from torch.utils._python_dispatch import TorchDispatchMode
 
 import __graft_entry__ as graft
 
@@ -89,3 +92,61 @@ def test_unpack_refuses_what_the_general_way_refuses(ut, seq_lens, tokens, width
     packed = torch.zeros(128 if len(seq_lens) > 1 else 64, 8, dtype=torch.float16, device="cuda")
     with pytest.raises((RuntimeError, TypeError)):
         ut.unpack_to_padded(packed, seq_lens, tokens, width)
+
+
+class SeenByDispatch(TorchDispatchMode):
+    def __init__(self):
+        super().__init__()
+        self.seen = 0
+
+    def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+        self.seen += 1
+        return func(*args, **(kwargs or {}))
+
+
+class SeenByFunction(TorchFunctionMode):
+    def __init__(self):
+        super().__init__()
+        self.seen = 0
+
+    def __torch_function__(self, func, types, args=(), kwargs=None):
+        self.seen += func is torch.Tensor.__setitem__
+        return func(*args, **(kwargs or {}))
+
+
+def test_unpack_traced_is_the_whole_computation(ut):
+    """What a tracer records, run on other rows, gives their padded batch; the same for a compiled call in one graph."""
+    seq_lens, tokens, width = [128, 64, 64], [70, 64, 1], 100
+    rows = [torch.randn(256, 8, generator=torch.Generator().manual_seed(i)).half() for i in range(2)]
+    call = lambda x: ut.unpack_to_padded(x, seq_lens, tokens, width)
+    torch.empty(3, width, 8, dtype=torch.float16, device="cuda").fill_(float("nan"))
+    graphs = [make_fx(call)(rows[0].cuda()), make_fx(call, pre_dispatch=True)(rows[0].cuda()), torch.jit.trace(call, rows[0].cuda()),
+              torch.compile(call, backend="eager", fullgraph=True)]
+    for graph in graphs:
+        assert torch.equal(graph(rows[1].cuda()).cpu(), call(rows[1]))
+
+
+@pytest.mark.parametrize("mode", [SeenByDispatch, SeenByFunction])
+def test_modes_see_the_operators(ut, mode):
+    packed = torch.randn(128, 8, device="cuda").half()
+    ids, mask = torch.arange(120, device="cuda").view(2, 60), mask_of([60, 3], 60, torch.int64).cuda()
+    with mode() as m:
+        out = ut.unpack_to_padded(packed, [64, 64], [60, 3], 64)
+        unpacked = m.seen
+        batch = ut.pack_padded_batch(ids, mask)
+    assert unpacked >= 2 and (mode is SeenByFunction or m.seen > unpacked + 2)
+    assert torch.equal(out, ut.unpack_to_padded(packed, [64, 64], [60, 3], 64))
+    assert torch.equal(batch["input_ids"], ut.pack_padded_batch(ids, mask)["input_ids"])
+
+
+def test_default_device_is_no_mode(ut):
+    with torch.device("cuda"):
+        assert not ut._watched()
+
+
+@pytest.mark.parametrize("lazy", ["conj", "neg", "zero"])
+def test_unpack_of_lazy_tensors(ut, lazy):
+    x = torch.randn(128, 8, dtype=torch.complex64 if lazy == "conj" else torch.float32)
+    make = {"conj": lambda t: t.conj(), "neg": torch._neg_view, "zero": lambda t: torch._efficientzerotensor(t.shape, device=t.device)}[lazy]
+    got = ut.unpack_to_padded(make(x.cuda()), [64, 64], [64, 5], 70)
+    assert torch.equal(got.cpu().resolve_conj().resolve_neg(), ut.unpack_to_padded(make(x), [64, 64], [64, 5], 70).resolve_conj().resolve_neg())
