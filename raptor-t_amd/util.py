@@ -184,23 +184,28 @@ def _pack_on_gpu(input_ids, attention_mask, token_type_ids, block_size, keep_wid
             "seq_tokens_tensor": tokens}
 
 
-def _unpacks_on_gpu(packed, starts, seq_lens, seq_tokens, length):
-    """Whether the unpacking kernel takes these rows: ordinary ones of whole 16-byte vectors on the current GPU, every
-    sequence inside of them and of the padded length.  (The general way has the words for what is wrong otherwise.)"""
+def _starts_on_gpu(packed, seq_lens, seq_tokens, length):
+    """First rows of the sequences where the unpacking kernel takes them: ordinary rows of whole 16-byte vectors on the current
+    GPU, every sequence inside of them and of the padded length; else None.  (The general way takes any iterable of counts, and has
+    the words for what is wrong.)"""
     if _watched() or not (_ordinary(packed) and packed.dim() == 2 and packed.is_contiguous() and packed.data_ptr() % 16 == 0):
-        return False
+        return None
+    if not (isinstance(seq_lens, (list, tuple)) and isinstance(seq_tokens, (list, tuple)) and len(seq_lens) == len(seq_tokens) >= 1 and
+            all(type(n) is int for n in (*seq_lens, *seq_tokens))):
+        return None
     row = packed.shape[1] * packed.element_size()
     if row == 0 or row % 16 or row >= 1 << 24 or type(length) is not int or not 1 <= length < 1 << 24 or length * row >= 1 << 37:
-        return False
-    return (len(starts) >= 1 and len(seq_lens) == len(seq_tokens) and all(type(n) is int for n in (*seq_lens, *seq_tokens)) and
-            all(n >= 0 and 0 <= t <= length and s + t <= packed.shape[0] for s, n, t in zip(starts, seq_lens, seq_tokens)))
+        return None
+    starts = list(itertools.accumulate(seq_lens, initial=0))[:-1]
+    inside = all(n >= 0 and 0 <= t <= length and s + t <= packed.shape[0] for s, n, t in zip(starts, seq_lens, seq_tokens))
+    return starts if inside else None
 
 
 def unpack_to_padded(packed, seq_lens, seq_tokens, length):
     """[T, D] packed encoder output -> [B, length, D] with zeros on the padded positions (the padded rows of
     the packed output are whatever the layers computed for padding tokens and are dropped here)."""
-    starts = list(itertools.accumulate(seq_lens, initial=0))[:-1]
-    if _unpacks_on_gpu(packed, starts, seq_lens, seq_tokens, length):
+    starts = _starts_on_gpu(packed, seq_lens, seq_tokens, length)
+    if starts is not None:
         out = torch.empty(len(seq_lens), length, packed.shape[1], dtype=packed.dtype, device=packed.device)
         return capi.unpack_rows(packed, starts, seq_tokens, out)
     out = packed.new_zeros(len(seq_lens), length, packed.shape[1])

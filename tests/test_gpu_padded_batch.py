@@ -150,3 +150,10 @@ def test_unpack_of_lazy_tensors(ut, lazy):
     make = {"conj": lambda t: t.conj(), "neg": torch._neg_view, "zero": lambda t: torch._efficientzerotensor(t.shape, device=t.device)}[lazy]
     got = ut.unpack_to_padded(make(x.cuda()), [64, 64], [64, 5], 70)
     assert torch.equal(got.cpu().resolve_conj().resolve_neg(), ut.unpack_to_padded(make(x), [64, 64], [64, 5], 70).resolve_conj().resolve_neg())
+
+
+def test_unpack_takes_any_iterable_of_counts(ut):
+    packed = torch.randn(128, 8)
+    want = ut.unpack_to_padded(packed, [64, 64], [64, 5], 70)
+    for tokens in (iter([64, 5]), (n for n in (64, 5)), torch.tensor([64, 5]), [64, 5, 9]):
+        assert torch.equal(ut.unpack_to_padded(packed.cuda(), [64, 64], tokens, 70).cpu(), want)
