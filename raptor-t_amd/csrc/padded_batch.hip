@@ -6,49 +6,47 @@
 // around a model call of 1.75 ms (8 sequences of 150-1700 tokens).
 #include <hip/hip_runtime.h>
 
+#include <climits>
+
 #include "rt_launch.h"
 
 namespace {
 
 constexpr int PACK_THREADS = 256;
 
-// One workgroup per sequence: its token count, or -1 where the mask is not ones on a prefix of the row.  A row qualifies if
-// its nonzero entries are as many as their sum and the last of them lies right there.
+// One workgroup per sequence: its token count, or -1 where the mask is not ones on a prefix of the row and zeros behind it.  A row
+// qualifies if no entry is another number and its ones are as many as the place of the last of them.
 template <typename T>
 __global__ __launch_bounds__(PACK_THREADS) void padded_tokens_kernel(const T* __restrict__ mask, int64_t row_stride, int64_t width,
                                                                     int* __restrict__ tokens) {
-  __shared__ long long sums[PACK_THREADS / 64];
   __shared__ int counts[PACK_THREADS / 64], ends[PACK_THREADS / 64];
   const T* const row = mask + blockIdx.x * row_stride;
-  long long sum = 0;
   int count = 0, end = 0;
   for (int64_t i = threadIdx.x; i < width; i += PACK_THREADS) {
     const T v = row[i];
-    sum += v;
-    if (v != 0) {
+    if (v == 1) {
       ++count;
-      end = int(i) + 1;
+      end = max(end, int(i) + 1);
+    } else if (v != 0) {
+      end = INT_MAX;                                   // no row has as many ones
     }
   }
 #pragma unroll
   for (int d = 32; d > 0; d >>= 1) {
-    sum += __shfl_xor(sum, d, 64);
     count += __shfl_xor(count, d, 64);
     end = max(end, __shfl_xor(end, d, 64));
   }
   if ((threadIdx.x & 63) == 0) {
-    sums[threadIdx.x >> 6] = sum;
     counts[threadIdx.x >> 6] = count;
     ends[threadIdx.x >> 6] = end;
   }
   __syncthreads();
   if (threadIdx.x == 0) {
     for (int w = 1; w < PACK_THREADS / 64; ++w) {
-      sum += sums[w];
       count += counts[w];
       end = max(end, ends[w]);
     }
-    tokens[blockIdx.x] = sum == count && end == count ? count : -1;
+    tokens[blockIdx.x] = end == count ? count : -1;
   }
 }
 

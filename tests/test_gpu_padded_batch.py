@@ -43,7 +43,7 @@ def test_pack_equals_the_general_way(ut, lens, width, ids_dtype, mask_dtype, typ
         assert torch.equal(got[name].cpu(), want[name]), name
 
 
-@pytest.mark.parametrize("change", ["hole", "empty", "left", "values", "float", "transposed"])
+@pytest.mark.parametrize("change", ["hole", "empty", "left", "values", "negative", "float", "transposed"])
 def test_pack_odd_masks_as_the_general_way(ut, change):
     """What the general way refuses is refused, what it accepts gives the same batch."""
     ids = torch.arange(3 * 200).view(3, 200) + 1
@@ -56,6 +56,8 @@ def test_pack_odd_masks_as_the_general_way(ut, change):
         mask = mask.flip(1)
     elif change == "values":                        # the sum of the entries counts: 100 places hold a token, 2 more are claimed
         mask[1, :2] = 2
+    elif change == "negative":                      # as many nonzero entries as their sum, the last of them there: accepted
+        mask[1, :2] = torch.tensor([3, -1])
     elif change == "float":
         mask = mask.float()
     elif change == "transposed":
@@ -71,6 +73,26 @@ def test_pack_odd_masks_as_the_general_way(ut, change):
         assert got == want
     else:
         assert got["seq_tokens"] == want["seq_tokens"] and torch.equal(got["input_ids"].cpu(), want["input_ids"])
+
+
+@pytest.mark.parametrize("dtype", [torch.bool, torch.uint8, torch.int8, torch.int32, torch.int64])
+def test_padded_tokens_counts_ones(dtype):
+    """The entry point by itself: -1 for every row that holds other numbers than ones in front and zeros behind them."""
+    capi = graft.load_package().capi
+    rows = [[1] * 300, [0] * 300, [1] * 7 + [0] * 293, [0, 1] + [0] * 298, [1] * 256 + [0] + [1] * 43, [1] * 299 + [0]]
+    want = [300, 0, 7, -1, -1, 299]
+    if dtype != torch.bool:
+        rows += [[2, 0] + [0] * 298, [1] * 100 + [0] * 199 + [2]]
+        want += [-1, -1]
+    if dtype in (torch.int8, torch.int32, torch.int64):
+        rows += [[3, -1, 1, 0] + [0] * 296, [-1] * 300, [2, 0] + [1] * 298]
+        want += [-1, -1, -1]
+    if dtype == torch.int64:
+        rows += [[1 << 32] + [0] * 299, [(1 << 32) + 1] + [0] * 299]
+        want += [-1, -1]
+    tokens = torch.full((len(rows),), -7, dtype=torch.int32, device="cuda")
+    capi.padded_tokens(torch.tensor(rows).to(dtype).cuda(), tokens)
+    assert tokens.tolist() == want
 
 
 @pytest.mark.parametrize("lens,width", [([1], 1), ([64, 1, 63, 65], 65), ([130, 64, 1], 150), ([0, 5, 0], 9), ([700, 3], 1100),
