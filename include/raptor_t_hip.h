@@ -219,6 +219,10 @@ int rt_bs_attention_fwd_qrows(const void* qkv, const void* qkv_bias, float q_sca
                               const int* from_idx, const int* from_pos, int n_wg, int dtype,
                               void* stream);
 
+/* How a launch of the 16-bit types cuts its rows: the shares that the tiles of a row which is not a global one (first or last
+ * block of a sparse sequence) and of one which is are dealt to, and the waves of a workgroup of the launch without a plan. */
+int rt_bs_attention_cut(int batch, int total_blocks, int heads, int* others, int* global, int* waves);
+
 /* rt_bs_attention_fwd_masked for callers that cannot allocate device memory (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc).  It has no counterpart in the
  * reference.  Its limits are stated as constants; it takes no from_idx/from_pos plan.  (None of the attention entry points

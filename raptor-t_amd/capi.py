@@ -24,7 +24,7 @@ EXPORTS = [
     "rt_last_error_string", "rt_abi_version", "rt_time_next_launch", "rt_meta_np_permutations", "rt_meta_seq_prefix_blocks",
     "rt_meta_rand_attn", "rt_meta_set_plan_cache", "rt_meta_to_index_size", "rt_meta_build_to_index", "rt_meta_block_costs",
     "rt_meta_partition_lpt", "rt_meta_check_partition", "rt_meta_check_to_index", "rt_qkv_bias_split", "rt_qkv_project", "rt_unpack_head_tiles", "rt_bs_attention_fwd",
-    "rt_bs_attention_fwd_masked", "rt_bs_attention_fwd_qrows", "rt_bs_attention_fwd_no_alloc",
+    "rt_bs_attention_fwd_masked", "rt_bs_attention_fwd_qrows", "rt_bs_attention_fwd_no_alloc", "rt_bs_attention_cut",
     "rt_bias_residual_layernorm", "rt_bias_gelu", "rt_embed_layernorm", "rt_gemm_create", "rt_gemm_destroy", "rt_gemm_set_tuning", "rt_gemm_set_retuning", "rt_gemm",
     "rt_gemm_bias_act", "rt_gemm_bt", "rt_gemm_bt_slices", "rt_gemm_bt_tile", "rt_slices_residual_layernorm", "rt_sequence_pool", "rt_pooler_dense_tanh",
     "rt_padded_tokens", "rt_pack_tokens", "rt_unpack_rows",
@@ -70,6 +70,7 @@ def lib():
         L.rt_bs_attention_fwd_masked.argtypes = [vp, vp, vp, vp, vp, vp, I, I, I, vp, vp, I, vp, vp, I, I, vp]
         L.rt_bs_attention_fwd_qrows.argtypes = [vp, vp, F, vp, vp, vp, vp, vp, I, I, I, vp, vp, I, vp, vp, I, I, vp]
         L.rt_bs_attention_fwd_no_alloc.argtypes = [vp, vp, vp, vp, vp, vp, I, I, I, vp, vp, I, I, vp]
+        L.rt_bs_attention_cut.argtypes = [I, I, I, i32p, i32p, i32p]
         L.rt_bias_residual_layernorm.argtypes = [vp, vp, vp, vp, vp, L64, I, F, I, vp]
         L.rt_bias_gelu.argtypes = [vp, vp, L64, I, I, vp]
         L.rt_gemm_create.argtypes = [ctypes.POINTER(vp)]
@@ -298,6 +299,13 @@ def bs_attention_fwd(q, k, vt, out, seq_blocks_dev, heads, to_idx, to_pos, plan_
     check(lib().rt_bs_attention_fwd_masked(_dp(q), _dp(k), _dp(vt), _dp(out), _dp(seq_blocks_dev), _dp(seq_tokens_dev),
                                            batch, nb, heads, _dp(to_idx), _dp(to_pos), plan_heads, _dp(from_idx),
                                            _dp(from_pos), n_wg, _dtype_code(out), _stream()))
+
+
+def bs_attention_cut(batch, total_blocks, heads):
+    """(shares of a row, shares of a global row, waves of a workgroup) of a launch in a 16-bit type."""
+    cut = [ctypes.c_int() for _ in range(3)]
+    check(lib().rt_bs_attention_cut(batch, total_blocks, heads, *(ctypes.byref(c) for c in cut)))
+    return tuple(c.value for c in cut)
 
 
 def bs_attention_fwd_no_alloc(q, k, vt, out, seq_blocks_dev, heads, to_idx, to_pos, plan_heads, seq_tokens_dev=None):

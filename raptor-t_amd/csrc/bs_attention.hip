@@ -1195,16 +1195,27 @@ int64_t most_pairs(int batch, int total_blocks, int heads) {
 // 37.2 / 37.6 / 37.6, 1 x 12288 55.7 / 50.8 / 52.0 / 48.0.
 struct Cut { int others, global, waves; };
 Cut cut_rows(int batch, int total_blocks, int heads) {
-  if (batch > 64) return {1, 4, 4};
-  const int64_t units = int64_t(total_blocks) * heads, global = 2 * most_pairs(batch, total_blocks, heads);
+  const Cut four{1, 4, 4}, eight{1, 8, 8};
+  if (batch > 64) return four;
+  const int64_t units = int64_t(total_blocks) * heads, pairs = most_pairs(batch, total_blocks, heads), global = 2 * pairs;
   const int longest = total_blocks - batch + 1;         // tiles that a row can have at most
+  const int likely = batch == 1 ? total_blocks : 3 * total_blocks / (2 * batch);
+  const bool one_round = global + (units - global) / 8 <= 256;                        // of workgroups of 8 waves
+  // Few units of long sequences: the global rows' chain is all of the time (f16, 4 4 4 / 2 4 4 / 1 8 8: 1 head 1 x 14080 tokens 38.3 / 38.0 /
+  // 33.5, 2 heads 9920 + 64 29.6 / 28.3 / 25.6, 1 x 8192 25.4 / 23.9 / 22.1; 1 head 1 x 3840 13.2 / 13.3 / 13.4, 2 x 3200 12.8 / 12.7 / 13.5).
+  if (likely > 75 && one_round) return eight;
   if (longest >= 3 && units <= 256) return {4, 4, 4};
   if (longest >= 2 && global + (units - global) / 2 <= 220) return {2, 4, 4};
-  const int likely = batch == 1 ? total_blocks : 3 * total_blocks / (2 * batch);
-  // one round of workgroups, or a single sequence whose chain, 5 us and 0.25 a tile, outlasts the units' 17 ns each
-  if (likely >= 60 && (global + (units - global) / 8 <= 256 || (batch == 1 && 5 + 0.25 * longest > 0.0167 * double(units))))
-    return {1, 8, 8};
-  return {1, 4, 4};
+  if (likely >= 60 && one_round) return eight;
+  // From about 1050 units on a round of workgroups of 8 waves takes as long as the same work by 4, whatever the lengths, and a
+  // sequence much longer than the others is done earlier (f16, 1 4 4 / 1 8 8: 12 heads 3 x 1920 tokens 16.6 / 17.0, 4 heads 10 x 1728 14.9 / 15.4, 6
+  // heads 7 x 1920 16.0 / 16.1; 4 heads 16000 + 9 x 128 50.1 / 42.4, 9600 + 11 x 896 33.6 / 27.5).  32 CUs to an XCD, as launch_rows deals them.
+  if (units >= 1056 && 2 * ((pairs + 7) / 8) + ((units + 7) / 8 + 7) / 8 <= 32) return eight;
+  // more rounds, and a chain, 5 us and 0.25 a tile, that outlasts the units' 17 ns each (f16, 1 4 4 / 1 8 8: 12 heads 12800 + 1280 tokens 50.0 /
+  // 41.0, 8 heads 2 x 11520 48.8 / 39.4, 4 heads 5 x 8192 38.7 / 35.3, 12 heads 2 x 7040 36.4 / 36.6; on the line 12 heads 2 x 8960 46.3 / 49.0; 4 heads
+  // 5 x 5760 29.3 / 32.0, whose second round is nearly empty)
+  if (likely >= 60 && 5 + 0.25 * likely > (batch == 1 ? 0.0167 : 0.0174) * double(units)) return eight;
+  return four;
 }
 
 template <typename T> int launch_rows(const Args<T>& a, int n_wg, hipStream_t st) {
@@ -1302,6 +1313,17 @@ extern "C" int rt_bs_attention_fwd(const void* q, const void* k, const void* vt,
                                    void* stream) {
   return rt_bs_attention_fwd_masked(q, k, vt, out, seq_blocks_dev, nullptr, batch, total_blocks, heads, to_idx, to_pos,
                                     plan_heads, from_idx, from_pos, n_wg, dtype, stream);
+}
+
+extern "C" int rt_bs_attention_cut(int batch, int total_blocks, int heads, int* others, int* global, int* waves) {
+  RT_REQUIRE(others && global && waves, RT_EINVAL, "NULL pointer");
+  RT_REQUIRE(batch >= 1 && total_blocks >= batch && heads >= 1, RT_EINVAL, "bad geometry: batch=%d total_blocks=%d heads=%d",
+             batch, total_blocks, heads);
+  const Cut cut = cut_rows(batch, total_blocks, heads);
+  *others = cut.others;
+  *global = cut.global;
+  *waves = cut.waves;
+  return RT_OK;
 }
 
 static_assert(RT_NO_ALLOC_MAX_BATCH <= MAX_BATCH && RT_NO_ALLOC_MAX_BLOCKS <= MAX_BLOCKS, "header limits exceed the kernel's");

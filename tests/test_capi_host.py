@@ -288,3 +288,23 @@ def test_padded_batch_adapters_round_trip():
         ut.pack_padded_batch(ids, torch.tensor([[1, 0, 1]]).expand(3, 3)[:, :3].repeat(1, 50))   # holes in the mask
     with pytest.raises(ValueError):
         ut.pack_padded_batch(ids, torch.zeros_like(mask))
+
+
+@pytest.mark.parametrize("heads,blocks,cut", [
+    # one long sequence, or one much longer than the others: its global rows' chain is the time of the launch
+    (4, [300, 300], (1, 8, 8)), (4, [300] + [2] * 9, (1, 8, 8)), (1, [300], (1, 8, 8)), (3, [300] * 3, (1, 8, 8)), (9, [300, 4], (1, 8, 8)),
+    (6, [300, 100], (1, 8, 8)), (12, [200, 20], (1, 8, 8)), (8, [256, 40, 40], (1, 8, 8)), (2, [155, 1], (1, 8, 8)),
+    (1, [220], (1, 8, 8)), (4, [250] + [2] * 9, (1, 8, 8)), (4, [128] * 5, (1, 8, 8)), (1, [128] * 16, (1, 8, 8)),
+    # the others as they were
+    (12, [1], (1, 4, 4)), (12, [3], (4, 4, 4)), (12, [8], (4, 4, 4)), (12, [24], (2, 4, 4)), (12, [40], (1, 4, 4)), (12, [64], (1, 8, 8)),
+    (12, [4, 16, 10, 14], (1, 4, 4)), (12, [64] * 8, (1, 4, 4)), (16, [200], (1, 8, 8)), (16, [256] * 4, (1, 4, 4)), (12, [8] * 16, (1, 4, 4)),
+    (1, [300] + [1] * 64, (1, 4, 4)), (1, [13] * 65, (1, 4, 4)),
+])
+def test_attention_cuts_rows(capi, heads, blocks, cut):
+    assert capi.bs_attention_cut(len(blocks), sum(blocks), heads) == cut
+
+
+def test_attention_cut_refuses_bad_geometry(capi):
+    for args in ((0, 1, 1), (2, 1, 1), (1, 1, 0)):
+        with pytest.raises(capi.RaptorError):
+            capi.bs_attention_cut(*args)
