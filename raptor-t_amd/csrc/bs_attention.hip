@@ -1081,6 +1081,21 @@ __device__ __forceinline__ void share_rows(const Args<T>& a, const Buffers<T>& b
   }
 }
 
+// share_rows as the launch's cut has it.  Four shares of a row of more than 256 tiles would be longer than the pipelined loop
+// takes: such a global row has eight, two to a wave (f16, us, moving-maximum loop / so: 16 heads 1 x 20480 tokens 114.5 / 88.3, 4 heads
+// 19200 + 30 x 640 98.0 / 72.0, 1 head 16448 + 8 x 640 116.8 / 52.8).  Beyond 512 tiles the moving-maximum loop has them still.
+constexpr int FOUR_SHARES = 4 * 64;
+template <typename T, bool MASKED, int OTHERS, int GLOBAL, int NW>
+__device__ __forceinline__ void cut_rows_of(const Args<T>& a, const Buffers<T>& b, Room<T, NW>& room, const QSide<T>& qbias, const Unit& u,
+                                            bool global, bool valid, int lane, int wave) {
+  if constexpr (OTHERS < GLOBAL) {
+    if (!global) return share_rows<T, MASKED, OTHERS, NW>(a, b, room, qbias, u, valid, lane, wave);
+    if constexpr (GLOBAL == 4)
+      if (u.n > FOUR_SHARES) return share_rows<T, MASKED, 8, NW>(a, b, room, qbias, u, valid, lane, wave);
+  }
+  share_rows<T, MASKED, GLOBAL, NW>(a, b, room, qbias, u, valid, lane, wave);
+}
+
 // Workgroup b looks its rows up from the batch's prefix, XCD x taking the x-th eighth of the global rows and then of the rest, both
 // head-major: the K / V^T tiles of a (sequence, head) are fetched into one L2.  A global row is a workgroup's, its tiles in
 // GLOBAL shares; of the others it takes NW / OTHERS, each in OTHERS shares.  Nothing persists and nothing is drawn: as its waves
@@ -1120,8 +1135,7 @@ __global__ __launch_bounds__(64 * NW, 2) void bs_attention_kernel(Args<T> a) {
   }
   __syncthreads();
   const Buffers<T> b = buffers_of(a);
-  if (OTHERS < GLOBAL && !global) share_rows<T, MASKED, OTHERS, NW>(a, b, room, qbias, u, valid, batch.lane, wave);
-  else share_rows<T, MASKED, GLOBAL, NW>(a, b, room, qbias, u, valid, batch.lane, wave);
+  cut_rows_of<T, MASKED, OTHERS, GLOBAL, NW>(a, b, room, qbias, u, global, valid, batch.lane, wave);
 }
 
 // With a caller's plan workgroup c walks its slice: four waves, two workgroups per CU, a global row by all of them, other
@@ -1171,8 +1185,7 @@ __global__ __launch_bounds__(256, 2) void bs_attention_plan_kernel(Args<T> a) {
     asm volatile("" : "+v"(lane));
     if (threadIdx.x < 8) room.failed(threadIdx.x) = 0;           // (the last rows' flags were read several barriers ago)
     __syncthreads();
-    if (OTHERS < GLOBAL && !whole) share_rows<T, MASKED, OTHERS, 4>(a, b, room, qbias, u, SIDE * wave / 4 < run, lane, wave);
-    else share_rows<T, MASKED, GLOBAL, 4>(a, b, room, qbias, u, true, lane, wave);
+    cut_rows_of<T, MASKED, OTHERS, GLOBAL, 4>(a, b, room, qbias, u, whole, whole || SIDE * wave / 4 < run, lane, wave);
     p += run;
   }
 }

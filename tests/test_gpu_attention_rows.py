@@ -31,7 +31,12 @@ def capi():
     (6, [90], 40.0, 30),
     (6, [100, 12, 90], 1.0, 1),
     (1, [600], 1.0, 0),                    # 75 tiles to a wave of a global row: the moving-maximum loop
-    (1, [300] + [1] * 64, 1.0, 2),         # the same with four waves; more sequences than lanes
+    (1, [300] + [1] * 64, 1.0, 2),         # two shares of 38 tiles to each of four waves; more sequences than lanes
+    (2, [300] + [10] * 30, 1.0, 0),        # the same with 31 sequences
+    (2, [300] + [10] * 30, 40.0, 9),       # beyond the pipelined loop's range
+    (1, [257] + [10] * 8, 1.0, 4),         # with two waves to the other rows, at the shortest sequence that takes them so
+    (1, [256] + [10] * 8, 1.0, 4),         # 64 tiles to each of four waves
+    (1, [600] + [1] * 64, 1.0, 1),         # 75 tiles to a share: the moving-maximum loop
     (2, [1 + i % 14 for i in range(65)], 1.0, 3),
     (1, [12 + i % 3 for i in range(130)], 40.0, 3),        # three chunks, every sequence with global rows
 ])
