@@ -777,20 +777,34 @@ template <typename T, int NW> struct Room {
   __device__ __forceinline__ int& failed(int row) { return reinterpret_cast<int&>(slots[NW - 1][row * SLOT_PITCH + 64]); }
 };
 
-// Lane l: where sequences l, l + 64, ... of the batch begin and end (CHUNKS of them).  Also fills the bias copy and clears the
-// flags; the caller's barrier follows.
+// The bias copy and cleared flags; the caller's barrier follows.
+template <typename T, int NW> __device__ __forceinline__ void ready_room(const Args<T>& a, Room<T, NW>& room) {
+  if (a.q_rows)
+    for (int i = threadIdx.x; i < a.heads * 64; i += 64 * NW) room.qbias[i] = a.q_bias ? a.q_bias[i] : static_cast<T>(0.f);
+  if (threadIdx.x < 8) room.failed(threadIdx.x) = 0;
+}
+
+// Padding of sequence s, which has u.n blocks
+template <typename T, bool MASKED> __device__ __forceinline__ void set_padding(const Args<T>& a, int s, Unit& u) {
+  u.tail = 64;
+  u.nbv = u.n;
+  if (MASKED) {
+    const int tokens = min(max(__builtin_amdgcn_readfirstlane(a.seq_tokens[s]), 1), 64 * u.n);
+    u.nbv = (tokens + 63) >> 6;
+    u.tail = tokens - 64 * (u.nbv - 1);
+  }
+}
+
+// Lane l: where sequences l, l + 64, ... of the batch begin and end (CHUNKS of them).
 template <typename T, int CHUNKS> struct Batch {
   int lane, sb0[CHUNKS], sb1[CHUNKS];
-  template <int NW> __device__ __forceinline__ Batch(const Args<T>& a, Room<T, NW>& room) {
+  __device__ __forceinline__ explicit Batch(const Args<T>& a) {
     lane = threadIdx.x & 63;
 #pragma unroll
     for (int c = 0; c < CHUNKS; ++c) {
       sb0[c] = a.seq_blocks[min(64 * c + lane, a.batch)];
       sb1[c] = a.seq_blocks[min(64 * c + lane + 1, a.batch)];
     }
-    if (a.q_rows)
-      for (int i = threadIdx.x; i < a.heads * 64; i += 64 * NW) room.qbias[i] = a.q_bias ? a.q_bias[i] : static_cast<T>(0.f);
-    if (threadIdx.x < 8) room.failed(threadIdx.x) = 0;
   }
   // which sequences of chunk c there are, and which have global rows
   __device__ __forceinline__ unsigned long long there(const Args<T>& a, int c) const { return __ballot(64 * c + lane < a.batch); }
@@ -810,13 +824,7 @@ template <typename T, int CHUNKS> struct Batch {
     u.n = __builtin_amdgcn_readlane(sb1[c], l) - u.g0;
     u.h = h;
     u.i = i;
-    u.tail = 64;
-    u.nbv = u.n;
-    if (MASKED) {
-      const int tokens = min(max(__builtin_amdgcn_readfirstlane(a.seq_tokens[64 * c + l]), 1), 64 * u.n);
-      u.nbv = (tokens + 63) >> 6;
-      u.tail = tokens - 64 * (u.nbv - 1);
-    }
+    set_padding<T, MASKED>(a, 64 * c + l, u);
     return u;
   }
   // the first row of the k-th sequence that has global rows
@@ -850,19 +858,50 @@ template <typename T, int CHUNKS> struct Batch {
     }
     return u;
   }
-  // the unit with the plan's id blk + head * n + first block * heads
-  template <bool MASKED> __device__ __forceinline__ Unit flat_unit(const Args<T>& a, int id) const {
+};
+
+// The units of a caller's plan, whose ids are blk + head * n + first block * heads, in a batch of up to 64 sequences: lane l
+// knows where sequence l begins and ends.
+template <typename T> struct UnitsOfFew {
+  struct Place {};
+  Batch<T, 1> batch;
+  __device__ __forceinline__ explicit UnitsOfFew(const Args<T>& a) : batch(a) {}
+  __device__ __forceinline__ Place place(const Args<T>&, int) const { return {}; }
+  template <bool MASKED> __device__ __forceinline__ Unit unit(const Args<T>& a, const Place&, int id) const {
     Unit u{};
-    bool found = false;
-#pragma unroll
-    for (int c = 0; c < CHUNKS; ++c)
-      if (!found && id < __builtin_amdgcn_readlane(sb1[c], 63) * a.heads) {
-        const int l = __popcll(there(a, c) & __ballot(sb0[c] * a.heads <= id)) - 1;
-        const int g0 = __builtin_amdgcn_readlane(sb0[c], l), n = __builtin_amdgcn_readlane(sb1[c], l) - g0;
-        const int rem = id - g0 * a.heads, h = rem / n;
-        u = unit_at<MASKED>(a, c, l, h, rem - h * n);
-        found = true;
-      }
+    if (id >= __builtin_amdgcn_readlane(batch.sb1[0], 63) * a.heads) return u;
+    const int l = __popcll(batch.there(a, 0) & __ballot(batch.sb0[0] * a.heads <= id)) - 1;
+    const int g0 = __builtin_amdgcn_readlane(batch.sb0[0], l), n = __builtin_amdgcn_readlane(batch.sb1[0], l) - g0;
+    const int rem = id - g0 * a.heads, h = rem / n;
+    return batch.template unit_at<MASKED>(a, 0, l, h, rem - h * n);
+  }
+};
+// The same in a batch of up to 1024: lane l knows where sequence 16 l begins, and the 16 that a unit may be of are looked up
+// (place requests them, unit waits).  All 1024 in the lanes are 32 registers that the pipelined loop does not have: it
+// spilled 47-66 (12 heads into 512, us, before / now: 65 sequences of 1-20 blocks f16 130 / 120, bf16 padded 144 / 122; 100 of 3 blocks 37.9 / 29.3).
+template <typename T> struct UnitsOfMany {
+  struct Place { int first, begins; };                 // lane l: where sequence first + l begins
+  static_assert(MAX_BATCH <= 64 * 16, "a lane for every 16 sequences");
+  int lane, begins16, total;
+  __device__ __forceinline__ explicit UnitsOfMany(const Args<T>& a) {
+    lane = threadIdx.x & 63;
+    begins16 = a.seq_blocks[min(16 * lane, a.batch)];
+    total = __builtin_amdgcn_readfirstlane(a.seq_blocks[a.batch]);
+  }
+  __device__ __forceinline__ Place place(const Args<T>& a, int id) const {
+    const int first = max(16 * __popcll(__ballot(16 * lane < a.batch && begins16 * a.heads <= id)) - 16, 0);
+    return {first, a.seq_blocks[min(first + lane, a.batch)]};
+  }
+  template <bool MASKED> __device__ __forceinline__ Unit unit(const Args<T>& a, const Place& p, int id) const {
+    Unit u{};
+    if (id >= total * a.heads) return u;
+    const int l = __popcll(__ballot(lane < 16 && p.first + lane < a.batch && p.begins * a.heads <= id)) - 1;
+    u.g0 = __builtin_amdgcn_readlane(p.begins, l);
+    u.n = __builtin_amdgcn_readlane(p.begins, l + 1) - u.g0;
+    const int rem = id - u.g0 * a.heads;
+    u.h = rem / u.n;
+    u.i = rem - u.h * u.n;
+    set_padding<T, MASKED>(a, p.first + l, u);
     return u;
   }
 };
@@ -1091,9 +1130,10 @@ __device__ __forceinline__ void cut_rows_of(const Args<T>& a, const Buffers<T>& 
   if constexpr (OTHERS < GLOBAL) {
     if (!global) return share_rows<T, MASKED, OTHERS, NW>(a, b, room, qbias, u, valid, lane, wave);
     if constexpr (GLOBAL == 4)
-      if (u.n > FOUR_SHARES) return share_rows<T, MASKED, 8, NW>(a, b, room, qbias, u, valid, lane, wave);
+      if (u.n > FOUR_SHARES) return share_rows<T, MASKED, 8, NW>(a, b, room, qbias, u, true, lane, wave);
   }
-  share_rows<T, MASKED, GLOBAL, NW>(a, b, room, qbias, u, valid, lane, wave);
+  static_assert(GLOBAL >= NW, "one row to the workgroup: it is there");
+  share_rows<T, MASKED, GLOBAL, NW>(a, b, room, qbias, u, true, lane, wave);
 }
 
 // Workgroup b looks its rows up from the batch's prefix, XCD x taking the x-th eighth of the global rows and then of the rest, both
@@ -1109,7 +1149,8 @@ __global__ __launch_bounds__(64 * NW, 2) void bs_attention_kernel(Args<T> a) {
   constexpr int ROWS = NW / OTHERS;
   __shared__ Room<T, NW> room;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const Batch<T, CHUNKS> batch(a, room);
+  const Batch<T, CHUNKS> batch(a);
+  ready_room<T, NW>(a, room);
   const QSide<T> qbias{room.qbias, room.stage(wave)};
   const int n_sparse = batch.sparse_count(a), n_rows = a.nb_total - 2 * n_sparse;
   const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
@@ -1143,7 +1184,7 @@ __global__ __launch_bounds__(64 * NW, 2) void bs_attention_kernel(Args<T> a) {
 // the bits are the same; a wave takes two of a global row's eight, or one of its four.  The slice is clamped to the list, ids
 // outside it are skipped.  An LPT plan spreads each (sequence, head) over many XCDs: 8 x 4096 tokens into 512 95 us, without a plan
 // 74; 16 x 512-4096 into 1024 116 / 84.
-template <typename T, bool MASKED, int OTHERS, int GLOBAL, int CHUNKS>
+template <typename T, bool MASKED, int OTHERS, int GLOBAL, bool MANY>
 __global__ __launch_bounds__(256, 2) void bs_attention_plan_kernel(Args<T> a) {
   constexpr int SIDE = OTHERS < 4 ? 4 / OTHERS : 1;    // rows side by side
   __shared__ Room<T, 4> room;
@@ -1152,7 +1193,8 @@ __global__ __launch_bounds__(256, 2) void bs_attention_plan_kernel(Args<T> a) {
   const int begin = min(max(a.from_pos[blockIdx.x], 0), n_units);
   const int end = min(max(a.from_pos[blockIdx.x + 1], begin), n_units);
   if (begin == end) return;
-  const Batch<T, CHUNKS> batch(a, room);
+  const std::conditional_t<MANY, UnitsOfMany<T>, UnitsOfFew<T>> units(a);
+  ready_room<T, 4>(a, room);
   const QSide<T> qbias{room.qbias, room.stage(wave)};
   const Buffers<T> b = buffers_of(a);
   for (int p = begin; p < end;) {
@@ -1163,7 +1205,10 @@ __global__ __launch_bounds__(256, 2) void bs_attention_plan_kernel(Args<T> a) {
       if (ids[w] >= n_units) ids[w] = -1;
     }
     if (ids[0] < 0) { ++p; continue; }
-    Unit u = batch.template flat_unit<MASKED>(a, ids[0]);
+    decltype(units.place(a, 0)) at[SIDE];
+#pragma unroll
+    for (int w = 0; w < SIDE; ++w) at[w] = units.place(a, max(ids[w], 0));
+    Unit u = units.template unit<MASKED>(a, at[0], ids[0]);
     const bool whole = is_global_row(u);
     int run = 1;
     if (!whole) {
@@ -1173,7 +1218,7 @@ __global__ __launch_bounds__(256, 2) void bs_attention_plan_kernel(Args<T> a) {
       for (int w = 1; w < SIDE; ++w) {
         more = more && ids[w] >= 0;
         if (more) {
-          const Unit v = batch.template flat_unit<MASKED>(a, ids[w]);
+          const Unit v = units.template unit<MASKED>(a, at[w], ids[w]);
           more = !is_global_row(v);
           if (more) ++run;
           if (more && w == mine) u = v;
@@ -1181,11 +1226,11 @@ __global__ __launch_bounds__(256, 2) void bs_attention_plan_kernel(Args<T> a) {
       }
     }
     // what the code below derives from the lane number is derived again for every unit, not kept in registers
-    int lane = batch.lane;
+    int lane = threadIdx.x & 63;
     asm volatile("" : "+v"(lane));
     if (threadIdx.x < 8) room.failed(threadIdx.x) = 0;           // (the last rows' flags were read several barriers ago)
     __syncthreads();
-    cut_rows_of<T, MASKED, OTHERS, GLOBAL, 4>(a, b, room, qbias, u, whole, whole || SIDE * wave / 4 < run, lane, wave);
+    cut_rows_of<T, MASKED, OTHERS, GLOBAL, 4>(a, b, room, qbias, u, whole, SIDE * wave / 4 < run, lane, wave);
     p += run;
   }
 }
@@ -1237,7 +1282,7 @@ template <typename T> int launch_rows(const Args<T>& a, int n_wg, hipStream_t st
     constexpr bool MASKED = decltype(masked)::value;
     constexpr int OTHERS = decltype(others)::value, GLOBAL = decltype(global)::value, NW = decltype(waves)::value, CHUNKS = decltype(chunks)::value;
     if (a.from_pos) {
-      RT_LAUNCH((bs_attention_plan_kernel<T, MASKED, OTHERS, GLOBAL, CHUNKS>), dim3(unsigned(n_wg)), dim3(256), 0, st, a);
+      RT_LAUNCH((bs_attention_plan_kernel<T, MASKED, OTHERS, GLOBAL, (CHUNKS > 1)>), dim3(unsigned(n_wg)), dim3(256), 0, st, a);
       return;
     }
     // every XCD's share of the global rows (two per head of each sequence that may have them) and of the others

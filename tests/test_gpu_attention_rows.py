@@ -39,6 +39,8 @@ def capi():
     (1, [600] + [1] * 64, 1.0, 1),         # 75 tiles to a share: the moving-maximum loop
     (2, [1 + i % 14 for i in range(65)], 1.0, 3),
     (1, [12 + i % 3 for i in range(130)], 40.0, 3),        # three chunks, every sequence with global rows
+    (2, [1] * 80 + [13] + [1] * 15 + [2, 12, 1], 1.0, 0),  # sequences that begin and end a sixteen
+    (1, [1] * 1023 + [14], 1.0, 1),        # the most sequences, the last of them with global rows
 ])
 def test_rows(capi, heads, blocks, scale, short):
     print("rows", heads, blocks[:4], scale, short, flush=True)
