@@ -1,6 +1,6 @@
-"""Block-sparse attention of batches with few units (rows shared by several waves): every number of rows to a
-workgroup, the edges of the rule that picks it, padding, scores that outgrow the pipelined loop's reference, and
-the caller's plan, against the oracle."""
+"""Block-sparse attention of batches with few units, whose rows several waves share: every cut of a row, padding, scores that
+outgrow the pipelined loop's reference, infinities, and the caller's plan, against the oracle.  Each case states the cut it is
+meant for (shares of a row, of a global row, waves of a workgroup) and asks the library for it."""
 import numpy as np
 import pytest
 import torch
@@ -19,25 +19,34 @@ def capi():
     return p.capi
 
 
-@pytest.mark.parametrize("heads,lens,scale", [
-    (1, [64], 1.0),                                   # one row, one tile: seven of its eight waves have none
-    (12, [512], 1.0),                                 # 8 waves to a row
-    (3, [704, 768, 64], 1.0),                         # sequences of 11 and 12 blocks: the last without and the first with global rows
-    (12, [1024, 1088], 1.0),                          # 4 waves to a row
-    (5, [2048, 832, 64], 40.0),                       # scores beyond the pipelined loop's range
-    (12, [256, 1024, 640, 896], 1.0),                 # 2 waves to a row
-    (12, [2048, 3008, 384], 1.0),                     # a wave to a row, global rows by 8 waves
-    (12, [2944, 3008, 2752], 1.0),                    # the two global rows of a head in one workgroup, by 4 waves each
-    (12, [4096, 2624, 1984], 40.0),                   # the same at the longest sequence that takes them so
-    (12, [4160, 2560, 1984], 1.0),                    # one block longer: by 8 waves each, in two rounds
-    (2, [64] * 64, 1.0),                              # as many sequences as lanes
-    (2, [64] * 64 + [128], 1.0),                      # one more
-    (8, [4096 * 4], 1.0),                             # global rows of 256 tiles
-    (11, [64 * 128, 64 * 128], 6.0),                  # 2816 units, the most the rule takes
+def cut_of(capi, heads, lens):
+    return capi.bs_attention_cut(len(lens), sum(lens) // 64, heads)
+
+
+@pytest.mark.parametrize("cut,heads,lens,scale", [
+    ((1, 4, 4), 1, [64], 1.0),                        # one row, one tile: three of the workgroup's waves have no row
+    ((4, 4, 4), 12, [512], 1.0),
+    ((4, 4, 4), 3, [704, 768, 64], 1.0),              # sequences of 11 and 12 blocks: the last without and the first with global rows
+    ((1, 4, 4), 12, [1024, 1088], 1.0),               # two workgroups too many for two waves to a row
+    ((2, 4, 4), 12, [1024, 1024], 1.0),
+    ((4, 4, 4), 5, [2048, 832, 64], 40.0),            # scores beyond the pipelined loop's range
+    ((2, 4, 4), 10, [1664, 512], 40.0),
+    ((1, 8, 8), 6, [5760], 40.0),
+    ((1, 4, 4), 12, [256, 1024, 640, 896], 1.0),
+    ((1, 4, 4), 12, [2048, 3008, 384], 1.0),
+    ((1, 4, 4), 12, [2944, 3008, 2752], 1.0),
+    ((1, 4, 4), 12, [4096, 2624, 1984], 40.0),
+    ((1, 4, 4), 12, [4160, 2560, 1984], 1.0),
+    ((1, 8, 8), 12, [1920] * 3, 1.0),                 # even sequences, one round of workgroups of eight waves
+    ((1, 4, 4), 2, [64] * 64, 1.0),                   # as many sequences as lanes
+    ((1, 4, 4), 2, [64] * 64 + [128], 1.0),           # one more
+    ((1, 8, 8), 8, [4096 * 4], 1.0),                  # global rows of 256 tiles
+    ((1, 8, 8), 11, [64 * 128, 64 * 128], 6.0),       # several rounds, and chains that outlast them
 ])
 @pytest.mark.parametrize("padded", [False, True])
-def test_few_units(capi, heads, lens, scale, padded):
-    print("few units", heads, lens[:4], scale, padded, flush=True)
+def test_few_units(capi, cut, heads, lens, scale, padded):
+    print("few units", cut, heads, lens[:4], scale, padded, flush=True)
+    assert cut_of(capi, heads, lens) == cut
     g = torch.Generator().manual_seed(heads + len(lens))
     t = sum(lens)
     q, k, v = (torch.randn(t, heads, 64, generator=g).half().cuda() for _ in range(3))
@@ -54,22 +63,29 @@ def test_few_units(capi, heads, lens, scale, padded):
         assert torch.equal(plan, out)                 # the caller's plan changes the order, not a unit's arithmetic
 
 
-@pytest.mark.parametrize("heads,lens,scale", [
-    (2, [512], 1.0),                                  # a unit in 8 shares: two to each of the workgroup's four waves
-    (2, [512], 40.0),                                 # the same with scores beyond the pipelined loop's range
-    (12, [1024, 1088], 1.0),                          # 4
-    (12, [256, 1024, 640, 896], 1.0),                 # 2: two units side by side
-    (12, [2048, 3008, 384], 6.0),                     # 1: four
-    (12, [2944, 3008, 2752], 6.0),                    # 1, global rows in 4 shares: one to a wave
+@pytest.mark.parametrize("cut,heads,lens,scale", [
+    ((4, 4, 4), 2, [512], 1.0),                       # a unit in 4 shares: one to each of the workgroup's four waves
+    ((4, 4, 4), 2, [512], 40.0),                      # the same with scores beyond the pipelined loop's range
+    ((2, 4, 4), 12, [1536, 512], 1.0),                # 2: two units side by side
+    ((2, 4, 4), 10, [1664], 40.0),
+    ((1, 4, 4), 12, [1024, 1088], 1.0),               # 1: four
+    ((1, 4, 4), 12, [256, 1024, 640, 896], 1.0),
+    ((1, 4, 4), 12, [2048, 3008, 384], 6.0),
+    ((1, 8, 8), 6, [5760], 1.0),                      # global rows in 8 shares: two to each wave
+    ((1, 8, 8), 6, [5760], 40.0),
+    ((1, 8, 8), 12, [4096], 6.0),
+    ((1, 4, 4), 12, [2944, 3008, 2752], 6.0),
+    ((2, 4, 4), 1, [64 * 257] + [640] * 8, 40.0),     # a sequence whose global rows have 8 shares all the same
 ])
 @pytest.mark.parametrize("padded", [False, True])
-def test_few_units_walk_the_plan(capi, heads, lens, scale, padded):
+def test_few_units_walk_the_plan(capi, cut, heads, lens, scale, padded):
     """Every workgroup walks the slice that the partition gives it, whatever its neighbours have: one slice with all units,
     more slices than units, and slices whose ends do not meet (the first is empty, the second begins before its end)."""
-    print("plan walk", heads, lens, scale, padded, flush=True)
+    print("plan walk", cut, heads, lens, scale, padded, flush=True)
+    assert cut_of(capi, heads, lens) == cut
     g = torch.Generator(device="cuda").manual_seed(3)
     t = sum(lens)
-    sb, _, _, ph, sb_d, idx_d, pos_d = lh.device_plan(capi, lens, heads, 3)
+    sb, _, _, ph, sb_d, idx_d, pos_d = lh.device_plan(capi, lens, heads, 3, max_pos=max(4096, max(lens)))
     q, k, v = (torch.randn(t, heads, 64, generator=g, device="cuda").half() for _ in range(3))
     operands = lh.pack_heads(q * (scale * lh.LOG2E / 8), sb), lh.pack_heads(k, sb), lh.pack_heads(v, sb, transpose_v=True)
     tokens = torch.tensor([max(1, n - 81 - 3 * i) for i, n in enumerate(lens)], dtype=torch.int32).cuda() if padded else None
@@ -91,20 +107,30 @@ def test_few_units_walk_the_plan(capi, heads, lens, scale, padded):
     assert torch.equal(run(ids, ends), want)
 
 
-@pytest.mark.parametrize("heads,lens", [
-    (2, [512]),                                       # 8 waves to a row: every tile is the first of its wave
-    (12, [1024, 256]),                                # 4 waves to a row, global rows by 8
-    (12, [512, 1024, 1280]),                          # 2
-    (12, [2048, 3008, 384]),                          # 1
-    (12, [2944, 3008, 2752]),                         # 1, global rows by 4
-    (16, [2048] * 6),                                 # 3072 units
+@pytest.mark.parametrize("cut,heads,lens,n_wg", [
+    ((4, 4, 4), 2, [512], 0),                         # two tiles to a wave
+    ((4, 4, 4), 2, [512], 5),
+    ((4, 4, 4), 12, [1024, 256], 0),
+    ((2, 4, 4), 12, [1536, 512], 0),
+    ((2, 4, 4), 12, [1536, 512], 31),
+    ((1, 4, 4), 12, [512, 1024, 1280], 0),
+    ((1, 4, 4), 12, [2048, 3008, 384], 0),
+    ((1, 4, 4), 12, [2944, 3008, 2752], 0),
+    ((1, 4, 4), 12, [2944, 3008, 2752], 300),
+    ((1, 8, 8), 6, [5120, 512], 0),
+    ((1, 8, 8), 6, [5120, 512], 40),                  # two shares to a wave
+    ((1, 8, 8), 2, [5120], 0),
+    ((1, 4, 4), 16, [2048] * 6, 0),                   # 3072 units
+    ((1, 4, 4), 2, [512] + [64] * 60 + [1024] * 5, 0),               # more sequences than lanes
+    ((1, 4, 4), 2, [512] + [64] * 60 + [1024] * 5, 20),
 ])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
-def test_infinite_and_very_low_scores(capi, heads, lens, dtype):
+def test_infinite_and_very_low_scores(capi, cut, heads, lens, n_wg, dtype):
     """Key blocks that a query scores with minus infinity throughout (first, in the middle, last in a wave's share),
     queries with no other keys, infinite and undefined values and, where the type reaches so far, rows whose scores
     all lie below -1e30: weights as a softmax over the whole row gives them."""
-    print("infinities", heads, lens, dtype, flush=True)
+    print("infinities", cut, heads, lens[:4], n_wg, dtype, flush=True)
+    assert cut_of(capi, heads, lens) == cut
     g = torch.Generator().manual_seed(1)
     t = sum(lens)
     q, k, v = (torch.randn(t, heads, 64, generator=g).to(dtype) for _ in range(3))
@@ -118,7 +144,7 @@ def test_infinite_and_very_low_scores(capi, heads, lens, dtype):
         q[:64, 1] = q[:64, 1].abs()
         k[:lens[0], 1] = -2e35 * k[:lens[0], 1].abs().clamp_min(.1)
         k[lens[0]:, 0, 9] = inf                        # the later sequences' head 0: every key, zeros or NaN
-    out, ref = lh.run_attention(capi, q.cuda(), k.cuda(), v.cuda(), lens, heads, seed=3)
+    out, ref = lh.run_attention(capi, q.cuda(), k.cuda(), v.cuda(), lens, heads, seed=3, n_wg=n_wg, max_pos=max(4096, max(lens)))
     out = out.float().cpu()
     assert torch.equal(out.isnan(), ref.isnan()) and torch.equal(out.isinf(), ref.isinf())
     ok = out.isfinite()                                # of the two heads with infinite keys half the queries, about

@@ -19,31 +19,37 @@ def capi():
     return p.capi
 
 
-@pytest.mark.parametrize("heads,blocks,scale,short", [
-    (16, [16], 1.0, 0),                    # 256 units: four waves to every row
-    (1, [3], 1.0, 63),                     # the shortest sequence whose rows are shared by four waves
-    (1, [2], 1.0, 0),                      # by two waves
-    (10, [26], 1.0, 9),                    # 260 units: two waves to a row, four to a global one
-    (10, [26], 40.0, 0),                   # the same beyond the pipelined loop's range
-    (12, [34], 1.0, 0),                    # 216 workgroups so
-    (12, [35], 1.0, 5),                    # 222 would be too many: a wave to a row
-    (6, [90], 1.0, 30),                    # a long sequence: eight waves to a global row
-    (6, [90], 40.0, 30),
-    (6, [100, 12, 90], 1.0, 1),
-    (1, [600], 1.0, 0),                    # 75 tiles to a wave of a global row: the moving-maximum loop
-    (1, [300] + [1] * 64, 1.0, 2),         # two shares of 38 tiles to each of four waves; more sequences than lanes
-    (2, [300] + [10] * 30, 1.0, 0),        # the same with 31 sequences
-    (2, [300] + [10] * 30, 40.0, 9),       # beyond the pipelined loop's range
-    (1, [257] + [10] * 8, 1.0, 4),         # with two waves to the other rows, at the shortest sequence that takes them so
-    (1, [256] + [10] * 8, 1.0, 4),         # 64 tiles to each of four waves
-    (1, [600] + [1] * 64, 1.0, 1),         # 75 tiles to a share: the moving-maximum loop
-    (2, [1 + i % 14 for i in range(65)], 1.0, 3),
-    (1, [12 + i % 3 for i in range(130)], 40.0, 3),        # three chunks, every sequence with global rows
-    (2, [1] * 80 + [13] + [1] * 15 + [2, 12, 1], 1.0, 0),  # sequences that begin and end a sixteen
-    (1, [1] * 1023 + [14], 1.0, 1),        # the most sequences, the last of them with global rows
+@pytest.mark.parametrize("cut,heads,blocks,scale,short", [
+    ((4, 4, 4), 16, [16], 1.0, 0),                   # 256 units, the most whose every row four waves share
+    ((4, 4, 4), 1, [3], 1.0, 63),                    # the shortest sequence whose rows are shared by four waves
+    ((2, 4, 4), 1, [2], 1.0, 0),                     # by two waves
+    ((2, 4, 4), 10, [26], 1.0, 9),                   # 260 units
+    ((2, 4, 4), 10, [26], 40.0, 0),                  # the same beyond the pipelined loop's range
+    ((2, 4, 4), 12, [34], 1.0, 0),                   # 216 workgroups so
+    ((1, 4, 4), 12, [35], 1.0, 5),                   # 222 would be too many: a wave to a row
+    ((4, 4, 4), 1, [75], 1.0, 0),                    # few units, on both sides of the line to workgroups of eight waves
+    ((1, 8, 8), 1, [76], 1.0, 0),
+    ((1, 4, 4), 12, [29] * 3, 1.0, 0),               # and where one round of those takes all
+    ((1, 8, 8), 12, [30] * 3, 1.0, 7),
+    ((1, 8, 8), 4, [250] + [2] * 9, 1.0, 7),         # one long sequence among short ones
+    ((1, 8, 8), 6, [90], 1.0, 30),                   # a long sequence: eight waves to a global row
+    ((1, 8, 8), 6, [90], 40.0, 30),
+    ((1, 8, 8), 6, [100, 12, 90], 1.0, 1),
+    ((1, 8, 8), 1, [600], 1.0, 0),                   # 75 tiles to a wave of a global row: the moving-maximum loop
+    ((1, 4, 4), 1, [300] + [1] * 64, 1.0, 2),        # two shares of 38 tiles to each of four waves; more sequences than lanes
+    ((1, 4, 4), 2, [300] + [10] * 30, 1.0, 0),       # the same with 31 sequences
+    ((1, 4, 4), 2, [300] + [10] * 30, 40.0, 9),      # beyond the pipelined loop's range
+    ((2, 4, 4), 1, [257] + [10] * 8, 1.0, 4),        # with two waves to the other rows, at the shortest sequence that takes them so
+    ((2, 4, 4), 1, [256] + [10] * 8, 1.0, 4),        # 64 tiles to each of four waves
+    ((1, 4, 4), 1, [600] + [1] * 64, 1.0, 1),        # 75 tiles to a share: the moving-maximum loop
+    ((1, 4, 4), 2, [1 + i % 14 for i in range(65)], 1.0, 3),
+    ((1, 4, 4), 1, [12 + i % 3 for i in range(130)], 40.0, 3),       # three chunks, every sequence with global rows
+    ((1, 4, 4), 2, [1] * 80 + [13] + [1] * 15 + [2, 12, 1], 1.0, 0),  # sequences that begin and end a sixteen
+    ((1, 4, 4), 1, [1] * 1023 + [14], 1.0, 1),       # the most sequences, the last of them with global rows
 ])
-def test_rows(capi, heads, blocks, scale, short):
-    print("rows", heads, blocks[:4], scale, short, flush=True)
+def test_rows(capi, cut, heads, blocks, scale, short):
+    print("rows", cut, heads, blocks[:4], scale, short, flush=True)
+    assert capi.bs_attention_cut(len(blocks), sum(blocks), heads) == cut
     lens = [64 * n for n in blocks]
     t, dtype = sum(lens), torch.float16
     gen = torch.Generator().manual_seed(t)
