@@ -1,7 +1,6 @@
-"""rt_bs_attention_fwd_no_alloc (queue counters in a static device array, no device allocation) against
-rt_bs_attention_fwd_masked on the same inputs: the two run the same kernel over the same plan, so the outputs
-must be the same bits.  Two calls in a row share the static counters, the second on a smaller batch; a third
-goes back to the larger one; both also match the CPU oracle.  Sizes beyond the stated limits are refused."""
+"""rt_bs_attention_fwd_no_alloc: the oracle's outputs, the bits of rt_bs_attention_fwd_masked (which is the same launch: what
+differs is the limits that it states), no device memory taken by its launches, calls that overlap on two streams, and sizes
+beyond the stated limits refused."""
 import pytest
 import torch
 
@@ -25,7 +24,7 @@ def _case(capi, dtype, seq_lens, heads, seed, padded):
     g = torch.Generator().manual_seed(seed)
     qkv = torch.randn(t, 3 * dm, generator=g).to(dtype).cuda()
     bias = (torch.randn(3 * dm, generator=g) * 0.5).to(dtype).cuda()
-    sb, idx, pos, ph, sb_d, idx_d, pos_d = lh.device_plan(capi, seq_lens, heads, seed, None)
+    sb, idx, pos, ph, sb_d, idx_d, pos_d = lh.device_plan(capi, seq_lens, heads, seed, None, max_pos=max(4096, max(seq_lens)))
     seq_tokens = [n - 9 for n in seq_lens] if padded else None
     tok_d = None if seq_tokens is None else torch.tensor(seq_tokens, dtype=torch.int32).cuda()
     q, k, vt = (torch.full((t * dm,), float("nan"), dtype=dtype, device="cuda") for _ in range(3))
@@ -38,8 +37,12 @@ def _case(capi, dtype, seq_lens, heads, seed, padded):
                 ref=ref, dtype=dtype)
 
 
-def _run(capi, c, no_alloc):
-    out = torch.full((c["t"], c["dm"]), float("nan"), dtype=c["dtype"], device="cuda")
+def _out(c):
+    return torch.full((c["t"], c["dm"]), float("nan"), dtype=c["dtype"], device="cuda")
+
+
+def _run(capi, c, no_alloc, out=None):
+    out = _out(c) if out is None else out
     if no_alloc:
         capi.bs_attention_fwd_no_alloc(c["q"], c["k"], c["vt"], out, c["sb_d"], c["heads"], c["idx_d"], c["pos_d"],
                                        c["ph"], c["tok_d"])
@@ -49,20 +52,45 @@ def _run(capi, c, no_alloc):
     return out
 
 
+# a batch for every cut of the rows, and more sequences than lanes
+SHAPES = [([64 * 13, 64], 3), ([64 * 26], 10), ([64 * 21, 64 * 3, 64 * 40, 64, 64 * 12], 6), ([64 * 80, 128], 6), ([64 * 12] + [64] * 64, 2)]
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
-def test_no_alloc_entry_point_matches_allocating_one(capi, dtype):
-    print("no_alloc", dtype, flush=True)
-    large = _case(capi, dtype, [64 * 21, 64 * 3, 64 * 40, 64, 64 * 12], 6, 11, padded=False)
-    small = _case(capi, dtype, [64 * 14, 64 * 2], 3, 12, padded=True)
-    want = {id(c): _run(capi, c, no_alloc=False) for c in (large, small)}
+def test_no_alloc_entry_point_against_the_oracle(capi, dtype):
+    """Launches take no device memory (behind the first of each kernel, for which the runtime takes some of its own)."""
+    cases = [_case(capi, dtype, lens, heads, 11 + i, padded) for i, (lens, heads) in enumerate(SHAPES) for padded in (False, True)]
+    outs = [_out(c) for c in cases]
+    for c, out in zip(cases, outs):
+        print("no_alloc", dtype, c["t"], c["heads"], c["tok_d"] is not None, flush=True)
+        _run(capi, c, True, out)
     torch.cuda.synchronize()
-    # back to back on one stream, nothing in between: the second call finds the first call's counters
-    got = [(c, _run(capi, c, no_alloc=True)) for c in (large, small, large)]
+    free, _ = torch.cuda.mem_get_info()
+    for _ in range(20):
+        for c, out in zip(cases, outs):
+            _run(capi, c, True, out)
     torch.cuda.synchronize()
-    for c, out in got:
-        assert torch.isfinite(out).all()
-        assert torch.equal(out, want[id(c)])
+    assert torch.cuda.mem_get_info()[0] == free
+    for c, out in zip(cases, outs):
+        assert torch.equal(_run(capi, c, False), out)
         assert (out.float().cpu() - c["ref"]).abs().max().item() <= 2e-2
+
+
+def test_no_alloc_calls_overlap_on_two_streams(capi):
+    """Nothing is shared between launches: two streams, a hundred calls each, every output with the bits of a call by itself."""
+    print("no_alloc two streams", flush=True)
+    cases = [_case(capi, torch.float16, lens, heads, 5, False) for lens, heads in (SHAPES[2], SHAPES[0])]
+    want = [_run(capi, c, True) for c in cases]
+    outs = [[_out(c) for _ in range(100)] for c in cases]
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream() for _ in cases]
+    for i in range(100):
+        for c, st, out in zip(cases, streams, outs):
+            with torch.cuda.stream(st):
+                _run(capi, c, True, out[i])
+    torch.cuda.synchronize()
+    for w, out in zip(want, outs):
+        assert all(torch.equal(o, w) for o in out)
 
 
 def test_no_alloc_entry_point_refuses_sizes_beyond_its_limits(capi):
