@@ -277,7 +277,7 @@ template <> struct Quad<__hip_bfloat16> {
 };
 
 // Bound by latency: the launch, one round trip for everything the row needs, the sums.  So the scales and every slice are
-// requested together with the row (P slices; 0: any number, four to a round trip).  512 x 768 (us in a graph; before: the
+// requested together with the row (P slices; 0: more than four, the others four to a round trip).  512 x 768 (us in a graph; before: the
 // scales requested behind the sums, those through LDS): one slice 2.54 -> 2.22, two 2.74 -> 2.36, four 2.74 -> 2.47.
 template <typename T, int CH, int P>
 __global__ __launch_bounds__(256) void slices_residual_layernorm_kernel(T* __restrict__ out, const float* __restrict__ parts,
@@ -294,11 +294,12 @@ __global__ __launch_bounds__(256) void slices_residual_layernorm_kernel(T* __res
   const float* src = parts + row * HIDDEN + lane * 4;
   float x[CH][4];
   uint2 res[CH], bi[CH], ga[CH], be[CH];
-  float4 v[P ? P : 1][CH];
+  constexpr int FIRST = P ? P : 4;
+  float4 v[FIRST][CH];
 #pragma unroll
   for (int c = 0; c < CH; ++c) {
 #pragma unroll
-    for (int u = 0; u < P; ++u) v[u][c] = *reinterpret_cast<const float4*>(src + u * slice + c * 256);
+    for (int u = 0; u < FIRST; ++u) v[u][c] = *reinterpret_cast<const float4*>(src + u * slice + c * 256);
     res[c] = *reinterpret_cast<const uint2*>(residual + row * HIDDEN + c * 256 + lane * 4);
     bi[c] = *reinterpret_cast<const uint2*>(bias + c * 256 + lane * 4);
     ga[c] = *reinterpret_cast<const uint2*>(gamma + c * 256 + lane * 4);
@@ -331,7 +332,8 @@ __global__ __launch_bounds__(256) void slices_residual_layernorm_kernel(T* __res
 #pragma unroll
       for (int c = 0; c < CH; ++c) add1(c, v[u][c]);
   } else {
-    int s = 0;
+    add4(v);
+    int s = 4;
     for (; s + 4 <= n_parts; s += 4) {
       float4 w[4][CH];
 #pragma unroll
@@ -356,6 +358,8 @@ __global__ __launch_bounds__(256) void slices_residual_layernorm_kernel(T* __res
   const float rstd = rsqrtf(group_sum<64>(sq) * (1.0f / HIDDEN) + eps);
 #pragma unroll
   for (int c = 0; c < CH; ++c) {
+    // behind a loop: converted here, where a product, its addition and the rounding to fp16 are one instruction (and one rounding)
+    if (P == 0) asm volatile("" : "+v"(ga[c].x), "+v"(ga[c].y), "+v"(be[c].x), "+v"(be[c].y));
     float g[4], b[4], y[4];
     Quad<T>::load(reinterpret_cast<const T*>(&ga[c]), g);
     Quad<T>::load(reinterpret_cast<const T*>(&be[c]), b);

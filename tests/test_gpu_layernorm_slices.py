@@ -32,3 +32,23 @@ def test_slices_residual_layernorm(parts, rows, hidden, dtype):
     ulp = torch.exp2(torch.floor(torch.log2(want.abs().clamp_min(2.0 ** -14))) - BITS[dtype])
     bound = 0.51 * ulp + 2.0 ** -20 * (1 + y.abs() * gamma.double().abs() + beta.double().abs())
     assert ((out.double() - want).abs() - bound).max().item() <= 0
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("hidden", [256, 512, 768, 1024])
+def test_slices_of_zeros_change_no_bit(hidden, dtype):
+    """Four slices, and the same with one or four of zeros behind them: the kernels differ, the sums and the one rounding do not."""
+    capi = graft.load_package().capi
+    g = torch.Generator(device="cuda").manual_seed(hidden)
+    r = lambda *shape: torch.randn(*shape, generator=g, device="cuda")
+    rows = 2000
+    slices = torch.cat([r(4, rows, hidden), torch.zeros(4, rows, hidden, device="cuda")])
+    residual, bias, gamma, beta = r(rows, hidden).to(dtype), r(hidden).to(dtype), r(hidden).to(dtype), r(hidden).to(dtype)
+    ptr = lambda t: ctypes.c_void_p(t.data_ptr())
+    outs = []
+    for parts in (4, 5, 8):
+        out = torch.empty(rows, hidden, dtype=dtype, device="cuda")
+        capi.check(capi.lib().rt_slices_residual_layernorm(ptr(out), ptr(slices), parts, ptr(residual), ptr(bias), ptr(gamma), ptr(beta),
+                                                           rows, hidden, 1e-5, capi._dtype_code(out), capi._stream()))
+        outs.append(out)
+    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
