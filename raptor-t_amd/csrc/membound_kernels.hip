@@ -567,9 +567,12 @@ __device__ inline float gelu_tanh(float x) {
 // takes vectors t, t + 256, ... of the run, all U requests issued before any is used.  No grid-stride
 // loop: with a capped grid the U requests of a thread lay a power of two apart (16 MiB), which on
 // this memory system falls into the same channel every time and costs a fifth of the bandwidth.
-// Bound by memory; stored through (us, plain / written through / non-temporal, buffers in rotation): fp16 8192 x 3072 18.3 / 16.4 /
-// 18.0, bf16 32768 x 3072 73.6 / 68.4 / 70.5, 60000 x 4096 172.8 / 167.9 / 172.0.
-template <typename T>
+// Bound by memory and stored through (us, plain / written through / non-temporal, buffers in rotation): fp16 8192 x 3072 18.3 / 16.4 /
+// 18.0, bf16 32768 x 3072 73.6 / 68.4 / 70.5, 60000 x 4096 172.8 / 167.9; 9000 x 264 4.05 / 4.02, 1024 x 3072 4.40 / 4.18.  Up to 4.4 MB the
+// launch is its latency, which a store's way to memory adds to: 64 x 3072 2.77 / 2.91, 512 x 3072 3.15 / 3.21, fp32 512 x 264 2.37 / 2.63,
+// 2048 x 1024 3.43 / 3.54.
+constexpr int64_t GELU_THROUGH_VECTORS = 275000;
+template <typename T, bool THROUGH>
 __global__ __launch_bounds__(256) void bias_gelu_kernel(T* __restrict__ out, const T* __restrict__ bias,
                                                         int64_t n_vec, int width_vec) {
   constexpr int N = Vec<T>::N;
@@ -578,18 +581,27 @@ __global__ __launch_bounds__(256) void bias_gelu_kernel(T* __restrict__ out, con
   const uint32_t col0 = uint32_t(v0 % width_vec);
   if (v0 + (U - 1) * 256 < n_vec) {
     const __amdgpu_buffer_rsrc_t dst = run_of(out + int64_t(blockIdx.x) * (U * 256) * N, U * 256 * N);
+    auto bias_of = [&](int u) { return bias + ((col0 + u * 256) % uint32_t(width_vec)) * N; };
     float a[U][N];
+    uint4 bi[U];
 #pragma unroll
-    for (int u = 0; u < U; ++u) Vec<T>::load(out + (v0 + u * 256) * N, a[u]);
+    for (int u = 0; u < U; ++u) {
+      Vec<T>::load(out + (v0 + u * 256) * N, a[u]);
+      if (THROUGH) bi[u] = *reinterpret_cast<const uint4*>(bias_of(u));         // ahead of the first store: no load passes a buffer store
+    }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       float b[N];
-      Vec<T>::load(bias + ((col0 + u * 256) % uint32_t(width_vec)) * N, b);
+      Vec<T>::load(THROUGH ? reinterpret_cast<const T*>(&bi[u]) : bias_of(u), b);
 #pragma unroll
       for (int i = 0; i < N; ++i) a[u][i] = gelu_tanh(a[u][i] + b[i]);
-      u32x4 packed;
-      Vec<T>::store(reinterpret_cast<T*>(&packed), a[u]);
-      store_through(packed, dst, uint32_t(threadIdx.x + u * 256) * 16u);
+      if (THROUGH) {
+        u32x4 packed;
+        Vec<T>::store(reinterpret_cast<T*>(&packed), a[u]);
+        store_through(packed, dst, uint32_t(threadIdx.x + u * 256) * 16u);
+      } else {
+        Vec<T>::store(out + (v0 + u * 256) * N, a[u]);
+      }
     }
     return;
   }
@@ -862,12 +874,17 @@ int rt_bias_gelu(void* out, const void* bias, int64_t rows, int width, int dtype
   RT_REQUIRE(want < (int64_t(1) << 31), RT_EINVAL, "rows=%lld x width=%d is too large for one launch", (long long)rows, width);
   const unsigned grid = unsigned(want);
   hipStream_t st = static_cast<hipStream_t>(stream);
-  if (dtype == RT_F16)
-    RT_LAUNCH(bias_gelu_kernel<__half>, dim3(grid), dim3(256), 0, st, (__half*)out, (const __half*)bias, n_vec, width / n);
-  else if (dtype == RT_BF16)
-    RT_LAUNCH(bias_gelu_kernel<__hip_bfloat16>, dim3(grid), dim3(256), 0, st, (__hip_bfloat16*)out, (const __hip_bfloat16*)bias, n_vec, width / n);
-  else
-    RT_LAUNCH(bias_gelu_kernel<float>, dim3(grid), dim3(256), 0, st, (float*)out, (const float*)bias, n_vec, width / n);
+  auto go = [&](auto* o, auto through) {
+    typedef std::remove_pointer_t<decltype(o)> T;
+    RT_LAUNCH((bias_gelu_kernel<T, decltype(through)::value>), dim3(grid), dim3(256), 0, st, o, static_cast<const T*>(bias), n_vec, width / n);
+  };
+  auto typed = [&](auto through) {
+    if (dtype == RT_F16) go(static_cast<__half*>(out), through);
+    else if (dtype == RT_BF16) go(static_cast<__hip_bfloat16*>(out), through);
+    else go(static_cast<float*>(out), through);
+  };
+  if (n_vec > GELU_THROUGH_VECTORS) typed(std::true_type());
+  else typed(std::false_type());
   return check_launch("bias_gelu");
 }
 

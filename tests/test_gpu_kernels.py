@@ -61,12 +61,30 @@ def test_bias_gelu(capi, dtype, rows, width):
     assert lh.excess(xd, want, dtype, k=1.0) <= 0
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("rows,width", [(8333, 264), (8334, 264), (537, 4096), (538, 4096)])
+def test_bias_gelu_where_rows_begin_to_be_written_through(capi, dtype, rows, width):
+    """Both sides of the line between the two kernels (275 000 vectors of 16 bytes; fp32 has twice as many to a row), the last
+    workgroup partly empty: against the oracle, and the same bits as in launches of a third of the rows."""
+    say("GELU, both kernels", dtype, rows, width)
+    if dtype == torch.float32:
+        rows = (rows + 1) // 2
+    g = torch.Generator().manual_seed(rows)
+    x, b = (torch.randn(rows, width, generator=g) * 2).to(dtype), torch.randn(width, generator=g).to(dtype)
+    whole, bd = x.cuda(), b.cuda()
+    capi.bias_gelu(whole, bd)
+    assert lh.excess(whole, ol.bias_gelu(x, b), dtype, k=1.0) <= 0
+    thirds = [t.contiguous() for t in x.cuda().chunk(3)]
+    for t in thirds:
+        capi.bias_gelu(t, bd)
+    assert torch.equal(torch.cat(thirds), whole)
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("rows", [32768, 65536])
 def test_memory_bound_kernels_at_benchmark_row_counts(capi, dtype, rows):
     """The row counts of the memory-bound benchmark (32 K and 64 K tokens; the reference sweeps them in
-    python/benchmark/mem_bound_op.py:93-108): bias + GELU over [rows, 3072], whose launch is capped so that every
-    workgroup walks its grid-stride loop several times, and bias + residual + LayerNorm over [rows, 768]."""
+    python/benchmark/mem_bound_op.py:93-108): bias + GELU over [rows, 3072] and bias + residual + LayerNorm over [rows, 768]."""
     say("membound at benchmark size", dtype, rows)
     g = torch.Generator().manual_seed(rows)
     x = (torch.randn(rows, 3072, generator=g) * 2).to(dtype)
