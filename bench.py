@@ -805,7 +805,7 @@ def main():
     ap.add_argument("--steps", type=int, default=20)
     ap.add_argument("--warmup", type=int, default=3)
     ap.add_argument("--workload", default="c3", choices=["c3", "c1", "c2", "c4", "c5", "ref_e2e", "stream", "overlap", "mfma_mix"])
-    ap.add_argument("--block-limit", type=int, default=1024, help="persistent workgroups of the balanced attention launch")
+    ap.add_argument("--block-limit", type=int, default=1024, help="workgroups of the balanced attention launch")
     ap.add_argument("--lpt-plan", action="store_true",
                     help="drive attention with the caller's LPT plan (the reference's balanced mode) instead of the kernel's own schedule")
     ap.add_argument("--sync-index", action="store_true", help="build the block index inline instead of on the workers")

@@ -73,7 +73,7 @@ int rt_abi_version(void);
  * launch (layers/kernels/add_bias_act.cu:109-131, the `info` map of every launcher); a pair of events recorded
  * around a launch also counts the gaps to the neighbouring kernels.  After this call the next kernel that one
  * of this library's kernel entry points (every one below, but not a product that goes to hipBLASLt; each launches one
- * kernel) launches from the calling
+ * kernel, rt_unpack_rows one for every 128 sequences, of which the pair gets the first) launches from the calling
  * thread writes the start and end timestamps of its dispatch into the two hipEvent_t (created by the caller,
  * either may be NULL); hipEventElapsedTime between them is the kernel's duration as a profiler reports it.
  * One launch consumes the pair; (NULL, NULL) withdraws a pair no launch has taken.  Returns 1 if the call

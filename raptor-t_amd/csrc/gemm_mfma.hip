@@ -319,8 +319,8 @@ __device__ __forceinline__ void main_loop(f32x4 (&acc)[MT][4], const f32x4 (&c0)
   v8 a[MT], b[2][4];
   // What may still be on its way at a step's barrier: the loads of A(s+2), which every wave has issued behind those of
   // s+1, or in a tile's first step, behind its loads of B(s+1), the stores of the last tile's outputs.  store_rows issues
-  // 2 * MT of them whatever it stores (past the ends of C the range check drops them); store_v and store_k issue none for
-  // rows and columns past the end, so behind them nothing may be left: B(s+1) could be what is.
+  // 2 * MT of them whatever it stores (past the ends of C the range check drops them), and so do store_v and store_k; but behind
+  // a V tile a wave whose columns lie past the end issues none, so with the head split nothing may be left: B(s+1) could be what is.
   constexpr int LEFT = TM / 64, STORES = EPI == EPI_QKV ? 0 : 2 * MT;
   enum { FIRST, INNER, LAST };
   // row i of a half: its four products, the columns in alternating direction (a row's last weights fragment is the
@@ -881,7 +881,7 @@ template <typename T, int MT, int NT, int WM, int WN, int STAGES, int EPI> int l
 // that share a CU, the launch, and what each round of workgroups spends on its first loads and its epilogue; plus the GELU
 // by the outputs of a round, and the slices' way to memory and back.  The figures are a least-squares fit to 940 launches
 // (15 row counts from 64 to 37184 at hidden 768, five from 128 to 40768 at 1024, all four products of a layer, up to six
-// slices; root mean square of the error 7 %), over which the kernel that the model picks is 0.6 % slower than the fastest on
+// slices; root mean square of the error 7 %; all with plain stores, where those below 192 x 256 are written through now), over which the kernel that the model picks is 0.6 % slower than the fastest on
 // average; with the LayerNorm behind it (20 row counts, up to eight slices) 1.3 %.  Where the lines fall, both sides (us):
 //   512 x 3072 x 768 + GELU   128 x 64: 6.9, 64 x 64: 7.2, 128 x 128: 8.5    1024 x 2304 x 768 split   128 x 128: 8.3, 128 x 64: 9.1
 //   2816 x 2304 x 768 split   128 x 256: 14.6, 128 x 128: 16.1, 192 x 256: 18.2    4096 x 2304 x 768 split   192 x 256: 21.2, 128 x 256: 23.9

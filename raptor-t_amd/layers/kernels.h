@@ -103,9 +103,9 @@ bool attention_q_from_rows();
 double tune_layer_gemms(const std::vector<int64_t>& token_counts, int64_t hidden, int64_t ffn, torch::ScalarType dtype);
 
 // What `balanced = true` means for the attention launch.  The reference's balanced kernel walks the
-// host's LPT partition (python/util.py:11-34); here the persistent kernel balances itself with an
-// XCD-aware schedule of its own that keeps each (sequence, head) group in one L2 and measures 20 %
-// faster than walking that partition, so by default (false) a balanced launch uses it and the
+// host's LPT partition (python/util.py:11-34); here the kernel has an XCD-aware schedule of its own that
+// keeps each (sequence, head) group in one L2 and measures 20 to 30 % faster than walking that
+// partition, so by default (false) a balanced launch uses it and the
 // partition tensors are only checked for shape.  true: walk the host's partition as the reference does.
 void set_attention_host_plan(bool on);
 bool attention_host_plan();
