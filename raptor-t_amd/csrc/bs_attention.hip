@@ -1267,10 +1267,11 @@ Cut cut_rows(int batch, int total_blocks, int heads) {
   if (longest >= 3 && units <= 256) return {4, 4, 4};
   if (longest >= 2 && global + (units - global) / 2 <= 220) return {2, 4, 4};
   if (likely >= 60 && one_round) return eight;
-  // From about 1050 units on a round of workgroups of 8 waves takes as long as the same work by 4, whatever the lengths, and a
-  // sequence much longer than the others is done earlier (f16, 1 4 4 / 1 8 8: 12 heads 3 x 1920 tokens 16.6 / 17.0, 4 heads 10 x 1728 14.9 / 15.4, 6
-  // heads 7 x 1920 16.0 / 16.1; 4 heads 16000 + 9 x 128 50.1 / 42.4, 9600 + 11 x 896 33.6 / 27.5).  32 CUs to an XCD, as launch_rows deals them.
-  if (units >= 1056 && 2 * ((pairs + 7) / 8) + ((units + 7) / 8 + 7) / 8 <= 32) return eight;
+  // From about 1050 units on a round of workgroups of 8 waves takes as long as the same work by 4 if the sequences are not short, and a
+  // sequence much longer than the others is done earlier (f16, 1 4 4 / 1 8 8: 12 heads 3 x 1920 tokens 16.8 / 17.2, 3 x 2432 19.4 / 19.2, 640 + 2560 +
+  // 2880 18.6 / 19.2, 3200 + 1920 + 1600 20.2 / 17.9, 4096 + 2 x 896 21.9 / 18.2, 4 heads 10 x 1728 14.9 / 15.4, 16000 + 9 x 128 50.1 / 42.4, 9600 + 11 x
+  // 896 33.6 / 27.5; below the line 16 heads 3 x 1408 15.7 / 16.8, 640 + 2 x 1920 17.9 / 19.1).  32 CUs to an XCD, as launch_rows deals them.
+  if (likely >= 38 && units >= 1056 && 2 * ((pairs + 7) / 8) + ((units + 7) / 8 + 7) / 8 <= 32) return eight;
   // more rounds, and a chain, 5 us and 0.25 a tile, that outlasts the units' 17 ns each (f16, 1 4 4 / 1 8 8: 12 heads 12800 + 1280 tokens 50.0 /
   // 41.0, 8 heads 2 x 11520 48.8 / 39.4, 4 heads 5 x 8192 38.7 / 35.3, 12 heads 2 x 7040 36.4 / 36.6; on the line 12 heads 2 x 8960 46.3 / 49.0; 4 heads
   // 5 x 5760 29.3 / 32.0, whose second round is nearly empty)

@@ -294,9 +294,10 @@ def test_padded_batch_adapters_round_trip():
     # one long sequence, or one much longer than the others: its global rows' chain is the time of the launch
     (4, [300, 300], (1, 8, 8)), (4, [300] + [2] * 9, (1, 8, 8)), (1, [300], (1, 8, 8)), (3, [300] * 3, (1, 8, 8)), (9, [300, 4], (1, 8, 8)),
     (6, [300, 100], (1, 8, 8)), (12, [200, 20], (1, 8, 8)), (8, [256, 40, 40], (1, 8, 8)), (2, [155, 1], (1, 8, 8)),
-    (1, [220], (1, 8, 8)), (4, [250] + [2] * 9, (1, 8, 8)), (4, [128] * 5, (1, 8, 8)), (1, [128] * 16, (1, 8, 8)),
+    (1, [220], (1, 8, 8)), (4, [250] + [2] * 9, (1, 8, 8)), (4, [150] + [14] * 11, (1, 8, 8)), (12, [64, 14, 14], (1, 8, 8)), (4, [128] * 5, (1, 8, 8)), (1, [128] * 16, (1, 8, 8)),
     # the others as they were
     (12, [1], (1, 4, 4)), (12, [3], (4, 4, 4)), (12, [8], (4, 4, 4)), (12, [24], (2, 4, 4)), (12, [40], (1, 4, 4)), (12, [64], (1, 8, 8)),
+    (16, [22] * 3, (1, 4, 4)), (12, [24] * 4, (1, 4, 4)), (16, [10, 30, 30], (1, 4, 4)),
     (12, [4, 16, 10, 14], (1, 4, 4)), (12, [64] * 8, (1, 4, 4)), (16, [200], (1, 8, 8)), (16, [256] * 4, (1, 4, 4)), (12, [8] * 16, (1, 4, 4)),
     (1, [300] + [1] * 64, (1, 4, 4)), (1, [13] * 65, (1, 4, 4)),
 ])
